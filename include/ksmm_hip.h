@@ -18,7 +18,7 @@
  * result is rounded to the output type.
  *
  * Alignment: x, w and y that start on 16-byte boundaries run on the vector kernels; tensors
- * that do not are still computed, by the one-thread-per-output kernel (a forced family
+ * that do not are still computed, by kernels that need element alignment only (a forced family
  * refuses them with KSMM_ERR_BAD_ALGO).  A bias vector needs the alignment of its element
  * type only.  Workspaces must be 16-byte aligned.
  *
@@ -128,7 +128,8 @@ int ksmm_query_tile(int64_t batch, int a, int b, int c, int d, int x_dtype, int 
 int ksmm_query_tile_variant(int64_t batch, int a, int b, int c, int d, int x_dtype, int w_dtype,
                             int y_dtype, int bs_last, int algo, int variant, ksmm_tile *out);
 
-/* The measured table KSMM_ALGO_AUTO consults for batches of 8192 and more: the counterpart
+/* The measured table KSMM_ALGO_AUTO consults for batches of 8192 and more (below, every instance is
+ * priced by a fitted model of its time, and the cheapest is taken): the counterpart
  * of the reference's tuned `*.best` files and the if-chains generated from them
  * (src/ksmm_py/layer/kronecker_sparse/kernel.py:151-257).  Row i is
  * {a, b, c, d, combo, bs_last, algo, instance id, parameter, variant}, combo 0 = fp32,
@@ -156,10 +157,12 @@ int ksmm_factor_forward(const void *x, const void *w, void *y, int64_t batch, in
 
 /* Same, with the kernel family (and optionally a variant, -1 = the family's own choice) forced;
  * used by the tuner and by tests that must exercise one family.  Variants: KSMM_ALGO_GENERIC
- * 0 = one thread per output, 1 = 16-byte vector form (batch-size-last); KSMM_ALGO_WAVE
+ * 0 = one thread per output, 1 = 16-byte vector form (batch-size-last), 16 + v = the KSMM_ALGO_TILE
+ * instance v (how the automatic choice reports an instance it takes for a problem that has no kernel
+ * of its own at full batches: a ragged batch, strided batch-size-first blocks); KSMM_ALGO_WAVE
  * instance | tiles-per-wave << 8 | round-robin << 16, 1000 + i = batch-size-first row kernel i;
  * KSMM_ALGO_TILE sub-family << 24 | instance (0 k-loop, 1 weight-stationary, 2 stream,
- * 3 batch-size-first d > 1, 4 direct-to-LDS GEMM); KSMM_ALGO_AUTO -1 = measured table, then
+ * 3 batch-size-first d > 1, 4 direct-to-LDS GEMM, 5 split-K: instance | waves << 8); KSMM_ALGO_AUTO -1 = measured table, then
  * heuristics, -3 = heuristics only.  An instance that cannot run the problem returns
  * KSMM_ERR_BAD_ALGO. */
 int ksmm_factor_forward_algo(const void *x, const void *w, void *y, int64_t batch, int a,
@@ -169,7 +172,8 @@ int ksmm_factor_forward_algo(const void *x, const void *w, void *y, int64_t batc
 /* Batch-size-first factors with d > 1 whose shape has no kernel of its own in that layout run
  * in batch-size-last layout between two transposes when the caller lends a workspace.
  * ksmm_factor_workspace returns the bytes ksmm_factor_forward_ws can use for a problem (0: a
- * direct kernel exists, the workspace is ignored).  With a smaller workspace (or NULL) it
+ * direct kernel exists, the workspace is ignored; a batch too small to pay for the copies runs on the
+ * tensors as they are, whatever the workspace).  With a smaller workspace (or NULL) it
  * returns KSMM_ERR_WORKSPACE; ksmm_factor_forward (no workspace) falls back to the generic
  * kernel for such shapes.  The reference has no counterpart: its batch-size-first kernels
  * gather with strided scalar loads (template_kernels_float.cuh:156-161).

@@ -3,7 +3,7 @@
 
 #include <atomic>
 
-#include "ksmm_common.h"
+#include "ksmm_choose.h"
 
 using namespace ksmm;
 
@@ -121,6 +121,7 @@ bool describe_variant(int algo, int variant, int combo, int bs_last, uint32_t *i
         case 2: *id = stream_inst_id(inst); break;
         case 3: *id = bf_inst_id(inst); break;
         case 4: *id = gemm_inst_id(inst); break;
+        case 5: *id = split_inst_id(inst); break;
         default: *id = 0;
         }
         return *id != 0;
@@ -159,6 +160,7 @@ bool resolve_variant(int algo, uint32_t id, int param, int combo, int bs_last, i
         else if ((i = find_id(stream_inst_count(), id, stream_inst_id)) >= 0) sub = 2;
         else if ((i = find_id(bf_inst_count(), id, bf_inst_id)) >= 0) sub = 3;
         else if ((i = find_id(gemm_inst_count(), id, gemm_inst_id)) >= 0) sub = 4;
+        else if ((i = find_id(split_inst_count(), id, split_inst_id)) >= 0) sub = 5;
         else return false;
         *variant = (sub << 24) | ((param & 0xffff) << 8) | i;
         return true;
@@ -192,42 +194,110 @@ const TunedRow *tuned_lookup(const Problem &p)
     return nullptr;
 }
 
-// Family order for KSMM_ALGO_AUTO: the table inside each family decides whether it takes the
-// problem; the generic family always does.
-int dispatch(const Problem &p, int algo, int variant, bool launch, ksmm_tile *tile)
+// A family's kernel, or its own choice (variant < 0).
+int family_run(const Problem &p, int algo, int variant, bool launch, ksmm_tile *tile)
 {
     switch (algo) {
     case KSMM_ALGO_GENERIC: return generic_run(p, variant, launch, tile);
     case KSMM_ALGO_WAVE: return wave_run(p, variant, launch, tile);
     case KSMM_ALGO_TILE: return tile_run(p, variant, launch, tile);
-    case KSMM_ALGO_AUTO: {
-        // variant -1: the tuned table first (large batches), then the heuristics below;
-        // variant -3: heuristics only (what the tuner compares against)
-        if (variant == -1 && p.batch >= TUNED_MIN_BATCH) {
-            const TunedRow *row = tuned_lookup(p);
-            int row_variant;
-            if (row && row->algo != KSMM_ALGO_AUTO &&
-                resolve_variant(row->algo, row->id, row->param, row->combo, row->bs_last, &row_variant)) {
-                const int rc = dispatch(p, row->algo, row_variant, launch, tile);
-                if (rc != KSMM_ERR_BAD_ALGO) return rc;
-            }
-        }
-        // Table order from sweeps at batch 25088: batch-size-first 16-bit mid-sized blocks
-        // (64x64 .. 192x192) go to the stream kernels of the tile family; batch-size-last blocks
-        // the wave family has an instance for (up to 96x96), and fp32, go to the wave family,
-        // larger 16-bit blocks to the stream kernels again (inside the tile family), the rest to
-        // the GEMM and k-loop tiles; shapes none of them takes run on the generic kernel.
-        int rc = KSMM_ERR_BAD_ALGO;
-        if (p.x_dtype == KSMM_F16 && !p.bs_last) rc = stream_run(p, -1, launch, tile);
-        if (rc != KSMM_ERR_BAD_ALGO) return rc;
-        rc = wave_run(p, -1, launch, tile);
-        if (rc != KSMM_ERR_BAD_ALGO) return rc;
-        rc = tile_run(p, -1, launch, tile);
-        if (rc != KSMM_ERR_BAD_ALGO) return rc;
-        return generic_run(p, -1, launch, tile);
-    }
     default: return KSMM_ERR_BAD_ALGO;
     }
+}
+
+// The choice measured at full batches: the tuned table (unless `table` is off, which is what the
+// tuner compares against), then the heuristics: the table inside each family decides whether it
+// takes the problem; the generic family always does.
+int table_run(const Problem &p, bool table, bool launch, ksmm_tile *tile)
+{
+    if (table && p.batch >= TUNED_MIN_BATCH) {
+        const TunedRow *row = tuned_lookup(p);
+        int row_variant;
+        if (row && row->algo != KSMM_ALGO_AUTO &&
+            resolve_variant(row->algo, row->id, row->param, row->combo, row->bs_last, &row_variant)) {
+            const int rc = family_run(p, row->algo, row_variant, launch, tile);
+            if (rc != KSMM_ERR_BAD_ALGO) return rc;
+        }
+    }
+    // Family order from sweeps at batch 25088: batch-size-first 16-bit mid-sized blocks
+    // (64x64 .. 192x192) go to the stream kernels of the tile family; batch-size-last blocks
+    // the wave family has an instance for (up to 96x96), and fp32, go to the wave family,
+    // larger 16-bit blocks to the stream kernels again (inside the tile family), the rest to
+    // the GEMM and k-loop tiles; shapes none of them takes run on the generic kernel.
+    int rc = KSMM_ERR_BAD_ALGO;
+    if (p.x_dtype == KSMM_F16 && !p.bs_last) rc = stream_run(p, -1, launch, tile);
+    if (rc != KSMM_ERR_BAD_ALGO) return rc;
+    rc = wave_run(p, -1, launch, tile);
+    if (rc != KSMM_ERR_BAD_ALGO) return rc;
+    rc = tile_run(p, -1, launch, tile);
+    if (rc != KSMM_ERR_BAD_ALGO) return rc;
+    return generic_run(p, -1, launch, tile);
+}
+
+// What takes a problem as it is.  `direct`: the full-batch choice is a kernel of its own, not the
+// one-thread-per-output one.
+struct Pick {
+    Choice c;     // AUTO: the full-batch choice
+    bool direct;
+    float us;     // predicted time, < 0: no model of it
+};
+
+// Below TUNED_MIN_BATCH, and where the full-batch choice is the one-thread-per-output kernel, the
+// cheapest instance by the model of ksmm_choose.hip; else the full-batch choice.  A function of the
+// sizes and types alone: each thread remembers its last answers (pricing every instance takes tens
+// of microseconds, a launch five).
+Pick pick_of(const Problem &p, bool table)
+{
+    struct Entry {
+        int64_t batch;
+        int key[8];
+        Pick pick;
+    };
+    constexpr unsigned SLOTS = 256;
+    static thread_local Entry memo[SLOTS];  // batch 0: empty
+    const int key[8] = {p.a, p.b, p.c, p.d, p.x_dtype, p.w_dtype, p.y_dtype, p.bs_last * 2 + (table ? 1 : 0)};
+    uint64_t h = (uint64_t)p.batch;
+    for (int v : key) h = (h ^ (uint64_t)v) * 0x9E3779B97F4A7C15ull;
+    Entry &e = memo[(h >> 40) % SLOTS];
+    if (e.batch == p.batch && memcmp(e.key, key, sizeof(key)) == 0) return e.pick;
+    ksmm_tile t;
+    memset(&t, 0, sizeof(t));
+    Pick k{{KSMM_ALGO_AUTO, -1, -1.f}, true, -1.f};
+    if (table_run(p, table, false, &t) == KSMM_OK) {
+        k.direct = t.algo != KSMM_ALGO_GENERIC || t.variant == 1;
+        k.us = predicted_us(p, t);
+        if (p.batch < TUNED_MIN_BATCH || !k.direct) {
+            const Choice c = cheapest_instance(p, false);
+            if (c.algo != KSMM_ALGO_AUTO && (k.us < 0.f || c.us < k.us)) {
+                k.c = c;
+                k.us = c.us;
+            }
+        }
+    }
+    e.batch = p.batch;
+    memcpy(e.key, key, sizeof(key));
+    e.pick = k;
+    return k;
+}
+
+int dispatch(const Problem &p, int algo, int variant, bool launch, ksmm_tile *tile)
+{
+    if (algo != KSMM_ALGO_AUTO) return family_run(p, algo, variant, launch, tile);
+    const bool table = variant == -1;
+    const Pick k = pick_of(p, table);
+    if (k.c.algo != KSMM_ALGO_AUTO) {
+        const int rc = family_run(p, k.c.algo, k.c.variant, launch, tile);
+        if (rc != KSMM_ERR_BAD_ALGO) {
+            // a problem without a kernel of its own at full batches is reported as the generic
+            // family's, which takes the same instance by that number
+            if (tile && !k.direct && tile->algo == KSMM_ALGO_TILE) {
+                tile->algo = KSMM_ALGO_GENERIC;
+                tile->variant += GENERIC_TILE;
+            }
+            return rc;
+        }
+    }
+    return table_run(p, table, launch, tile);
 }
 
 // Rows of a batch-size-last workspace copy are padded to a multiple of 16 columns (the 16-byte
@@ -242,7 +312,7 @@ bool wants_transposed(const Problem &p)
     if (p.bs_last) return false;
     ksmm_tile t;
     memset(&t, 0, sizeof(t));
-    if (dispatch(p, KSMM_ALGO_AUTO, -1, false, &t) != KSMM_OK || t.algo != KSMM_ALGO_GENERIC) return false;
+    if (table_run(p, true, false, &t) != KSMM_OK || t.algo != KSMM_ALGO_GENERIC) return false;
     Problem q = p;
     q.bs_last = 1;
     q.batch = padded_batch(p.batch);
@@ -250,7 +320,7 @@ bool wants_transposed(const Problem &p)
     if (check_shape(q.batch, p.a, p.b, p.c, p.d, p.x_dtype, p.w_dtype, p.y_dtype) != KSMM_OK) return false;
     memset(&t, 0, sizeof(t));
     // (the vector form of the generic kernel counts as a real kernel: variant 1)
-    return dispatch(q, KSMM_ALGO_AUTO, -1, false, &t) == KSMM_OK && (t.algo != KSMM_ALGO_GENERIC || t.variant == 1);
+    return table_run(q, true, false, &t) == KSMM_OK && (t.algo != KSMM_ALGO_GENERIC || t.variant == 1);
 }
 
 // Batch-size-last rows are `batch` elements long: when that is not a multiple of the 16-byte
@@ -262,13 +332,35 @@ bool wants_padded(const Problem &p)
     if (!p.bs_last || p.batch % 16 == 0) return false;
     ksmm_tile t;
     memset(&t, 0, sizeof(t));
-    if (dispatch(p, KSMM_ALGO_AUTO, -1, false, &t) != KSMM_OK || t.algo != KSMM_ALGO_GENERIC || t.variant == 1)
+    if (table_run(p, true, false, &t) != KSMM_OK || t.algo != KSMM_ALGO_GENERIC || t.variant == 1)
         return false;
     Problem q = p;
     q.batch = padded_batch(p.batch);
     if (check_shape(q.batch, p.a, p.b, p.c, p.d, p.x_dtype, p.w_dtype, p.y_dtype) != KSMM_OK) return false;
     memset(&t, 0, sizeof(t));
-    return dispatch(q, KSMM_ALGO_AUTO, -1, false, &t) == KSMM_OK && (t.algo != KSMM_ALGO_GENERIC || t.variant == 1);
+    return table_run(q, true, false, &t) == KSMM_OK && (t.algo != KSMM_ALGO_GENERIC || t.variant == 1);
+}
+
+// The same problem in batch-size-last layout with padded rows (what both routes run in the middle).
+Problem twin_of(const Problem &p)
+{
+    Problem q = p;
+    q.bs_last = 1;
+    q.batch = padded_batch(p.batch);
+    return q;
+}
+
+// Whether the transposed or padded-rows route of a problem that has one beats the kernel that takes
+// it as it is: small problems are done before the first copy would be.
+bool route_pays(const Problem &p)
+{
+    const Pick k = pick_of(p, true);
+    if (k.us < 0.f) return true;
+    const Pick q = pick_of(twin_of(p), true);
+    const int64_t bp = padded_batch(p.batch);
+    const float copies = copy_us((int64_t)p.a * p.c * p.d, p.batch, bp, (int)dtype_size(p.x_dtype), !p.bs_last) +
+                         copy_us((int64_t)p.a * p.b * p.d, p.batch, bp, (int)dtype_size(p.y_dtype), !p.bs_last);
+    return q.us >= 0.f && copies + q.us < k.us;
 }
 
 int64_t align256(int64_t v) { return (v + 255) / 256 * 256; }
@@ -325,11 +417,12 @@ int factor_forward_impl(const void *x, const void *w, void *y, int64_t batch, in
         p.bias = ep->bias;
         p.act = ep->act;
     }
-    // Every kernel but the one-thread-per-output one moves 16-byte vectors: tensors that do not
-    // start on a 16-byte boundary run on that kernel (a forced family refuses them).
+    // Every kernel but the split-K and the one-thread-per-output ones moves aligned 16-byte vectors:
+    // tensors that do not start on a 16-byte boundary run on those (a forced family refuses them).
     if ((((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)p.bias) & 15) != 0) {
         if (algo != KSMM_ALGO_AUTO && !(algo == KSMM_ALGO_GENERIC && variant <= 0)) return KSMM_ERR_BAD_ALGO;
-        return generic_run(p, 0, true, nullptr);
+        const Choice c = algo == KSMM_ALGO_AUTO ? cheapest_instance(p, true) : Choice{KSMM_ALGO_AUTO, -1, -1.f};
+        return c.algo != KSMM_ALGO_AUTO ? family_run(p, c.algo, c.variant, true, nullptr) : generic_run(p, 0, true, nullptr);
     }
     return dispatch(p, algo, variant, true, nullptr);
 }
@@ -351,6 +444,10 @@ int factor_forward_ws_impl(const void *x, const void *w, void *y, int64_t batch,
     if (overlaps(x, xbytes, y, ybytes) || overlaps(workspace, need, x, xbytes) || overlaps(workspace, need, y, ybytes))
         return KSMM_ERR_ALIAS;
     if (((uintptr_t)workspace & 15) != 0) return KSMM_ERR_WORKSPACE;
+    Problem p{x, w, y, batch, a, b, c, d, x_dtype, w_dtype, y_dtype, bs_last ? 1 : 0, scale, (hipStream_t)stream};
+    if (!route_pays(p))
+        return factor_forward_impl(x, w, y, batch, a, b, c, d, x_dtype, w_dtype, y_dtype, bs_last, scale,
+                                   KSMM_ALGO_AUTO, -1, ep, stream);
     if (bs_last) {
         // rows padded to the vector (see wants_padded)
         const int64_t bp = padded_batch(batch);
@@ -420,6 +517,57 @@ bool chain_wants_padded(const ksmm_factor_desc *f, int n, int64_t batch, int x_d
     return false;
 }
 
+// Predicted time of the fused radix-16 chain (< 0: it does not take the chain).  Measured in
+// microseconds at batches 16 .. 25088: 2 factors of 256 features 5.4, 3 of 512 8.1, 3 of 1024 10.7 with
+// e4m3 weights, 1.3 times that with fp16 ones, plus the input and output at 5 TB/s.
+float chain16_us(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype)
+{
+    if (chain16_run(f, n, nullptr, nullptr, batch, x_dtype, y_dtype, 1, false, nullptr, nullptr) != KSMM_OK) return -1.f;
+    const double features = (double)f[0].a * f[0].c * f[0].d;
+    const double base = (2.7 * n + (features > 512 ? 2.6 : 0.)) * (f[0].w_dtype == KSMM_F16 ? 1.3 : 1.);
+    return (float)(base + features * batch * (double)(dtype_size(x_dtype) + dtype_size(y_dtype)) / 5e6);
+}
+
+// Predicted time of a chain factor by factor, as given or in batch-size-last layout with padded rows
+// (< 0: a factor has no price)
+float chain_us(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype, int bs_last, bool twin)
+{
+    float sum = 0.f;
+    for (int i = 0; i < n; ++i) {
+        Problem p{nullptr, nullptr, nullptr, batch, f[i].a, f[i].b, f[i].c, f[i].d, i == 0 ? x_dtype : y_dtype,
+                  f[i].w_dtype, y_dtype, bs_last, 1.f, nullptr};
+        const Pick k = pick_of(twin ? twin_of(p) : p, true);
+        if (k.us < 0.f) return -1.f;
+        sum += k.us;
+    }
+    return sum;
+}
+
+// Whether the fused chain is the faster way through a batch-size-last chain that it takes: at full
+// batches it saves the intermediates' traffic; on a few thousand columns a launch per factor is
+// done first (2.4 us each on the wave kernels against 3 to 4 us a factor in the fused one).
+bool fused_pays(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype)
+{
+    if (batch >= TUNED_MIN_BATCH) return true;
+    const float fused = chain16_us(f, n, batch, x_dtype, y_dtype), each = chain_us(f, n, batch, x_dtype, y_dtype, 1, false);
+    return fused < 0.f || each < 0.f || fused < each;
+}
+
+// Whether a chain that has a transposed or padded-rows route should take it.
+bool chain_route_pays(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype, int bs_last, bool fuse)
+{
+    const float direct = chain_us(f, n, batch, x_dtype, y_dtype, bs_last, false);
+    if (direct < 0.f) return true;
+    const int64_t bp = padded_batch(batch);
+    float middle = chain_us(f, n, batch, x_dtype, y_dtype, bs_last, true);
+    const float fused = fuse ? chain16_us(f, n, bp, x_dtype, y_dtype) : -1.f;
+    if (fused >= 0.f && (middle < 0.f || fused < middle)) middle = fused;
+    if (middle < 0.f) return true;
+    const ksmm_factor_desc &l = f[n - 1];
+    return copy_us((int64_t)f[0].a * f[0].c * f[0].d, batch, bp, (int)dtype_size(x_dtype), !bs_last) +
+               copy_us((int64_t)l.a * l.b * l.d, batch, bp, (int)dtype_size(y_dtype), !bs_last) + middle < direct;
+}
+
 // The chain launcher behind ksmm_chain_forward, ksmm_chain_forward_ep and
 // ksmm_chain_forward_static: `ep` (may be null) belongs to the last factor.
 int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const void *x, void *y, void *workspace,
@@ -448,7 +596,7 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
     // ping-pong buffers of `one` bytes at pp; *result = where the last factor's output is.
     auto run_bs_last = [&](const void *x0, char *pp, int64_t one, int64_t nb, const void **result) -> int {
         int rc2 = KSMM_ERR_BAD_ALGO;
-        if (fuse)
+        if (fuse && fused_pays(factors, n_factors, nb, x_dtype, y_dtype))
             rc2 = chain16_run(factors, n_factors, x0, pp, nb, x_dtype, y_dtype, 1, true, (hipStream_t)stream, ep);
         if (rc2 == KSMM_OK) {
             *result = pp;
@@ -476,7 +624,7 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
         // kernel without a word)
         const int64_t need_t = ksmm_chain_workspace_layout(factors, n_factors, batch, x_dtype, y_dtype, 0);
         if (!workspace || workspace_bytes < need_t) return KSMM_ERR_WORKSPACE;
-        {
+        if (chain_route_pays(factors, n_factors, batch, x_dtype, y_dtype, 0, fuse != 0)) {
             const int64_t bp = padded_batch(batch);  // row length of the transposed copies
             const int64_t xt_bytes = align256(in0 * bp * (int64_t)dtype_size(x_dtype));
             char *xt = (char *)workspace;
@@ -491,7 +639,7 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
         // pad the rows once, run the whole chain at the padded batch, cut the result rows back
         const int64_t need_p = ksmm_chain_workspace_layout(factors, n_factors, batch, x_dtype, y_dtype, 1);
         if (!workspace || workspace_bytes < need_p) return KSMM_ERR_WORKSPACE;
-        {
+        if (chain_route_pays(factors, n_factors, batch, x_dtype, y_dtype, 1, fuse != 0)) {
             const int64_t bp = padded_batch(batch);
             const int64_t xp_bytes = align256(in0 * bp * (int64_t)dtype_size(x_dtype));
             char *xp = (char *)workspace;
@@ -503,7 +651,7 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
             return repitch_run(cur, y, out_n, bp, batch, (int)dtype_size(y_dtype), (hipStream_t)stream);
         }
     }
-    if (fuse) {
+    if (fuse && (!bs_last || fused_pays(factors, n_factors, batch, x_dtype, y_dtype))) {
         // chains whose intermediates fit LDS run as one kernel (no workspace traffic)
         rc = chain16_run(factors, n_factors, x, y, batch, x_dtype, y_dtype, bs_last ? 1 : 0, true,
                          (hipStream_t)stream, ep);

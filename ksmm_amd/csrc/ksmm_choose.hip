@@ -1,0 +1,149 @@
+// Which kernel instance takes a problem the measured table does not cover: small and medium
+// batches, and batch-size-last batches off the vector.
+//
+// The table and the heuristics of the families were measured at full batches, where the tile with
+// the fewest re-reads wins.  Below a few thousand rows that tile leaves most of the chip idle and
+// walks c alone: over 2400 problems drawn from the layers' shapes (batches 1 .. 25088, all types,
+// both layouts) the heuristics' choice took 1.4 to 2.2 times the time of the fastest instance in the
+// geometric mean, and up to 12 times.  Here every instance that takes the problem is priced by a
+// linear model of its time in microseconds,
+//     t = f . (1, s, cu s, s w, cu s w, cu, by, by w)
+//   s   steps of a workgroup's loop over c (wave and row kernels: size of a tile)
+//   cu  rounds of workgroups over the 256 CUs (split-K kernel: of its waves over the SIMDs)
+//   w   share of a 64-byte line a batch-size-first tile does not use, as a factor
+//   by  bytes of input, output and weights at 5 TB/s
+// with non-negative coefficients fitted per instance (wave and row kernels: per family) to their
+// measured times, and the cheapest one is taken: 1.03 to 1.06 times the fastest instance in the
+// geometric mean on problems that were held back from the fit.
+#include <string.h>
+
+#include "ksmm_choose.h"
+
+namespace ksmm {
+
+namespace {
+
+constexpr int FAM_SPLIT = 5, FAM_WAVE = 14, FAM_ROWS = 15;  // tile sub-families have their own numbers
+constexpr int COST_TERMS = 8;
+struct CostRow {
+    int family, combo, bs_last;
+    uint32_t id;
+    float f[COST_TERMS];
+};
+const CostRow cost_rows[] = {
+#include "ksmm_cost.inc"
+};
+constexpr int N_COST = (int)(sizeof(cost_rows) / sizeof(CostRow));
+
+constexpr int N_SUBS = 6, MAX_INST = 128;
+struct CostIndex {  // rows by family and instance
+    const CostRow *tile[N_SUBS][4][2][MAX_INST];
+    const CostRow *wave[4][2], *rows[4][2];
+    int count[N_SUBS];
+    CostIndex()
+    {
+        memset(this, 0, sizeof(*this));
+        const int n[N_SUBS] = {ktile_inst_count(), ws_inst_count(), stream_inst_count(),
+                               bf_inst_count(), gemm_inst_count(), split_inst_count()};
+        uint32_t (*const id[N_SUBS])(int) = {ktile_inst_id, ws_inst_id, stream_inst_id,
+                                             bf_inst_id, gemm_inst_id, split_inst_id};
+        for (int s = 0; s < N_SUBS; ++s) count[s] = n[s] < MAX_INST ? n[s] : MAX_INST;
+        for (int i = 0; i < N_COST; ++i) {
+            const CostRow &r = cost_rows[i];
+            if (r.family == FAM_WAVE) wave[r.combo][r.bs_last] = &r;
+            if (r.family == FAM_ROWS) rows[r.combo][r.bs_last] = &r;
+            if (r.family >= N_SUBS) continue;
+            for (int k = 0; k < count[r.family]; ++k)
+                if (id[r.family](k) == r.id) tile[r.family][r.combo][r.bs_last][k] = &r;
+        }
+    }
+};
+const CostIndex &cost_index()
+{
+    static const CostIndex index;
+    return index;
+}
+
+int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+float price(const CostRow &r, const Problem &p, const ksmm_tile &t)
+{
+    const double ex = (double)dtype_size(p.x_dtype), ew = (double)dtype_size(p.w_dtype), ey = (double)dtype_size(p.y_dtype);
+    const double n = (double)p.batch, ad = (double)p.a * p.d;
+    const int64_t blocks = r.family == FAM_ROWS ? ceil_div((int64_t)p.a * p.d, t.tile_d) : (int64_t)p.a * (p.d / t.tile_d);
+    int64_t groups = blocks * ceil_div(p.b, t.tile_m) * ceil_div(p.batch, t.tile_n);
+    double s = (double)ceil_div(p.c, t.tile_k);
+    int64_t cu = ceil_div(groups, 256);
+    if (r.family == FAM_SPLIT) {
+        const int ks = t.threads / 64;
+        s = (double)ceil_div((int64_t)s, ks);
+        cu = ceil_div(groups * ks, 1024);
+    } else if (r.family == FAM_WAVE || r.family == FAM_ROWS) {
+        s = (double)t.tile_m * t.tile_n * t.tile_d * p.c / 65536.;
+    }
+    const double by = (n * ad * (p.c * ex + p.b * ey) + ad * p.b * p.c * ew) / 5e6;
+    double w = 1.;
+    if (!p.bs_last && t.tile_d < p.d) {
+        const double line = p.d * ex < 64. ? p.d * ex : 64.;
+        w = line / (t.tile_d * ex) > 1. ? line / (t.tile_d * ex) : 1.;
+    }
+    const double v[COST_TERMS] = {1., s, cu * s, s * w, cu * s * w, (double)cu, by, by * w};
+    double us = 0.;
+    for (int i = 0; i < COST_TERMS; ++i) us += r.f[i] * v[i];
+    return (float)us;
+}
+
+const CostRow *row_of(const Problem &p, int combo, int algo, int variant)
+{
+    const CostIndex &ix = cost_index();
+    if (algo == KSMM_ALGO_WAVE) return variant >= 1000 ? ix.rows[combo][p.bs_last] : ix.wave[combo][p.bs_last];
+    if (algo != KSMM_ALGO_TILE) return nullptr;
+    const int sub = variant >> 24, inst = variant & 0xff;
+    return sub < N_SUBS && inst < MAX_INST ? ix.tile[sub][combo][p.bs_last][inst] : nullptr;
+}
+
+}  // namespace
+
+float predicted_us(const Problem &p, const ksmm_tile &t)
+{
+    const int combo = combo_of(p.x_dtype, p.w_dtype, p.y_dtype);
+    const CostRow *r = combo < 0 ? nullptr : row_of(p, combo, t.algo, t.variant);
+    return r ? price(*r, p, t) : -1.f;
+}
+
+Choice cheapest_instance(const Problem &p, bool split_only)
+{
+    Choice best{KSMM_ALGO_AUTO, -1, -1.f};
+    const int combo = combo_of(p.x_dtype, p.w_dtype, p.y_dtype);
+    if (combo < 0) return best;
+    auto offer = [&](int algo, int variant) {
+        ksmm_tile t;
+        memset(&t, 0, sizeof(t));
+        const int rc = algo == KSMM_ALGO_WAVE ? wave_run(p, variant, false, &t) : tile_run(p, variant, false, &t);
+        if (rc != KSMM_OK) return;
+        const CostRow *r = row_of(p, combo, t.algo, t.variant);
+        if (!r || (t.threads & 63) || t.tile_d < 1) return;
+        const float us = price(*r, p, t);
+        if (best.us < 0.f || us < best.us) best = Choice{t.algo, t.variant, us};
+    };
+    const CostIndex &ix = cost_index();
+    if (!split_only) {
+        offer(KSMM_ALGO_WAVE, -1);
+        for (int sub = 0; sub < FAM_SPLIT; ++sub)
+            for (int i = 0; i < ix.count[sub]; ++i)
+                if (ix.tile[sub][combo][p.bs_last][i]) offer(KSMM_ALGO_TILE, (sub << 24) | i);
+    }
+    for (int i = 0; i < ix.count[FAM_SPLIT]; ++i) {
+        if (!ix.tile[FAM_SPLIT][combo][p.bs_last][i]) continue;
+        for (int waves = 1; waves <= 16; waves *= 2) offer(KSMM_ALGO_TILE, (FAM_SPLIT << 24) | (waves << 8) | i);
+    }
+    return best;
+}
+
+float copy_us(int64_t rows, int64_t cols_in, int64_t cols_out, int elem_bytes, bool transpose)
+{
+    // measured: 7.4 us for 19 + 19 MB transposed, 28 us for 77 + 77; 8.3 us for 10 + 10 MB re-pitched
+    return 2.5f + (float)((double)rows * (cols_in + cols_out) * elem_bytes / (transpose ? 5.2e6 : 3e6));
+}
+
+}  // namespace ksmm

@@ -172,10 +172,14 @@ int bf_inst_count();
 uint32_t bf_inst_id(int i);
 int gemm_inst_count();
 uint32_t gemm_inst_id(int i);
+int split_inst_count();
+uint32_t split_inst_id(int i);
 
 // Launchers, one per kernel family.  Each fills `tile` and, when `launch` is true, enqueues
 // the kernel on p.stream.  They return KSMM_ERR_BAD_ALGO when the family (or the requested
 // variant) cannot run the problem.
+// (generic variants from GENERIC_TILE on: the tile instance of that variant, see ksmm_hip.h)
+constexpr int GENERIC_TILE = 16;
 int generic_run(const Problem &p, int variant, bool launch, ksmm_tile *tile);
 int wave_run(const Problem &p, int variant, bool launch, ksmm_tile *tile);
 int tile_run(const Problem &p, int variant, bool launch, ksmm_tile *tile);
@@ -183,6 +187,7 @@ int stream_run(const Problem &p, int variant, bool launch, ksmm_tile *tile);  //
 int rows_bf_run(const Problem &p, int variant, bool launch, ksmm_tile *tile);  // part of the wave family
 int gemm_run(const Problem &p, int variant, bool launch, ksmm_tile *tile);  // part of the tile family
 int tile_bf_run(const Problem &p, int variant, bool launch, ksmm_tile *tile);  // part of the tile family
+int split_run(const Problem &p, int variant, bool launch, ksmm_tile *tile);  // part of the tile family
 
 // Backward pass pieces (ksmm_backward.hip): blockwise transpose of a kernel-format weight, and the
 // weight gradient (acc: fp32 scratch of wgrad_partial_floats() elements, one slice of a*b*c*d per

@@ -172,9 +172,18 @@ static void launch_generic(const Problem &p, dim3 grid, dim3 block)
 }
 
 // variant 0: one thread per output; 1: the vector form (batch-size-last, batch a multiple of the
-// 16-byte vector); -1: the vector form where it applies and the block is small
+// 16-byte vector); -1: the vector form where it applies and the block is small; GENERIC_TILE + v: the
+// tile instance v, for problems without a kernel of their own at full batches
 int generic_run(const Problem &p, int variant, bool launch, ksmm_tile *tile)
 {
+    if (variant >= GENERIC_TILE) {
+        const int rc = tile_run(p, variant - GENERIC_TILE, launch, tile);
+        if (rc == KSMM_OK && tile) {
+            tile->algo = KSMM_ALGO_GENERIC;
+            tile->variant = variant;
+        }
+        return rc;
+    }
     if (variant > 1) return KSMM_ERR_BAD_ALGO;
     const int combo = combo_of(p.x_dtype, p.w_dtype, p.y_dtype);
     const int vec = 16 / (int)dtype_size(p.x_dtype);

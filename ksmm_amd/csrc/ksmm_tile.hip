@@ -663,6 +663,7 @@ int tile_run(const Problem &p, int variant, bool launch, ksmm_tile *tile)
     // sub-family parameter (persistent workgroups per block); -1: everything automatic
     if (variant >= 0) {
         const int sub = (variant >> 24) & 15, inst = variant & 0xff, par = (variant >> 8) & 0xffff;
+        if (sub == 5) return split_run(p, inst == 0xff ? -1 : inst | (par << 8), launch, tile);
         if (sub == 4) return gemm_run(p, inst == 0xff ? -1 : inst, launch, tile);
         if (sub == 3) return tile_bf_run(p, inst == 0xff ? -1 : inst, launch, tile);
         if (sub == 2) return stream_run(p, (inst == 0xff ? 0x7f : inst) | (par << 7), launch, tile);

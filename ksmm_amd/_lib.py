@@ -81,6 +81,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_native = None
 
 
 class KsmmError(RuntimeError):
@@ -108,6 +109,20 @@ def load():
                           "`python -m ksmm_amd.build`" % (lib.ksmm_version(), ABI_VERSION))
     _lib = lib
     return lib
+
+
+def native():
+    """The CPython module KSLinear calls the library through (loaded once, with the library)."""
+    global _native
+    if _native is None:
+        load()
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise ImportError("ksmm_amd/_native.so is not built or does not load (%s): run `python -m ksmm_amd.build`. "
+                              "algo='kernel' has no fallback." % e)
+        _native = module
+    return _native
 
 
 def strerror(status):

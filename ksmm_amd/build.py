@@ -1,4 +1,5 @@
-"""Builds libksmm_hip.so for gfx950 with hipcc (cross-compiles without a GPU).
+"""Builds libksmm_hip.so for gfx950 with hipcc (cross-compiles without a GPU), and the CPython module
+_native.so that KSLinear calls it through.
 
     python -m ksmm_amd.build          # rebuild everything
 """
@@ -15,6 +16,9 @@ SOURCES = ["ksmm_api.hip", "ksmm_generic.hip", "ksmm_wave.hip", "ksmm_tile.hip",
 # measurement aids of bench.py: a library of their own, outside the drop-in ABI
 BENCH_LIB = os.path.join(HERE, "libksmm_bench.so")
 BENCH_SOURCES = ["ksmm_probe.hip"]
+# host side of KSLinear: a CPython module that links the library
+NATIVE = os.path.join(HERE, "_native.so")
+NATIVE_SOURCE = "ksmm_torch.cpp"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # packed fp32 VALU ops are switched off on purpose for this hardware pool
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function", "-Wno-inline-asm",
@@ -32,17 +36,48 @@ def _compile(src):
     return obj, warn
 
 
+def _compile_native():
+    import sysconfig
+
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    obj = os.path.join(OBJ, NATIVE_SOURCE.replace(".cpp", ".o"))
+    inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI), *("-I" + i for i in inc),
+           "-c", os.path.join(CSRC, NATIVE_SOURCE), "-o", obj]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed for %s:\n%s" % (NATIVE_SOURCE, r.stderr[-8000:]))
+    return obj, ""
+
+
+def _link_native(obj):
+    import torch
+
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ["g++", "-shared", "-o", NATIVE, obj, LIB, "-L" + lib, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python",
+           "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("link failed:\n" + r.stderr[-4000:])
+
+
 def build(verbose=False, jobs=8):
     os.makedirs(OBJ, exist_ok=True)
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as ex:
+        native = ex.submit(_compile_native)
         results = list(ex.map(_compile, SOURCES + BENCH_SOURCES))
+        native_obj, _ = native.result()
     objs = [o for o, _ in results[:len(SOURCES)]]
     bench_objs = [o for o, _ in results[len(SOURCES):]]
     if verbose:
         for _, w in results:
             if w:
                 print(w, file=sys.stderr)
-    r = subprocess.run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs,
+    r = subprocess.run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-Wl,-soname,libksmm_hip.so", "-o", LIB] + objs,
                        capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("link failed:\n" + r.stderr[-4000:])
@@ -50,6 +85,7 @@ def build(verbose=False, jobs=8):
                        capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("link failed:\n" + r.stderr[-4000:])
+    _link_native(native_obj)
     return LIB
 
 

@@ -234,11 +234,53 @@ int table_run(const Problem &p, bool table, bool launch, ksmm_tile *tile)
     return generic_run(p, -1, launch, tile);
 }
 
+// Rows of a batch-size-last workspace copy are padded to a multiple of 16 columns (the 16-byte
+// vector of every type).
+int64_t padded_batch(int64_t batch) { return (batch + 15) / 16 * 16; }
+
+// A batch-size-first problem that only the generic kernel takes, while its batch-size-last
+// twin has a real kernel: worth two transposes.  (The transposed copy has padded rows, so the
+// twin runs at the padded batch.)
+bool find_transposed(const Problem &p)
+{
+    if (p.bs_last) return false;
+    ksmm_tile t;
+    memset(&t, 0, sizeof(t));
+    if (table_run(p, true, false, &t) != KSMM_OK || t.algo != KSMM_ALGO_GENERIC) return false;
+    Problem q = p;
+    q.bs_last = 1;
+    q.batch = padded_batch(p.batch);
+    // (a batch whose padded copies would pass the size limit stays on the kernel it has)
+    if (check_shape(q.batch, p.a, p.b, p.c, p.d, p.x_dtype, p.w_dtype, p.y_dtype) != KSMM_OK) return false;
+    memset(&t, 0, sizeof(t));
+    // (the vector form of the generic kernel counts as a real kernel: variant 1)
+    return table_run(q, true, false, &t) == KSMM_OK && (t.algo != KSMM_ALGO_GENERIC || t.variant == 1);
+}
+
+// Batch-size-last rows are `batch` elements long: when that is not a multiple of the 16-byte
+// vector only the one-thread-per-output kernel takes the problem.  With a workspace it runs on a
+// copy whose rows are zero-filled to the next multiple of 16 columns (the vector of every type)
+// and the result rows are cut back: two copies more, but on the kernel of the padded batch.
+bool find_padded(const Problem &p)
+{
+    if (!p.bs_last || p.batch % 16 == 0) return false;
+    ksmm_tile t;
+    memset(&t, 0, sizeof(t));
+    if (table_run(p, true, false, &t) != KSMM_OK || t.algo != KSMM_ALGO_GENERIC || t.variant == 1)
+        return false;
+    Problem q = p;
+    q.batch = padded_batch(p.batch);
+    if (check_shape(q.batch, p.a, p.b, p.c, p.d, p.x_dtype, p.w_dtype, p.y_dtype) != KSMM_OK) return false;
+    memset(&t, 0, sizeof(t));
+    return table_run(q, true, false, &t) == KSMM_OK && (t.algo != KSMM_ALGO_GENERIC || t.variant == 1);
+}
+
 // What takes a problem as it is.  `direct`: the full-batch choice is a kernel of its own, not the
 // one-thread-per-output one.
 struct Pick {
     Choice c;     // AUTO: the full-batch choice
     bool direct;
+    bool transposed, padded;  // the problem has that route
     float us;     // predicted time, < 0: no model of it
 };
 
@@ -262,7 +304,7 @@ Pick pick_of(const Problem &p, bool table)
     if (e.batch == p.batch && memcmp(e.key, key, sizeof(key)) == 0) return e.pick;
     ksmm_tile t;
     memset(&t, 0, sizeof(t));
-    Pick k{{KSMM_ALGO_AUTO, -1, -1.f}, true, -1.f};
+    Pick k{{KSMM_ALGO_AUTO, -1, -1.f}, true, find_transposed(p), find_padded(p), -1.f};
     if (table_run(p, table, false, &t) == KSMM_OK) {
         k.direct = t.algo != KSMM_ALGO_GENERIC || t.variant == 1;
         k.us = predicted_us(p, t);
@@ -279,6 +321,9 @@ Pick pick_of(const Problem &p, bool table)
     e.pick = k;
     return k;
 }
+
+bool wants_transposed(const Problem &p) { return pick_of(p, true).transposed; }
+bool wants_padded(const Problem &p) { return pick_of(p, true).padded; }
 
 int dispatch(const Problem &p, int algo, int variant, bool launch, ksmm_tile *tile)
 {
@@ -298,47 +343,6 @@ int dispatch(const Problem &p, int algo, int variant, bool launch, ksmm_tile *ti
         }
     }
     return table_run(p, table, launch, tile);
-}
-
-// Rows of a batch-size-last workspace copy are padded to a multiple of 16 columns (the 16-byte
-// vector of every type).
-int64_t padded_batch(int64_t batch) { return (batch + 15) / 16 * 16; }
-
-// A batch-size-first problem that only the generic kernel takes, while its batch-size-last
-// twin has a real kernel: worth two transposes.  (The transposed copy has padded rows, so the
-// twin runs at the padded batch.)
-bool wants_transposed(const Problem &p)
-{
-    if (p.bs_last) return false;
-    ksmm_tile t;
-    memset(&t, 0, sizeof(t));
-    if (table_run(p, true, false, &t) != KSMM_OK || t.algo != KSMM_ALGO_GENERIC) return false;
-    Problem q = p;
-    q.bs_last = 1;
-    q.batch = padded_batch(p.batch);
-    // (a batch whose padded copies would pass the size limit stays on the kernel it has)
-    if (check_shape(q.batch, p.a, p.b, p.c, p.d, p.x_dtype, p.w_dtype, p.y_dtype) != KSMM_OK) return false;
-    memset(&t, 0, sizeof(t));
-    // (the vector form of the generic kernel counts as a real kernel: variant 1)
-    return table_run(q, true, false, &t) == KSMM_OK && (t.algo != KSMM_ALGO_GENERIC || t.variant == 1);
-}
-
-// Batch-size-last rows are `batch` elements long: when that is not a multiple of the 16-byte
-// vector only the one-thread-per-output kernel takes the problem.  With a workspace it runs on a
-// copy whose rows are zero-filled to the next multiple of 16 columns (the vector of every type)
-// and the result rows are cut back: two copies more, but on the kernel of the padded batch.
-bool wants_padded(const Problem &p)
-{
-    if (!p.bs_last || p.batch % 16 == 0) return false;
-    ksmm_tile t;
-    memset(&t, 0, sizeof(t));
-    if (table_run(p, true, false, &t) != KSMM_OK || t.algo != KSMM_ALGO_GENERIC || t.variant == 1)
-        return false;
-    Problem q = p;
-    q.batch = padded_batch(p.batch);
-    if (check_shape(q.batch, p.a, p.b, p.c, p.d, p.x_dtype, p.w_dtype, p.y_dtype) != KSMM_OK) return false;
-    memset(&t, 0, sizeof(t));
-    return table_run(q, true, false, &t) == KSMM_OK && (t.algo != KSMM_ALGO_GENERIC || t.variant == 1);
 }
 
 // The same problem in batch-size-last layout with padded rows (what both routes run in the middle).

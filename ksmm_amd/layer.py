@@ -15,6 +15,8 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from . import _lib
+
 ALGOS = ("dense", "einsum", "kernel", "bmm")
 FP8 = torch.float8_e4m3fn
 FP8_MAX = 448.0
@@ -236,7 +238,26 @@ class KSLinear(nn.Module):
                 output = output.reshape(a * b * d, *lead)
         return output
 
+    def _infer(self, tensor, x_scale):
+        """The layer in one native call, or None where gradients are wanted or the call is unusual."""
+        factors = list(self.factors._parameters.values())
+        if torch.is_grad_enabled() and self.dtype != FP8 and (
+                tensor.requires_grad or any(f.requires_grad for f in factors)):
+            return None
+        scales = self.w_scales
+        if self.dtype == FP8:
+            if tensor.dtype != FP8:
+                return None
+            if x_scale is not None:
+                scales = [scales[0] * float(x_scale)] + scales[1:]
+        return _lib.native().infer(tensor, factors, self.patterns, self.bs_last, scales, self.fuse,
+                                   self._parameters["bias"], self.act)
+
     def forward(self, tensor, x_scale=None):
+        if self.algo == "kernel":
+            output = self._infer(tensor, x_scale)
+            if output is not None:
+                return output
         output = self.pre_process(tensor)
         if self.dtype == FP8 and self.algo != "kernel":
             # PyTorch algorithms work on the dequantised input in fp32

@@ -3,13 +3,14 @@
 //   dX = K^T dY   is itself a KS factor: pattern (a, c, b, d) with every b x c block transposed,
 //                 so it runs on the forward kernels once the blocks are transposed (ks_block_transpose_kernel)
 //   dW[a_i, b_i, c_i, d_i] = sum_n dY[a_i, b_i, d_i, n] * X[a_i, c_i, d_i, n]
-//                 one (b x B) @ (B x c) product per (a_i, d_i) block, reduced over the batch:
-//                 MFMA kernel for batch-size-last (operand rows are batch-contiguous, so both
-//                 operands come straight from global memory in MFMA layout, no LDS), an
-//                 LDS-tiled FMA kernel for everything else; every batch split writes its partial
-//                 sums to a slice of its own in the workspace, and a finish kernel adds the slices
-//                 in a fixed order, scales, converts and writes kernel format (a*d*c, b): the
-//                 result is the same bit for bit from run to run (no atomics).
+//                 one (b x B) @ (B x c) product per (a_i, d_i) block, reduced over the batch.
+//                 Batch-size-last: MFMA kernels below (operand rows are batch-contiguous, so both
+//                 operands come straight from global memory in MFMA layout); batch-size-first:
+//                 ksmm_wgrad_bf.hip; rows shorter than a 16-byte vector: an LDS-tiled FMA kernel.
+//                 Every batch split writes its partial sums to a slice of its own in the
+//                 workspace, and a finish kernel adds the slices in a fixed order, scales, converts
+//                 and writes kernel format (a*d*c, b): the result is the same bit for bit from run
+//                 to run (no atomics).
 //
 // The reference has no backward pass (src/ksmm_py/layer/kronecker_sparse/kernel.py:319-329 refers
 // to an undefined symbol; forward_bmm.py:12-15 is `pass`); the definition above is the adjoint of
@@ -63,6 +64,30 @@ __global__ __launch_bounds__(256) void ks_wgrad_finish_kernel(const float *__res
     if (g == 0 && i < n) dw[i] = (T)((((part[0][l] + part[1][l]) + part[2][l]) + part[3][l]) * scale);
 }
 
+// One 16-byte vector; ANY: at element alignment.  fp16 vectors at odd elements come as aligned words
+// that are shifted into place (a 2-byte aligned vector load takes about twice as long); no word is
+// read that does not hold one of the elements.
+template <bool NTL, bool ANY, typename V, typename T> __device__ __forceinline__ V wg_load(const T *p)
+{
+    if (ANY && sizeof(T) == 2) {
+        const uintptr_t at = (uintptr_t)p;
+        const uint32_t *w = (const uint32_t *)(at & ~(uintptr_t)3);
+        const uint32_t odd = (uint32_t)at & 2;
+        uint4_t v;
+        __builtin_memcpy(&v, w, 16);
+        const uint32_t last = w[odd ? 4 : 3];
+        v = uint4_t{__builtin_amdgcn_alignbyte(v[1], v[0], odd), __builtin_amdgcn_alignbyte(v[2], v[1], odd),
+                    __builtin_amdgcn_alignbyte(v[3], v[2], odd), __builtin_amdgcn_alignbyte(last, v[3], odd)};
+        return __builtin_bit_cast(V, v);
+    }
+    if (ANY) {
+        V v;
+        __builtin_memcpy(&v, p, sizeof(V));
+        return v;
+    }
+    return NTL ? __builtin_nontemporal_load((const V *)p) : *(const V *)p;
+}
+
 template <typename T> struct wg_vec;
 template <> struct wg_vec<float> {
     static constexpr int N = 4, MFMAS = 4;  // elements per 16-byte load; MFMAs fed by one load pair
@@ -83,14 +108,17 @@ template <> struct wg_vec<half_t> {
     }
 };
 
-// Batch-size-last, batch a multiple of the 16-byte vector.  One wavefront owns a (16*MT) x (16*NT)
+// Batch-size-last.  One wavefront owns a (16*MT) x (16*NT)
 // tile of one block's b x c gradient and a range of batch columns.  Lane (r = lane % 16,
 // q = lane / 16) loads N consecutive batch elements of operand row r at column n + N*q; MFMA e
 // multiplies element group e of every lane, i.e. its k-set is {n + N*q + e ...}: the same set for
 // both operands, and the order of a sum's terms is free.
 // NTL: non-temporal loads, for blocks of a single tile (every operand row is read by one wave only;
 // with several tiles per block the rows are shared through the caches)
-template <typename T, int MT, int NT, bool NTL>
+// ANY: rows of any length and alignment (a batch that the vector does not divide): vectors at element
+// alignment, and the last one of a row pulled back to end with it, its first elements cleared where
+// the vector before has them.
+template <typename T, int MT, int NT, bool NTL, bool ANY>
 __global__ __launch_bounds__(256) void ks_wgrad_bl_kernel(const T *__restrict__ dy, const T *__restrict__ x,
                                                           float *__restrict__ acc_out, int batch, int a, int b,
                                                           int c, int d, int m_tiles, int n_tiles, int splits,
@@ -135,25 +163,26 @@ __global__ __launch_bounds__(256) void ks_wgrad_bl_kernel(const T *__restrict__ 
         for (int u = 0; u < U; ++u) {
             const int col = n + u * STEP + V::N * q;
             const bool live = col < n_end;          // whole vectors: batch and the split are multiples of N
-            const int lcol = live ? col : n_begin;  // (a valid address; the value is zeroed)
+            const int lcol = ANY ? min(col, batch - V::N) : live ? col : n_begin;  // (a valid address; the value is zeroed)
 #pragma unroll
-            for (int i = 0; i < MT; ++i)
-                av[u][i] = NTL ? __builtin_nontemporal_load((const vec_t *)(ap[i] + lcol)) : *(const vec_t *)(ap[i] + lcol);
+            for (int i = 0; i < MT; ++i) av[u][i] = wg_load<NTL, ANY, vec_t>(ap[i] + lcol);
 #pragma unroll
-            for (int j = 0; j < NT; ++j)
-                bv[u][j] = NTL ? __builtin_nontemporal_load((const vec_t *)(bp[j] + lcol)) : *(const vec_t *)(bp[j] + lcol);
+            for (int j = 0; j < NT; ++j) bv[u][j] = wg_load<NTL, ANY, vec_t>(bp[j] + lcol);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            if (n + u * STEP + V::N * q >= n_end) {
+            const int col = n + u * STEP + V::N * q;
+            if (ANY ? col + V::N > n_end : col >= n_end) {
+                // elements in front of `drop` are not this vector's (n_end is the batch where ANY gets here with col < n_end)
+                const int drop = ANY && col < n_end ? col - min(col, batch - V::N) : V::N;
 #pragma unroll
                 for (int i = 0; i < MT; ++i)
 #pragma unroll
-                    for (int e = 0; e < V::N; ++e) av[u][i][e] = 0;
+                    for (int e = 0; e < V::N; ++e) av[u][i][e] = e < drop ? (T)0 : av[u][i][e];
 #pragma unroll
                 for (int j = 0; j < NT; ++j)
 #pragma unroll
-                    for (int e = 0; e < V::N; ++e) bv[u][j][e] = 0;
+                    for (int e = 0; e < V::N; ++e) bv[u][j][e] = e < drop ? (T)0 : bv[u][j][e];
             }
 #pragma unroll
             for (int e = 0; e < V::MFMAS; ++e)
@@ -243,7 +272,9 @@ template <typename T> int launch_block_transpose(const void *w, void *wt, int64_
 // which re-reads every operand row once per 64 x 64 tile through L2 (1.85 GB for (1,1536,384,2) at
 // batch 25088), the traffic drops to a quarter.  D = X-rows x dY-rows^T, so a lane holds one output
 // feature m (contiguous in kernel format) and 16 inputs k.
+// ANY as in the kernel above.
 constexpr int WG_TM = 128, WG_TN = 128, WG_TK = 64;
+template <bool ANY>
 __global__ __launch_bounds__(256, 2) void ks_wgrad_gemm_h_kernel(const half_t *__restrict__ dy,
                                                                  const half_t *__restrict__ x,
                                                                  float *__restrict__ acc_out, int batch, int a, int b,
@@ -277,9 +308,20 @@ __global__ __launch_bounds__(256, 2) void ks_wgrad_gemm_h_kernel(const half_t *_
     auto gload = [&](int k) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const bool in = k + lcol[i] < k_end;  // (k_end is a multiple of 8)
-            ra[i] = in ? *(const uint4_t *)(ga[i] + k) : uint4_t{0u, 0u, 0u, 0u};
-            rb[i] = in ? *(const uint4_t *)(gb[i] + k) : uint4_t{0u, 0u, 0u, 0u};
+            const int col = k + lcol[i];
+            ra[i] = rb[i] = uint4_t{0u, 0u, 0u, 0u};
+            if (col >= k_end) continue;  // (without ANY, k_end is a multiple of 8)
+            const int back = ANY ? max(col + 8 - batch, 0) : 0;
+            ra[i] = wg_load<false, ANY, uint4_t>(ga[i] + k - back);
+            rb[i] = wg_load<false, ANY, uint4_t>(gb[i] + k - back);
+            if (ANY && back > 0) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t keep = (2 * e >= back ? 0xffffu : 0u) | (2 * e + 1 >= back ? 0xffff0000u : 0u);
+                    ra[i][e] &= keep;
+                    rb[i][e] &= keep;
+                }
+            }
         }
     };
     auto lstore = [&](int buf) {
@@ -384,11 +426,14 @@ int wgrad_bl_tile(int b, int c)
     return (b <= 16 && c <= 16) ? 1 : (b <= 32 && c <= 32) ? 2 : (b % 64 && c % 64 && b % 48 == 0 && c % 48 == 0) ? 3 : 4;
 }
 
-bool wgrad_mfma_ok(const void *dy, const void *x, int64_t batch, int b, int c, int d, int dtype, int bs_last)
+// Batch-size-last with at least one vector per row.  Against the tiled kernel at 6501 columns, which
+// the vector does not divide: (1,768,192,2) fp16 310 -> 58 us, fp32 310 -> 82.
+bool wgrad_mfma_ok(int64_t batch, int dtype, int bs_last) { return bs_last && batch >= 16 / (int)dtype_size(dtype); }
+
+// rows of whole, aligned vectors
+bool wgrad_aligned(const void *dy, const void *x, int64_t batch, int dtype)
 {
-    const int vec = 16 / (int)dtype_size(dtype);
-    return bs_last && batch % vec == 0 && ((((uintptr_t)dy | (uintptr_t)x) & 15) == 0) &&
-           (int64_t)(b > c ? b : c) * d * batch < 0x7fffffffLL;
+    return batch % (16 / (int)dtype_size(dtype)) == 0 && ((((uintptr_t)dy | (uintptr_t)x) & 15) == 0);
 }
 
 template <typename T, int MT, int NT>
@@ -403,14 +448,12 @@ int launch_wgrad_bl(const void *dy, const void *x, float *acc, int64_t batch, in
     const int64_t waves = tiles * splits, blocks = (waves + 3) / 4;
     if (blocks > 0x7fffffffLL) return KSMM_ERR_TOO_LARGE;
     *splits_used = (int)splits;
-    if (m_tiles == 1 && n_tiles == 1)
-        hipLaunchKernelGGL((ks_wgrad_bl_kernel<T, MT, NT, true>), dim3((unsigned)blocks), dim3(256), 0, s, (const T *)dy,
-                           (const T *)x, acc, (int)batch, a, b, c, d, m_tiles, n_tiles, (int)splits, (int)cols,
-                           (int64_t)a * b * c * d);
-    else
-        hipLaunchKernelGGL((ks_wgrad_bl_kernel<T, MT, NT, false>), dim3((unsigned)blocks), dim3(256), 0, s, (const T *)dy,
-                           (const T *)x, acc, (int)batch, a, b, c, d, m_tiles, n_tiles, (int)splits, (int)cols,
-                           (int64_t)a * b * c * d);
+    const bool one = m_tiles == 1 && n_tiles == 1, any = !wgrad_aligned(dy, x, batch, elem<T>::dtype);
+    const auto fn = any   ? &ks_wgrad_bl_kernel<T, MT, NT, false, true>
+                    : one ? &ks_wgrad_bl_kernel<T, MT, NT, true, false>
+                          : &ks_wgrad_bl_kernel<T, MT, NT, false, false>;
+    hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(256), 0, s, (const T *)dy, (const T *)x, acc, (int)batch, a, b, c, d,
+                       m_tiles, n_tiles, (int)splits, (int)cols, (int64_t)a * b * c * d);
     return hipGetLastError() == hipSuccess ? KSMM_OK : KSMM_ERR_LAUNCH;
 }
 
@@ -445,7 +488,8 @@ int launch_wgrad_gemm(const void *dy, const void *x, float *acc, int64_t batch, 
     const int64_t blocks = tiles * splits;
     if (blocks > 0x7fffffffLL) return KSMM_ERR_TOO_LARGE;
     *splits_used = (int)splits;
-    hipLaunchKernelGGL(ks_wgrad_gemm_h_kernel, dim3((unsigned)blocks), dim3(256), 0, s, (const half_t *)dy,
+    const auto fn = wgrad_aligned(dy, x, batch, KSMM_F16) ? &ks_wgrad_gemm_h_kernel<false> : &ks_wgrad_gemm_h_kernel<true>;
+    hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(256), 0, s, (const half_t *)dy,
                        (const half_t *)x, acc, (int)batch, a, b, c, d, m_tiles, n_tiles, (int)splits, (int)cols,
                        (int64_t)a * b * c * d);
     return hipGetLastError() == hipSuccess ? KSMM_OK : KSMM_ERR_LAUNCH;
@@ -466,10 +510,10 @@ int block_transpose_run(const void *w, void *wt, int a, int b, int c, int d, int
 }
 
 // Floats of partial sums the weight gradient of this problem writes (slices of a*b*c*d, one per
-// batch split), whichever kernel takes it: the larger of the two kernels' needs, so that the
-// answer does not depend on pointer alignment.
-int64_t wgrad_partial_floats(int64_t batch, int a, int b, int c, int d, int dtype)
+// batch split), whichever kernel takes it: the largest of the kernels' needs.
+int64_t wgrad_partial_floats(int64_t batch, int a, int b, int c, int d, int dtype, int bs_last)
 {
+    if (!bs_last && wgrad_bf_ok(a, b, c, d, dtype)) return wgrad_bf_partial_floats(batch, a, b, c, d, dtype);
     const int64_t n = (int64_t)a * b * c * d;
     int64_t splits, cols, most = 1;
     const int t = wgrad_bl_tile(b, c);
@@ -486,18 +530,20 @@ int64_t wgrad_partial_floats(int64_t batch, int a, int b, int c, int d, int dtyp
 }
 
 // dw (kernel format, type `dtype`) <- scale * sum over the batch of dY x X^T per block; acc is an
-// fp32 buffer of wgrad_partial_floats() elements.  kernel_used: 1 = MFMA kernel, 0 = tiled kernel.
+// fp32 buffer of wgrad_partial_floats() elements.
 int wgrad_run(const void *dy, const void *x, void *dw, float *acc, int64_t batch, int a, int b, int c, int d,
-              int dtype, int bs_last, float scale, hipStream_t stream, int *kernel_used)
+              int dtype, int bs_last, float scale, hipStream_t stream)
 {
     const int64_t n = (int64_t)a * b * c * d;
     const int64_t fin_blocks = (n + 63) / 64;
     if (fin_blocks > 0x7fffffffLL) return KSMM_ERR_TOO_LARGE;
-    const bool mfma_ok = wgrad_mfma_ok(dy, x, batch, b, c, d, dtype, bs_last);
-    if (kernel_used) *kernel_used = mfma_ok ? 1 : 0;
+    const bool mfma_ok = wgrad_mfma_ok(batch, dtype, bs_last);
     const int t = wgrad_bl_tile(b, c);
     int rc, splits = 1;
-    if (dtype == KSMM_F32) {
+    if (!bs_last && wgrad_bf_ok(a, b, c, d, dtype)) {
+        rc = wgrad_bf_run(dy, x, dw, acc, batch, a, b, c, d, dtype, scale, stream, &splits);
+        if (rc != KSMM_OK || splits == 1) return rc;
+    } else if (dtype == KSMM_F32) {
         if (mfma_ok)
             rc = t == 1   ? launch_wgrad_bl<float, 1, 1>(dy, x, acc, batch, a, b, c, d, stream, &splits)
                  : t == 2 ? launch_wgrad_bl<float, 2, 2>(dy, x, acc, batch, a, b, c, d, stream, &splits)

@@ -1,0 +1,45 @@
+"""Weight gradients at the edges of their kernels: the batch-size-first kernel (ksmm_wgrad_bf.hip) and
+the batch-size-last ones on rows of any length and alignment, against float64 products of the values
+the device holds.
+
+Tolerance: a gradient is a sum of n products rounded once to its type; the fp32 accumulation is off by
+at most n * 2^-24 of the sum of the magnitudes, sqrt(n) * 2^-24 for inputs of random sign, so for
+n <= 4200 the relative Frobenius error is below 1e-5 in fp32 and that of the last rounding, 2^-11 at
+most, in fp16."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TOL = {torch.float32: 1e-5, torch.float16: 5e-4}
+
+# block edges of 16, 32, 48 and 64 and one more; d of one pass (1 .. 8) and in eights with an overlap (9,
+# 12); blocks shared by a workgroup with a remainder; one row, one slab, a ragged one, several splits
+CASES = [((1, 16, 16, 64), 130), ((5, 16, 9, 1), 333), ((3, 17, 33, 1), 64), ((7, 32, 20, 3), 129), ((1, 48, 144, 5), 1),
+         ((2, 65, 64, 2), 31), ((1, 64, 129, 7), 97), ((2, 40, 24, 9), 261), ((1, 70, 130, 12), 40), ((1, 192, 64, 8), 515),
+         ((3, 64, 64, 1), 4197), ((1, 451, 64, 1), 77), ((2, 130, 260, 4), 1030), ((1, 3, 500, 1), 50), ((1, 128, 128, 1), 3),
+         ((1, 128, 256, 2), 777), ((2, 48, 48, 3), 2003)]
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16])
+@pytest.mark.parametrize("bs_last", [False, True])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_weight_gradient_edges(dt, bs_last, offset):
+    """``offset``: the operands start one element behind a 16-byte boundary."""
+    from ksmm_amd import Kernel
+
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    for (a, b, c, d), n in CASES:
+        def tensor(features):
+            t = torch.randn(offset + features * n, generator=gen, device="cuda").to(dt)[offset:]
+            return t.view(features, n) if bs_last else t.view(n, features)
+
+        x, dy = tensor(a * c * d), tensor(a * b * d)
+        factor = torch.zeros(a * c * d, b, device="cuda", dtype=dt)
+        got = Kernel.backward(dy, x, factor, bs_last, a, b, c, d, scale=0.5, need_input=False)[1]
+        xs, ys = (x, dy) if bs_last else (x.t(), dy.t())
+        xs = xs.double().reshape(a, c, d, n).permute(0, 2, 1, 3).reshape(a * d, c, n)
+        ys = ys.double().reshape(a, b, d, n).permute(0, 2, 3, 1).reshape(a * d, n, b).contiguous()
+        want = 0.5 * torch.bmm(xs, ys).reshape(a * d * c, b)
+        err = ((got.double() - want).norm() / want.norm()).item()
+        assert err <= TOL[dt], ((a, b, c, d), n, err)

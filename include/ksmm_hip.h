@@ -252,6 +252,16 @@ int ksmm_factor_backward_weight(const void *dy, const void *x, void *dw, int64_t
                                 int c, int d, int dtype, int bs_last, float scale, void *workspace,
                                 int64_t workspace_bytes, void *stream);
 
+/* Backward pass of an epilogue y = act(z), z = K x + bias (fp32 and fp16):
+ *   dz = dy * act'(z)   (dy, z, dz: y's shape and layout; with KSMM_ACT_NONE dz is dy: z and dz are
+ *                       not touched and may be NULL),
+ *   dbias[f] = the sum of dz over the batch, in fp32 and in a fixed order (NULL: not wanted).
+ * Needs ksmm_epilogue_backward_workspace() bytes of 16-byte aligned device memory for dbias. */
+int64_t ksmm_epilogue_backward_workspace(int64_t batch, int64_t features, int dtype, int bs_last);
+int ksmm_epilogue_backward(const void *dy, const void *z, void *dz, void *dbias, int64_t batch,
+                           int64_t features, int dtype, int bs_last, int act, void *workspace,
+                           int64_t workspace_bytes, void *stream);
+
 /* ksmm_chain_forward_ep for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc): the ping-pong intermediates
  * and the transposed-route and padded-rows buffers live in a fixed device array inside the library,

@@ -916,6 +916,27 @@ int ksmm_factor_backward_weight(const void *dy, const void *x, void *dw, int64_t
     return wgrad_run(dy, x, dw, acc, batch, a, b, c, d, dtype, bs_last ? 1 : 0, scale, (hipStream_t)stream);
 }
 
+int64_t ksmm_epilogue_backward_workspace(int64_t batch, int64_t features, int dtype, int bs_last)
+{
+    if (features < 1) return KSMM_ERR_BAD_PATTERN;
+    if (batch < 1) return KSMM_ERR_BAD_BATCH;
+    if (dtype != KSMM_F32 && dtype != KSMM_F16) return KSMM_ERR_BAD_DTYPE;
+    if (batch > 0x7fffffffLL / features) return KSMM_ERR_TOO_LARGE;
+    return align256(4 * act_bwd_partial_floats(batch, features, dtype, bs_last ? 1 : 0));
+}
+
+int ksmm_epilogue_backward(const void *dy, const void *z, void *dz, void *dbias, int64_t batch, int64_t features, int dtype,
+                           int bs_last, int act, void *workspace, int64_t workspace_bytes, void *stream)
+{
+    const int64_t need = ksmm_epilogue_backward_workspace(batch, features, dtype, bs_last);
+    if (need < 0) return (int)need;
+    if (act != KSMM_ACT_NONE && act != KSMM_ACT_GELU) return KSMM_ERR_BAD_EPILOGUE;
+    if (!dy || (act != KSMM_ACT_NONE && (!z || !dz))) return KSMM_ERR_NULL_POINTER;
+    if (dbias && (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15) != 0)) return KSMM_ERR_WORKSPACE;
+    if (!dbias && act == KSMM_ACT_NONE) return KSMM_OK;
+    return act_bwd_run(dy, z, dz, dbias, (float *)workspace, batch, features, dtype, bs_last ? 1 : 0, act, (hipStream_t)stream);
+}
+
 int64_t ksmm_static_scratch_bytes(void) { return KSMM_STATIC_SCRATCH_BYTES; }
 
 int ksmm_chain_forward_static(const ksmm_factor_desc *factors, int n_factors, const void *x, void *y,

@@ -529,14 +529,26 @@ int64_t wgrad_partial_floats(int64_t batch, int a, int b, int c, int d, int dtyp
     return most * n;
 }
 
+// out[i] (type `dtype`, i < n) <- scale * the sum of acc's slices of n floats
+int slices_finish_run(const float *acc, void *out, int64_t n, int splits, int dtype, float scale, hipStream_t stream)
+{
+    const int64_t blocks = (n + 63) / 64;
+    if (blocks > 0x7fffffffLL) return KSMM_ERR_TOO_LARGE;
+    if (dtype == KSMM_F32)
+        hipLaunchKernelGGL((ks_wgrad_finish_kernel<float>), dim3((unsigned)blocks), dim3(256), 0, stream, acc, (float *)out, n,
+                           splits, scale);
+    else
+        hipLaunchKernelGGL((ks_wgrad_finish_kernel<half_t>), dim3((unsigned)blocks), dim3(256), 0, stream, acc, (half_t *)out, n,
+                           splits, scale);
+    return hipGetLastError() == hipSuccess ? KSMM_OK : KSMM_ERR_LAUNCH;
+}
+
 // dw (kernel format, type `dtype`) <- scale * sum over the batch of dY x X^T per block; acc is an
 // fp32 buffer of wgrad_partial_floats() elements.
 int wgrad_run(const void *dy, const void *x, void *dw, float *acc, int64_t batch, int a, int b, int c, int d,
               int dtype, int bs_last, float scale, hipStream_t stream)
 {
     const int64_t n = (int64_t)a * b * c * d;
-    const int64_t fin_blocks = (n + 63) / 64;
-    if (fin_blocks > 0x7fffffffLL) return KSMM_ERR_TOO_LARGE;
     const bool mfma_ok = wgrad_mfma_ok(batch, dtype, bs_last);
     const int t = wgrad_bl_tile(b, c);
     int rc, splits = 1;
@@ -565,13 +577,7 @@ int wgrad_run(const void *dy, const void *x, void *dw, float *acc, int64_t batch
         return KSMM_ERR_BAD_DTYPE;
     }
     if (rc != KSMM_OK) return rc;
-    if (dtype == KSMM_F32)
-        hipLaunchKernelGGL((ks_wgrad_finish_kernel<float>), dim3((unsigned)fin_blocks), dim3(256), 0, stream, acc,
-                           (float *)dw, n, splits, scale);
-    else
-        hipLaunchKernelGGL((ks_wgrad_finish_kernel<half_t>), dim3((unsigned)fin_blocks), dim3(256), 0, stream, acc,
-                           (half_t *)dw, n, splits, scale);
-    return hipGetLastError() == hipSuccess ? KSMM_OK : KSMM_ERR_LAUNCH;
+    return slices_finish_run(acc, dw, n, splits, dtype, scale, stream);
 }
 
 }  // namespace ksmm

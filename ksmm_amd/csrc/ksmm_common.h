@@ -201,6 +201,11 @@ bool wgrad_bf_ok(int a, int b, int c, int d, int dtype);
 int64_t wgrad_bf_partial_floats(int64_t batch, int a, int b, int c, int d, int dtype);
 int wgrad_bf_run(const void *dy, const void *x, void *dw, float *acc, int64_t batch, int a, int b, int c, int d, int dtype,
                  float scale, hipStream_t stream, int *splits);
+int slices_finish_run(const float *acc, void *out, int64_t n, int splits, int dtype, float scale, hipStream_t stream);
+// Backward pass of the epilogue (ksmm_act_bwd.hip; acc: fp32 scratch of act_bwd_partial_floats() elements)
+int64_t act_bwd_partial_floats(int64_t batch, int64_t features, int dtype, int bs_last);
+int act_bwd_run(const void *dy, const void *z, void *dz, void *dbias, float *acc, int64_t batch, int64_t features, int dtype,
+                int bs_last, int act, hipStream_t stream);
 
 // Fused radix-16 chain (intermediates in LDS); KSMM_ERR_BAD_ALGO when the chain does not qualify.
 // out (cols x rows) = transpose of in (rows x cols); pitches in elements per row, 0 = dense

@@ -9,6 +9,8 @@ with raw device pointers on the current PyTorch stream.
 import ctypes
 
 import torch
+import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -160,6 +162,35 @@ class Kernel:
         return grad_input, grad_factor
 
     @staticmethod
+    def epilogue_backward(grad_output, z, bs_last, act=None, need_bias=True):
+        """(grad_z, grad_bias) of ``y = act(z)``, ``z = K x + bias``, for fp32 / fp16 tensors of y's
+        layout; ``grad_bias`` holds one value per feature (None unless ``need_bias``).  Without an
+        activation grad_z is grad_output itself and ``z`` is not read."""
+        lib = _lib.load()
+        code = _ACTS[act]
+        _check_input(grad_output, "grad_output")
+        features, batch = grad_output.shape if bs_last else reversed(grad_output.shape)
+        grad_z = grad_output
+        if code != _lib.ACT_NONE:
+            _check_input(z, "z")
+            assert z.shape == grad_output.shape and z.dtype == grad_output.dtype
+            grad_z = torch.empty_like(z)
+        dt = dtype_code(grad_output.dtype)
+        need = lib.ksmm_epilogue_backward_workspace(batch, features, dt, int(bs_last))
+        if need < 0:
+            _lib.check(int(need))
+        grad_bias = workspace = None
+        if need_bias:
+            grad_bias = torch.empty(features, dtype=grad_output.dtype, device=grad_output.device)
+            workspace = torch.empty(need, dtype=torch.uint8, device=grad_output.device)
+        with torch.cuda.device(grad_output.device):
+            _lib.check(lib.ksmm_epilogue_backward(
+                grad_output.data_ptr(), z.data_ptr() if z is not None else None, grad_z.data_ptr(),
+                grad_bias.data_ptr() if need_bias else None, batch, features, dt, int(bs_last), code,
+                workspace.data_ptr() if need_bias else None, need if need_bias else 0, _stream_ptr(grad_output)))
+        return grad_z, grad_bias
+
+    @staticmethod
     def chain_forward(input, factors, patterns, bs_last, scales=None, fuse=True, workspace=None,
                       bias=None, act=None, static_scratch=False, out=None):
         """All factors of a KSLinear in one call (factor-chain launcher).  ``bias``/``act`` are
@@ -233,6 +264,68 @@ class KSFactorFunction(torch.autograd.Function):
         gi, gf = Kernel.backward(grad_output.contiguous(), input, factor, ctx.bs_last, *ctx.pattern,
                                  need_input=ctx.needs_input_grad[0], need_weight=ctx.needs_input_grad[1])
         return gi, gf, None, None
+
+
+def layer_by_factors(x, bias, act, bs_last, patterns, factors):
+    """act(K_n .. K_1 x + bias) with an autograd node per factor; bias and activation are PyTorch's."""
+    for f, p in zip(factors, patterns):
+        x = KSFactorFunction.apply(x, f, bs_last, p)
+    if bias is not None:
+        x = x + bias
+    return F.gelu(x) if act == "gelu" else x
+
+
+class KSLayerFunction(torch.autograd.Function):
+    """A layer with a backward pass: ``apply(x, bias, act, bs_last, patterns, *factors)``.
+
+    Against ``layer_by_factors`` it adds the bias in the last factor's kernel and takes the gradients
+    of activation and bias in one pass.  Per tensor of the result that is two reads and two writes less."""
+
+    @staticmethod
+    def takes(x, bias, patterns, bs_last):
+        """Whether ``bias`` is what the kernels add: one value of the result's type per feature.  Forward-mode
+        gradients go through PyTorch's own addition and activation."""
+        if forward_ad._current_level >= 0:
+            return False
+        a, b, _, d = patterns[-1]
+        n = a * b * d
+        return bias is None or (bias.dtype == x.dtype and bias.device == x.device and bias.is_contiguous()
+                                and tuple(bias.shape) == ((n, 1) if bs_last else (n,)))
+
+    @staticmethod
+    def forward(ctx, x, bias, act, bs_last, patterns, *factors):
+        ctx.act, ctx.bs_last, ctx.patterns = act, bs_last, patterns
+        inputs, last = [x], len(factors) - 1
+        for i, (f, p) in enumerate(zip(factors, patterns)):
+            inputs.append(Kernel.forward(inputs[-1], f, bs_last, *p, bias=bias if i == last else None))
+        z = inputs.pop()
+        ctx.save_for_backward(bias, *factors, *inputs, z if act else None)
+        return F.gelu(z) if act else z
+
+    @staticmethod
+    def backward(ctx, grad_output):
+        n, bs_last = len(ctx.patterns), ctx.bs_last
+        saved = ctx.saved_tensors
+        bias, factors, inputs, z = saved[0], saved[1:n + 1], saved[n + 1:-1], saved[-1]
+        need_x, need_bias = ctx.needs_input_grad[:2]
+        need_factors = ctx.needs_input_grad[5:]
+        if torch.is_grad_enabled() and (ctx.act or bias is not None):  # create_graph: what can be differentiated again is
+            args = [t for t, need in zip((inputs[0], bias) + factors, (need_x, need_bias) + need_factors) if need]
+            y = layer_by_factors(inputs[0], bias, ctx.act, bs_last, ctx.patterns, factors)
+            grads = iter(torch.autograd.grad(y, args, grad_output, create_graph=True))
+            gx, gb, *gf = [next(grads) if need else None for need in (need_x, need_bias) + need_factors]
+            return (gx, gb, None, None, None, *gf)
+        grad = grad_output.contiguous()
+        grad_bias, grad_factors = None, [None] * n
+        if ctx.act or need_bias:
+            grad, grad_bias = Kernel.epilogue_backward(grad, z, bs_last, ctx.act, need_bias)
+            grad_bias = grad_bias.view_as(bias) if need_bias else None
+        for i in reversed(range(n)):
+            need_input = need_x or any(need_factors[:i])
+            if need_input or need_factors[i]:
+                grad, grad_factors[i] = Kernel.backward(grad, inputs[i], factors[i], bs_last, *ctx.patterns[i],
+                                                        need_input=need_input, need_weight=need_factors[i])
+        return (grad if need_x else None, grad_bias, None, None, None, *grad_factors)
 
 
 def query_tile(batch, pattern, x_dtype, w_dtype=None, bs_last=True, algo=_lib.ALGO_AUTO, variant=-1):

@@ -111,8 +111,9 @@ class KSLinear(nn.Module):
     the whole layer is one call of the chain launcher: intermediates in a workspace or in LDS,
     bias and activation inside the last factor's kernel.  With gradients enabled and trainable
     factors (the state of a freshly built layer, ``eval()`` included) it runs factor by factor
-    through an autograd function that keeps the intermediates for the backward pass, and bias
-    and activation are PyTorch operations; both modes compute the same function.
+    inside an autograd function that keeps the intermediates for the backward pass; the bias is
+    added in the last factor's kernel and the activation is a PyTorch operation; both modes
+    compute the same function.
 
     Beyond the reference's signature: ``fuse`` lets the chain launcher keep intermediates in
     LDS where it has a kernel for the chain, and ``act='gelu'`` applies GELU (erf form) after
@@ -187,16 +188,13 @@ class KSLinear(nn.Module):
 
         if torch.is_grad_enabled() and self.dtype != FP8 and (
                 x.requires_grad or any(f.requires_grad for f in self.factors)):
-            # training: factor by factor through the autograd function (intermediates are kept for
-            # the weight gradients); bias and activation stay PyTorch ops so that autograd sees them
-            from .kernel import KSFactorFunction
+            # training: intermediates are kept for the weight gradients
+            from .kernel import KSLayerFunction, layer_by_factors
 
-            out = x
-            for f, p in zip(self.factors, self.patterns):
-                out = KSFactorFunction.apply(out, f, self.bs_last, p)
-            if self.bias is not None:
-                out = out + self.bias
-            return F.gelu(out) if self.act == "gelu" else out
+            args = x, self.bias, self.act, self.bs_last, self.patterns
+            if KSLayerFunction.takes(x, self.bias, self.patterns, self.bs_last):
+                return KSLayerFunction.apply(*args, *self.factors)
+            return layer_by_factors(*args, self.factors)
         scales = list(self.w_scales)
         if self.dtype == FP8:
             if x.dtype != FP8:

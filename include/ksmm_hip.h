@@ -252,6 +252,17 @@ int ksmm_factor_backward_weight(const void *dy, const void *x, void *dw, int64_t
                                 int c, int d, int dtype, int bs_last, float scale, void *workspace,
                                 int64_t workspace_bytes, void *stream);
 
+/* ksmm_chain_forward_ep on an fp32 or fp16 input that the call quantises to e4m3 itself: one scale for
+ * the tensor (largest magnitude / 448, or 1 where that is 0 or NaN), codes rounded to nearest even.
+ * The scale stays on the device and multiplies the first factor's, whose weights must be e4m3.
+ * Needs ksmm_chain_quant_workspace() bytes of 16-byte aligned device memory. */
+int64_t ksmm_chain_quant_workspace(const ksmm_factor_desc *factors, int n_factors, int64_t batch,
+                                   int x_dtype, int y_dtype, int bs_last);
+int ksmm_chain_forward_quant(const ksmm_factor_desc *factors, int n_factors, const void *x, void *y,
+                             void *workspace, int64_t workspace_bytes, int64_t batch, int x_dtype,
+                             int y_dtype, int bs_last, int fuse, const ksmm_epilogue *epilogue,
+                             void *stream);
+
 /* Backward pass of an epilogue y = act(z), z = K x + bias (fp32 and fp16):
  *   dz = dy * act'(z)   (dy, z, dz: y's shape and layout; with KSMM_ACT_NONE dz is dy: z and dz are
  *                       not touched and may be NULL),

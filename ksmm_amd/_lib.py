@@ -75,6 +75,9 @@ SIGNATURES = {
                                            ctypes.c_float, c_vp, c_i64, c_vp]),
     "ksmm_factor_backward_weight": (c_int, [c_vp, c_vp, c_vp, c_i64, c_int, c_int, c_int, c_int, c_int, c_int,
                                             ctypes.c_float, c_vp, c_i64, c_vp]),
+    "ksmm_chain_quant_workspace": (c_i64, [ctypes.POINTER(KsmmFactorDesc), c_int, c_i64, c_int, c_int, c_int]),
+    "ksmm_chain_forward_quant": (c_int, [ctypes.POINTER(KsmmFactorDesc), c_int, c_vp, c_vp, c_vp, c_i64, c_i64, c_int, c_int,
+                                         c_int, c_int, ctypes.POINTER(KsmmEpilogue), c_vp]),
     "ksmm_epilogue_backward_workspace": (c_i64, [c_i64, c_i64, c_int, c_int]),
     "ksmm_epilogue_backward": (c_int, [c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_int, c_int, c_int, c_vp, c_i64, c_vp]),
     "ksmm_static_scratch_bytes": (c_i64, []),

@@ -391,7 +391,7 @@ int check_epilogue(const ksmm_epilogue *ep)
 
 int factor_forward_impl(const void *x, const void *w, void *y, int64_t batch, int a, int b, int c, int d,
                         int x_dtype, int w_dtype, int y_dtype, int bs_last, float scale, int algo, int variant,
-                        const ksmm_epilogue *ep, void *stream)
+                        const ksmm_epilogue *ep, void *stream, const float *x_scale = nullptr)
 {
     int rc = check_shape(batch, a, b, c, d, x_dtype, w_dtype, y_dtype);
     if (rc != KSMM_OK) return rc;
@@ -406,6 +406,7 @@ int factor_forward_impl(const void *x, const void *w, void *y, int64_t batch, in
         p.bias = ep->bias;
         p.act = ep->act;
     }
+    p.x_scale = x_scale;
     // Every kernel but the split-K and the one-thread-per-output ones moves aligned 16-byte vectors:
     // tensors that do not start on a 16-byte boundary run on those (a forced family refuses them).
     if ((((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)p.bias) & 15) != 0) {
@@ -558,10 +559,11 @@ bool chain_route_pays(const ksmm_factor_desc *f, int n, int64_t batch, int x_dty
 }
 
 // The chain launcher behind ksmm_chain_forward, ksmm_chain_forward_ep and
-// ksmm_chain_forward_static: `ep` (may be null) belongs to the last factor.
+// ksmm_chain_forward_static: `ep` (may be null) belongs to the last factor, `x_scale` (device
+// memory, may be null) multiplies the first one's scale.
 int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const void *x, void *y, void *workspace,
                        int64_t workspace_bytes, int64_t batch, int x_dtype, int y_dtype, int bs_last, int fuse,
-                       const ksmm_epilogue *ep, void *stream)
+                       const ksmm_epilogue *ep, void *stream, const float *x_scale = nullptr)
 {
     int rc = check_chain(factors, n_factors, batch, x_dtype, y_dtype);
     if (rc != KSMM_OK) return rc;
@@ -586,7 +588,7 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
     auto run_bs_last = [&](const void *x0, char *pp, int64_t one, int64_t nb, const void **result) -> int {
         int rc2 = KSMM_ERR_BAD_ALGO;
         if (fuse && fused_pays(factors, n_factors, nb, x_dtype, y_dtype))
-            rc2 = chain16_run(factors, n_factors, x0, pp, nb, x_dtype, y_dtype, 1, true, (hipStream_t)stream, ep);
+            rc2 = chain16_run(factors, n_factors, x0, pp, nb, x_dtype, y_dtype, 1, true, (hipStream_t)stream, ep, x_scale);
         if (rc2 == KSMM_OK) {
             *result = pp;
             return KSMM_OK;
@@ -598,7 +600,7 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
             void *dst = pp + (i & 1) * one;
             rc2 = factor_forward_impl(cur, factors[i].w, dst, nb, factors[i].a, factors[i].b, factors[i].c,
                                       factors[i].d, cur_dtype, factors[i].w_dtype, y_dtype, 1, factors[i].scale,
-                                      KSMM_ALGO_AUTO, -1, ep_of(i), stream);
+                                      KSMM_ALGO_AUTO, -1, ep_of(i), stream, i == 0 ? x_scale : nullptr);
             if (rc2 != KSMM_OK) return rc2;
             cur = dst;
             cur_dtype = y_dtype;
@@ -643,7 +645,7 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
     if (fuse && (!bs_last || fused_pays(factors, n_factors, batch, x_dtype, y_dtype))) {
         // chains whose intermediates fit LDS run as one kernel (no workspace traffic)
         rc = chain16_run(factors, n_factors, x, y, batch, x_dtype, y_dtype, bs_last ? 1 : 0, true,
-                         (hipStream_t)stream, ep);
+                         (hipStream_t)stream, ep, x_scale);
         if (rc != KSMM_ERR_BAD_ALGO) return rc;
     }
     const int64_t need = ksmm_chain_workspace(factors, n_factors, batch, y_dtype);
@@ -655,7 +657,7 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
         void *dst = (i == n_factors - 1) ? y : (void *)buf[i & 1];
         rc = factor_forward_impl(cur, factors[i].w, dst, batch, factors[i].a, factors[i].b, factors[i].c,
                                  factors[i].d, cur_dtype, factors[i].w_dtype, y_dtype, bs_last, factors[i].scale,
-                                 KSMM_ALGO_AUTO, -1, ep_of(i), stream);
+                                 KSMM_ALGO_AUTO, -1, ep_of(i), stream, i == 0 ? x_scale : nullptr);
         if (rc != KSMM_OK) return rc;
         cur = dst;
         cur_dtype = y_dtype;
@@ -870,6 +872,50 @@ int ksmm_chain_forward_ep(const ksmm_factor_desc *factors, int n_factors, const 
 {
     return chain_forward_impl(factors, n_factors, x, y, workspace, workspace_bytes, batch, x_dtype, y_dtype,
                               bs_last, fuse, epilogue, stream);
+}
+
+// workspace of the chain that quantises its input: codes | partial maxima | scale | the chain's own
+static int64_t quant_layout(const ksmm_factor_desc *f, int64_t batch, int64_t *maxima)
+{
+    *maxima = align256((int64_t)f[0].a * f[0].c * f[0].d * batch);
+    return *maxima + align256(quantize_scratch_bytes()) + 256;
+}
+
+int64_t ksmm_chain_quant_workspace(const ksmm_factor_desc *factors, int n_factors, int64_t batch, int x_dtype, int y_dtype,
+                                   int bs_last)
+{
+    if (x_dtype != KSMM_F32 && x_dtype != KSMM_F16) return KSMM_ERR_BAD_DTYPE;
+    const int64_t chain = ksmm_chain_workspace_layout(factors, n_factors, batch, KSMM_FP8_E4M3, y_dtype, bs_last);
+    if (chain < 0) return chain;
+    int64_t maxima;
+    return quant_layout(factors, batch, &maxima) + chain;
+}
+
+int ksmm_chain_forward_quant(const ksmm_factor_desc *factors, int n_factors, const void *x, void *y, void *workspace,
+                             int64_t workspace_bytes, int64_t batch, int x_dtype, int y_dtype, int bs_last, int fuse,
+                             const ksmm_epilogue *epilogue, void *stream)
+{
+    const int64_t need = ksmm_chain_quant_workspace(factors, n_factors, batch, x_dtype, y_dtype, bs_last);
+    if (need < 0) return (int)need;
+    int rc = check_epilogue(epilogue);
+    if (rc != KSMM_OK) return rc;
+    if (!x || !y) return KSMM_ERR_NULL_POINTER;
+    for (int i = 0; i < n_factors; ++i)
+        if (!factors[i].w) return KSMM_ERR_NULL_POINTER;
+    if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15) != 0) return KSMM_ERR_WORKSPACE;
+    const ksmm_factor_desc &last = factors[n_factors - 1];
+    const int64_t n = (int64_t)factors[0].a * factors[0].c * factors[0].d * batch, xbytes = n * (int64_t)dtype_size(x_dtype);
+    const int64_t ybytes = (int64_t)last.a * last.b * last.d * batch * (int64_t)dtype_size(y_dtype);
+    if (overlaps(x, xbytes, y, ybytes) || overlaps(workspace, need, x, xbytes) || overlaps(workspace, need, y, ybytes))
+        return KSMM_ERR_ALIAS;
+    int64_t maxima;
+    const int64_t own = quant_layout(factors, batch, &maxima);
+    char *ws = (char *)workspace;
+    float *scale = (float *)(ws + own - 256);
+    rc = quantize_run(x, x_dtype, ws, scale, ws + maxima, n, (hipStream_t)stream);
+    if (rc != KSMM_OK) return rc;
+    return chain_forward_impl(factors, n_factors, ws, y, need > own ? ws + own : nullptr, need - own, batch, KSMM_FP8_E4M3, y_dtype,
+                              bs_last, fuse, epilogue, stream, scale);
 }
 
 int64_t ksmm_factor_backward_workspace(int64_t batch, int a, int b, int c, int d, int dtype, int bs_last)

@@ -37,6 +37,7 @@ struct Chain16Args {
     float scale[4];
     const void *bias;  // of the last factor's outputs (fp16), or none
     int act;
+    const float *x_scale;  // device: factor of scale[0] that only the GPU knows, or none
 };
 
 namespace {
@@ -88,6 +89,8 @@ __global__ __launch_bounds__(CH_THREADS) void ks_chain16_kernel(const TX *__rest
     if (gridDim.x % 16 == 0) c0 = 2 * (8 * (c0 / 16) + c0 % 8) + (c0 / 8) % 2;
     const int c_begin = c0 * CH_TN, c_step = gridDim.x * CH_TN, c_end = batch;
     if (c_begin >= c_end) return;
+    float scale0 = args.scale[0];
+    if (sizeof(TX) == 1 && args.x_scale) scale0 *= *args.x_scale;
     const int c_last = c_begin + ((c_end - 1 - c_begin) / c_step) * c_step;  // this workgroup's last chunk
     const int n_blocks = n_feat / 16;  // blocks per factor
     constexpr int MAXB = 64 / CH_WAVES;  // blocks per wave and factor (n_feat <= 1024)
@@ -208,7 +211,7 @@ __global__ __launch_bounds__(CH_THREADS) void ks_chain16_kernel(const TX *__rest
 #pragma unroll
         for (int f = 0; f < NF; ++f) {
             const int ld = args.log2d[f];
-            const float scale = args.scale[f];
+            const float scale = f == 0 ? scale0 : args.scale[f];
             // first row of block g (scalar) and the A operand of its four sub-tiles
             auto block_row0 = [&](int g) { return ((g >> ld) << (ld + 4)) | (g & ((1 << ld) - 1)); };
             auto read_block = [&](int g, half4_t(&xa)[4]) {
@@ -236,7 +239,7 @@ __global__ __launch_bounds__(CH_THREADS) void ks_chain16_kernel(const TX *__rest
                 const int row0 = block_row0(g);
                 if (f + 1 == NF && (args.bias != nullptr || args.act != KSMM_ACT_NONE)) {
                     // the chain's epilogue: the lane's output row is row0 + r * d
-                    const Epi ep{scale, args.act, args.bias};
+                    const Epi ep{scale, args.act, args.bias, nullptr};
                     const float bv = epi_bias<half_t>(ep, (size_t)(row0 + (r << ld)));
 #pragma unroll
                     for (int s = 0; s < 4; ++s)
@@ -299,7 +302,8 @@ template <typename TX, typename TW> const void *chain16_fn(int nf, bool full)
 
 // Returns KSMM_ERR_BAD_ALGO when the chain is not a radix-16 butterfly this kernel takes.
 int chain16_run(const ksmm_factor_desc *f, int n, const void *x, void *y, int64_t batch, int x_dtype,
-                int y_dtype, int bs_last, bool launch, hipStream_t stream, const ksmm_epilogue *ep)
+                int y_dtype, int bs_last, bool launch, hipStream_t stream, const ksmm_epilogue *ep,
+                const float *x_scale)
 {
     if (!bs_last || n < 2 || n > 4 || y_dtype != KSMM_F16) return KSMM_ERR_BAD_ALGO;
     if (x_dtype != KSMM_FP8_E4M3 && x_dtype != KSMM_F16) return KSMM_ERR_BAD_ALGO;
@@ -338,6 +342,7 @@ int chain16_run(const ksmm_factor_desc *f, int n, const void *x, void *y, int64_
     }
     args.bias = ep ? ep->bias : nullptr;
     args.act = ep ? ep->act : KSMM_ACT_NONE;
+    args.x_scale = x_scale;
     const int lds = (int)n_feat * CH_ROW;
     if (ensure_dynamic_lds(fn, lds) != KSMM_OK) return KSMM_ERR_LAUNCH;
     int batch_i = (int)batch, n_feat_i = (int)n_feat;

@@ -77,16 +77,24 @@ struct Problem {
     hipStream_t stream;
     const void *bias = nullptr;  // one value of y's type per output feature, or none
     int act = KSMM_ACT_NONE;
+    const float *x_scale = nullptr;  // device: scale of an e4m3 input that was quantised on the GPU, or none
 };
 
 // What a kernel does to an fp32 accumulator before rounding it to the output type:
-// v = act(acc * scale + bias[output feature]).  Passed to the kernels by value.
+// v = act(acc * scale + bias[output feature]).  Passed to the kernels by value.  With e4m3 inputs scale
+// may lack a factor that only the GPU knows, *x_scale: kernels on such inputs begin with epi_load().
 struct Epi {
     float scale;
     int act;
     const void *bias;
+    const float *x_scale;
 };
-static inline Epi epi_of(const Problem &p) { return Epi{p.scale, p.act, p.bias}; }
+static inline Epi epi_of(const Problem &p) { return Epi{p.scale, p.act, p.bias, p.x_scale}; }
+template <typename TX> __device__ __forceinline__ void epi_load(Epi &e)
+{
+    if constexpr (sizeof(TX) == 1)
+        if (e.x_scale) e.scale *= *e.x_scale;
+}
 
 // GELU, erf form: x * Phi(x) = max(x, 0) - |x| * erfc(|x| / sqrt 2) / 2.  erfc by Abramowitz &
 // Stegun 7.1.26 (|error| <= 1.5e-7, branch-free: one reciprocal, one exponential, a degree-4
@@ -215,6 +223,10 @@ int transpose_run(const void *in, void *out, int64_t rows, int64_t cols, int ele
 int repitch_run(const void *in, void *out, int64_t rows, int64_t cols_in, int64_t cols_out, int elem_bytes,
                 hipStream_t stream);
 int chain16_run(const ksmm_factor_desc *f, int n, const void *x, void *y, int64_t batch, int x_dtype,
-                int y_dtype, int bs_last, bool launch, hipStream_t stream, const ksmm_epilogue *ep);
+                int y_dtype, int bs_last, bool launch, hipStream_t stream, const ksmm_epilogue *ep,
+                const float *x_scale = nullptr);
+// codes (e4m3fn) and scale of a tensor of n values (ksmm_quant.hip)
+int64_t quantize_scratch_bytes();
+int quantize_run(const void *x, int x_dtype, void *codes, float *scale, void *scratch, int64_t n, hipStream_t stream);
 
 }  // namespace ksmm

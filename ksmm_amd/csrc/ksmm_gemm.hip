@@ -164,6 +164,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void ks_gemm_kernel(const CT *__
                                                               int b, int c, int d, Epi ep,
                                                               int m_tiles, int n_tiles, int blocks, int pf_dist)
 {
+    epi_load<CT>(ep);
     const float scale = ep.scale;
     // bias and activation live in an instantiation of their own: next to the accumulators their
     // registers would push the plain one into scratch memory
@@ -1012,6 +1013,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void ks_gemm_pbl_kernel(const CT
     constexpr int OP = 128 + 16;          // bytes per row of a wave's output piece
     constexpr int OUT_BASE = C::LDS_BYTES;  // the pieces follow the ring
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    epi_load<CT>(ep);
     const float scale = ep.scale;
     // bias and activation live in an instantiation of their own: next to the accumulators their
     // registers would push the plain one into scratch memory

@@ -25,6 +25,7 @@ __global__ __launch_bounds__(256) void ks_generic_kernel(const TX *__restrict__ 
                                                          TY *__restrict__ y, int64_t batch, int a,
                                                          int b, int c, int d, Epi ep)
 {
+    epi_load<TX>(ep);
     const int64_t in_size = (int64_t)a * c * d;
     const int64_t out_size = (int64_t)a * b * d;
     // 1-D grid: blockIdx.x = slow * fast_blocks + fast_block
@@ -102,6 +103,7 @@ __global__ __launch_bounds__(256) void ks_small_bl_kernel(const TX *__restrict__
                                                           TY *__restrict__ y, int64_t batch, int a, int b, int c,
                                                           int d, Epi ep, int n_blocks, int b_chunks)
 {
+    epi_load<TX>(ep);
     constexpr int V = vec16<TX>::N;
     const int bc = blockIdx.x % b_chunks;
     const int rest = blockIdx.x / b_chunks;

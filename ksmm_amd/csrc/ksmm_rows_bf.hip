@@ -249,6 +249,7 @@ __global__ __launch_bounds__(64 * DD * MS) void ks_rows_bf_h_kernel(const TX *__
                                                               half_t *__restrict__ y, int batch, int a, int d,
                                                               Epi ep, int wgs_per_a, int n_tiles)
 {
+    epi_load<TX>(ep);
     typedef RowCfgH<TX, BB, CC, DD, TN, MS> C;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     TX *const xs = (TX *)smem;                         // [2][TN][LDX]

@@ -68,6 +68,7 @@ template <typename TX, typename TW, typename TY, bool LAST, bool RUN, int VM, in
 __global__ __launch_bounds__(64 * split_waves(VM, NT, DD), 2) void ks_split_kernel(
     const TX *__restrict__ x, const TW *__restrict__ w, TY *__restrict__ y, SplitArgs s, Epi ep)
 {
+    epi_load<TX>(ep);
     typedef typename op_type<TX>::type op_t;
     constexpr bool F32 = sizeof(op_t) == 4;
     constexpr int KV = F32 ? 4 : 8, KSTEP = 4 * KV, TM = 16 * VM, TN = 16 * NT, TILES = VM * NT * DD;

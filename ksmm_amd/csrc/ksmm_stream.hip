@@ -140,6 +140,7 @@ __global__ __launch_bounds__(64 * WM * WN) void ks_stream_kernel(const CT *__res
                                                                 TY *__restrict__ y, int batch, int a,
                                                                 int d, Epi ep, int wgs_per_group)
 {
+    epi_load<CT>(ep);
     const float scale = ep.scale;
     const bool has_epi = ep.bias != nullptr || ep.act != KSMM_ACT_NONE;  // uniform
     typedef StreamCfg<CT, TW, BS_LAST, BB, CC, TN, WM, WN, ST> C;

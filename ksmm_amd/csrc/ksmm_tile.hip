@@ -62,6 +62,7 @@ __global__ __launch_bounds__(64 * WM * WN) void ks_tile_kernel(const TX *__restr
                                                               int b, int c, int d, Epi ep,
                                                               int m_tiles, int n_tiles, int blocks)
 {
+    epi_load<TX>(ep);
     typedef TileCfg<CT, TX, TW, TY, BS_LAST, TM, TN, TK, WM, WN> C;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     CT *const lds = (CT *)smem;
@@ -307,6 +308,7 @@ __global__ __launch_bounds__(64 * WM * WN) void ks_ws_kernel(const TX *__restric
                                                             int d, Epi ep, int wgs_per_group,
                                                             int n_tiles)
 {
+    epi_load<TX>(ep);
     typedef WsCfg<CT, TX, TW, TY, BS_LAST, BB, CC, TN, WM, WN> C;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     CT *const lds = (CT *)smem;

@@ -60,6 +60,7 @@ __global__ __launch_bounds__(64 * WM * WN) void ks_tile_bf_kernel(const TX *__re
                                                                  int b, int c, int d, Epi ep,
                                                                  int m_tiles, int n_tiles, int blocks)
 {
+    epi_load<TX>(ep);
     typedef BfCfg<CT, TW, DD, TM, TN, TK, WM, WN, TX> C;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     CT *const lds = (CT *)smem;
@@ -244,6 +245,7 @@ __global__ __launch_bounds__(64 * WM * WN * NG, (WM * WN * NG >= 8 ? 1 : 2)) voi
                                                                 int b, int c, int d, Epi ep,
                                                                 int m_tiles, int n_tiles, int blocks)
 {
+    epi_load<TX>(ep);
     constexpr int DD = 8, DDA = DD * NG, KH = TK / 2, THREADS = 64 * WM * WN * NG;
     constexpr bool FL = NG > 1;  // whole lines: results leave through LDS
     constexpr int NBUF = 2;

@@ -118,33 +118,35 @@ bool read_epilogue(PyObject *bias, PyObject *act, const at::Device &dev, at::Sca
     return true;
 }
 
-// The whole layer without gradients: y = act(scale K_n .. K_1 x + bias), or KSMM error < 0.
+// The whole layer without gradients: y = act(scale K_n .. K_1 x + bias), or KSMM error < 0.  quantise:
+// x goes through e4m3 codes and a scale that the call finds itself.
 int forward(const at::Tensor &x, const Layer &l, int64_t batch, const c10::SmallVector<int64_t, 6> &shape, bool bs_last,
-            bool fuse, const ksmm_epilogue &ep, at::ScalarType out_type, at::Tensor *y)
+            bool fuse, bool quantise, const ksmm_epilogue &ep, at::ScalarType out_type, at::Tensor *y)
 {
     const int xd = code_of(x.scalar_type()), yd = code_of(out_type);
-    const int64_t need = ksmm_chain_workspace_layout(l.f, l.n, batch, xd, yd, bs_last);
+    const int64_t need = quantise ? ksmm_chain_quant_workspace(l.f, l.n, batch, xd, yd, bs_last)
+                                  : ksmm_chain_workspace_layout(l.f, l.n, batch, xd, yd, bs_last);
     if (need < 0) return (int)need;
     *y = at::empty(shape, x.options().dtype(out_type));
     at::Tensor ws;
     if (need > 0) ws = at::empty({need}, x.options().dtype(at::kByte));
-    return ksmm_chain_forward_ep(l.f, l.n, x.const_data_ptr(), y->mutable_data_ptr(), need > 0 ? ws.mutable_data_ptr() : nullptr,
-                                 need, batch, xd, yd, bs_last, fuse, ep.bias || ep.act ? &ep : nullptr,
-                                 c10::hip::getCurrentHIPStream(x.device().index()).stream());
+    const auto run = quantise ? ksmm_chain_forward_quant : ksmm_chain_forward_ep;
+    return run(l.f, l.n, x.const_data_ptr(), y->mutable_data_ptr(), need > 0 ? ws.mutable_data_ptr() : nullptr, need, batch, xd, yd,
+               bs_last, fuse, ep.bias || ep.act ? &ep : nullptr, c10::hip::getCurrentHIPStream(x.device().index()).stream());
 }
 
-// infer(x, factors, patterns, bs_last, scales, fuse, bias, act) -> y or None
+// infer(x, factors, patterns, bs_last, scales, fuse, bias, act, quantise) -> y or None
 PyObject *py_infer(PyObject *, PyObject *const *args, Py_ssize_t n)
 {
-    if (n != 8) {
-        PyErr_SetString(PyExc_TypeError, "infer() takes 8 arguments");
+    if (n != 9) {
+        PyErr_SetString(PyExc_TypeError, "infer() takes 9 arguments");
         return nullptr;
     }
     try {
         if (!THPVariable_Check(args[0])) Py_RETURN_NONE;
         const at::Tensor &x = THPVariable_Unpack(args[0]);
         if (!x.is_cuda()) Py_RETURN_NONE;
-        const bool bs_last = args[3] == Py_True, fuse = args[5] == Py_True;
+        const bool bs_last = args[3] == Py_True, fuse = args[5] == Py_True, quantise = args[8] == Py_True;
         Layer l;
         int64_t batch;
         c10::SmallVector<int64_t, 6> shape;
@@ -157,7 +159,7 @@ PyObject *py_infer(PyObject *, PyObject *const *args, Py_ssize_t n)
             if (read_epilogue(args[6], args[7], x.device(), out, l.out_size, &ep)) {
                 DeviceScope scope(x.device().index());
                 at::Tensor y;
-                if (forward(x, l, batch, shape, bs_last, fuse, ep, out, &y) == KSMM_OK) return THPVariable_Wrap(std::move(y));
+                if (forward(x, l, batch, shape, bs_last, fuse, quantise, ep, out, &y) == KSMM_OK) return THPVariable_Wrap(std::move(y));
             }
         }
         PyErr_Clear();

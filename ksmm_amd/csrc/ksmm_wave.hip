@@ -529,6 +529,7 @@ __global__ __launch_bounds__(256, OCC) void ks_wave_bl_h(const TX *__restrict__ 
                                                    half_t *__restrict__ y, int batch, int a, int b,
                                                    int c, int d, Epi ep, int n_slabs, int iters, int rr)
 {
+    epi_load<TX>(ep);
     const float scale = ep.scale;
     constexpr int TN = 16 * VEC, KSTEP = 4 * KL;
     typedef typename hvec<KL>::type frag_t;

@@ -243,13 +243,11 @@ class KSLinear(nn.Module):
                 tensor.requires_grad or any(f.requires_grad for f in factors)):
             return None
         scales = self.w_scales
-        if self.dtype == FP8:
-            if tensor.dtype != FP8:
-                return None
-            if x_scale is not None:
-                scales = [scales[0] * float(x_scale)] + scales[1:]
+        quantise = self.dtype == FP8 and tensor.dtype != FP8
+        if self.dtype == FP8 and not quantise and x_scale is not None:
+            scales = [scales[0] * float(x_scale)] + scales[1:]
         return _lib.native().infer(tensor, factors, self.patterns, self.bs_last, scales, self.fuse,
-                                   self._parameters["bias"], self.act)
+                                   self._parameters["bias"], self.act, quantise)
 
     def forward(self, tensor, x_scale=None):
         if self.algo == "kernel":

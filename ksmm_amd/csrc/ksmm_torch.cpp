@@ -6,7 +6,8 @@
 // remembered between calls: pointers, sizes and types are read from the tensors each time.
 //
 // Every entry returns None when it does not take a call (an unusual argument, an error of the
-// library): the caller then goes through ksmm_amd/kernel.py, which raises what is wrong with it.
+// library, no memory): the caller then goes through ksmm_amd/kernel.py, which raises what is wrong
+// with it.  The GIL is released from the first allocation on: both that and a launch can wait.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -44,6 +45,11 @@ struct DeviceScope {
     {
         if (before >= 0) c10::hip::set_device(before);
     }
+};
+
+struct WithoutGil {
+    PyThreadState *state = PyEval_SaveThread();
+    ~WithoutGil() { PyEval_RestoreThread(state); }
 };
 
 struct Layer {
@@ -146,7 +152,7 @@ PyObject *py_infer(PyObject *, PyObject *const *args, Py_ssize_t n)
         if (!THPVariable_Check(args[0])) Py_RETURN_NONE;
         const at::Tensor &x = THPVariable_Unpack(args[0]);
         if (!x.is_cuda()) Py_RETURN_NONE;
-        const bool bs_last = args[3] == Py_True, fuse = args[5] == Py_True, quantise = args[8] == Py_True;
+        const bool bs_last = PyObject_IsTrue(args[3]) == 1, fuse = PyObject_IsTrue(args[5]) == 1, quantise = PyObject_IsTrue(args[8]) == 1;
         Layer l;
         int64_t batch;
         c10::SmallVector<int64_t, 6> shape;
@@ -157,17 +163,20 @@ PyObject *py_infer(PyObject *, PyObject *const *args, Py_ssize_t n)
             for (int i = 0; i < l.n; ++i) fp8 |= l.f[i].w_dtype == KSMM_FP8_E4M3;
             const at::ScalarType out = fp8 ? at::kHalf : x.scalar_type();
             if (read_epilogue(args[6], args[7], x.device(), out, l.out_size, &ep)) {
-                DeviceScope scope(x.device().index());
                 at::Tensor y;
-                if (forward(x, l, batch, shape, bs_last, fuse, quantise, ep, out, &y) == KSMM_OK) return THPVariable_Wrap(std::move(y));
+                int status;
+                {
+                    WithoutGil released;
+                    DeviceScope scope(x.device().index());
+                    status = forward(x, l, batch, shape, bs_last, fuse, quantise, ep, out, &y);
+                }
+                if (status == KSMM_OK) return THPVariable_Wrap(std::move(y));
             }
         }
-        PyErr_Clear();
-        Py_RETURN_NONE;
-    } catch (const std::exception &e) {
-        if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
-        return nullptr;
+    } catch (const std::exception &) {
     }
+    PyErr_Clear();
+    Py_RETURN_NONE;
 }
 
 PyMethodDef methods[] = {

@@ -247,7 +247,7 @@ class KSLinear(nn.Module):
         if self.dtype == FP8 and not quantise and x_scale is not None:
             scales = [scales[0] * float(x_scale)] + scales[1:]
         return _lib.native().infer(tensor, factors, self.patterns, self.bs_last, scales, self.fuse,
-                                   self._parameters["bias"], self.act, quantise)
+                                   self.bias, self.act, quantise)
 
     def forward(self, tensor, x_scale=None):
         if self.algo == "kernel":

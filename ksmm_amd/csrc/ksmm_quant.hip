@@ -5,12 +5,13 @@
 // Two passes over the input.  What bounds them: HBM (or the cache that the layer before left the input in),
 // 2 + 2 + 1 bytes a value in fp16.  The same steps as tensor operations (to fp32, abs, max, compare, select,
 // divide, to e4m3) move about 40 bytes a value, and reading the scale on the host waits for them: a ViT-B
-// feed-forward block on 6304 rows took 324 us with them and takes 115, 34 of them here (6304 x 3072 fp16:
-// 8 us for the maximum, 15 for the codes; 6304 x 768: 4 and 6).
+// feed-forward block on 6304 rows took 324 us with them and takes 111, 30 of them here (6304 x 3072 fp16:
+// 8 us for the maximum, 12.8 for the codes, 15 when they divided; 6304 x 768: 2.5 and 5.3).  Fewer workgroups with
+// the loads ahead of the scale's reduction: the same time.
 //
 // Bit for bit what those operations give on this GPU: amax is the largest magnitude as an integer (a NaN is
 // above infinity and stays), the division by 448 is the product with its rounded reciprocal, values are
-// divided, and what rounds beyond 448 (scales that under- or overflowed, NaN) is the NaN code.
+// divided (or given the quotient's bits by residuals), and what rounds beyond 448 (scales that under- or overflowed, NaN) is the NaN code.
 #include "ksmm_common.h"
 
 namespace ksmm {
@@ -94,6 +95,17 @@ __device__ __forceinline__ uint32_t quant_code(float t, float scale)
     return fabsf(v) <= 464.f ? code : ((__builtin_bit_cast(uint32_t, v) >> 24) & 0x80u) | 0x7fu;
 }
 
+// t / scale correctly rounded, for r = 1 / scale correctly rounded: the first residual brings the quotient
+// within one unit in the last place, the second to the nearest (Markstein's theorem; both residuals are exact
+// in an fma).  The sign is t's, which a residual of zero would lose for t = -0.
+__device__ __forceinline__ float quotient(float t, float scale, float r)
+{
+    float q = t * r;
+    q = fmaf(fmaf(-q, scale, t), r, q);
+    q = fmaf(fmaf(-q, scale, t), r, q);
+    return copysignf(q, t);
+}
+
 template <typename T, bool ALIGNED>
 __global__ __launch_bounds__(256) void ks_quant_kernel(const T *__restrict__ x, uint8_t *__restrict__ q,
                                                        const uint32_t *__restrict__ part, int parts, float *__restrict__ scale_out,
@@ -108,15 +120,29 @@ __global__ __launch_bounds__(256) void ks_quant_kernel(const T *__restrict__ x, 
     const int64_t stride = (int64_t)gridDim.x * 256, me = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (me == 0) *scale_out = scale;
     const int64_t runs = ALIGNED ? n / RUN : 0;
+    // A division is ten instructions, a quarter-rate one among them, and bounded the codes.  For ordinary scales
+    // seven do: every quotient that is not rounded to zero has residuals above the subnormals, and none is
+    // beyond 448 by more than its rounding, so nothing is tested.  0, infinite and NaN maxima divide.
+    const bool ordinary = amax > 0.f && scale >= 0x1p-60f && scale <= 0x1p60f;
+    const float r = 1.0f / scale;
     for (int64_t i = me; i < runs; i += stride) {
         uint4_t v[LOADS];
 #pragma unroll
         for (int l = 0; l < LOADS; ++l) v[l] = ((const uint4_t *)x)[i * LOADS + l];
         uint4_t o = {0u, 0u, 0u, 0u};
+        if (ordinary) {
 #pragma unroll
-        for (int e = 0; e < RUN; ++e) {
-            const T *t = (const T *)&v[e / N];
-            o[e / 4] |= quant_code((float)t[e % N], scale) << (8 * (e % 4));
+            for (int e = 0; e < RUN; e += 4) {
+                const T *t = (const T *)&v[e / N] + e % N;
+                const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(quotient((float)t[0], scale, r), quotient((float)t[1], scale, r), 0, false);
+                o[e / 4] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(quotient((float)t[2], scale, r), quotient((float)t[3], scale, r), lo, true);
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < RUN; ++e) {
+                const T *t = (const T *)&v[e / N];
+                o[e / 4] |= quant_code((float)t[e % N], scale) << (8 * (e % 4));
+            }
         }
         ((uint4_t *)q)[i] = o;
     }

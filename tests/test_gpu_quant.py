@@ -69,3 +69,22 @@ def test_quantising_layers_replay_in_a_graph():
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(y, layers[1](layers[0](x))), k
+
+
+@pytest.mark.parametrize("dt,exponents", [(torch.float16, range(-22, 15, 4)), (torch.float32, (-120, -53, -52, -51, -20, 0, 33, 67, 68, 69, 120))])
+def test_scales_with_and_without_a_division(dt, exponents):
+    """Scales from 2^-60 to 2^60 take the quotient by residuals, others divide: the same bits."""
+    from ksmm_amd import KSLinear, quantize_fp8
+
+    gen = torch.Generator(device="cuda").manual_seed(12)
+    w = torch.eye(128).reshape(1, 128, 128, 1)
+    with torch.no_grad():
+        layer = KSLinear([(1, 128, 128, 1)], weights=[w], bias=False, algo="kernel", dtype=FP8, device="cuda")
+        for e in exponents:
+            x = torch.rand(512, 128, generator=gen, device="cuda") * 2 - 1
+            x[::2] *= torch.exp2(-20 * torch.rand(256, 128, generator=gen, device="cuda"))
+            x = (x * 2.0 ** e).to(dt)
+            codes, scale = quantize_fp8(x)
+            layer.w_scales[0] = 2.0 ** -e  # fp16 results in range
+            got, want = layer(x), layer(codes, x_scale=float(scale))
+            assert torch.equal(got.nan_to_num(), want.nan_to_num()), (dt, e)

@@ -20,6 +20,7 @@ from . import _lib
 ALGOS = ("dense", "einsum", "kernel", "bmm")
 FP8 = torch.float8_e4m3fn
 FP8_MAX = 448.0
+_KEYS = tuple(str(i) for i in range(_lib.MAX_FACTORS))  # of a ParameterList's entries
 
 
 def quantize_fp8(t):
@@ -236,9 +237,19 @@ class KSLinear(nn.Module):
                 output = output.reshape(a * b * d, *lead)
         return output
 
+    def _factor_list(self):
+        """The factors in the order they are applied in.  The parameters of the list in the order they were
+        registered in are the same thing, without a look-up by index each (1 us a factor), only where every
+        entry is a parameter and none came back later: pruning and parametrisations replace entries by what
+        they compute, and leave their parameter at the end."""
+        factors = self.factors
+        if type(factors) is nn.ParameterList and tuple(factors._parameters) == _KEYS[:len(factors)]:
+            return list(factors._parameters.values())
+        return list(factors)
+
     def _infer(self, tensor, x_scale):
         """The layer in one native call, or None where gradients are wanted or the call is unusual."""
-        factors = list(self.factors._parameters.values())
+        factors = self._factor_list()
         if torch.is_grad_enabled() and self.dtype != FP8 and (
                 tensor.requires_grad or any(f.requires_grad for f in factors)):
             return None

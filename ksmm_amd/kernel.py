@@ -276,7 +276,8 @@ def layer_by_factors(x, bias, act, bs_last, patterns, factors):
 
 
 class KSLayerFunction(torch.autograd.Function):
-    """A layer with a backward pass: ``apply(x, bias, act, bs_last, patterns, *factors)``.
+    """A layer with a backward pass: ``apply(x, bias, act, bs_last, patterns, *factors)`` is the result,
+    with an activation (result, what the activation was applied to).
 
     Against ``layer_by_factors`` it adds the bias in the last factor's kernel and takes the gradients
     of activation and bias in one pass.  Per tensor of the result that is two reads and two writes less."""
@@ -295,30 +296,37 @@ class KSLayerFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, bias, act, bs_last, patterns, *factors):
         ctx.act, ctx.bs_last, ctx.patterns = act, bs_last, patterns
+        ctx.set_materialize_grads(False)
         inputs, last = [x], len(factors) - 1
         for i, (f, p) in enumerate(zip(factors, patterns)):
             inputs.append(Kernel.forward(inputs[-1], f, bs_last, *p, bias=bias if i == last else None))
         z = inputs.pop()
         ctx.save_for_backward(bias, *factors, *inputs, z if act else None)
-        return F.gelu(z) if act else z
+        return (F.gelu(z), z) if act else z
 
     @staticmethod
-    def backward(ctx, grad_output):
-        n, bs_last = len(ctx.patterns), ctx.bs_last
+    def backward(ctx, grad_y, grad_z=None):
+        n, bs_last, act = len(ctx.patterns), ctx.bs_last, ctx.act
         saved = ctx.saved_tensors
         bias, factors, inputs, z = saved[0], saved[1:n + 1], saved[n + 1:-1], saved[-1]
         need_x, need_bias = ctx.needs_input_grad[:2]
         need_factors = ctx.needs_input_grad[5:]
-        if torch.is_grad_enabled() and (ctx.act or bias is not None):  # create_graph: what can be differentiated again is
-            args = [t for t, need in zip((inputs[0], bias) + factors, (need_x, need_bias) + need_factors) if need]
-            y = layer_by_factors(inputs[0], bias, ctx.act, bs_last, ctx.patterns, factors)
-            grads = iter(torch.autograd.grad(y, args, grad_output, create_graph=True))
-            gx, gb, *gf = [next(grads) if need else None for need in (need_x, need_bias) + need_factors]
-            return (gx, gb, None, None, None, *gf)
-        grad = grad_output.contiguous()
+        again = torch.is_grad_enabled()  # create_graph: the epilogue in operations that can be differentiated
+        grad = grad_y
+        if act and grad_y is None:
+            grad, act = grad_z, None
+        elif act and (again or grad_z is not None):
+            # z is an output of this node: derivatives of its slope come back here as grad_z
+            grad, act = torch.ops.aten.gelu_backward(grad_y, z), None
+            grad = grad if grad_z is None else grad + grad_z
         grad_bias, grad_factors = None, [None] * n
-        if ctx.act or need_bias:
-            grad, grad_bias = Kernel.epilogue_backward(grad, z, bs_last, ctx.act, need_bias)
+        if grad is None:
+            return (None,) * (5 + n)
+        if again and need_bias:
+            grad_bias = grad.sum_to_size(bias.shape)
+        grad = grad.contiguous()
+        if act or (need_bias and not again):
+            grad, grad_bias = Kernel.epilogue_backward(grad, z, bs_last, act, need_bias)
             grad_bias = grad_bias.view_as(bias) if need_bias else None
         for i in reversed(range(n)):
             need_input = need_x or any(need_factors[:i])

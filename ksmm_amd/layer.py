@@ -194,7 +194,8 @@ class KSLinear(nn.Module):
 
             args = x, self.bias, self.act, self.bs_last, self.patterns
             if KSLayerFunction.takes(x, self.bias, self.patterns, self.bs_last):
-                return KSLayerFunction.apply(*args, *self.factors)
+                out = KSLayerFunction.apply(*args, *self.factors)
+                return out[0] if self.act else out
             return layer_by_factors(*args, self.factors)
         scales = list(self.w_scales)
         if self.dtype == FP8:

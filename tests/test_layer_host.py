@@ -14,9 +14,7 @@ SQUARE = [(1, 4, 4, 2), (2, 4, 4, 1), (1, 4, 4, 2)]  # equally shaped factors: a
 
 def cpu_layer(patterns, cls=KSLinear, **kw):
     """A layer whose kernel-format factors live on the CPU."""
-    kw = dict(dtype=torch.float32, **kw)
-    layer = cls(patterns, algo="kernel", device="cpu:0", **kw)
-    return layer
+    return cls(patterns, algo="kernel", device="cpu:0", dtype=torch.float32, **kw)
 
 
 def dense_product(x, factors, patterns, bs_last, bias=None):
@@ -84,3 +82,91 @@ def test_wanted_gradients_are_those_of_the_layers_factors(native_stub):
             f.requires_grad_(False)
         assert layer.factors[1].requires_grad  # the masked tensor keeps its history
         assert layer._infer(torch.randn(3, layer.in_size), None) is None
+
+
+class DenseKernel:
+    """What the kernels compute, as dense products."""
+
+    @staticmethod
+    def forward(x, factor, bs_last, a, b, c, d, bias=None, **kw):
+        with torch.no_grad():
+            return dense_product(x, [factor], [(a, b, c, d)], bs_last, bias)
+
+    @staticmethod
+    def backward(grad, x, factor, bs_last, a, b, c, d, need_input=True, need_weight=True, **kw):
+        with torch.enable_grad():
+            xs, fs = x.detach().requires_grad_(), factor.detach().requires_grad_()
+            y = dense_product(xs, [fs], [(a, b, c, d)], bs_last)
+            return torch.autograd.grad(y, (xs, fs), grad.detach())
+
+    @staticmethod
+    def epilogue_backward(grad, z, bs_last, act=None, need_bias=True):
+        with torch.no_grad():
+            grad = torch.ops.aten.gelu_backward(grad, z) if act else grad
+            return grad, grad.sum(1 if bs_last else 0) if need_bias else None
+
+
+@pytest.fixture
+def dense_kernel(monkeypatch):
+    from ksmm_amd import kernel
+
+    for name in ("forward", "backward", "epilogue_backward"):
+        monkeypatch.setattr(kernel.Kernel, name, staticmethod(getattr(DenseKernel, name)))
+
+
+def hooked(layer, x):
+    """Hooks on a factor, the bias and an input with a history: each runs once a backward pass."""
+    x = x * 1.0
+    for t in (x, layer.bias, layer.factors[1]):
+        if t is not None:
+            t.register_hook(lambda g: 2 * g)
+    return layer(x)
+
+
+def tied(layer, x):
+    layer.factors[2] = layer.factors[0]
+    return layer(x)
+
+
+def shared(layer, x):
+    return layer(layer(x))
+
+
+@pytest.mark.parametrize("call", [hooked, tied, shared])
+@pytest.mark.parametrize("bs_last", [False, True])
+@pytest.mark.parametrize("act", [None, "gelu"])
+@pytest.mark.parametrize("bias", [False, True])
+def test_gradients_with_a_graph(dense_kernel, monkeypatch, call, bs_last, act, bias):
+    """create_graph=True: the gradients, and what can be differentiated again, as with a node per factor
+    and PyTorch's bias and activation."""
+    from ksmm_amd import kernel
+
+    torch.manual_seed(3)
+    weights = [torch.randn(p) / 2 for p in SQUARE]
+    start, x0, g0 = torch.randn(8, 1) if bs_last else torch.randn(8), torch.randn(8, 8), torch.randn(8, 8)
+
+    def gradients(one_node, create_graph):
+        with monkeypatch.context() as m, torch.enable_grad():
+            if not one_node:
+                m.setattr(kernel.KSLayerFunction, "takes", staticmethod(lambda *a: False))
+            layer = cpu_layer(SQUARE, weights=weights, bs_last=bs_last, act=act, bias=bias).double()
+            if bias:
+                layer.bias.data.copy_(start)
+            x, g = x0.double().requires_grad_(), g0.double().requires_grad_()
+            y = call(layer, x)
+            args = [x] + list(layer.parameters())
+            first = torch.autograd.grad(y, args, g, create_graph=create_graph)
+            if not create_graph or not bias:
+                return first
+            assert args[1] is layer.bias and first[1].requires_grad
+            again = torch.autograd.grad(first[1].pow(2).sum(), args + [g], allow_unused=True)
+            return first + tuple(torch.zeros(1) if t is None else t for t in again)
+
+    plain = gradients(False, False)
+    for create_graph in (False, True):
+        want, got = gradients(False, create_graph), gradients(True, create_graph)
+        assert len(want) == len(got)
+        for t, u in zip(got, want):
+            torch.testing.assert_close(t, u, rtol=1e-12, atol=1e-12)
+        for t, u in zip(got, plain):
+            torch.testing.assert_close(t, u, rtol=1e-12, atol=1e-12)

@@ -301,14 +301,16 @@ class KSLayerFunction(torch.autograd.Function):
         for i, (f, p) in enumerate(zip(factors, patterns)):
             inputs.append(Kernel.forward(inputs[-1], f, bs_last, *p, bias=bias if i == last else None))
         z = inputs.pop()
-        ctx.save_for_backward(bias, *factors, *inputs, z if act else None)
+        # (the bias is not saved: no gradient needs its values, and it may change before the backward pass)
+        ctx.bias_shape = None if bias is None else bias.shape
+        ctx.save_for_backward(*factors, *inputs, z if act else None)
         return (F.gelu(z), z) if act else z
 
     @staticmethod
     def backward(ctx, grad_y, grad_z=None):
         n, bs_last, act = len(ctx.patterns), ctx.bs_last, ctx.act
         saved = ctx.saved_tensors
-        bias, factors, inputs, z = saved[0], saved[1:n + 1], saved[n + 1:-1], saved[-1]
+        factors, inputs, z = saved[:n], saved[n:-1], saved[-1]
         need_x, need_bias = ctx.needs_input_grad[:2]
         need_factors = ctx.needs_input_grad[5:]
         again = torch.is_grad_enabled()  # create_graph: the epilogue in operations that can be differentiated
@@ -323,11 +325,11 @@ class KSLayerFunction(torch.autograd.Function):
         if grad is None:
             return (None,) * (5 + n)
         if again and need_bias:
-            grad_bias = grad.sum_to_size(bias.shape)
+            grad_bias = grad.sum_to_size(ctx.bias_shape)
         grad = grad.contiguous()
         if act or (need_bias and not again):
             grad, grad_bias = Kernel.epilogue_backward(grad, z, bs_last, act, need_bias)
-            grad_bias = grad_bias.view_as(bias) if need_bias else None
+            grad_bias = grad_bias.view(ctx.bias_shape) if need_bias else None
         for i in reversed(range(n)):
             need_input = need_x or any(need_factors[:i])
             if need_input or need_factors[i]:

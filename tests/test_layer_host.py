@@ -170,3 +170,17 @@ def test_gradients_with_a_graph(dense_kernel, monkeypatch, call, bs_last, act, b
             torch.testing.assert_close(t, u, rtol=1e-12, atol=1e-12)
         for t, u in zip(got, plain):
             torch.testing.assert_close(t, u, rtol=1e-12, atol=1e-12)
+
+
+@pytest.mark.parametrize("act", [None, "gelu"])
+@pytest.mark.parametrize("create_graph", [False, True])
+def test_bias_may_change_before_the_backward_pass(dense_kernel, act, create_graph):
+    with torch.enable_grad():
+        layer = cpu_layer(SQUARE, act=act).double()
+        x, g = torch.randn(5, 8, dtype=torch.float64), torch.randn(5, 8, dtype=torch.float64)
+        want = torch.autograd.grad(layer(x), list(layer.parameters()), g)
+        y = layer(x)
+        with torch.no_grad():
+            layer.bias += 1
+        for got, t in zip(torch.autograd.grad(y, list(layer.parameters()), g, create_graph=create_graph), want):
+            torch.testing.assert_close(got, t, rtol=1e-12, atol=1e-12)

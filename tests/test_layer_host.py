@@ -184,3 +184,37 @@ def test_bias_may_change_before_the_backward_pass(dense_kernel, act, create_grap
             layer.bias += 1
         for got, t in zip(torch.autograd.grad(y, list(layer.parameters()), g, create_graph=create_graph), want):
             torch.testing.assert_close(got, t, rtol=1e-12, atol=1e-12)
+
+
+class Doubled(KSLinear):
+    def post_process(self, tensor, output):
+        return 2 * super().post_process(tensor, output)
+
+
+class Shifted(KSLinear):
+    def pre_process(self, tensor):
+        return super().pre_process(tensor) + 1
+
+
+class Negated(KSLinear):
+    def forward_bs_first(self, output, x_scale=None):
+        return -super().forward_bs_first(output, x_scale)
+
+
+@pytest.mark.parametrize("cls,expected", [(Doubled, lambda layer, x: 2 * layer(x)), (Shifted, lambda layer, x: layer(x + 1)),
+                                          (Negated, lambda layer, x: -layer(x))])
+def test_steps_of_a_subclass_are_kept(native_stub, monkeypatch, cls, expected):
+    from ksmm_amd import kernel
+
+    def chain(x, factors, patterns, bs_last, bias=None, **kw):
+        return dense_product(x, factors, patterns, bs_last, bias)
+
+    monkeypatch.setattr(kernel.Kernel, "chain_forward", staticmethod(chain))
+    plain, layer = cpu_layer(SQUARE), cpu_layer(SQUARE, cls=cls)
+    layer.load_state_dict(plain.state_dict())
+    x = torch.randn(5, 8)
+    torch.testing.assert_close(layer(x), expected(plain, x))
+    patched = cpu_layer(SQUARE)
+    patched.post_process = lambda tensor, output: output + 3
+    patched.load_state_dict(plain.state_dict())
+    torch.testing.assert_close(patched(x), plain(x) + 3)

@@ -5,6 +5,7 @@ missing: there is no CPU or eager-PyTorch stand-in for ``algo='kernel'``.
 """
 import ctypes
 import os
+import warnings
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libksmm_hip.so")
@@ -116,16 +117,27 @@ def load():
     return lib
 
 
+class _NoNative:
+    """In place of the CPython module: takes no call, so that each goes through ksmm_amd/kernel.py."""
+
+    @staticmethod
+    def infer(*args):
+        return None
+
+
 def native():
-    """The CPython module KSLinear calls the library through (loaded once, with the library)."""
+    """The CPython module KSLinear calls the library through (loaded once, with the library).  It saves host
+    time only: where it is not built (no g++, no PyTorch headers) or does not load, the same kernels are launched
+    through ctypes, and a warning says so once."""
     global _native
     if _native is None:
         load()
         try:
             from . import _native as module
         except ImportError as e:
-            raise ImportError("ksmm_amd/_native.so is not built or does not load (%s): run `python -m ksmm_amd.build`. "
-                              "algo='kernel' has no fallback." % e)
+            warnings.warn("ksmm_amd/_native.so is not built or does not load (%s): layers are launched through ctypes, which takes "
+                          "10 to 20 us more host time a call; run `python -m ksmm_amd.build`" % e, RuntimeWarning, stacklevel=2)
+            module = _NoNative
         _native = module
     return _native
 

@@ -56,3 +56,10 @@ def test_full_device_raises_out_of_memory():
         torch.cuda.set_per_process_memory_fraction(1.0)
     with torch.no_grad():
         assert not layer(x).any()
+
+
+@pytest.mark.gpu
+def test_native_module_loads():
+    from ksmm_amd import _lib
+
+    assert _lib.native().__name__ == "ksmm_amd._native"

@@ -218,3 +218,45 @@ def test_steps_of_a_subclass_are_kept(native_stub, monkeypatch, cls, expected):
     patched.post_process = lambda tensor, output: output + 3
     patched.load_state_dict(plain.state_dict())
     torch.testing.assert_close(patched(x), plain(x) + 3)
+
+
+def test_without_the_native_module(monkeypatch):
+    """A module that does not load costs a warning and host time, no call."""
+    import sys
+    import warnings
+
+    import ksmm_amd
+    from ksmm_amd import kernel
+
+    monkeypatch.setattr(kernel.Kernel, "chain_forward",
+                        staticmethod(lambda x, f, p, last, bias=None, **kw: dense_product(x, f, p, last, bias)))
+    monkeypatch.setattr(_lib, "_native", None)
+    monkeypatch.delattr(ksmm_amd, "_native", raising=False)
+    monkeypatch.setitem(sys.modules, "ksmm_amd._native", None)  # as if it were not there
+    layer, x = cpu_layer(SQUARE), torch.randn(5, 8)
+    with pytest.warns(RuntimeWarning, match="_native"):
+        got = layer(x)
+    assert torch.equal(got, dense_product(x, layer.factors, SQUARE, False, layer.bias))
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        layer(x)
+
+
+def test_build_without_a_host_compiler(monkeypatch, tmp_path):
+    from ksmm_amd import build
+
+    for name in ("OBJ", "LIB", "BENCH_LIB", "NATIVE"):
+        monkeypatch.setattr(build, name, str(tmp_path / name))
+    (tmp_path / "NATIVE").write_text("of an earlier build")
+    monkeypatch.setattr(build, "_compile", lambda src: (src, ""))
+    run = build.subprocess.run
+
+    def no_gxx(cmd, **kw):
+        if cmd[0] == "g++":
+            raise FileNotFoundError("g++")
+        return run(["true"], **kw)
+
+    monkeypatch.setattr(build.subprocess, "run", no_gxx)
+    with pytest.warns(RuntimeWarning, match="g\\+\\+"):
+        assert build.build() == build.LIB
+    assert not (tmp_path / "NATIVE").exists()

@@ -409,7 +409,8 @@ int factor_forward_impl(const void *x, const void *w, void *y, int64_t batch, in
     p.x_scale = x_scale;
     // Every kernel but the split-K and the one-thread-per-output ones moves aligned 16-byte vectors:
     // tensors that do not start on a 16-byte boundary run on those (a forced family refuses them).
-    if ((((uintptr_t)x | (uintptr_t)w | (uintptr_t)y | (uintptr_t)p.bias) & 15) != 0) {
+    // All of them read a bias at the alignment of its elements.
+    if ((((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) != 0) {
         if (algo != KSMM_ALGO_AUTO && !(algo == KSMM_ALGO_GENERIC && variant <= 0)) return KSMM_ERR_BAD_ALGO;
         const Choice c = algo == KSMM_ALGO_AUTO ? cheapest_instance(p, true) : Choice{KSMM_ALGO_AUTO, -1, -1.f};
         return c.algo != KSMM_ALGO_AUTO ? family_run(p, c.algo, c.variant, true, nullptr) : generic_run(p, 0, true, nullptr);

@@ -504,13 +504,14 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void ks_gemm_kernel(const CT *__
                 } else {
                     // element u of group eg is output m0 + mb + 4*lq + 8*eg + u (x DD interleaved
                     // d_i): the lane's 4 * DD bias values of a group are consecutive, one vector load
+                    // (at element alignment: a bias may be a slice of a longer buffer)
                     static_assert(BS_LAST || sizeof(TY) == 2, "batch-size-first tiles write fp16");
                     typedef TY bias_v __attribute__((ext_vector_type(4 * DD)));
                     const size_t f0 = ((size_t)a_i * b + m0 + mb + 4 * lq) * DD;
 #pragma unroll
                     for (int eg = 0; eg < 4; ++eg) {
                         bias_v bb = {};
-                        if (ep.bias) bb = *(const bias_v *)((const TY *)ep.bias + f0 + 8 * eg * DD);
+                        if (ep.bias) __builtin_memcpy(&bb, (const TY *)ep.bias + f0 + 8 * eg * DD, sizeof(bb));
 #pragma unroll
                         for (int j = 0; j < C::NT; ++j)
 #pragma unroll
@@ -913,9 +914,10 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void ks_gemm_pbf_kernel(const CT
 #pragma unroll
                 for (int eg = 0; eg < 4; ++eg) {
                     // the lane's bias values of this group: (4 outputs) x (DD d_i), one vector load
+                    // (at element alignment)
                     typedef TY bias_v __attribute__((ext_vector_type(4 * DD)));
                     bias_v bb = {};
-                    if (ep.bias) bb = *(const bias_v *)((const TY *)ep.bias + f0 + 8 * DD * eg);
+                    if (ep.bias) __builtin_memcpy(&bb, (const TY *)ep.bias + f0 + 8 * DD * eg, sizeof(bb));
 #pragma unroll
                     for (int j = 0; j < C::NT; ++j)
 #pragma unroll

@@ -128,6 +128,11 @@ int ksmm_query_tile(int64_t batch, int a, int b, int c, int d, int x_dtype, int 
 int ksmm_query_tile_variant(int64_t batch, int a, int b, int c, int d, int x_dtype, int w_dtype,
                             int y_dtype, int bs_last, int algo, int variant, ksmm_tile *out);
 
+/* What the model of kernel times says of the kernel that ksmm_query_tile_variant reports, in microseconds;
+ * negative where it has no price for that kernel.  Host only. */
+int ksmm_price(int64_t batch, int a, int b, int c, int d, int x_dtype, int w_dtype, int y_dtype,
+               int bs_last, int algo, int variant, float *us);
+
 /* The measured table KSMM_ALGO_AUTO consults for batches of 8192 and more (below, every instance is
  * priced by a fitted model of its time, and the cheapest is taken): the counterpart
  * of the reference's tuned `*.best` files and the if-chains generated from them

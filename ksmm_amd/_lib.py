@@ -48,6 +48,8 @@ SIGNATURES = {
                                 ctypes.POINTER(KsmmTile)]),
     "ksmm_query_tile_variant": (c_int, [c_i64, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                                         c_int, ctypes.POINTER(KsmmTile)]),
+    "ksmm_price": (c_int, [c_i64, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
+                           ctypes.POINTER(ctypes.c_float)]),
     "ksmm_tuned_count": (c_int, []),
     "ksmm_tuned_row": (c_int, [c_int, ctypes.POINTER(c_int * 10)]),
     "ksmm_variant_id": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, ctypes.POINTER(ctypes.c_uint32),

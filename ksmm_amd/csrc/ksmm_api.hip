@@ -742,6 +742,22 @@ int ksmm_query_tile_variant(int64_t batch, int a, int b, int c, int d, int x_dty
     return dispatch(p, algo, variant, false, out);
 }
 
+int ksmm_price(int64_t batch, int a, int b, int c, int d, int x_dtype, int w_dtype, int y_dtype, int bs_last,
+               int algo, int variant, float *us)
+{
+    if (!us) return KSMM_ERR_NULL_POINTER;
+    ksmm_tile t;
+    const int rc = ksmm_query_tile_variant(batch, a, b, c, d, x_dtype, w_dtype, y_dtype, bs_last, algo, variant, &t);
+    if (rc != KSMM_OK) return rc;
+    if (t.algo == KSMM_ALGO_GENERIC && t.variant >= GENERIC_TILE) {  // a tile instance by the number it is reported under
+        t.algo = KSMM_ALGO_TILE;
+        t.variant -= GENERIC_TILE;
+    }
+    const Problem p{nullptr, nullptr, nullptr, batch, a, b, c, d, x_dtype, w_dtype, y_dtype, bs_last ? 1 : 0, 1.f, nullptr};
+    *us = predicted_us(p, t);
+    return KSMM_OK;
+}
+
 int ksmm_tuned_count(void) { return N_TUNED; }
 
 int ksmm_tuned_row(int index, int row[10])

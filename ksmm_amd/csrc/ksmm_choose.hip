@@ -8,13 +8,15 @@
 // geometric mean, and up to 12 times.  Here every instance that takes the problem is priced by a
 // linear model of its time in microseconds,
 //     t = f . (1, s, cu s, s w, cu s w, cu, by, by w)
-//   s   steps of a workgroup's loop over c (wave and row kernels: size of a tile)
-//   cu  rounds of workgroups over the 256 CUs (split-K kernel: of its waves over the SIMDs)
+//   s   steps of a workgroup's loop over c (wave and row kernels: size of a tile times the tiles of a wave
+//       or workgroup)
+//   cu  rounds of workgroups over the 256 CUs (split-K, wave and row kernels: of waves over the SIMDs)
 //   w   share of a 64-byte line a batch-size-first tile does not use, as a factor
 //   by  bytes of input, output and weights at 5 TB/s
-// with non-negative coefficients fitted per instance (wave and row kernels: per family) to their
-// measured times, and the cheapest one is taken: 1.03 to 1.06 times the fastest instance in the
-// geometric mean on problems that were held back from the fit.
+// with non-negative coefficients fitted per instance to its measured times, and the cheapest one is
+// taken.  The table comes from `python -m ksmm_amd.prices`, which also says how good the choice is on
+// problems that were held back from the fit; instances that it lists as having no price are not
+// offered.
 #include <string.h>
 
 #include "ksmm_choose.h"
@@ -23,11 +25,12 @@ namespace ksmm {
 
 namespace {
 
-constexpr int FAM_SPLIT = 5, FAM_WAVE = 14, FAM_ROWS = 15;  // tile sub-families have their own numbers
+// tile sub-families have their own numbers
+constexpr int FAM_SPLIT = 5, FAM_WAVE = 14, FAM_ROWS = 15;
 constexpr int COST_TERMS = 8;
 struct CostRow {
     int family, combo, bs_last;
-    uint32_t id;
+    uint32_t id;  // of the instance
     float f[COST_TERMS];
 };
 const CostRow cost_rows[] = {
@@ -35,10 +38,10 @@ const CostRow cost_rows[] = {
 };
 constexpr int N_COST = (int)(sizeof(cost_rows) / sizeof(CostRow));
 
-constexpr int N_SUBS = 6, MAX_INST = 128;
+constexpr int N_SUBS = 6, MAX_INST = 128, MAX_ROWS = 1024;
 struct CostIndex {  // rows by family and instance
     const CostRow *tile[N_SUBS][4][2][MAX_INST];
-    const CostRow *wave[4][2], *rows[4][2];
+    const CostRow *wave[4][MAX_INST], *rows[4][MAX_ROWS];  // batch-size-last, batch-size-first
     int count[N_SUBS];
     CostIndex()
     {
@@ -50,8 +53,12 @@ struct CostIndex {  // rows by family and instance
         for (int s = 0; s < N_SUBS; ++s) count[s] = n[s] < MAX_INST ? n[s] : MAX_INST;
         for (int i = 0; i < N_COST; ++i) {
             const CostRow &r = cost_rows[i];
-            if (r.family == FAM_WAVE) wave[r.combo][r.bs_last] = &r;
-            if (r.family == FAM_ROWS) rows[r.combo][r.bs_last] = &r;
+            if (r.family == FAM_WAVE)
+                for (int k = 0; k < wave_inst_count(r.combo) && k < MAX_INST; ++k)
+                    if (wave_inst_id(r.combo, k) == r.id) wave[r.combo][k] = &r;
+            if (r.family == FAM_ROWS)
+                for (int k = 0; k < rows_inst_count() && k < MAX_ROWS; ++k)
+                    if (rows_inst_id(k) == r.id) rows[r.combo][k] = &r;
             if (r.family >= N_SUBS) continue;
             for (int k = 0; k < count[r.family]; ++k)
                 if (id[r.family](k) == r.id) tile[r.family][r.combo][r.bs_last][k] = &r;
@@ -79,7 +86,10 @@ float price(const CostRow &r, const Problem &p, const ksmm_tile &t)
         s = (double)ceil_div((int64_t)s, ks);
         cu = ceil_div(groups * ks, 1024);
     } else if (r.family == FAM_WAVE || r.family == FAM_ROWS) {
-        s = (double)t.tile_m * t.tile_n * t.tile_d * p.c / 65536.;
+        // workers (waves, or a row kernel's workgroups) walk over tiles of the whole of c
+        const int64_t waves = t.grid * (t.threads / 64), workers = r.family == FAM_WAVE ? waves : t.grid;
+        s = (double)t.tile_m * t.tile_n * t.tile_d * p.c / 65536. * (double)ceil_div(groups, workers);
+        cu = ceil_div(waves, 1024);
     }
     const double by = (n * ad * (p.c * ex + p.b * ey) + ad * p.b * p.c * ew) / 5e6;
     double w = 1.;
@@ -96,7 +106,11 @@ float price(const CostRow &r, const Problem &p, const ksmm_tile &t)
 const CostRow *row_of(const Problem &p, int combo, int algo, int variant)
 {
     const CostIndex &ix = cost_index();
-    if (algo == KSMM_ALGO_WAVE) return variant >= 1000 ? ix.rows[combo][p.bs_last] : ix.wave[combo][p.bs_last];
+    if (variant < 0) return nullptr;
+    if (algo == KSMM_ALGO_WAVE) {
+        if (p.bs_last) return (variant & 0xff) < MAX_INST ? ix.wave[combo][variant & 0xff] : nullptr;
+        return variant >= 1000 ? ix.rows[combo][(variant - 1000) & (MAX_ROWS - 1)] : nullptr;
+    }
     if (algo != KSMM_ALGO_TILE) return nullptr;
     const int sub = variant >> 24, inst = variant & 0xff;
     return sub < N_SUBS && inst < MAX_INST ? ix.tile[sub][combo][p.bs_last][inst] : nullptr;

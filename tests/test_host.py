@@ -587,3 +587,76 @@ def test_bench_csv_writes_the_reference_schema_and_replaces_rows(tmp_path, capsy
     with pytest.raises(ValueError):
         bench_csv.main(["--saving-csv", str(bad), "--device", "cpu", "--patterns", "2,3,5,4", "--algo", "bmm",
                         "--min-run-time", "0.01"])
+
+
+def _price_table():
+    from ksmm_amd import prices
+
+    path = os.path.join(os.path.dirname(prices.__file__), "csrc", "ksmm_cost.inc")
+    listed = {tuple(int(v) for v in re.match(r"// no price: (\d+) (\d+)u", l).groups())
+              for l in open(path) if l.startswith("// no price")}
+    return prices, prices.read(path), listed
+
+
+def test_every_price_has_an_instance_and_every_instance_a_price(lib):
+    """Rows of the price table name instances of this library, and an instance without one is listed as such:
+    one that is added or changed cannot drop out of the choice unseen."""
+    prices, rows, listed = _price_table()
+    for combo in range(4):
+        for bs_last in (False, True):
+            have = {(f, i) for f, i, _, _ in prices.instances(combo, bs_last)}
+            assert {(k[0], k[3]) for k in rows if (k[1], k[2]) == (combo, int(bs_last))} <= have
+    assert set(prices.unpriced(rows)) == listed
+
+
+def test_prices_of_the_library_are_those_of_the_fit(lib):
+    """The model in Python, which the table is fitted with, and the one the library chooses by."""
+    import random
+
+    prices, rows, _ = _price_table()
+    seen = set()
+    for combo in range(4):
+        for bs_last in (False, True):
+            insts, rng = prices.instances(combo, bs_last), random.Random(combo)
+            for _ in range(40):
+                a, b, c, d, batch = problem = prices.draw(rng)
+                for family, iid, algo, variant in insts:
+                    t = prices.query(problem, combo, bs_last, algo, variant)
+                    if t is None or family == prices.FAM_GENERIC:
+                        continue
+                    us = ctypes.c_float()
+                    assert lib.ksmm_price(batch, a, b, c, d, *prices._COMBO_DTYPES[combo], int(bs_last), algo, variant, us) == 0
+                    f = rows.get((family, combo, int(bs_last), iid))
+                    want = -1. if f is None else float(f @ prices.features(problem, combo, bs_last, family, t))
+                    assert us.value == pytest.approx(want, rel=1e-5), (problem, combo, bs_last, family, variant)
+                    seen.add(family)
+    assert seen == {0, 1, 2, 3, 4, 5, 14, 15}
+
+
+def test_prices_do_not_drop_as_the_batch_grows(lib):
+    """One pattern at doubled batches: the automatic choice gets no cheaper."""
+    import random
+
+    prices, _, _ = _price_table()
+    for combo in range(4):
+        for bs_last in (False, True):
+            rng = random.Random(7 + combo)
+            for _ in range(150):
+                a, b, c, d, _ = prices.draw(rng)
+                last = 0.
+                for batch in (64, 128, 256, 512, 1024, 2048, 4096):
+                    us = ctypes.c_float()
+                    assert lib.ksmm_price(batch, a, b, c, d, *prices._COMBO_DTYPES[combo], int(bs_last), 0, -1, us) == 0
+                    if us.value < 0:  # a generic kernel
+                        break
+                    assert us.value >= last, ((a, b, c, d), combo, bs_last, batch, last, us.value)
+                    last = us.value
+
+
+def test_tile_instances_of_small_problems_are_priced_by_the_number_they_are_reported_under(lib):
+    from ksmm_amd.kernel import query_tile
+
+    us = ctypes.c_float()
+    t = query_tile(33 * 197, (4, 192, 192, 1), torch.float16, None, True)  # ragged rows: a split-K tile, as generic 16 + v
+    assert t["algo"] == 1 and t["variant"] >= 16
+    assert lib.ksmm_price(33 * 197, 4, 192, 192, 1, 1, 1, 1, 1, 0, -1, us) == 0 and us.value > 0

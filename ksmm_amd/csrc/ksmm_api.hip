@@ -310,7 +310,8 @@ Pick pick_of(const Problem &p, bool table)
         k.us = predicted_us(p, t);
         if (p.batch < TUNED_MIN_BATCH || !k.direct) {
             const Choice c = cheapest_instance(p, false);
-            if (c.algo != KSMM_ALGO_AUTO && (k.us < 0.f || c.us < k.us)) {
+            // (a kernel of its own that has no price is not known to be slower: it stays)
+            if (c.algo != KSMM_ALGO_AUTO && (k.us < 0.f ? !k.direct : c.us < k.us)) {
                 k.c = c;
                 k.us = c.us;
             }
@@ -358,13 +359,12 @@ Problem twin_of(const Problem &p)
 // it as it is: small problems are done before the first copy would be.
 bool route_pays(const Problem &p)
 {
-    const Pick k = pick_of(p, true);
-    if (k.us < 0.f) return true;
-    const Pick q = pick_of(twin_of(p), true);
+    const Pick k = pick_of(p, true), q = pick_of(twin_of(p), true);
+    if (k.us < 0.f || q.us < 0.f) return true;
     const int64_t bp = padded_batch(p.batch);
     const float copies = copy_us((int64_t)p.a * p.c * p.d, p.batch, bp, (int)dtype_size(p.x_dtype), !p.bs_last) +
                          copy_us((int64_t)p.a * p.b * p.d, p.batch, bp, (int)dtype_size(p.y_dtype), !p.bs_last);
-    return q.us >= 0.f && copies + q.us < k.us;
+    return copies + q.us < k.us;
 }
 
 int64_t align256(int64_t v) { return (v + 255) / 256 * 256; }

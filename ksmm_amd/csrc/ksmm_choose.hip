@@ -9,14 +9,15 @@
 // linear model of its time in microseconds,
 //     t = f . (1, s, cu s, s w, cu s w, cu, by, by w)
 //   s   steps of a workgroup's loop over c (wave and row kernels: size of a tile times the tiles of a wave
-//       or workgroup)
+//       or workgroup; one thread per output and vector form: eighths of c)
 //   cu  rounds of workgroups over the 256 CUs (split-K, wave and row kernels: of waves over the SIMDs)
 //   w   share of a 64-byte line a batch-size-first tile does not use, as a factor
 //   by  bytes of input, output and weights at 5 TB/s
 // with non-negative coefficients fitted per instance to its measured times, and the cheapest one is
 // taken.  The table comes from `python -m ksmm_amd.prices`, which also says how good the choice is on
 // problems that were held back from the fit; instances that it lists as having no price are not
-// offered.
+// offered.  The generic kernels are priced for the comparison only: they are the choice at full batches
+// of what has no other kernel, or of blocks of a few elements.
 #include <string.h>
 
 #include "ksmm_choose.h"
@@ -26,11 +27,11 @@ namespace ksmm {
 namespace {
 
 // tile sub-families have their own numbers
-constexpr int FAM_SPLIT = 5, FAM_WAVE = 14, FAM_ROWS = 15;
+constexpr int FAM_SPLIT = 5, FAM_GENERIC = 13, FAM_WAVE = 14, FAM_ROWS = 15;
 constexpr int COST_TERMS = 8;
 struct CostRow {
     int family, combo, bs_last;
-    uint32_t id;  // of the instance
+    uint32_t id;  // of the instance (generic family: the variant)
     float f[COST_TERMS];
 };
 const CostRow cost_rows[] = {
@@ -40,7 +41,7 @@ constexpr int N_COST = (int)(sizeof(cost_rows) / sizeof(CostRow));
 
 constexpr int N_SUBS = 6, MAX_INST = 128, MAX_ROWS = 1024;
 struct CostIndex {  // rows by family and instance
-    const CostRow *tile[N_SUBS][4][2][MAX_INST];
+    const CostRow *tile[N_SUBS][4][2][MAX_INST], *generic[4][2][2];
     const CostRow *wave[4][MAX_INST], *rows[4][MAX_ROWS];  // batch-size-last, batch-size-first
     int count[N_SUBS];
     CostIndex()
@@ -53,6 +54,7 @@ struct CostIndex {  // rows by family and instance
         for (int s = 0; s < N_SUBS; ++s) count[s] = n[s] < MAX_INST ? n[s] : MAX_INST;
         for (int i = 0; i < N_COST; ++i) {
             const CostRow &r = cost_rows[i];
+            if (r.family == FAM_GENERIC) generic[r.combo][r.bs_last][r.id & 1] = &r;
             if (r.family == FAM_WAVE)
                 for (int k = 0; k < wave_inst_count(r.combo) && k < MAX_INST; ++k)
                     if (wave_inst_id(r.combo, k) == r.id) wave[r.combo][k] = &r;
@@ -90,6 +92,9 @@ float price(const CostRow &r, const Problem &p, const ksmm_tile &t)
         const int64_t waves = t.grid * (t.threads / 64), workers = r.family == FAM_WAVE ? waves : t.grid;
         s = (double)t.tile_m * t.tile_n * t.tile_d * p.c / 65536. * (double)ceil_div(groups, workers);
         cu = ceil_div(waves, 1024);
+    } else if (r.family == FAM_GENERIC) {  // one thread's loop over c; workgroups of 256
+        s = (double)p.c / 8.;
+        cu = ceil_div(t.grid, 256);
     }
     const double by = (n * ad * (p.c * ex + p.b * ey) + ad * p.b * p.c * ew) / 5e6;
     double w = 1.;
@@ -107,6 +112,7 @@ const CostRow *row_of(const Problem &p, int combo, int algo, int variant)
 {
     const CostIndex &ix = cost_index();
     if (variant < 0) return nullptr;
+    if (algo == KSMM_ALGO_GENERIC) return variant < 2 ? ix.generic[combo][p.bs_last][variant] : nullptr;
     if (algo == KSMM_ALGO_WAVE) {
         if (p.bs_last) return (variant & 0xff) < MAX_INST ? ix.wave[combo][variant & 0xff] : nullptr;
         return variant >= 1000 ? ix.rows[combo][(variant - 1000) & (MAX_ROWS - 1)] : nullptr;

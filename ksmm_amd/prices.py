@@ -3,13 +3,17 @@ not apply (small and medium batches, ragged ones): measures every kernel instanc
 model of ``csrc/ksmm_choose.hip`` to the times.
 
     python -m ksmm_amd.prices --measure OUT.json [--problems 400] [--seed 0] [--made-for] [--combos 0,1,2,3]   (on the GPU)
-    python -m ksmm_amd.prices --fit A.json B.json ... --emit ksmm_amd/csrc/ksmm_cost.inc
+    python -m ksmm_amd.prices --fit A.json B.json ... --emit ksmm_amd/csrc/ksmm_cost.inc [--keep OLD.inc [--families 13,14,15]]
     python -m ksmm_amd.prices --check A.json ...          how good the choice by the present table is
 
 A problem is a factor pattern, a batch, an element-type combination (0 = fp32, 1 = fp16, 2 = e4m3 -> fp16,
 3 = e4m3 weights on fp16 input) and a layout.  Its instances are timed as launches of a HIP graph on one set of
 buffers, the way a layer finds its input: just written.  A quarter of the problems is held back from the fit; what
 is printed for them is the geometric mean of (time of the cheapest priced instance) / (time of the fastest).
+
+``--keep`` leaves the prices that a table has as they are, and with them the choices among those instances, except
+for the families named (0 .. 5 the tile sub-families, 13 generic, 14 wave, 15 row kernels); instances without one
+get the fitted price.
 
 Instances with fewer than ``ENOUGH`` measured problems get no price and are listed at the end of the file: they are
 never offered, and only run where the measured table or a family's own choice names them.
@@ -18,6 +22,7 @@ import argparse
 import ctypes
 import json
 import math
+import os
 import random
 import re
 import sys
@@ -201,14 +206,19 @@ def measure(path, combos, problems, seed, made_for):
 
 def load(paths):
     """Entries of measured files, with the terms of each instance as the library reports it now, and whether
-    it is among those the choice is made from (of the wave and row kernels one: the family's own choice)."""
+    it is among those the choice is made from: of the wave and row kernels the family's own choice, of the
+    generic ones that of full batches, if it is one."""
     entries = [e for p in paths for e in json.load(open(p))]
     for e in entries:
         problem, times = tuple(e["problem"]), []
         own = query(problem, e["combo"], e["bs_last"], _lib.ALGO_WAVE, -1)
+        full = query(problem[:4] + (16384 + problem[4] % 16,), e["combo"], e["bs_last"], _lib.ALGO_AUTO, -3)
         for family, iid, algo, variant, us in e["times"]:
             t = query(problem, e["combo"], e["bs_last"], algo, variant)
-            offered = family < FAM_WAVE or (own is not None and own.variant == variant)
+            if family == FAM_GENERIC:
+                offered = full is not None and full.algo == _lib.ALGO_GENERIC and (full.variant == 1) == (variant == 1)
+            else:
+                offered = family < FAM_GENERIC or (own is not None and own.variant == variant)
             times.append((family, iid, us, features(problem, e["combo"], e["bs_last"], family, t), offered))
         e["times"] = times
     return entries
@@ -316,20 +326,22 @@ def main():
     ap.add_argument("--combos", default="0,1,2,3")
     ap.add_argument("--fit", nargs="*")
     ap.add_argument("--emit")
+    ap.add_argument("--keep", help="a table whose prices stay")
+    ap.add_argument("--families", default="", help="families that --keep does not hold for")
     ap.add_argument("--check", nargs="*")
     args = ap.parse_args()
     if args.measure:
         measure(args.measure, [int(c) for c in args.combos.split(",")], args.problems, args.seed, args.made_for)
     if args.fit:
         entries = load(args.fit)
-        check(entries, fit(entries, whole=False))
-        rows = fit(entries)
+        again = {int(f) for f in args.families.split(",") if f}
+        kept = {k: f for k, f in read(args.keep).items() if k[0] not in again} if args.keep else {}
+        check(entries, {**fit(entries, whole=False), **kept})
+        rows = {**fit(entries), **kept}
         print("%d prices, %d instances without one" % (len(rows), len(unpriced(rows))))
         if args.emit:
             emit(rows, args.emit)
     if args.check:
-        import os
-
         check(load(args.check), read(os.path.join(os.path.dirname(__file__), "csrc", "ksmm_cost.inc")),
               only=lambda e: True)
     return 0

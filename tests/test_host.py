@@ -589,6 +589,18 @@ def test_bench_csv_writes_the_reference_schema_and_replaces_rows(tmp_path, capsy
                         "--min-run-time", "0.01"])
 
 
+def test_kernels_of_small_blocks_stay_below_full_batches(lib):
+    """Blocks of a few elements keep the vector form below batch 8192: 64-row tiles would compute mostly
+    rows that are not there."""
+    from ksmm_amd.kernel import query_tile
+
+    for dt in (torch.float32, torch.float16):
+        for pattern in [(32, 4, 4, 64), (16, 8, 8, 64), (64, 4, 4, 64), (1024, 4, 4, 1)]:
+            for batch in (4096, 8176):
+                t = query_tile(batch, pattern, dt, None, True)
+                assert (t["algo"], t["variant"]) == (1, 1), (pattern, batch, t)
+
+
 def _price_table():
     from ksmm_amd import prices
 
@@ -622,7 +634,7 @@ def test_prices_of_the_library_are_those_of_the_fit(lib):
                 a, b, c, d, batch = problem = prices.draw(rng)
                 for family, iid, algo, variant in insts:
                     t = prices.query(problem, combo, bs_last, algo, variant)
-                    if t is None or family == prices.FAM_GENERIC:
+                    if t is None:
                         continue
                     us = ctypes.c_float()
                     assert lib.ksmm_price(batch, a, b, c, d, *prices._COMBO_DTYPES[combo], int(bs_last), algo, variant, us) == 0
@@ -630,7 +642,7 @@ def test_prices_of_the_library_are_those_of_the_fit(lib):
                     want = -1. if f is None else float(f @ prices.features(problem, combo, bs_last, family, t))
                     assert us.value == pytest.approx(want, rel=1e-5), (problem, combo, bs_last, family, variant)
                     seen.add(family)
-    assert seen == {0, 1, 2, 3, 4, 5, 14, 15}
+    assert seen == {0, 1, 2, 3, 4, 5, 13, 14, 15}
 
 
 def test_prices_do_not_drop_as_the_batch_grows(lib):
@@ -647,8 +659,6 @@ def test_prices_do_not_drop_as_the_batch_grows(lib):
                 for batch in (64, 128, 256, 512, 1024, 2048, 4096):
                     us = ctypes.c_float()
                     assert lib.ksmm_price(batch, a, b, c, d, *prices._COMBO_DTYPES[combo], int(bs_last), 0, -1, us) == 0
-                    if us.value < 0:  # a generic kernel
-                        break
                     assert us.value >= last, ((a, b, c, d), combo, bs_last, batch, last, us.value)
                     last = us.value
 

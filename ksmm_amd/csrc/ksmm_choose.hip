@@ -18,6 +18,7 @@
 // problems that were held back from the fit; instances that it lists as having no price are not
 // offered.  The generic kernels are priced for the comparison only: they are the choice at full batches
 // of what has no other kernel, or of blocks of a few elements.
+#include <math.h>
 #include <string.h>
 
 #include "ksmm_choose.h"
@@ -162,8 +163,10 @@ Choice cheapest_instance(const Problem &p, bool split_only)
 
 float copy_us(int64_t rows, int64_t cols_in, int64_t cols_out, int elem_bytes, bool transpose)
 {
-    // measured: 7.4 us for 19 + 19 MB transposed, 28 us for 77 + 77; 8.3 us for 10 + 10 MB re-pitched
-    return 2.5f + (float)((double)rows * (cols_in + cols_out) * elem_bytes / (transpose ? 5.2e6 : 3e6));
+    // measured: 7.4 us for 19 + 19 MB transposed, 28 us for 77 + 77; 8.3 us for 10 + 10 MB re-pitched, 68 us for
+    // 205 + 205, 280 us for 822 + 822 (5.9 TB/s)
+    const float bytes = (float)((double)rows * (cols_in + cols_out) * elem_bytes);
+    return 2.5f + (transpose ? bytes / 5.2e6f : fminf(bytes / 3e6f, 3.5f + bytes / 5.9e6f));
 }
 
 }  // namespace ksmm

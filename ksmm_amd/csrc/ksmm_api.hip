@@ -284,12 +284,20 @@ struct Pick {
     float us;     // predicted time, < 0: no model of it
 };
 
+// Whether the kernels that move aligned 16-byte vectors take a problem's tensors (null: they will be).
+bool on_vectors(const Problem &p) { return (((uintptr_t)p.x | (uintptr_t)p.w | (uintptr_t)p.y) & 15) == 0; }
+
 // Below TUNED_MIN_BATCH, and where the full-batch choice is the one-thread-per-output kernel, the
-// cheapest instance by the model of ksmm_choose.hip; else the full-batch choice.  A function of the
-// sizes and types alone: each thread remembers its last answers (pricing every instance takes tens
+// cheapest instance by the model of ksmm_choose.hip; else the full-batch choice.  Tensors off the
+// vector take the cheapest of the kernels that do not need it.  A function of the sizes, types and that
+// alignment alone: each thread remembers its last answers (pricing every instance takes tens
 // of microseconds, a launch five).
-Pick pick_of(const Problem &p, bool table)
+Pick pick_of(const Problem &given, bool table)
 {
+    const bool aligned = on_vectors(given);
+    Problem p = given;  // (the routes of a problem are those the workspace query sees)
+    p.x = p.w = nullptr;
+    p.y = nullptr;
     struct Entry {
         int64_t batch;
         int key[8];
@@ -297,7 +305,7 @@ Pick pick_of(const Problem &p, bool table)
     };
     constexpr unsigned SLOTS = 256;
     static thread_local Entry memo[SLOTS];  // batch 0: empty
-    const int key[8] = {p.a, p.b, p.c, p.d, p.x_dtype, p.w_dtype, p.y_dtype, p.bs_last * 2 + (table ? 1 : 0)};
+    const int key[8] = {p.a, p.b, p.c, p.d, p.x_dtype, p.w_dtype, p.y_dtype, p.bs_last * 4 + (table ? 2 : 0) + (aligned ? 1 : 0)};
     uint64_t h = (uint64_t)p.batch;
     for (int v : key) h = (h ^ (uint64_t)v) * 0x9E3779B97F4A7C15ull;
     Entry &e = memo[(h >> 40) % SLOTS];
@@ -305,7 +313,17 @@ Pick pick_of(const Problem &p, bool table)
     ksmm_tile t;
     memset(&t, 0, sizeof(t));
     Pick k{{KSMM_ALGO_AUTO, -1, -1.f}, true, find_transposed(p), find_padded(p), -1.f};
-    if (table_run(p, table, false, &t) == KSMM_OK) {
+    if (!aligned) {
+        // (the alternative is the one-thread-per-output kernel)
+        k.direct = false;
+        generic_run(p, 0, false, &t);
+        k.us = predicted_us(p, t);
+        const Choice c = cheapest_instance(p, true);
+        if (c.algo != KSMM_ALGO_AUTO && (k.us < 0.f || c.us < k.us)) {
+            k.c = c;
+            k.us = c.us;
+        }
+    } else if (table_run(p, table, false, &t) == KSMM_OK) {
         k.direct = t.algo != KSMM_ALGO_GENERIC || t.variant == 1;
         k.us = predicted_us(p, t);
         if (p.batch < TUNED_MIN_BATCH || !k.direct) {
@@ -343,13 +361,15 @@ int dispatch(const Problem &p, int algo, int variant, bool launch, ksmm_tile *ti
             return rc;
         }
     }
-    return table_run(p, table, launch, tile);
+    return on_vectors(p) ? table_run(p, table, launch, tile) : generic_run(p, 0, launch, tile);
 }
 
 // The same problem in batch-size-last layout with padded rows (what both routes run in the middle).
 Problem twin_of(const Problem &p)
 {
     Problem q = p;
+    q.x = nullptr;  // (copies in a workspace)
+    q.y = nullptr;
     q.bs_last = 1;
     q.batch = padded_batch(p.batch);
     return q;
@@ -410,11 +430,8 @@ int factor_forward_impl(const void *x, const void *w, void *y, int64_t batch, in
     // Every kernel but the split-K and the one-thread-per-output ones moves aligned 16-byte vectors:
     // tensors that do not start on a 16-byte boundary run on those (a forced family refuses them).
     // All of them read a bias at the alignment of its elements.
-    if ((((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) != 0) {
-        if (algo != KSMM_ALGO_AUTO && !(algo == KSMM_ALGO_GENERIC && variant <= 0)) return KSMM_ERR_BAD_ALGO;
-        const Choice c = algo == KSMM_ALGO_AUTO ? cheapest_instance(p, true) : Choice{KSMM_ALGO_AUTO, -1, -1.f};
-        return c.algo != KSMM_ALGO_AUTO ? family_run(p, c.algo, c.variant, true, nullptr) : generic_run(p, 0, true, nullptr);
-    }
+    if (algo != KSMM_ALGO_AUTO && !on_vectors(p))
+        return algo == KSMM_ALGO_GENERIC && variant <= 0 ? generic_run(p, 0, true, nullptr) : KSMM_ERR_BAD_ALGO;
     return dispatch(p, algo, variant, true, nullptr);
 }
 
@@ -519,14 +536,14 @@ float chain16_us(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, i
     return (float)(base + features * batch * (double)(dtype_size(x_dtype) + dtype_size(y_dtype)) / 5e6);
 }
 
-// Predicted time of a chain factor by factor, as given or in batch-size-last layout with padded rows
-// (< 0: a factor has no price)
-float chain_us(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype, int bs_last, bool twin)
+// Predicted time of a chain factor by factor, as given (x and y: its tensors) or in batch-size-last
+// layout with padded rows (< 0: a factor has no price)
+float chain_us(const ksmm_factor_desc *f, int n, const void *x, void *y, int64_t batch, int x_dtype, int y_dtype, int bs_last, bool twin)
 {
     float sum = 0.f;
     for (int i = 0; i < n; ++i) {
-        Problem p{nullptr, nullptr, nullptr, batch, f[i].a, f[i].b, f[i].c, f[i].d, i == 0 ? x_dtype : y_dtype,
-                  f[i].w_dtype, y_dtype, bs_last, 1.f, nullptr};
+        Problem p{i == 0 ? x : nullptr, f[i].w, i == n - 1 ? y : nullptr, batch, f[i].a, f[i].b, f[i].c, f[i].d,
+                  i == 0 ? x_dtype : y_dtype, f[i].w_dtype, y_dtype, bs_last, 1.f, nullptr};
         const Pick k = pick_of(twin ? twin_of(p) : p, true);
         if (k.us < 0.f) return -1.f;
         sum += k.us;
@@ -537,20 +554,21 @@ float chain_us(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int
 // Whether the fused chain is the faster way through a batch-size-last chain that it takes: at full
 // batches it saves the intermediates' traffic; on a few thousand columns a launch per factor is
 // done first (2.4 us each on the wave kernels against 3 to 4 us a factor in the fused one).
-bool fused_pays(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype)
+bool fused_pays(const ksmm_factor_desc *f, int n, const void *x, void *y, int64_t batch, int x_dtype, int y_dtype)
 {
     if (batch >= TUNED_MIN_BATCH) return true;
-    const float fused = chain16_us(f, n, batch, x_dtype, y_dtype), each = chain_us(f, n, batch, x_dtype, y_dtype, 1, false);
+    const float fused = chain16_us(f, n, batch, x_dtype, y_dtype), each = chain_us(f, n, x, y, batch, x_dtype, y_dtype, 1, false);
     return fused < 0.f || each < 0.f || fused < each;
 }
 
 // Whether a chain that has a transposed or padded-rows route should take it.
-bool chain_route_pays(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype, int bs_last, bool fuse)
+bool chain_route_pays(const ksmm_factor_desc *f, int n, const void *x, void *y, int64_t batch, int x_dtype, int y_dtype, int bs_last,
+                      bool fuse)
 {
-    const float direct = chain_us(f, n, batch, x_dtype, y_dtype, bs_last, false);
+    const float direct = chain_us(f, n, x, y, batch, x_dtype, y_dtype, bs_last, false);
     if (direct < 0.f) return true;
     const int64_t bp = padded_batch(batch);
-    float middle = chain_us(f, n, batch, x_dtype, y_dtype, bs_last, true);
+    float middle = chain_us(f, n, x, y, batch, x_dtype, y_dtype, bs_last, true);
     const float fused = fuse ? chain16_us(f, n, bp, x_dtype, y_dtype) : -1.f;
     if (fused >= 0.f && (middle < 0.f || fused < middle)) middle = fused;
     if (middle < 0.f) return true;
@@ -588,7 +606,7 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
     // ping-pong buffers of `one` bytes at pp; *result = where the last factor's output is.
     auto run_bs_last = [&](const void *x0, char *pp, int64_t one, int64_t nb, const void **result) -> int {
         int rc2 = KSMM_ERR_BAD_ALGO;
-        if (fuse && fused_pays(factors, n_factors, nb, x_dtype, y_dtype))
+        if (fuse && fused_pays(factors, n_factors, x0, pp, nb, x_dtype, y_dtype))
             rc2 = chain16_run(factors, n_factors, x0, pp, nb, x_dtype, y_dtype, 1, true, (hipStream_t)stream, ep, x_scale);
         if (rc2 == KSMM_OK) {
             *result = pp;
@@ -616,7 +634,7 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
         // kernel without a word)
         const int64_t need_t = ksmm_chain_workspace_layout(factors, n_factors, batch, x_dtype, y_dtype, 0);
         if (!workspace || workspace_bytes < need_t) return KSMM_ERR_WORKSPACE;
-        if (chain_route_pays(factors, n_factors, batch, x_dtype, y_dtype, 0, fuse != 0)) {
+        if (chain_route_pays(factors, n_factors, x, y, batch, x_dtype, y_dtype, 0, fuse != 0)) {
             const int64_t bp = padded_batch(batch);  // row length of the transposed copies
             const int64_t xt_bytes = align256(in0 * bp * (int64_t)dtype_size(x_dtype));
             char *xt = (char *)workspace;
@@ -631,7 +649,7 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
         // pad the rows once, run the whole chain at the padded batch, cut the result rows back
         const int64_t need_p = ksmm_chain_workspace_layout(factors, n_factors, batch, x_dtype, y_dtype, 1);
         if (!workspace || workspace_bytes < need_p) return KSMM_ERR_WORKSPACE;
-        if (chain_route_pays(factors, n_factors, batch, x_dtype, y_dtype, 1, fuse != 0)) {
+        if (chain_route_pays(factors, n_factors, x, y, batch, x_dtype, y_dtype, 1, fuse != 0)) {
             const int64_t bp = padded_batch(batch);
             const int64_t xp_bytes = align256(in0 * bp * (int64_t)dtype_size(x_dtype));
             char *xp = (char *)workspace;
@@ -643,7 +661,7 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
             return repitch_run(cur, y, out_n, bp, batch, (int)dtype_size(y_dtype), (hipStream_t)stream);
         }
     }
-    if (fuse && (!bs_last || fused_pays(factors, n_factors, batch, x_dtype, y_dtype))) {
+    if (fuse && (!bs_last || fused_pays(factors, n_factors, x, y, batch, x_dtype, y_dtype))) {
         // chains whose intermediates fit LDS run as one kernel (no workspace traffic)
         rc = chain16_run(factors, n_factors, x, y, batch, x_dtype, y_dtype, bs_last ? 1 : 0, true,
                          (hipStream_t)stream, ep, x_scale);

@@ -23,3 +23,31 @@ def test_bias_needs_the_alignment_of_its_elements(dt, bs_last, batch):
                 bias = flat[offset:offset + a * b * d]
                 got = Kernel.forward(x, w, bs_last, a, b, c, d, bias=bias, act=act)
                 assert torch.equal(got, Kernel.forward(x, w, bs_last, a, b, c, d, bias=bias.clone(), act=act)), (a, b, c, d, offset)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16])
+@pytest.mark.parametrize("bs_last", [False, True])
+def test_unaligned_tensors_between_aligned_ones(dt, bs_last):
+    """The choice is remembered by sizes and by whether the tensors start on 16 bytes: calls of both kinds in
+    turn get their own each time, whichever tensor is off, and agree with float64."""
+    from ksmm_amd import Kernel
+    from ksmm_amd.layer import from_kernel_format_to_dense
+
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    for (a, b, c, d), batch in [((1, 96, 48, 2), 200), ((2, 64, 64, 1), 33), ((1, 3, 5, 4), 77), ((1, 256, 256, 2), 8200)]:
+        def tensor(rows, cols, off):
+            t = torch.empty(rows * cols + 1, device="cuda", dtype=dt)[off:off + rows * cols].view(rows, cols)
+            return t.copy_(torch.randn(rows, cols, generator=gen, device="cuda"))
+
+        w, x = [tensor(a * d * c, b, off) for off in (0, 1)], [tensor(*((a * c * d, batch) if bs_last else (batch, a * c * d)), off) for off in (0, 1)]
+        w[1].copy_(w[0])
+        x[1].copy_(x[0])
+        k = from_kernel_format_to_dense(w[0].double(), (a, b, c, d))
+        want = k @ x[0].double() if bs_last else x[0].double() @ k.t()
+        bits = {}
+        for _ in range(2):
+            for i, j in ((0, 0), (1, 0), (0, 1), (1, 1)):
+                y = Kernel.forward(x[i], w[j], bs_last, a, b, c, d)
+                # sums of c products of type dt in fp32, one rounding: 2e-7 sqrt(c) in fp32, 2.9e-4 in fp16
+                assert ((y.double() - want).norm() / want.norm()).item() <= (5e-6 if dt == torch.float32 else 4e-4)
+                assert torch.equal(y, bits.setdefault((i, j), y)), (i, j)

@@ -296,15 +296,16 @@ class KSLayerFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, bias, act, bs_last, patterns, *factors):
         ctx.act, ctx.bs_last, ctx.patterns = act, bs_last, patterns
-        ctx.set_materialize_grads(False)
         inputs, last = [x], len(factors) - 1
         for i, (f, p) in enumerate(zip(factors, patterns)):
             inputs.append(Kernel.forward(inputs[-1], f, bs_last, *p, bias=bias if i == last else None))
         z = inputs.pop()
         # (the bias is not saved: no gradient needs its values, and it may change before the backward pass)
-        ctx.bias_shape = None if bias is None else bias.shape
         ctx.save_for_backward(*factors, *inputs, z if act else None)
-        return (F.gelu(z), z) if act else z
+        if not act:
+            return z
+        ctx.set_materialize_grads(False)
+        return F.gelu(z), z
 
     @staticmethod
     def backward(ctx, grad_y, grad_z=None):
@@ -325,11 +326,11 @@ class KSLayerFunction(torch.autograd.Function):
         if grad is None:
             return (None,) * (5 + n)
         if again and need_bias:
-            grad_bias = grad.sum_to_size(ctx.bias_shape)
+            grad_bias = grad.sum(1, keepdim=True) if bs_last else grad.sum(0)
         grad = grad.contiguous()
         if act or (need_bias and not again):
             grad, grad_bias = Kernel.epilogue_backward(grad, z, bs_last, act, need_bias)
-            grad_bias = grad_bias.view(ctx.bias_shape) if need_bias else None
+            grad_bias = grad_bias.unsqueeze(1) if need_bias and bs_last else grad_bias
         for i in reversed(range(n)):
             need_input = need_x or any(need_factors[:i])
             if need_input or need_factors[i]:

@@ -81,3 +81,25 @@ def test_layer_gradients_equal_those_factor_by_factor(bs_last, act):
                 second = [torch.autograd.grad(torch.autograd.grad(out, layer.bias, g, create_graph=True)[0].sum(), layer.bias)[0]
                           for out in (y, ref)]
                 assert rel(second[0], second[1].double()) <= 1e-5
+
+
+@pytest.mark.parametrize("bs_last", [False, True])
+@pytest.mark.parametrize("act", [None, "gelu"])
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16])
+def test_gradients_with_a_graph_on_shared_parameters(bs_last, act, dt):
+    """create_graph=True through a layer applied twice, with one parameter for two factors and a hook on the bias:
+    as without a graph, where the same kernels run (a sum rounds apart)."""
+    from ksmm_amd import KSLinear
+
+    patterns = [(1, 16, 16, 4), (4, 16, 16, 1), (1, 16, 16, 4)]
+    with torch.enable_grad():
+        layer = KSLinear(patterns, algo="kernel", dtype=dt, bs_last=bs_last, device="cuda", act=act)
+        layer.factors[2] = layer.factors[0]
+        layer.bias.register_hook(lambda g: 2 * g)
+        x = torch.randn(64, 64, device="cuda", dtype=dt, requires_grad=True)
+        g = torch.randn(64, 64, device="cuda", dtype=dt)
+        args = [x] + list(layer.parameters())
+        want = torch.autograd.grad(layer(layer(x)), args, g)
+        for got, ref in zip(torch.autograd.grad(layer(layer(x)), args, g, create_graph=True), want):
+            # fp16: the slope by PyTorch's kernel or the series, rounded to 2^-11 in each of two layers
+            assert rel(got, ref.double()) <= (1e-5 if dt == torch.float32 else 2e-3)

@@ -35,6 +35,29 @@ def test_bias_that_is_pruned(bs_last):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("bs_last", [True, False])
+@pytest.mark.parametrize("for_good", [False, True])
+def test_factor_that_is_pruned(bs_last, for_good):
+    """Factors of one shape: unpruned or out of order they would fit as well."""
+    from ksmm_amd import KSLinear
+    from ksmm_amd.layer import from_kernel_format_to_abcd
+    from torch.nn.utils import prune
+
+    patterns = [(1, 16, 16, 4), (4, 16, 16, 1)]
+    layer = KSLinear(patterns, algo="kernel", dtype=torch.float32, bs_last=bs_last, device="cuda")
+    prune.l1_unstructured(layer.factors, "0", 0.5)
+    if for_good:
+        prune.remove(layer.factors, "0")
+    with torch.no_grad():
+        ref = KSLinear(patterns, weights=[from_kernel_format_to_abcd(f, p).cpu() for f, p in zip(layer.factors, patterns)],
+                       algo="einsum", dtype=torch.float64, bs_last=bs_last, device="cuda")
+        ref.bias.copy_(layer.bias)
+        x = _input(bs_last)
+        # two sums of 16 products in fp32
+        torch.testing.assert_close(layer(x).double(), ref(x.double()), rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bs_last", [True, False])
 def test_flags_need_not_be_bool(bs_last):
     with torch.no_grad():
         x = _input(bs_last)

@@ -7,9 +7,10 @@
 // What bounds it: HBM, 6 bytes a value in fp16.  The sums cost no traffic of their own; apart they are a
 // pass over dz that reads it back.  Batch-size-first, a thread keeps the sums of one 16-byte vector of
 // features and walks down the rows; batch-size-last, a wavefront walks along one feature's row.
-// fp16, 25088 x 1536 with GELU: 43 us (5.3 TB/s).  With the bias added in the last factor's kernel a
+// fp16, 25088 x 1536 with GELU: 44 us (5.3 TB/s).  With the bias added in the last factor's kernel a
 // training step of a ViT-S feed-forward block on 25088 rows went from 489 to 447 us, one of the fp32 layer
-// (6,64,64,1)+(1,768,192,2) on 6272 batch-size-last columns (bias only: 10 us here) from 266 to 242.
+// (6,64,64,1)+(1,768,192,2) on 6272 batch-size-last columns (bias only: 10 us here) from 266 to 242 (on one
+// box each; such a step varies by a tenth between boxes and with the host).
 #include "ksmm_common.h"
 
 namespace ksmm {
@@ -24,8 +25,8 @@ template <> __device__ __forceinline__ float gelu_slope<float>(float x)
 {
     return fmaf(x * INV_SQRT_2PI, expf(-0.5f * x * x), fmaf(0.5f, erff(x * 0.70710678118654752f), 0.5f));
 }
-// fp16: the series of gelu_erf (|error of Phi| < 1e-7, next to 5e-4 in the type), whose exponential is phi's as
-// well: erff and expf would take longer than the loads
+// fp16: the series of gelu_erf, whose exponential is phi's as well: erff and expf would take longer than the loads.
+// Largest error of the slope over all fp16 values 3.0e-7 (1.3e-7 with erff), next to the type's 5e-4
 template <> __device__ __forceinline__ float gelu_slope<half_t>(float x)
 {
     const float z = fabsf(x) * 0.84932180028801907f;

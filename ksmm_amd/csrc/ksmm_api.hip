@@ -258,9 +258,10 @@ bool find_transposed(const Problem &p)
 }
 
 // Batch-size-last rows are `batch` elements long: when that is not a multiple of the 16-byte
-// vector only the one-thread-per-output kernel takes the problem.  With a workspace it runs on a
+// vector only the split-K and the one-thread-per-output kernels take the problem.  With a workspace it runs on a
 // copy whose rows are zero-filled to the next multiple of 16 columns (the vector of every type)
-// and the result rows are cut back: two copies more, but on the kernel of the padded batch.
+// and the result rows are cut back: two copies more, but on the kernel of the padded batch, where that
+// is priced lower (route_pays).
 bool find_padded(const Problem &p)
 {
     if (!p.bs_last || p.batch % 16 == 0) return false;

@@ -19,7 +19,7 @@
 // shape below.  128 registers a wave (four waves a SIMD) spill: 74 us.
 // Against transposed copies of both operands in HBM and the batch-size-last kernel on them, fp16 at
 // 25088 rows: (1,768,192,2) 156 -> 52 us, (6,64,256,1) 90 -> 35, (1,128,128,3) 38 -> 23,
-// (1,1536,384,2) 213 -> 157, (1,16,16,64) 70 -> 46; fp32: 323 -> 200, 193 -> 72, 108 -> 52, 1083 -> 680, 148 -> 52.
+// (1,1536,384,2) 213 -> 157 (180 on another box), (1,16,16,64) 70 -> 46; fp32: 323 -> 200, 193 -> 72, 108 -> 52, 1083 -> 680, 148 -> 52.
 #include "ksmm_common.h"
 
 namespace ksmm {

@@ -7,12 +7,13 @@
 // both layouts) the heuristics' choice took 1.4 to 2.2 times the time of the fastest instance in the
 // geometric mean, and up to 12 times.  Here every instance that takes the problem is priced by a
 // linear model of its time in microseconds,
-//     t = f . (1, s, cu s, s w, cu s w, cu, by, by w)
+//     t = f . (1, s, cu s, s w, cu s w, cu, by, by w, far)
 //   s   steps of a workgroup's loop over c (wave and row kernels: size of a tile times the tiles of a wave
 //       or workgroup; one thread per output and vector form: eighths of c)
 //   cu  rounds of workgroups over the 256 CUs (split-K, wave and row kernels: of waves over the SIMDs)
 //   w   share of a 64-byte line a batch-size-first tile does not use, as a factor
 //   by  bytes of input, output and weights at 5 TB/s
+//   far those beyond 125 MB, which the last-level cache does not keep for the next kernel
 // with non-negative coefficients fitted per instance to its measured times, and the cheapest one is
 // taken.  The table comes from `python -m ksmm_amd.prices`, which also says how good the choice is on
 // problems that were held back from the fit (1.05 to 1.07 times the fastest instance in the geometric
@@ -29,7 +30,7 @@ namespace {
 
 // tile sub-families have their own numbers
 constexpr int FAM_SPLIT = 5, FAM_GENERIC = 13, FAM_WAVE = 14, FAM_ROWS = 15;
-constexpr int COST_TERMS = 8;
+constexpr int COST_TERMS = 9;
 struct CostRow {
     int family, combo, bs_last;
     uint32_t id;  // of the instance (generic family: the variant)
@@ -103,7 +104,7 @@ float price(const CostRow &r, const Problem &p, const ksmm_tile &t)
         const double line = p.d * ex < 64. ? p.d * ex : 64.;
         w = line / (t.tile_d * ex) > 1. ? line / (t.tile_d * ex) : 1.;
     }
-    const double v[COST_TERMS] = {1., s, cu * s, s * w, cu * s * w, (double)cu, by, by * w};
+    const double v[COST_TERMS] = {1., s, cu * s, s * w, cu * s * w, (double)cu, by, by * w, by > 25. ? by - 25. : 0.};
     double us = 0.;
     for (int i = 0; i < COST_TERMS; ++i) us += r.f[i] * v[i];
     return (float)us;
@@ -163,10 +164,10 @@ Choice cheapest_instance(const Problem &p, bool split_only)
 
 float copy_us(int64_t rows, int64_t cols_in, int64_t cols_out, int elem_bytes, bool transpose)
 {
-    // measured: 7.4 us for 19 + 19 MB transposed, 28 us for 77 + 77; 8.3 us for 10 + 10 MB re-pitched, 68 us for
-    // 205 + 205, 280 us for 822 + 822 (5.9 TB/s)
+    // measured: 7.4 us for 19 + 19 MB transposed, 28 us for 77 + 77; 8.3 us for 10 + 10 MB re-pitched from memory
+    // that no kernel has just read (3 TB/s), 68 us for 205 + 205, 280 us for 822 + 822 (5.9 TB/s)
     const float bytes = (float)((double)rows * (cols_in + cols_out) * elem_bytes);
-    return 2.5f + (transpose ? bytes / 5.2e6f : fminf(bytes / 3e6f, 3.5f + bytes / 5.9e6f));
+    return 2.5f + (transpose ? bytes / 5.2e6f : fminf(bytes / 3e6f, 20.f + bytes / 5.9e6f));
 }
 
 }  // namespace ksmm

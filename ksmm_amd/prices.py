@@ -36,6 +36,7 @@ from .kernel import _COMBO_DTYPES, variant_id
 FAM_SPLIT, FAM_GENERIC, FAM_WAVE, FAM_ROWS = 5, 13, 14, 15
 SIZE = {_lib.KSMM_F32: 4, _lib.KSMM_F16: 2, _lib.KSMM_FP8_E4M3: 1}
 ENOUGH = 12  # problems a price is fitted to
+TERMS = 9
 MOST = 1 << 27  # elements of a problem's input or output
 ROW = re.compile(r"^\{(\d+), (\d+), (\d+), (\d+)u, \{([^}]*)\}\}")
 
@@ -122,7 +123,7 @@ def features(problem, combo, bs_last, family, t):
     w = 1.
     if not bs_last and t.tile_d < d:
         w = max(1., min(d * ex, 64.) / (t.tile_d * ex))
-    return [1., s, cu * s, s * w, cu * s * w, float(cu), by, by * w]
+    return [1., s, cu * s, s * w, cu * s * w, float(cu), by, by * w, max(0., by - 25.)]
 
 
 # ---- measuring --------------------------------------------------------------------------------------------------
@@ -249,7 +250,9 @@ def fit(entries, whole=True):
     for e in entries:
         if not whole and held_back(e):
             continue
-        for family, iid, us, v, _ in e["times"]:
+        for family, iid, us, v, offered in e["times"]:
+            if family == FAM_GENERIC and not offered:
+                continue  # (large blocks on these kernels say little about the small ones they run on)
             data.setdefault((family, e["combo"], int(e["bs_last"]), iid), []).append((us, v))
     rows = {}
     for key, samples in data.items():
@@ -268,7 +271,8 @@ def read(path):
     for line in open(path):
         m = ROW.match(line)
         if m:
-            rows[tuple(int(g) for g in m.groups()[:4])] = np.array([float(v.rstrip("f")) for v in m.group(5).split(", ")])
+            terms = [float(v.rstrip("f")) for v in m.group(5).split(", ")]
+            rows[tuple(int(g) for g in m.groups()[:4])] = np.array(terms + [0.] * (TERMS - len(terms)))
     return rows
 
 

@@ -304,13 +304,16 @@ Pick pick_of(const Problem &given, bool table)
         int key[8];
         Pick pick;
     };
-    constexpr unsigned SLOTS = 256;
-    static thread_local Entry memo[SLOTS];  // batch 0: empty
+    // sets of four: with one entry a hash, two factors of a chain that share it cost 3 to 5 us a call
+    constexpr unsigned SETS = 64, WAYS = 4;
+    static thread_local Entry memo[SETS][WAYS];  // batch 0: empty
+    static thread_local uint8_t oldest[SETS];
     const int key[8] = {p.a, p.b, p.c, p.d, p.x_dtype, p.w_dtype, p.y_dtype, p.bs_last * 4 + (table ? 2 : 0) + (aligned ? 1 : 0)};
     uint64_t h = (uint64_t)p.batch;
     for (int v : key) h = (h ^ (uint64_t)v) * 0x9E3779B97F4A7C15ull;
-    Entry &e = memo[(h >> 40) % SLOTS];
-    if (e.batch == p.batch && memcmp(e.key, key, sizeof(key)) == 0) return e.pick;
+    const unsigned set = (h >> 40) % SETS;
+    for (const Entry &e : memo[set])
+        if (e.batch == p.batch && memcmp(e.key, key, sizeof(key)) == 0) return e.pick;
     ksmm_tile t;
     memset(&t, 0, sizeof(t));
     Pick k{{KSMM_ALGO_AUTO, -1, -1.f}, true, find_transposed(p), find_padded(p), -1.f};
@@ -333,6 +336,7 @@ Pick pick_of(const Problem &given, bool table)
         k.us = predicted_us(p, t);
         if (p.batch < TUNED_MIN_BATCH || !k.direct) replace(cheapest_instance(p, false));
     }
+    Entry &e = memo[set][oldest[set]++ % WAYS];
     e.batch = p.batch;
     memcpy(e.key, key, sizeof(key));
     e.pick = k;

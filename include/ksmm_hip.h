@@ -278,6 +278,18 @@ int ksmm_epilogue_backward(const void *dy, const void *z, void *dz, void *dbias,
                            int64_t features, int dtype, int bs_last, int act, void *workspace,
                            int64_t workspace_bytes, void *stream);
 
+/* Backward pass of a whole layer y = act(K_n ... K_1 x + bias) in one call (fp32 and fp16; every factor,
+ * input and gradient of one type): inputs[i] is what factor i was applied to (inputs[0] = x), z what the
+ * activation was applied to (KSMM_ACT_NONE: not read).  Writes dx, dw[i] (kernel format) and dbias, each
+ * of which may be NULL where it is not wanted.  Against one call per factor and epilogue it transposes
+ * all blocks in one launch and adds all partial sums in one.  Needs ksmm_layer_backward_workspace() bytes
+ * of 16-byte aligned device memory. */
+int64_t ksmm_layer_backward_workspace(const ksmm_factor_desc *factors, int n_factors, int64_t batch, int dtype,
+                                      int bs_last, int act);
+int ksmm_layer_backward(const ksmm_factor_desc *factors, int n_factors, const void *const *inputs, const void *z,
+                        const void *dy, void *dx, void *const *dw, void *dbias, void *workspace,
+                        int64_t workspace_bytes, int64_t batch, int dtype, int bs_last, int act, void *stream);
+
 /* ksmm_chain_forward_ep for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc): the ping-pong intermediates
  * and the transposed-route and padded-rows buffers live in a fixed device array inside the library,

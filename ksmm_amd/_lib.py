@@ -83,6 +83,9 @@ SIGNATURES = {
                                          c_int, c_int, ctypes.POINTER(KsmmEpilogue), c_vp]),
     "ksmm_epilogue_backward_workspace": (c_i64, [c_i64, c_i64, c_int, c_int]),
     "ksmm_epilogue_backward": (c_int, [c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_int, c_int, c_int, c_vp, c_i64, c_vp]),
+    "ksmm_layer_backward_workspace": (c_i64, [ctypes.POINTER(KsmmFactorDesc), c_int, c_i64, c_int, c_int, c_int]),
+    "ksmm_layer_backward": (c_int, [ctypes.POINTER(KsmmFactorDesc), c_int, ctypes.POINTER(c_vp), c_vp, c_vp, c_vp, ctypes.POINTER(c_vp),
+                                    c_vp, c_vp, c_i64, c_i64, c_int, c_int, c_int, c_vp]),
     "ksmm_static_scratch_bytes": (c_i64, []),
     "ksmm_chain_forward_static": (c_int, [ctypes.POINTER(KsmmFactorDesc), c_int, c_vp, c_vp, c_i64, c_int,
                                           c_int, c_int, c_int, ctypes.POINTER(KsmmEpilogue), c_vp]),
@@ -125,6 +128,8 @@ class _NoNative:
     @staticmethod
     def infer(*args):
         return None
+
+    train_forward = train_backward = infer
 
 
 def native():

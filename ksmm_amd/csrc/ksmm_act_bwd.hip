@@ -267,7 +267,7 @@ int64_t act_bwd_partial_floats(int64_t batch, int64_t features, int dtype, int b
 }
 
 int act_bwd_run(const void *dy, const void *z, void *dz, void *dbias, float *acc, int64_t batch, int64_t features, int dtype,
-                int bs_last, int act, hipStream_t stream)
+                int bs_last, int act, hipStream_t stream, FinishJob *rest)
 {
     const bool on = act != KSMM_ACT_NONE;
     const uintptr_t at = (uintptr_t)dy | (on ? (uintptr_t)z | (uintptr_t)dz : 0);
@@ -282,8 +282,8 @@ int act_bwd_run(const void *dy, const void *z, void *dz, void *dbias, float *acc
     else
         rc = on ? launch_vec<half_t, true>(vec, dy, z, dz, part, one, batch, features, p, bs_last, stream)
                 : launch_vec<half_t, false>(vec, dy, z, dz, part, one, batch, features, p, bs_last, stream);
-    if (rc != KSMM_OK || !part) return rc;
-    return slices_finish_run(acc, dbias, features, (int)p.splits, dtype, 1.f, stream);
+    *rest = FinishJob{acc, dbias, features, part ? (int)p.splits : 0, 1.f};
+    return rc;
 }
 
 }  // namespace ksmm

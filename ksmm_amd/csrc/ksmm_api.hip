@@ -686,6 +686,45 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
     return KSMM_OK;
 }
 
+// Offsets in the workspace of a layer's backward pass
+struct LayerBackward {
+    int64_t dz, bias_sums;               // gradient of what the activation was applied to; partial sums of the bias's
+    int64_t blocks[KSMM_MAX_FACTORS];    // transposed blocks of each factor
+    int64_t sums[KSMM_MAX_FACTORS];      // partial sums of each weight gradient: all are added at the end
+    int64_t grads[2];                    // gradients between factors
+    int64_t forward;                     // what the forward kernels of the transposed factors ask for
+};
+
+// bytes of it, or an error
+int64_t layer_backward_layout(const ksmm_factor_desc *f, int n, int64_t batch, int dtype, int bs_last, int act, LayerBackward *l)
+{
+    if (dtype != KSMM_F32 && dtype != KSMM_F16) return KSMM_ERR_BAD_DTYPE;
+    int rc = check_chain(f, n, batch, dtype, dtype);
+    if (rc != KSMM_OK) return rc;
+    const int64_t es = (int64_t)dtype_size(dtype), out = (int64_t)f[n - 1].a * f[n - 1].b * f[n - 1].d;
+    int64_t at = 0, widest = 0, forward = 0;
+    auto take = [&](int64_t bytes) {
+        const int64_t was = at;
+        at += align256(bytes);
+        return was;
+    };
+    l->dz = take(act != KSMM_ACT_NONE ? out * batch * es : 0);
+    l->bias_sums = take(4 * act_bwd_partial_floats(batch, out, dtype, bs_last));
+    for (int i = 0; i < n; ++i) {
+        l->blocks[i] = take((int64_t)f[i].a * f[i].b * f[i].c * f[i].d * es);
+        l->sums[i] = take(wgrad_partial_bytes(batch, f[i].a, f[i].b, f[i].c, f[i].d, dtype, bs_last));
+        const int64_t need = ksmm_factor_workspace(batch, f[i].a, f[i].c, f[i].b, f[i].d, dtype, dtype, dtype, bs_last);
+        if (need < 0) return need;
+        if (need > forward) forward = need;
+        const int64_t in = (int64_t)f[i].a * f[i].c * f[i].d;
+        if (i > 0 && in > widest) widest = in;
+    }
+    l->grads[0] = take(widest * batch * es);
+    l->grads[1] = take(widest * batch * es);
+    l->forward = take(forward);
+    return at;
+}
+
 // ---- scratch of ksmm_chain_forward_static ---------------------------------------------------
 // The device address of the array is asked for once per device, with that device current, and
 // kept; kernels and copies only ever see that address.
@@ -979,7 +1018,8 @@ int ksmm_factor_backward_input(const void *dy, const void *w, void *dx, int64_t 
     const int64_t nnz = (int64_t)a * b * c * d;
     char *wt = (char *)workspace;
     char *fwd_ws = wt + align256(nnz * (int64_t)dtype_size(dtype)) + wgrad_partial_bytes(batch, a, b, c, d, dtype, bs_last ? 1 : 0);
-    int rc = block_transpose_run(w, wt, a, b, c, d, dtype, (hipStream_t)stream);
+    const TransposeJob job{w, wt, (int64_t)a * d, b, c};
+    int rc = block_transpose_run(&job, 1, dtype, (hipStream_t)stream);
     if (rc != KSMM_OK) return rc;
     // dX = K^T dY: the factor with pattern (a, c, b, d) and transposed blocks
     return factor_forward_ws_impl(dy, wt, dx, batch, a, c, b, d, dtype, dtype, dtype, bs_last, scale, nullptr, fwd_ws,
@@ -996,7 +1036,9 @@ int ksmm_factor_backward_weight(const void *dy, const void *x, void *dw, int64_t
     if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15) != 0) return KSMM_ERR_WORKSPACE;
     const int64_t nnz = (int64_t)a * b * c * d;
     float *acc = (float *)((char *)workspace + align256(nnz * (int64_t)dtype_size(dtype)));
-    return wgrad_run(dy, x, dw, acc, batch, a, b, c, d, dtype, bs_last ? 1 : 0, scale, (hipStream_t)stream);
+    FinishJob rest;
+    const int rc = wgrad_run(dy, x, dw, acc, batch, a, b, c, d, dtype, bs_last ? 1 : 0, scale, (hipStream_t)stream, &rest);
+    return rc == KSMM_OK ? finish_run(&rest, 1, dtype, (hipStream_t)stream) : rc;
 }
 
 int64_t ksmm_epilogue_backward_workspace(int64_t batch, int64_t features, int dtype, int bs_last)
@@ -1017,7 +1059,72 @@ int ksmm_epilogue_backward(const void *dy, const void *z, void *dz, void *dbias,
     if (!dy || (act != KSMM_ACT_NONE && (!z || !dz))) return KSMM_ERR_NULL_POINTER;
     if (dbias && (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15) != 0)) return KSMM_ERR_WORKSPACE;
     if (!dbias && act == KSMM_ACT_NONE) return KSMM_OK;
-    return act_bwd_run(dy, z, dz, dbias, (float *)workspace, batch, features, dtype, bs_last ? 1 : 0, act, (hipStream_t)stream);
+    FinishJob rest;
+    const int rc = act_bwd_run(dy, z, dz, dbias, (float *)workspace, batch, features, dtype, bs_last ? 1 : 0, act, (hipStream_t)stream, &rest);
+    return rc == KSMM_OK ? finish_run(&rest, 1, dtype, (hipStream_t)stream) : rc;
+}
+
+int64_t ksmm_layer_backward_workspace(const ksmm_factor_desc *factors, int n_factors, int64_t batch, int dtype, int bs_last,
+                                      int act)
+{
+    LayerBackward l;
+    return layer_backward_layout(factors, n_factors, batch, dtype, bs_last ? 1 : 0, act, &l);
+}
+
+int ksmm_layer_backward(const ksmm_factor_desc *factors, int n_factors, const void *const *inputs, const void *z, const void *dy,
+                        void *dx, void *const *dw, void *dbias, void *workspace, int64_t workspace_bytes, int64_t batch, int dtype,
+                        int bs_last, int act, void *stream)
+{
+    LayerBackward l;
+    const int64_t need = layer_backward_layout(factors, n_factors, batch, dtype, bs_last ? 1 : 0, act, &l);
+    if (need < 0) return (int)need;
+    if (act != KSMM_ACT_NONE && act != KSMM_ACT_GELU) return KSMM_ERR_BAD_EPILOGUE;
+    if (!inputs || !dw || !dy || (act != KSMM_ACT_NONE && !z)) return KSMM_ERR_NULL_POINTER;
+    if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15) != 0) return KSMM_ERR_WORKSPACE;
+    int lowest = -1;  // the first factor that a gradient goes through or to
+    for (int i = n_factors - 1; i >= 0; --i) {
+        if (dw[i] && !inputs[i]) return KSMM_ERR_NULL_POINTER;
+        if (dw[i] || dx) lowest = i;
+    }
+    if (dx) lowest = 0;
+    char *ws = (char *)workspace;
+    const hipStream_t s = (hipStream_t)stream;
+    const ksmm_factor_desc &last = factors[n_factors - 1];
+    const int64_t out_size = (int64_t)last.a * last.b * last.d;
+    FinishJob rest[KSMM_MAX_FACTORS + 1];
+    TransposeJob flips[KSMM_MAX_FACTORS];
+    int jobs = 0, n_flips = 0, rc;
+    const void *grad = dy;
+    if (act != KSMM_ACT_NONE || dbias) {
+        void *dz = act != KSMM_ACT_NONE ? ws + l.dz : nullptr;
+        rc = act_bwd_run(dy, z, dz, dbias, (float *)(ws + l.bias_sums), batch, out_size, dtype, bs_last ? 1 : 0, act, s, &rest[jobs++]);
+        if (rc != KSMM_OK) return rc;
+        if (dz) grad = dz;
+    }
+    // factors whose input's gradient is needed: all behind the first one wanted, and that one for dx
+    for (int i = lowest < 0 ? n_factors : dx ? 0 : lowest + 1; i < n_factors; ++i) {
+        const ksmm_factor_desc &f = factors[i];
+        if (!f.w) return KSMM_ERR_NULL_POINTER;
+        flips[n_flips++] = TransposeJob{f.w, ws + l.blocks[i], (int64_t)f.a * f.d, f.b, f.c};
+    }
+    rc = block_transpose_run(flips, n_flips, dtype, s);
+    if (rc != KSMM_OK) return rc;
+    for (int i = n_factors - 1; i >= 0 && i >= lowest && lowest >= 0; --i) {
+        const ksmm_factor_desc &f = factors[i];
+        if (dw[i]) {
+            rc = wgrad_run(grad, inputs[i], dw[i], (float *)(ws + l.sums[i]), batch, f.a, f.b, f.c, f.d, dtype, bs_last ? 1 : 0,
+                           f.scale, s, &rest[jobs++]);
+            if (rc != KSMM_OK) return rc;
+        }
+        if (i == lowest && !dx) break;
+        void *to = i == 0 ? dx : ws + l.grads[i & 1];
+        // dX = K^T dY: the factor with pattern (a, c, b, d) and transposed blocks
+        rc = factor_forward_ws_impl(grad, ws + l.blocks[i], to, batch, f.a, f.c, f.b, f.d, dtype, dtype, dtype, bs_last, f.scale, nullptr,
+                                    ws + l.forward, workspace_bytes - l.forward, stream);
+        if (rc != KSMM_OK) return rc;
+        grad = to;
+    }
+    return finish_run(rest, jobs, dtype, s);
 }
 
 int64_t ksmm_static_scratch_bytes(void) { return KSMM_STATIC_SCRATCH_BYTES; }

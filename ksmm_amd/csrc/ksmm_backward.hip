@@ -22,50 +22,126 @@ namespace ksmm {
 namespace {
 
 // out block g (b x c, c contiguous)  <-  in block g (c x b, b contiguous); both in "kernel format"
-// of their own pattern: in = (a*d*c, b) of (a,b,c,d), out = (a*d*b, c) of (a,c,b,d)
-template <typename T>
-__global__ __launch_bounds__(256) void ks_block_transpose_kernel(const T *__restrict__ in, T *__restrict__ out,
-                                                                 int64_t total, int b, int c)
+// of their own pattern: in = (a*d*c, b) of (a,b,c,d), out = (a*d*b, c) of (a,c,b,d).  One launch takes
+// the weights of a whole layer.  A workgroup moves a 64 x 64 square through LDS, so that both sides are
+// whole lines; what bounds it is the launch.
+struct TransposeArgs {
+    struct {
+        const void *in;
+        void *out;
+        int b, c, b_tiles, c_tiles;
+        uint32_t first;  // the job's first workgroup
+    } job[KSMM_MAX_FACTORS];
+    int jobs;
+};
+
+template <typename T> __global__ __launch_bounds__(256) void ks_block_transpose_kernel(TransposeArgs t)
 {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;  // index into out
-    if (i >= total) return;
-    const int64_t g = i / ((int64_t)b * c);
-    const int rem = (int)(i - g * b * c);
-    const int bi = rem / c, ci = rem - bi * c;
-    out[i] = in[(g * c + ci) * b + bi];
+    __shared__ T square[64][64 + 4 / sizeof(T)];
+    int k = 0;
+    while (k + 1 < t.jobs && blockIdx.x >= t.job[k + 1].first) ++k;
+    const int b = t.job[k].b, c = t.job[k].c, bt = t.job[k].b_tiles, ct = t.job[k].c_tiles;
+    const T *in = (const T *)t.job[k].in;
+    T *out = (T *)t.job[k].out;
+    uint32_t id = blockIdx.x - t.job[k].first;
+    const int b0 = (int)(id % bt) * 64;
+    id /= bt;
+    const int c0 = (int)(id % ct) * 64;
+    const size_t block = (size_t)(id / ct) * b * c;
+    const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
+    if (b0 + x < b)
+#pragma unroll 4
+        for (int i = y; i < 64; i += 4)
+            if (c0 + i < c) square[i][x] = in[block + (size_t)(c0 + i) * b + b0 + x];
+    __syncthreads();
+    if (c0 + x < c)
+#pragma unroll 4
+        for (int i = y; i < 64; i += 4)
+            if (b0 + i < b) out[block + (size_t)(b0 + i) * c + c0 + x] = square[x][i];
 }
 
-// dw[i] = scale * (sum of the slices); slices are n floats apart.  A workgroup takes 64 outputs;
-// its G 64-thread groups add a G-th of the slices each, in slice order, and the G partial sums are
-// added in group order: the association is fixed by (splits) alone, so the result has the same bits
+// out[i] = scale * (sum of the slices); slices are n floats apart.  One launch takes all the sums of a
+// layer's backward pass: weight gradients and the bias's.  A workgroup's G groups of 256 / G threads add a
+// G-th of the slices each, in slice order, for V outputs a thread, and the G partial sums are added
+// in group order: the association is fixed by (splits) alone, so the result has the same bits
 // on every run.  What bounds it: the latency of a thread's loads, so eight are in flight, the last few
-// slices among them, and many slices (a bias gradient's: few outputs) are shared by more groups.
-// Six of these launches in a training step of a ViT-S feed-forward block (25088 rows, fp16): 38 us together, 44
-// with four groups and single loads at the end.
-template <typename T, int G>
-__global__ __launch_bounds__(64 * G) void ks_wgrad_finish_kernel(const float *__restrict__ acc, T *__restrict__ dw,
-                                                                 int64_t n, int splits, float scale)
+// slices among them, and many slices (a bias gradient's: few outputs) are shared by more groups; the launch
+// itself where the slices are few.
+struct FinishArgs {
+    struct {
+        const float *acc;
+        void *out;
+        int64_t n;
+        int splits;
+        float scale;
+        uint32_t first;  // the job's first workgroup
+    } job[KSMM_MAX_FACTORS + 1];
+    int jobs;
+};
+
+template <int V> struct FinishVec {
+    float v[V];
+};
+template <typename T, int G, int V>
+__device__ __forceinline__ void finish_part(const float *__restrict__ acc, T *__restrict__ out, int64_t n, int splits, float scale,
+                                            uint32_t block, float *part)
 {
-    __shared__ float part[G][64];
-    const int g = threadIdx.x >> 6, l = threadIdx.x & 63;
-    const int64_t i = (int64_t)blockIdx.x * 64 + l;
+    constexpr int LANES = 256 / G;
+    const int g = threadIdx.x / LANES, l = threadIdx.x % LANES;
+    const int64_t i = ((int64_t)block * LANES + l) * V;
     const int per = (splits + G - 1) / G, k0 = g * per, k1 = min(k0 + per, splits);
-    float s = 0.f;
-    if (i < n) {
+    float s[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) s[e] = 0.f;
+    if (i < n) {  // (V divides n)
         for (int k = k0; k < k1; k += 8) {
-            float v[8];
+            FinishVec<V> v[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = k + j < k1 ? acc[(int64_t)(k + j) * n + i] : 0.f;
+            for (int j = 0; j < 8; ++j) {
+                if (k + j < k1) __builtin_memcpy(&v[j], __builtin_assume_aligned(acc + (int64_t)(k + j) * n + i, 4 * V), 4 * V);
+                else v[j] = FinishVec<V>{};
+            }
 #pragma unroll
-            for (int j = 0; j < 8; ++j) s += v[j];
+            for (int j = 0; j < 8; ++j)
+#pragma unroll
+                for (int e = 0; e < V; ++e) s[e] += v[j].v[e];
         }
     }
-    part[g][l] = s;
+#pragma unroll
+    for (int e = 0; e < V; ++e) part[(e * G + g) * LANES + l] = s[e];
     __syncthreads();
     if (g || i >= n) return;
 #pragma unroll
-    for (int k = 1; k < G; ++k) s += part[k][l];
-    dw[i] = (T)(s * scale);
+    for (int e = 0; e < V; ++e) {
+#pragma unroll
+        for (int k = 1; k < G; ++k) s[e] += part[(e * G + k) * LANES + l];
+        out[i + e] = (T)(s[e] * scale);
+    }
+}
+
+// where the slices are shared by 16 groups: four have more than one round of loads each
+__host__ __device__ inline bool finish_wide(int splits) { return splits > 32; }
+// outputs per workgroup: a vector of four a thread where that divides n (slices stay aligned)
+__host__ __device__ inline int finish_outputs(int64_t n, int splits) { return (finish_wide(splits) ? 16 : 64) * (n % 4 == 0 ? 4 : 1); }
+
+template <typename T> __global__ __launch_bounds__(256) void ks_finish_kernel(FinishArgs f)
+{
+    __shared__ float part[4 * 256];
+    int k = 0;
+    while (k + 1 < f.jobs && blockIdx.x >= f.job[k + 1].first) ++k;
+    const float *acc = f.job[k].acc;
+    T *out = (T *)f.job[k].out;
+    const int64_t n = f.job[k].n;
+    const int splits = f.job[k].splits;
+    const float scale = f.job[k].scale;
+    const uint32_t block = blockIdx.x - f.job[k].first;
+    if (n % 4 == 0) {
+        if (finish_wide(splits)) finish_part<T, 16, 4>(acc, out, n, splits, scale, block, part);
+        else finish_part<T, 4, 4>(acc, out, n, splits, scale, block, part);
+    } else {
+        if (finish_wide(splits)) finish_part<T, 16, 1>(acc, out, n, splits, scale, block, part);
+        else finish_part<T, 4, 1>(acc, out, n, splits, scale, block, part);
+    }
 }
 
 // One 16-byte vector; ANY: at element alignment.  fp16 vectors at odd elements come as aligned words
@@ -254,15 +330,6 @@ __global__ __launch_bounds__(256) void ks_wgrad_tiled_kernel(const T *__restrict
     }
     const int m = mt * 16 + tx, cc = nt * 16 + ty;  // consecutive threads: consecutive b_i (contiguous in dW)
     if (m < b && cc < c) acc_out[(size_t)split * slice + ((size_t)g * c + cc) * b + m] = acc;
-}
-
-template <typename T> int launch_block_transpose(const void *w, void *wt, int64_t total, int b, int c, hipStream_t s)
-{
-    const int64_t blocks = (total + 255) / 256;
-    if (blocks > 0x7fffffffLL) return KSMM_ERR_TOO_LARGE;
-    hipLaunchKernelGGL((ks_block_transpose_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, s, (const T *)w, (T *)wt,
-                       total, b, c);
-    return hipGetLastError() == hipSuccess ? KSMM_OK : KSMM_ERR_LAUNCH;
 }
 
 // Batch splits of the two weight-gradient kernels (every split is non-empty and writes a slice of
@@ -501,16 +568,31 @@ int launch_wgrad_gemm(const void *dy, const void *x, float *acc, int64_t batch, 
 
 }  // namespace
 
-// wt <- the b x c blocks of w transposed: kernel format (a*d*b, c) of pattern (a, c, b, d)
-int block_transpose_run(const void *w, void *wt, int a, int b, int c, int d, int dtype, hipStream_t stream)
+// the b x c blocks of each job's w transposed: kernel format (a*d*b, c) of pattern (a, c, b, d)
+int block_transpose_run(const TransposeJob *jobs, int n, int dtype, hipStream_t stream)
 {
-    const int64_t total = (int64_t)a * b * c * d;
-    switch (dtype) {
-    case KSMM_F32: return launch_block_transpose<float>(w, wt, total, b, c, stream);
-    case KSMM_F16: return launch_block_transpose<half_t>(w, wt, total, b, c, stream);
-    case KSMM_FP8_E4M3: return launch_block_transpose<uint8_t>(w, wt, total, b, c, stream);
-    default: return KSMM_ERR_BAD_DTYPE;
+    TransposeArgs t;
+    int64_t blocks = 0;
+    t.jobs = n;
+    for (int i = 0; i < n; ++i) {
+        const TransposeJob &j = jobs[i];
+        auto &o = t.job[i];
+        o.in = j.w;
+        o.out = j.wt;
+        o.b = j.b;
+        o.c = j.c;
+        o.b_tiles = (j.b + 63) / 64;
+        o.c_tiles = (j.c + 63) / 64;
+        o.first = (uint32_t)blocks;
+        blocks += j.blocks * o.b_tiles * o.c_tiles;
+        if (blocks > 0x7fffffffLL) return KSMM_ERR_TOO_LARGE;
     }
+    if (n < 1) return KSMM_OK;
+    if (dtype == KSMM_F32)
+        hipLaunchKernelGGL((ks_block_transpose_kernel<float>), dim3((unsigned)blocks), dim3(256), 0, stream, t);
+    else
+        hipLaunchKernelGGL((ks_block_transpose_kernel<half_t>), dim3((unsigned)blocks), dim3(256), 0, stream, t);
+    return hipGetLastError() == hipSuccess ? KSMM_OK : KSMM_ERR_LAUNCH;
 }
 
 // Floats of partial sums the weight gradient of this problem writes (slices of a*b*c*d, one per
@@ -533,34 +615,44 @@ int64_t wgrad_partial_floats(int64_t batch, int a, int b, int c, int d, int dtyp
     return most * n;
 }
 
-// out[i] (type `dtype`, i < n) <- scale * the sum of acc's slices of n floats
-template <typename T> int launch_finish(const float *acc, void *out, int64_t n, int splits, float scale, hipStream_t stream)
+// out[i] (type `dtype`, i < n) of each job <- scale * the sum of its slices of n floats
+int finish_run(const FinishJob *jobs, int n, int dtype, hipStream_t stream)
 {
-    const int64_t blocks = (n + 63) / 64;
-    if (blocks > 0x7fffffffLL) return KSMM_ERR_TOO_LARGE;
-    // four groups have more than one round of loads each
-    if (splits > 32)
-        hipLaunchKernelGGL((ks_wgrad_finish_kernel<T, 16>), dim3((unsigned)blocks), dim3(1024), 0, stream, acc, (T *)out, n, splits, scale);
+    FinishArgs f;
+    int64_t blocks = 0;
+    f.jobs = 0;
+    for (int i = 0; i < n; ++i) {
+        const FinishJob &j = jobs[i];
+        if (j.splits < 1) continue;  // complete already
+        auto &o = f.job[f.jobs++];
+        o.acc = j.acc;
+        o.out = j.out;
+        o.n = j.n;
+        o.splits = j.splits;
+        o.scale = j.scale;
+        o.first = (uint32_t)blocks;
+        const int64_t per = finish_outputs(j.n, j.splits);
+        blocks += (j.n + per - 1) / per;
+        if (blocks > 0x7fffffffLL) return KSMM_ERR_TOO_LARGE;
+    }
+    if (f.jobs < 1) return KSMM_OK;
+    if (dtype == KSMM_F32)
+        hipLaunchKernelGGL((ks_finish_kernel<float>), dim3((unsigned)blocks), dim3(256), 0, stream, f);
     else
-        hipLaunchKernelGGL((ks_wgrad_finish_kernel<T, 4>), dim3((unsigned)blocks), dim3(256), 0, stream, acc, (T *)out, n, splits, scale);
+        hipLaunchKernelGGL((ks_finish_kernel<half_t>), dim3((unsigned)blocks), dim3(256), 0, stream, f);
     return hipGetLastError() == hipSuccess ? KSMM_OK : KSMM_ERR_LAUNCH;
 }
 
-int slices_finish_run(const float *acc, void *out, int64_t n, int splits, int dtype, float scale, hipStream_t stream)
-{
-    return dtype == KSMM_F32 ? launch_finish<float>(acc, out, n, splits, scale, stream)
-                             : launch_finish<half_t>(acc, out, n, splits, scale, stream);
-}
-
 // dw (kernel format, type `dtype`) <- scale * sum over the batch of dY x X^T per block; acc is an
-// fp32 buffer of wgrad_partial_floats() elements.
+// fp32 buffer of wgrad_partial_floats() elements.  dw is complete once *rest has been finished.
 int wgrad_run(const void *dy, const void *x, void *dw, float *acc, int64_t batch, int a, int b, int c, int d,
-              int dtype, int bs_last, float scale, hipStream_t stream)
+              int dtype, int bs_last, float scale, hipStream_t stream, FinishJob *rest)
 {
     const int64_t n = (int64_t)a * b * c * d;
     const bool mfma_ok = wgrad_mfma_ok(batch, dtype, bs_last);
     const int t = wgrad_bl_tile(b, c);
     int rc, splits = 1;
+    *rest = FinishJob{acc, dw, n, 0, scale};
     if (!bs_last && wgrad_bf_ok(a, b, c, d, dtype)) {
         rc = wgrad_bf_run(dy, x, dw, acc, batch, a, b, c, d, dtype, scale, stream, &splits);
         if (rc != KSMM_OK || splits == 1) return rc;
@@ -585,8 +677,8 @@ int wgrad_run(const void *dy, const void *x, void *dw, float *acc, int64_t batch
     } else {
         return KSMM_ERR_BAD_DTYPE;
     }
-    if (rc != KSMM_OK) return rc;
-    return slices_finish_run(acc, dw, n, splits, dtype, scale, stream);
+    rest->splits = splits;
+    return rc;
 }
 
 }  // namespace ksmm

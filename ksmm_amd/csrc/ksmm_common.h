@@ -197,23 +197,37 @@ int gemm_run(const Problem &p, int variant, bool launch, ksmm_tile *tile);  // p
 int tile_bf_run(const Problem &p, int variant, bool launch, ksmm_tile *tile);  // part of the tile family
 int split_run(const Problem &p, int variant, bool launch, ksmm_tile *tile);  // part of the tile family
 
-// Backward pass pieces (ksmm_backward.hip): blockwise transpose of a kernel-format weight, and the
-// weight gradient (acc: fp32 scratch of wgrad_partial_floats() elements, one slice of a*b*c*d per
-// batch split).
-int block_transpose_run(const void *w, void *wt, int a, int b, int c, int d, int dtype, hipStream_t stream);
+// Backward pass pieces (ksmm_backward.hip): blockwise transposes of kernel-format weights, the weight
+// gradient (acc: fp32 scratch of wgrad_partial_floats() elements, one slice of a*b*c*d per
+// batch split), and the sums of such slices, each for a whole layer in one launch.
+struct TransposeJob {
+    const void *w;
+    void *wt;
+    int64_t blocks;  // a * d of them
+    int b, c;
+};
+int block_transpose_run(const TransposeJob *jobs, int n, int dtype, hipStream_t stream);
+struct FinishJob {
+    const float *acc;
+    void *out;
+    int64_t n;
+    int splits;  // 0: nothing to do
+    float scale;
+};
+int finish_run(const FinishJob *jobs, int n, int dtype, hipStream_t stream);
 int64_t wgrad_partial_floats(int64_t batch, int a, int b, int c, int d, int dtype, int bs_last);
 int wgrad_run(const void *dy, const void *x, void *dw, float *acc, int64_t batch, int a, int b, int c, int d,
-              int dtype, int bs_last, float scale, hipStream_t stream);
+              int dtype, int bs_last, float scale, hipStream_t stream, FinishJob *rest);
 // Batch-size-first weight gradient (ksmm_wgrad_bf.hip)
 bool wgrad_bf_ok(int a, int b, int c, int d, int dtype);
 int64_t wgrad_bf_partial_floats(int64_t batch, int a, int b, int c, int d, int dtype);
 int wgrad_bf_run(const void *dy, const void *x, void *dw, float *acc, int64_t batch, int a, int b, int c, int d, int dtype,
                  float scale, hipStream_t stream, int *splits);
-int slices_finish_run(const float *acc, void *out, int64_t n, int splits, int dtype, float scale, hipStream_t stream);
-// Backward pass of the epilogue (ksmm_act_bwd.hip; acc: fp32 scratch of act_bwd_partial_floats() elements)
+// Backward pass of the epilogue (ksmm_act_bwd.hip; acc: fp32 scratch of act_bwd_partial_floats() elements);
+// dbias is complete once *rest has been finished
 int64_t act_bwd_partial_floats(int64_t batch, int64_t features, int dtype, int bs_last);
 int act_bwd_run(const void *dy, const void *z, void *dz, void *dbias, float *acc, int64_t batch, int64_t features, int dtype,
-                int bs_last, int act, hipStream_t stream);
+                int bs_last, int act, hipStream_t stream, FinishJob *rest);
 
 // Fused radix-16 chain (intermediates in LDS); KSMM_ERR_BAD_ALGO when the chain does not qualify.
 // out (cols x rows) = transpose of in (rows x cols); pitches in elements per row, 0 = dense

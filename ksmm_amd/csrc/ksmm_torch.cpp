@@ -58,12 +58,12 @@ struct Layer {
     int64_t in_size = 0, out_size = 0;
 };
 
-// factor tensors (an iterable of them), patterns (tuple of 4-tuples) and scales (list of floats)
+// factor tensors, patterns (4-tuples) and scales (floats), lists of them; scales may be null: 1 each
 bool read_layer(PyObject *params, PyObject *patterns, PyObject *scales, const at::Device &dev, Layer *l)
 {
-    if (!PyList_Check(params) || !PyList_Check(patterns) || !PyList_Check(scales)) return false;
+    if (!PyList_Check(params) || !PyList_Check(patterns) || (scales && !PyList_Check(scales))) return false;
     const Py_ssize_t n = PyList_GET_SIZE(params);
-    if (n < 1 || n > KSMM_MAX_FACTORS || PyList_GET_SIZE(patterns) != n || PyList_GET_SIZE(scales) != n) return false;
+    if (n < 1 || n > KSMM_MAX_FACTORS || PyList_GET_SIZE(patterns) != n || (scales && PyList_GET_SIZE(scales) != n)) return false;
     for (Py_ssize_t i = 0; i < n; ++i) {
         PyObject *w = PyList_GET_ITEM(params, i), *p = PyList_GET_ITEM(patterns, i);
         if (!THPVariable_Check(w) || !PyTuple_Check(p) || PyTuple_GET_SIZE(p) != 4) return false;
@@ -79,7 +79,7 @@ bool read_layer(PyObject *params, PyObject *patterns, PyObject *scales, const at
         f.c = (int)v[2];
         f.d = (int)v[3];
         f.w_dtype = code_of(t.scalar_type());
-        const double s = PyFloat_AsDouble(PyList_GET_ITEM(scales, i));
+        const double s = scales ? PyFloat_AsDouble(PyList_GET_ITEM(scales, i)) : 1.0;
         if (s == -1.0 && PyErr_Occurred()) return false;
         f.scale = (float)s;
         if (f.w_dtype < 0 || t.device() != dev || !t.is_contiguous() || t.dim() != 2 || t.size(0) != v[0] * v[2] * v[3] ||
@@ -179,7 +179,162 @@ PyObject *py_infer(PyObject *, PyObject *const *args, Py_ssize_t n)
     Py_RETURN_NONE;
 }
 
+bool trainable(at::ScalarType t) { return t == at::kFloat || t == at::kHalf; }
+
+// every factor of type t and in line with its neighbours (a chain's own check comes too late for the intermediates' sizes)
+bool of_type(const Layer &l, at::ScalarType t)
+{
+    for (int i = 0; i < l.n; ++i) {
+        if (l.f[i].w_dtype != code_of(t)) return false;
+        if (i > 0 && (int64_t)l.f[i].a * l.f[i].c * l.f[i].d != (int64_t)l.f[i - 1].a * l.f[i - 1].b * l.f[i - 1].d) return false;
+    }
+    return true;
+}
+
+PyObject *wrapped(const at::Tensor &t)
+{
+    if (t.defined()) return THPVariable_Wrap(t);
+    Py_RETURN_NONE;
+}
+
+// train_forward(x, factors, patterns, bs_last, bias, act) -> (y, what each factor but the first was applied to.., z) or
+// None; z is what the activation was applied to (None without one).
+PyObject *py_train_forward(PyObject *, PyObject *const *args, Py_ssize_t n_args)
+{
+    if (n_args != 6) {
+        PyErr_SetString(PyExc_TypeError, "train_forward() takes 6 arguments");
+        return nullptr;
+    }
+    try {
+        if (!THPVariable_Check(args[0])) Py_RETURN_NONE;
+        const at::Tensor &x = THPVariable_Unpack(args[0]);
+        const bool bs_last = PyObject_IsTrue(args[3]) == 1;
+        Layer l;
+        int64_t batch;
+        c10::SmallVector<int64_t, 6> shape;
+        ksmm_epilogue ep;
+        if (x.is_cuda() && x.dim() == 2 && trainable(x.scalar_type()) && read_layer(args[1], args[2], nullptr, x.device(), &l) &&
+            of_type(l, x.scalar_type()) && result_shape(x, bs_last, l, &batch, &shape) &&
+            read_epilogue(args[4], args[5], x.device(), x.scalar_type(), l.out_size, &ep)) {
+            const int dt = code_of(x.scalar_type());
+            at::Tensor out[KSMM_MAX_FACTORS], y;
+            int status = KSMM_OK;
+            {
+                WithoutGil released;
+                DeviceScope scope(x.device().index());
+                void *const stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
+                const ksmm_epilogue bias_only{ep.bias, KSMM_ACT_NONE};
+                const void *in = x.const_data_ptr();
+                for (int i = 0; i < l.n && status == KSMM_OK; ++i) {
+                    const ksmm_factor_desc &f = l.f[i];
+                    const int64_t size = (int64_t)f.a * f.b * f.d;
+                    const int64_t need = ksmm_factor_workspace(batch, f.a, f.b, f.c, f.d, dt, dt, dt, bs_last);
+                    if (need < 0) {
+                        status = (int)need;
+                        break;
+                    }
+                    out[i] = at::empty({bs_last ? size : batch, bs_last ? batch : size}, x.options());
+                    at::Tensor ws;
+                    if (need > 0) ws = at::empty({need}, x.options().dtype(at::kByte));
+                    status = ksmm_factor_forward_ep(in, f.w, out[i].mutable_data_ptr(), batch, f.a, f.b, f.c, f.d, dt, dt, dt, bs_last, 1.f,
+                                                    i + 1 == l.n && ep.bias ? &bias_only : nullptr,
+                                                    need > 0 ? ws.mutable_data_ptr() : nullptr, need, stream);
+                    in = out[i].const_data_ptr();
+                }
+                if (status == KSMM_OK) y = ep.act ? at::gelu(out[l.n - 1]) : out[l.n - 1];
+            }
+            if (status == KSMM_OK) {
+                PyObject *r = PyTuple_New(l.n + 1);
+                if (!r) return nullptr;
+                PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(y));
+                for (int i = 0; i + 1 < l.n; ++i) PyTuple_SET_ITEM(r, i + 1, THPVariable_Wrap(out[i]));
+                PyTuple_SET_ITEM(r, l.n, wrapped(ep.act ? out[l.n - 1] : at::Tensor()));
+                return r;
+            }
+        }
+    } catch (const std::exception &) {
+    }
+    PyErr_Clear();
+    Py_RETURN_NONE;
+}
+
+// train_backward(grad, factors, patterns, inputs, z, bs_last, act, need_x, need_bias, need_factors) -> (grad_x, grad_bias, [grad_factors])
+// or None; lists but for grad, z (None without an activation) and need_factors (a tuple).  What is not needed is None.
+PyObject *py_train_backward(PyObject *, PyObject *const *args, Py_ssize_t n_args)
+{
+    if (n_args != 10) {
+        PyErr_SetString(PyExc_TypeError, "train_backward() takes 10 arguments");
+        return nullptr;
+    }
+    try {
+        if (!THPVariable_Check(args[0])) Py_RETURN_NONE;
+        const at::Tensor &grad = THPVariable_Unpack(args[0]);
+        const bool bs_last = PyObject_IsTrue(args[5]) == 1, need_x = PyObject_IsTrue(args[7]) == 1, need_bias = PyObject_IsTrue(args[8]) == 1;
+        Layer l;
+        ksmm_epilogue ep;
+        bool taken = grad.is_cuda() && grad.dim() == 2 && grad.is_contiguous() && grad.numel() > 0 && trainable(grad.scalar_type()) &&
+                     read_layer(args[1], args[2], nullptr, grad.device(), &l) && of_type(l, grad.scalar_type()) &&
+                     read_epilogue(Py_None, args[6], grad.device(), grad.scalar_type(), l.out_size, &ep) &&
+                     grad.size(bs_last ? 0 : 1) == l.out_size && PyList_Check(args[3]) && PyList_GET_SIZE(args[3]) == l.n &&
+                     PyTuple_Check(args[9]) && PyTuple_GET_SIZE(args[9]) == l.n;
+        const int64_t batch = taken ? grad.size(bs_last ? 1 : 0) : 0;
+        const void *inputs[KSMM_MAX_FACTORS], *z = nullptr;
+        bool need[KSMM_MAX_FACTORS];
+        // a tensor of the pass: the gradient's type, as many features as factor i takes (i == n: as the layer gives)
+        auto fits = [&](PyObject *o, int i, const void **p) {
+            if (!THPVariable_Check(o)) return false;
+            const at::Tensor &t = THPVariable_Unpack(o);
+            const int64_t size = i == l.n ? l.out_size : (int64_t)l.f[i].a * l.f[i].c * l.f[i].d;
+            *p = t.scalar_type() == grad.scalar_type() && t.device() == grad.device() && t.dim() == 2 && t.is_contiguous() &&
+                         t.size(bs_last ? 0 : 1) == size && t.size(bs_last ? 1 : 0) == batch
+                     ? t.const_data_ptr() : nullptr;
+            return *p != nullptr;
+        };
+        for (int i = 0; taken && i < l.n; ++i) {
+            need[i] = PyObject_IsTrue(PyTuple_GET_ITEM(args[9], i)) == 1;
+            taken = fits(PyList_GET_ITEM(args[3], i), i, &inputs[i]);
+        }
+        if (taken && ep.act) taken = fits(args[4], l.n, &z);
+        if (taken) {
+            const int dt = code_of(grad.scalar_type());
+            at::Tensor dx, dbias, dw[KSMM_MAX_FACTORS];
+            int status;
+            {
+                WithoutGil released;
+                DeviceScope scope(grad.device().index());
+                const int64_t bytes = ksmm_layer_backward_workspace(l.f, l.n, batch, dt, bs_last, ep.act);
+                status = bytes < 0 ? (int)bytes : KSMM_OK;
+                if (status == KSMM_OK) {
+                    const auto opts = grad.options();
+                    void *to[KSMM_MAX_FACTORS];
+                    if (need_x) dx = at::empty({bs_last ? l.in_size : batch, bs_last ? batch : l.in_size}, opts);
+                    if (need_bias) dbias = bs_last ? at::empty({l.out_size, 1}, opts) : at::empty({l.out_size}, opts);
+                    for (int i = 0; i < l.n; ++i) {
+                        if (need[i]) dw[i] = at::empty({(int64_t)l.f[i].a * l.f[i].c * l.f[i].d, l.f[i].b}, opts);
+                        to[i] = need[i] ? dw[i].mutable_data_ptr() : nullptr;
+                    }
+                    const at::Tensor ws = at::empty({bytes}, opts.dtype(at::kByte));
+                    status = ksmm_layer_backward(l.f, l.n, inputs, z, grad.const_data_ptr(), need_x ? dx.mutable_data_ptr() : nullptr, to,
+                                                 need_bias ? dbias.mutable_data_ptr() : nullptr, ws.mutable_data_ptr(), bytes, batch, dt,
+                                                 bs_last, ep.act, c10::hip::getCurrentHIPStream(grad.device().index()).stream());
+                }
+            }
+            if (status == KSMM_OK) {
+                PyObject *ws = PyList_New(l.n);
+                if (!ws) return nullptr;
+                for (int i = 0; i < l.n; ++i) PyList_SET_ITEM(ws, i, wrapped(dw[i]));
+                return Py_BuildValue("(NNN)", wrapped(dx), wrapped(dbias), ws);
+            }
+        }
+    } catch (const std::exception &) {
+    }
+    PyErr_Clear();
+    Py_RETURN_NONE;
+}
+
 PyMethodDef methods[] = {
+    {"train_forward", (PyCFunction)(void (*)(void))py_train_forward, METH_FASTCALL, "one layer, its intermediates kept"},
+    {"train_backward", (PyCFunction)(void (*)(void))py_train_backward, METH_FASTCALL, "gradients of one layer"},
     {"infer", (PyCFunction)(void (*)(void))py_infer, METH_FASTCALL, "one layer without gradients"},
     {nullptr, nullptr, 0, nullptr},
 };

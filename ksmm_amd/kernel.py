@@ -280,7 +280,8 @@ class KSLayerFunction(torch.autograd.Function):
     with an activation (result, what the activation was applied to).
 
     Against ``layer_by_factors`` it adds the bias in the last factor's kernel and takes the gradients
-    of activation and bias in one pass.  Per tensor of the result that is two reads and two writes less."""
+    of activation and bias in one pass.  Per tensor of the result that is two reads and two writes less.
+    Both directions are one native call each where that takes the tensors."""
 
     @staticmethod
     def takes(x, bias, patterns, bs_last):
@@ -296,16 +297,19 @@ class KSLayerFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, bias, act, bs_last, patterns, *factors):
         ctx.act, ctx.bs_last, ctx.patterns = act, bs_last, patterns
-        inputs, last = [x], len(factors) - 1
-        for i, (f, p) in enumerate(zip(factors, patterns)):
-            inputs.append(Kernel.forward(inputs[-1], f, bs_last, *p, bias=bias if i == last else None))
-        z = inputs.pop()
+        done = _lib.native().train_forward(x, [*factors], patterns, bs_last, bias, act)
+        if done is None:
+            inputs, last = [x], len(factors) - 1
+            for i, (f, p) in enumerate(zip(factors, patterns)):
+                inputs.append(Kernel.forward(inputs[-1], f, bs_last, *p, bias=bias if i == last else None))
+            z = inputs.pop()
+            done = (F.gelu(z) if act else z, *inputs[1:], z if act else None)
         # (the bias is not saved: no gradient needs its values, and it may change before the backward pass)
-        ctx.save_for_backward(*factors, *inputs, z if act else None)
+        ctx.save_for_backward(*factors, x, *done[1:])
         if not act:
-            return z
+            return done[0]
         ctx.set_materialize_grads(False)
-        return F.gelu(z), z
+        return done[0], done[-1]
 
     @staticmethod
     def backward(ctx, grad_y, grad_z=None):
@@ -328,6 +332,10 @@ class KSLayerFunction(torch.autograd.Function):
         if again and need_bias:
             grad_bias = grad.sum(1, keepdim=True) if bs_last else grad.sum(0)
         grad = grad.contiguous()
+        done = _lib.native().train_backward(grad, [*factors], ctx.patterns, [*inputs], z, bs_last, act, need_x,
+                                            need_bias and not again, need_factors)
+        if done is not None:
+            return (done[0], grad_bias if again else done[1], None, None, None, *done[2])
         if act or (need_bias and not again):
             grad, grad_bias = Kernel.epilogue_backward(grad, z, bs_last, act, need_bias)
             grad_bias = grad_bias.unsqueeze(1) if need_bias and bs_last else grad_bias

@@ -2,7 +2,7 @@
 // to nearest even.  The scale stays on the device: the first factor's kernel reads it (Epi::x_scale), so
 // nothing waits for the GPU.
 //
-// Two passes over the input.  What bounds them: HBM (or the cache that the layer before left the input in),
+// Two passes over the input, in one launch where it is small.  What bounds them: HBM (or the cache that the layer before left the input in),
 // 2 + 2 + 1 bytes a value in fp16.  The same steps as tensor operations (to fp32, abs, max, compare, select,
 // divide, to e4m3) move about 40 bytes a value, and reading the scale on the host waits for them: a ViT-B
 // feed-forward block on 6304 rows took 324 us with them and takes 111, 30 of them here (6304 x 3072 fp16:
@@ -43,22 +43,23 @@ template <> __device__ __forceinline__ uint32_t as_f32_bits<half_t>(uint32_t m)
     return __builtin_bit_cast(uint32_t, (float)__builtin_bit_cast(half_t, h));
 }
 
-__device__ __forceinline__ uint32_t block_max(uint32_t m, uint32_t *red)
+// largest value over a workgroup of W waves
+template <int W> __device__ __forceinline__ uint32_t block_max(uint32_t m, uint32_t *red)
 {
 #pragma unroll
     for (int s = 32; s; s >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, s, 64));
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
-    return max(max(red[0], red[1]), max(red[2], red[3]));
+#pragma unroll
+    for (int w = 0; w < W; ++w) m = max(m, red[w]);
+    return m;
 }
 
+// Largest magnitude (its bits in fp32) of the values that thread `me` of `stride` takes.
 // ALIGNED: x starts on a 16-byte boundary (else single elements)
-template <typename T, bool ALIGNED>
-__global__ __launch_bounds__(256) void ks_amax_kernel(const T *__restrict__ x, uint32_t *__restrict__ part, int64_t n)
+template <typename T, bool ALIGNED> __device__ __forceinline__ uint32_t max_of(const T *__restrict__ x, int64_t n, int64_t me, int64_t stride)
 {
     constexpr int N = qvec<T>::N, U = 4;
-    __shared__ uint32_t red[4];
-    const int64_t stride = (int64_t)gridDim.x * 256, me = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int64_t vecs = ALIGNED ? n / N : 0;
     const uint4_t *xv = (const uint4_t *)x;
     uint32_t m = 0;
@@ -82,7 +83,14 @@ __global__ __launch_bounds__(256) void ks_amax_kernel(const T *__restrict__ x, u
         const float v = (float)x[k];
         m = max(m, __builtin_bit_cast(uint32_t, v) & 0x7fffffffu);
     }
-    m = block_max(m, red);
+    return m;
+}
+
+template <typename T, bool ALIGNED>
+__global__ __launch_bounds__(256) void ks_amax_kernel(const T *__restrict__ x, uint32_t *__restrict__ part, int64_t n)
+{
+    __shared__ uint32_t red[4];
+    const uint32_t m = block_max<4>(max_of<T, ALIGNED>(x, n, (int64_t)blockIdx.x * 256 + threadIdx.x, (int64_t)gridDim.x * 256), red);
     if (threadIdx.x == 0) part[blockIdx.x] = m;
 }
 
@@ -106,18 +114,14 @@ __device__ __forceinline__ float quotient(float t, float scale, float r)
     return copysignf(q, t);
 }
 
+// codes of the whole tensor for its largest magnitude (the bits of it); one run a thread at a time
 template <typename T, bool ALIGNED>
-__global__ __launch_bounds__(256) void ks_quant_kernel(const T *__restrict__ x, uint8_t *__restrict__ q,
-                                                       const uint32_t *__restrict__ part, int parts, float *__restrict__ scale_out,
-                                                       int64_t n)
+__device__ __forceinline__ void quant_all(const T *__restrict__ x, uint8_t *__restrict__ q, uint32_t max_f32, float *__restrict__ scale_out,
+                                          int64_t n, int64_t me, int64_t stride)
 {
     constexpr int N = qvec<T>::N, LOADS = qvec<T>::LOADS;
-    __shared__ uint32_t red[4];
-    uint32_t m = 0;
-    for (int i = threadIdx.x; i < parts; i += 256) m = max(m, part[i]);
-    const float amax = __builtin_bit_cast(float, block_max(m, red));
+    const float amax = __builtin_bit_cast(float, max_f32);
     const float scale = amax > 0.f ? amax * (1.0f / 448.0f) : 1.0f;
-    const int64_t stride = (int64_t)gridDim.x * 256, me = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (me == 0) *scale_out = scale;
     const int64_t runs = ALIGNED ? n / RUN : 0;
     // A division is ten instructions, a quarter-rate one among them, and bounded the codes.  For ordinary scales
@@ -149,9 +153,42 @@ __global__ __launch_bounds__(256) void ks_quant_kernel(const T *__restrict__ x, 
     for (int64_t k = runs * RUN + me; k < n; k += stride) q[k] = (uint8_t)quant_code((float)x[k], scale);
 }
 
+template <typename T, bool ALIGNED>
+__global__ __launch_bounds__(256) void ks_quant_kernel(const T *__restrict__ x, uint8_t *__restrict__ q,
+                                                       const uint32_t *__restrict__ part, int parts, float *__restrict__ scale_out,
+                                                       int64_t n)
+{
+    __shared__ uint32_t red[4];
+    uint32_t m = 0;
+    for (int i = threadIdx.x; i < parts; i += 256) m = max(m, part[i]);
+    m = block_max<4>(m, red);
+    quant_all<T, ALIGNED>(x, q, m, scale_out, n, (int64_t)blockIdx.x * 256 + threadIdx.x, (int64_t)gridDim.x * 256);
+}
+
+// Both passes of a small tensor in one launch: every workgroup looks for the maximum itself.  What bounds it up to
+// 64 KB is the launch, then one CU's rate of loads from L2 (about 100 GB/s).
+template <typename T>
+__global__ __launch_bounds__(1024) void ks_quant_small_kernel(const T *__restrict__ x, uint8_t *__restrict__ q, float *__restrict__ scale_out,
+                                                              int n)
+{
+    __shared__ uint32_t red[16];
+    const uint32_t m = block_max<16>(max_of<T, true>(x, n, threadIdx.x, 1024), red);
+    quant_all<T, true>(x, q, m, scale_out, n, blockIdx.x * 1024 + threadIdx.x, gridDim.x * 1024);
+}
+
+// Bytes up to which one launch is the faster.  Layers of (4,64,64,1) / (1,128,128,16), us a call with two launches and
+// with one: fp16 64 KB 11.5 / 11.4 and 9.7 / 8.9, 256 KB 11.6 / 11.5 and 10.8 / 9.4, 384 KB 14.7 / 13.2 and 12.5 / 10.9,
+// 512 KB 13.4 / 13.2 and 13.0 / 11.7, 768 KB 13.3 / 13.3 and 14.7 / 13.5; fp32 within 0.5 of these.
+constexpr int64_t SMALL_BYTES = 384 << 10;
+
 template <typename T> int launch(const void *x, void *q, uint32_t *part, float *scale, int64_t n, hipStream_t s)
 {
     const bool aligned = ((uintptr_t)x & 15) == 0;
+    if (aligned && n * (int64_t)sizeof(T) <= SMALL_BYTES) {
+        const int64_t blocks = (n + 1024 * RUN - 1) / (1024 * RUN);
+        hipLaunchKernelGGL(ks_quant_small_kernel<T>, dim3((unsigned)blocks), dim3(1024), 0, s, (const T *)x, (uint8_t *)q, scale, (int)n);
+        return hipGetLastError() == hipSuccess ? KSMM_OK : KSMM_ERR_LAUNCH;
+    }
     // first pass: four vectors a thread, four workgroups a CU at most; second: one run a thread
     int64_t parts = (n + 256 * 4 * qvec<T>::N - 1) / (256 * 4 * qvec<T>::N), blocks = (n + 256 * RUN - 1) / (256 * RUN);
     if (parts > QUANT_BLOCKS) parts = QUANT_BLOCKS;

@@ -30,6 +30,24 @@ def test_quantised_inputs_give_the_same_bits(dt, bs_last):
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.float16])
+def test_one_launch_and_two_give_the_same_codes(dt):
+    """Sizes around the 384 KB up to which one launch takes the input, whole runs of 16 values and not; the largest
+    value is the last, which the last thread alone sees."""
+    from ksmm_amd import KSLinear, quantize_fp8
+
+    edge = (384 << 10) // (2 if dt == torch.float16 else 4)
+    w = torch.eye(8).reshape(1, 8, 8, 1)
+    with torch.no_grad():
+        layer = KSLinear([(1, 8, 8, 1)], weights=[w], bias=False, algo="kernel", dtype=FP8, device="cuda")
+        for rows in (1, 2, 3, 2049, edge // 8 - 1, edge // 8, edge // 8 + 1):
+            x = torch.randn(rows, 8, device="cuda").to(dt)
+            x[-1, -1] = -9.5
+            codes, scale = quantize_fp8(x)
+            assert float(scale) == pytest.approx(9.5 / 448, rel=1e-3)
+            assert torch.equal(layer(x), layer(codes, x_scale=float(scale))), rows
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16])
 def test_quantisation_of_special_values(dt):
     """Zeros, one value, infinities, NaN, denormals, halfway codes: a layer of the identity shows the codes."""
     from ksmm_amd import KSLinear, quantize_fp8

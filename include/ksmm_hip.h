@@ -235,6 +235,12 @@ int ksmm_chain_forward_ep(const ksmm_factor_desc *factors, int n_factors, const 
                           int y_dtype, int bs_last, int fuse, const ksmm_epilogue *epilogue,
                           void *stream);
 
+/* The chain in one launch that needs no workspace, where that is the fastest way through it (radix-16 chains of at most
+ * 1024 features); KSMM_ERR_BAD_ALGO, and nothing launched, otherwise.  ksmm_chain_forward_ep with `fuse` takes the same
+ * launch. */
+int ksmm_chain_forward_fused(const ksmm_factor_desc *factors, int n_factors, const void *x, void *y, int64_t batch,
+                             int x_dtype, int y_dtype, int bs_last, const ksmm_epilogue *epilogue, void *stream);
+
 /* Backward pass of one factor y = scale_fwd * K x, for F32 and F16 tensors (all three of one
  * type).  The reference has none that works (src/ksmm_py/layer/kronecker_sparse/kernel.py:319-329
  * names an undefined symbol, forward_bmm.py:12-15 is `pass`); these are the adjoints of its

@@ -563,6 +563,24 @@ bool fused_pays(const ksmm_factor_desc *f, int n, const void *x, void *y, int64_
     return fused < 0.f || each < 0.f || fused < each;
 }
 
+// Whether the fused chain of ksmm_chain16r.hip is the fastest way through a chain that it takes.  Measured on chains of
+// 256, 512 and 1024 features in three types, us a call of the routes below / this one at 197, 2050, 9408 and 25088 rows:
+// batch-size-first always (1024 features: fp32 14 / 11, 21 / 12, 51 / 32, 119 / 68; fp16 14 / 8, 16 / 9, 39 / 20, 81 / 35;
+// e4m3 21 / 9, 24 / 9, 29 / 20, 54 / 32).  Batch-size-last fp32 as well (13 / 12, 29 / 15, 49 / 31, 108 / 64), but where
+// a second round of chunks is nearly empty (1024 features at 4800 columns: 24.1 / 25.8, at 5300 equal).  The 16-bit
+// kernel for whole batch-size-last vectors (ksmm_chain16.hip) has longer chunks and is ahead once this one needs a second
+// round (fp16 4800 columns 17 / 11, 9408 19 / 23; e4m3 13 / 11.5, 14.5 / 23); on other row lengths it needs
+// padded copies (9409 columns: 38 / 28).  Narrower chains leave most of a workgroup idle: one round only.
+bool fused_rows_pay(const ksmm_factor_desc *f, int n, const void *x, void *y, int64_t batch, int x_dtype, int y_dtype, int bs_last)
+{
+    if (chain16r_run(f, n, x, y, batch, x_dtype, y_dtype, bs_last ? 1 : 0, false, nullptr, nullptr) != KSMM_OK) return false;
+    const int64_t features = (int64_t)f[0].a * f[0].c * f[0].d, round = 256 * 16;
+    if (features < 256) return batch <= round;
+    if (!bs_last) return true;
+    if (x_dtype == KSMM_F32) return !(features > 512 && batch > round && batch <= round + round / 4);
+    return batch <= 2 * round || chain16_run(f, n, x, y, batch, x_dtype, y_dtype, 1, false, nullptr, nullptr) != KSMM_OK;
+}
+
 // Whether a chain that has a transposed or padded-rows route should take it.
 bool chain_route_pays(const ksmm_factor_desc *f, int n, const void *x, void *y, int64_t batch, int x_dtype, int y_dtype, int bs_last,
                       bool fuse)
@@ -604,6 +622,14 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
         if (((uintptr_t)workspace & 15) != 0) return KSMM_ERR_WORKSPACE;
     }
     auto ep_of = [&](int i) { return i == n_factors - 1 ? ep : nullptr; };
+    // (with the workspace that the other routes ask for: a call that lacks it is refused whichever route is the faster)
+    if (fuse && fused_rows_pay(factors, n_factors, x, y, batch, x_dtype, y_dtype, bs_last)) {
+        const int64_t asked = ksmm_chain_workspace_layout(factors, n_factors, batch, x_dtype, y_dtype, bs_last);
+        if (asked <= 0 || (workspace && workspace_bytes >= asked)) {
+            rc = chain16r_run(factors, n_factors, x, y, batch, x_dtype, y_dtype, bs_last ? 1 : 0, true, (hipStream_t)stream, ep, x_scale);
+            if (rc != KSMM_ERR_BAD_ALGO) return rc;
+        }
+    }
     // The whole chain in batch-size-last layout on workspace buffers: input x0 (nb columns), two
     // ping-pong buffers of `one` bytes at pp; *result = where the last factor's output is.
     auto run_bs_last = [&](const void *x0, char *pp, int64_t one, int64_t nb, const void **result) -> int {
@@ -948,6 +974,23 @@ int ksmm_chain_forward_ep(const ksmm_factor_desc *factors, int n_factors, const 
 {
     return chain_forward_impl(factors, n_factors, x, y, workspace, workspace_bytes, batch, x_dtype, y_dtype,
                               bs_last, fuse, epilogue, stream);
+}
+
+int ksmm_chain_forward_fused(const ksmm_factor_desc *factors, int n_factors, const void *x, void *y, int64_t batch, int x_dtype,
+                             int y_dtype, int bs_last, const ksmm_epilogue *epilogue, void *stream)
+{
+    int rc = check_chain(factors, n_factors, batch, x_dtype, y_dtype);
+    if (rc != KSMM_OK) return rc;
+    if ((rc = check_epilogue(epilogue)) != KSMM_OK) return rc;
+    if (!x || !y) return KSMM_ERR_NULL_POINTER;
+    for (int i = 0; i < n_factors; ++i)
+        if (!factors[i].w) return KSMM_ERR_NULL_POINTER;
+    const ksmm_factor_desc &l = factors[n_factors - 1];
+    if (overlaps(x, (int64_t)factors[0].a * factors[0].c * factors[0].d * batch * (int64_t)dtype_size(x_dtype), y,
+                 (int64_t)l.a * l.b * l.d * batch * (int64_t)dtype_size(y_dtype)))
+        return KSMM_ERR_ALIAS;
+    if (!fused_rows_pay(factors, n_factors, x, y, batch, x_dtype, y_dtype, bs_last)) return KSMM_ERR_BAD_ALGO;
+    return chain16r_run(factors, n_factors, x, y, batch, x_dtype, y_dtype, bs_last ? 1 : 0, true, (hipStream_t)stream, epilogue);
 }
 
 // workspace of the chain that quantises its input: codes | partial maxima | scale | the chain's own

@@ -239,6 +239,9 @@ int repitch_run(const void *in, void *out, int64_t rows, int64_t cols_in, int64_
 int chain16_run(const ksmm_factor_desc *f, int n, const void *x, void *y, int64_t batch, int x_dtype,
                 int y_dtype, int bs_last, bool launch, hipStream_t stream, const ksmm_epilogue *ep,
                 const float *x_scale = nullptr);
+// the same chains in either layout, fp32 and any batch (ksmm_chain16r.hip)
+int chain16r_run(const ksmm_factor_desc *f, int n, const void *x, void *y, int64_t batch, int x_dtype, int y_dtype, int bs_last,
+                 bool launch, hipStream_t stream, const ksmm_epilogue *ep, const float *x_scale = nullptr);
 // codes (e4m3fn) and scale of a tensor of n values (ksmm_quant.hip)
 int64_t quantize_scratch_bytes();
 int quantize_run(const void *x, int x_dtype, void *codes, float *scale, void *scratch, int64_t n, hipStream_t stream);

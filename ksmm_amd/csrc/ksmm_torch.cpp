@@ -130,15 +130,23 @@ int forward(const at::Tensor &x, const Layer &l, int64_t batch, const c10::Small
             bool fuse, bool quantise, const ksmm_epilogue &ep, at::ScalarType out_type, at::Tensor *y)
 {
     const int xd = code_of(x.scalar_type()), yd = code_of(out_type);
+    void *const stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
+    const ksmm_epilogue *const epilogue = ep.bias || ep.act ? &ep : nullptr;
+    if (fuse && !quantise && l.n > 1) {  // chains of one launch need no workspace (1.7 us)
+        at::Tensor out = at::empty(shape, x.options().dtype(out_type));
+        const int rc = ksmm_chain_forward_fused(l.f, l.n, x.const_data_ptr(), out.mutable_data_ptr(), batch, xd, yd, bs_last, epilogue, stream);
+        *y = std::move(out);
+        if (rc != KSMM_ERR_BAD_ALGO) return rc;
+    }
     const int64_t need = quantise ? ksmm_chain_quant_workspace(l.f, l.n, batch, xd, yd, bs_last)
                                   : ksmm_chain_workspace_layout(l.f, l.n, batch, xd, yd, bs_last);
     if (need < 0) return (int)need;
-    *y = at::empty(shape, x.options().dtype(out_type));
+    if (!y->defined()) *y = at::empty(shape, x.options().dtype(out_type));
     at::Tensor ws;
     if (need > 0) ws = at::empty({need}, x.options().dtype(at::kByte));
     const auto run = quantise ? ksmm_chain_forward_quant : ksmm_chain_forward_ep;
     return run(l.f, l.n, x.const_data_ptr(), y->mutable_data_ptr(), need > 0 ? ws.mutable_data_ptr() : nullptr, need, batch, xd, yd,
-               bs_last, fuse, ep.bias || ep.act ? &ep : nullptr, c10::hip::getCurrentHIPStream(x.device().index()).stream());
+               bs_last, fuse, epilogue, stream);
 }
 
 // infer(x, factors, patterns, bs_last, scales, fuse, bias, act, quantise) -> y or None

@@ -487,41 +487,49 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void ks_gemm_kernel(const CT *__
         // the passes below then store them as they are
         float st_scale = scale;
         if constexpr (has_epi) {
-            const bool gelu = ep.act == KSMM_ACT_GELU;
+            // (per TM-block the bias values the lane needs are in flight together, and one branch decides on the
+            // activation: a value's GELU is a chain of dependent instructions, which overlap only with other values'.  All
+            // blocks at once spill on the tiles with 256 accumulators)
+            auto finish = [&](auto gelu, int i, const auto &bias_at) {
 #pragma unroll
-            for (int i = 0; i < C::MT; ++i) {
-                const int mb = (wm * C::MT + i) * 32;
-                if constexpr (BS_LAST) {
-                    // the lane's row is one output feature
-                    const float bl = epi_bias<TY>(ep, ((size_t)a_i * b + m0 + mb + l32) * d + d_i);
+                for (int j = 0; j < C::NT; ++j)
 #pragma unroll
-                    for (int j = 0; j < C::NT; ++j)
+                    for (int e = 0; e < 16; ++e)
 #pragma unroll
-                        for (int e = 0; e < 16; ++e) {
-                            const float v = fmaf(acc[0][i][j][e], scale, bl);
-                            acc[0][i][j][e] = gelu_if(gelu, v);
+                        for (int dd = 0; dd < DD; ++dd) {
+                            const float v = fmaf(acc[dd][i][j][e], scale, bias_at(e, dd));
+                            acc[dd][i][j][e] = decltype(gelu)::value ? gelu_erf(v) : v;
                         }
-                } else {
-                    // element u of group eg is output m0 + mb + 4*lq + 8*eg + u (x DD interleaved
-                    // d_i): the lane's 4 * DD bias values of a group are consecutive, one vector load
-                    // (at element alignment: a bias may be a slice of a longer buffer)
-                    static_assert(BS_LAST || sizeof(TY) == 2, "batch-size-first tiles write fp16");
-                    typedef TY bias_v __attribute__((ext_vector_type(4 * DD)));
-                    const size_t f0 = ((size_t)a_i * b + m0 + mb + 4 * lq) * DD;
+            };
+            auto finish_act = [&](int i, const auto &bias_at) {
+                if (ep.act == KSMM_ACT_GELU) finish(std::true_type(), i, bias_at);
+                else finish(std::false_type(), i, bias_at);
+            };
+            if constexpr (BS_LAST) {
+                // the lane's row is one output feature
+                float bl[C::MT] = {};
+                if (ep.bias) {
 #pragma unroll
-                    for (int eg = 0; eg < 4; ++eg) {
-                        bias_v bb = {};
-                        if (ep.bias) __builtin_memcpy(&bb, (const TY *)ep.bias + f0 + 8 * eg * DD, sizeof(bb));
+                    for (int i = 0; i < C::MT; ++i)
+                        bl[i] = (float)((const TY *)ep.bias)[((size_t)a_i * b + m0 + (wm * C::MT + i) * 32 + l32) * d + d_i];
+                }
 #pragma unroll
-                        for (int j = 0; j < C::NT; ++j)
+                for (int i = 0; i < C::MT; ++i) finish_act(i, [&](int, int) { return bl[i]; });
+            } else {
+                // element u of group eg is output m0 + mb + 4*lq + 8*eg + u (x DD interleaved d_i): the lane's
+                // 4 * DD bias values of a group are consecutive, one vector load (at element alignment: a bias
+                // may be a slice of a longer buffer)
+                static_assert(BS_LAST || sizeof(TY) == 2, "batch-size-first tiles write fp16");
+                typedef TY bias_v __attribute__((ext_vector_type(4 * DD)));
 #pragma unroll
-                            for (int u = 0; u < 4; ++u)
+                for (int i = 0; i < C::MT; ++i) {
+                    bias_v bb[4] = {};
+                    if (ep.bias) {
+                        const size_t f0 = ((size_t)a_i * b + m0 + (wm * C::MT + i) * 32 + 4 * lq) * DD;
 #pragma unroll
-                                for (int dd = 0; dd < DD; ++dd) {
-                                    const float v = fmaf(acc[dd][i][j][4 * eg + u], scale, (float)bb[u * DD + dd]);
-                                    acc[dd][i][j][4 * eg + u] = gelu_if(gelu, v);
-                                }
+                        for (int eg = 0; eg < 4; ++eg) __builtin_memcpy(&bb[eg], (const TY *)ep.bias + f0 + 8 * DD * eg, sizeof(bias_v));
                     }
+                    finish_act(i, [&](int e, int dd) { return (float)bb[e >> 2][DD * (e & 3) + dd]; });
                 }
             }
             st_scale = 1.f;
@@ -908,27 +916,37 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void ks_gemm_pbf_kernel(const CT
         // eight neighbouring lanes get the eight pieces of a row: whole lines, 8 per store.
         // LDS accesses of one wave execute in order, so the piece needs no barrier.
         if constexpr (has_epi) {
+            // the lane's bias values, per group (4 outputs) x (DD d_i) one vector load (at element alignment): all of
+            // them in flight before the first is used
+            typedef TY bias_v __attribute__((ext_vector_type(4 * DD)));
+            bias_v bb[C::MT][4] = {};
+            if (ep.bias) {
 #pragma unroll
-            for (int i = 0; i < C::MT; ++i) {
-                const size_t f0 = ((size_t)cur.a_i * b + cur.m0 + (wm * C::MT + i) * 32 + 4 * lq) * DD;
+                for (int i = 0; i < C::MT; ++i) {
+                    const size_t f0 = ((size_t)cur.a_i * b + cur.m0 + (wm * C::MT + i) * 32 + 4 * lq) * DD;
 #pragma unroll
-                for (int eg = 0; eg < 4; ++eg) {
-                    // the lane's bias values of this group: (4 outputs) x (DD d_i), one vector load
-                    // (at element alignment)
-                    typedef TY bias_v __attribute__((ext_vector_type(4 * DD)));
-                    bias_v bb = {};
-                    if (ep.bias) __builtin_memcpy(&bb, (const TY *)ep.bias + f0 + 8 * DD * eg, sizeof(bb));
-#pragma unroll
-                    for (int j = 0; j < C::NT; ++j)
-#pragma unroll
-                        for (int u = 0; u < 4; ++u)
-#pragma unroll
-                            for (int dd = 0; dd < DD; ++dd) {
-                                const float v = fmaf(acc[dd][i][j][4 * eg + u], scale, (float)bb[DD * u + dd]);
-                                acc[dd][i][j][4 * eg + u] = gelu_if(ep.act == KSMM_ACT_GELU, v);
-                            }
+                    for (int eg = 0; eg < 4; ++eg) __builtin_memcpy(&bb[i][eg], (const TY *)ep.bias + f0 + 8 * DD * eg, sizeof(bias_v));
                 }
             }
+            auto finish = [&](auto gelu) {
+#pragma unroll
+                for (int i = 0; i < C::MT; ++i)
+#pragma unroll
+                    for (int eg = 0; eg < 4; ++eg)
+#pragma unroll
+                        for (int j = 0; j < C::NT; ++j)
+#pragma unroll
+                            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                                for (int dd = 0; dd < DD; ++dd) {
+                                    const float v = fmaf(acc[dd][i][j][4 * eg + u], scale, (float)bb[i][eg][DD * u + dd]);
+                                    acc[dd][i][j][4 * eg + u] = decltype(gelu)::value ? gelu_erf(v) : v;
+                                }
+            };
+            // one branch for the tile, as in ks_gemm_kernel.  (1,1536,384,2) at 25088 rows with bias / and GELU: 99.9 / 120.9 us
+            // with a load and a branch where a value needs them, 95.1 / 117.2 like this, 93.5 without either
+            if (ep.act == KSMM_ACT_GELU) finish(std::true_type());
+            else finish(std::false_type());
         }
         const float st_scale = has_epi ? 1.f : scale;
         {
@@ -1226,19 +1244,26 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void ks_gemm_pbl_kernel(const CT
         // lanes get the eight 16-byte parts of a row: whole lines, 8 rows per store.  LDS
         // accesses of one wave execute in order, so the piece needs no barrier.
         if constexpr (has_epi) {
-            const bool gelu = ep.act == KSMM_ACT_GELU;
+            // (all bias values in flight at once, one branch on the activation: see ks_gemm_kernel)
+            float bl[C::MT] = {};
+            if (ep.bias) {
 #pragma unroll
-            for (int i = 0; i < C::MT; ++i) {
-                const int mb = (wm * C::MT + i) * 32;
-                const float bl = epi_bias<TY>(ep, ((size_t)cur.a_i * b + min(cur.m0 + mb + l32, b - 1)) * d + cur.d_i);
-#pragma unroll
-                for (int j = 0; j < C::NT; ++j)
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        const float v = fmaf(acc[i][j][e], scale, bl);
-                        acc[i][j][e] = gelu_if(gelu, v);
-                    }
+                for (int i = 0; i < C::MT; ++i)
+                    bl[i] = (float)((const TY *)ep.bias)[((size_t)cur.a_i * b + min(cur.m0 + (wm * C::MT + i) * 32 + l32, b - 1)) * d + cur.d_i];
             }
+            auto finish = [&](auto gelu) {
+#pragma unroll
+                for (int i = 0; i < C::MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < C::NT; ++j)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) {
+                            const float v = fmaf(acc[i][j][e], scale, bl[i]);
+                            acc[i][j][e] = decltype(gelu)::value ? gelu_erf(v) : v;
+                        }
+            };
+            if (ep.act == KSMM_ACT_GELU) finish(std::true_type());
+            else finish(std::false_type());
         }
         const float st_scale = has_epi ? 1.f : scale;
         {

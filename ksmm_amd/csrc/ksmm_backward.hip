@@ -49,13 +49,14 @@ template <typename T> __global__ __launch_bounds__(256) void ks_block_transpose_
     const int c0 = (int)(id % ct) * 64;
     const size_t block = (size_t)(id / ct) * b * c;
     const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
-    if (b0 + x < b)
-#pragma unroll 4
-        for (int i = y; i < 64; i += 4)
-            if (c0 + i < c) square[i][x] = in[block + (size_t)(c0 + i) * b + b0 + x];
+    T v[16];  // (every load in flight before the first is waited for: none is behind a branch)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = in[block + (size_t)min(c0 + y + 4 * i, c - 1) * b + min(b0 + x, b - 1)];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) square[y + 4 * i][x] = v[i];
     __syncthreads();
     if (c0 + x < c)
-#pragma unroll 4
+#pragma unroll
         for (int i = y; i < 64; i += 4)
             if (b0 + i < b) out[block + (size_t)(b0 + i) * c + c0 + x] = square[x][i];
 }

@@ -96,25 +96,24 @@ template <typename TX> __device__ __forceinline__ void epi_load(Epi &e)
         if (e.x_scale) e.scale *= *e.x_scale;
 }
 
-// GELU, erf form: x * Phi(x) = max(x, 0) - |x| * tail, tail = erfc(|x| / sqrt 2) / 2 = 2^P(|x|).  log2 of the tail is
-// smooth, and a polynomial of degree 8, fitted to the smallest largest error of the GELU, gives that to 1e-8 before
-// rounding; its leading coefficient is negative, so the tail falls to 0 behind the fitted range (6.5) as well.  11 vector
-// instructions per value, one of them transcendental, which is what an epilogue with GELU costs next to the
-// multiplications.  Against Abramowitz & Stegun 7.1.26 for the tail (12 instructions, a reciprocal and an exponential):
-// largest error in fp32 2.5e-7 for 3.3e-7, root mean square over normal values 2.0e-8 for 5.4e-8, and
-// (1,1536,384,2) fp16 at 25088 rows 118.6 -> 109.5 us, (1,768,192,2) 51.4 -> 46.8.
+// GELU, erf form: x * Phi(x) = max(x, 0) - |x| * erfc(|x| / sqrt 2) / 2.  erfc by Abramowitz &
+// Stegun 7.1.26 (|error| <= 1.5e-7, branch-free: one reciprocal, one exponential, a degree-4
+// polynomial in t = 1 / (1 + p z)), far inside fp32 storage rounding of the result for the
+// value range of activations.  The constants carry the factors the formula would multiply by:
+// with z' = |x| sqrt(log2(e) / 2) the exponential is 2^(-z'^2), p is divided by sqrt(log2 e),
+// and the polynomial's coefficients are halved: 12 vector instructions per value, two of them
+// transcendental, which is what an epilogue with GELU costs next to the multiplications.
 __device__ __forceinline__ float gelu_erf(float x)
 {
     const float ax = fabsf(x);
-    float p = fmaf(-1.99189935e-06f, ax, 2.9272016e-05f);
-    p = fmaf(p, ax, -0.000138088333f);
-    p = fmaf(p, ax, -0.000253436272f);
-    p = fmaf(p, ax, 0.00721638929f);
-    p = fmaf(p, ax, -0.0526030511f);
-    p = fmaf(p, ax, -0.459172219f);
-    p = fmaf(p, ax, -1.1511097f);
-    p = fmaf(p, ax, -0.999999881f);
-    return fmaf(-ax, __builtin_amdgcn_exp2f(p), fmaxf(x, 0.f));
+    const float z = ax * 0.84932180028801907f;
+    const float t = __builtin_amdgcn_rcpf(fmaf(0.2727374808792225f, z, 1.0f));
+    float poly = fmaf(0.5307027145f, t, -0.7265760135f);
+    poly = fmaf(poly, t, 0.7107068705f);
+    poly = fmaf(poly, t, -0.142248368f);
+    poly = fmaf(poly, t, 0.127414796f);
+    const float tail = (poly * t) * __builtin_amdgcn_exp2f(-(z * z));  // erfc(|x| / sqrt 2) / 2
+    return fmaf(-ax, tail, fmaxf(x, 0.f));
 }
 
 // GELU of v when `on` (uniform over the wave), v otherwise: a branch, never a select, so that a

@@ -276,6 +276,33 @@ def test_gelu_constants_of_the_kernel_epilogue():
     assert np.linalg.norm(got - want) <= 1e-7 * np.linalg.norm(want)
 
 
+def test_gelu_of_the_gemm_tiles():
+    """gelu_pow2 in ksmm_gemm.hip, the same way: max(x, 0) - |x| 2^P(|x|) with the coefficients of P read from the
+    source, in float32 Horner form, against the erf form in float64; nothing comes back behind the fitted range."""
+    import os
+    import re
+
+    import torch
+
+    src = open(os.path.join(os.path.dirname(__file__), "..", "ksmm_amd", "csrc", "ksmm_gemm.hip")).read()
+    body = src[src.index("float gelu_pow2(float x)"):]
+    coefs = [np.float32(v) for v in re.findall(r"(-?\d+\.\d{5,}(?:e-\d+)?)f", body[:body.index("\n}\n")])]
+    assert len(coefs) == 9
+    x = np.concatenate([np.linspace(-12, 12, 240001), [0.0, -0.0, 1e-20, -1e-20, 60.0, -60.0, -65504.0, 65504.0, -3e38]]).astype(np.float32)
+    ax = np.abs(x)
+    p = np.full_like(ax, coefs[0])
+    with np.errstate(over="ignore"):
+        for c in coefs[1:]:
+            p = p * ax + c
+    got = np.maximum(x, np.float32(0)) - ax * np.exp2(p)
+    want = torch.nn.functional.gelu(torch.from_numpy(x).double()).numpy()
+    assert got.dtype == np.float32
+    # (the product and the sum of a Horner step round apart here: the kernel's fused ones are within 2.5e-7)
+    assert np.abs(got - want).max() <= 5e-7
+    normal = ax <= 12
+    assert np.linalg.norm((got - want)[normal]) <= 1e-7 * np.linalg.norm(want[normal])
+
+
 def test_unaligned_batch_asks_for_room_for_padded_rows():
     """Batch-size-last rows are `batch` elements long; when that is not a multiple of the
     16-byte vector the library asks for room for the input and the output with rows padded to a

@@ -214,7 +214,9 @@ int64_t ksmm_chain_workspace(const ksmm_factor_desc *factors, int n_factors, int
  * KSMM_ERR_WORKSPACE when the workspace it is given is smaller than this (or NULL while this
  * is not 0), like ksmm_factor_forward_ws: it never falls back to a slower route silently.
  * A batch-size-last chain whose batch is not a multiple of the 16-byte vector asks for the same
- * buffers with rows padded to a multiple of 16 columns and runs the whole chain there. */
+ * buffers with rows padded to a multiple of 16 columns and runs the whole chain there.
+ * An e4m3 chain that is faster with its weights decoded to fp16 asks for room for these too, and runs without them on
+ * a workspace that holds the rest. */
 int64_t ksmm_chain_workspace_layout(const ksmm_factor_desc *factors, int n_factors, int64_t batch,
                                     int x_dtype, int y_dtype, int bs_last);
 

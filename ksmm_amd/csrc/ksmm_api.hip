@@ -597,6 +597,92 @@ bool chain_route_pays(const ksmm_factor_desc *f, int n, const void *x, void *y, 
                copy_us((int64_t)l.a * l.b * l.d, batch, bp, (int)dtype_size(y_dtype), !bs_last) + middle < direct;
 }
 
+// What a chain cannot do without (a chain with decoded weights uses more, see decode_pays)
+int64_t chain_layout(const ksmm_factor_desc *factors, int n_factors, int64_t batch, int x_dtype, int y_dtype, int bs_last)
+{
+    int rc = check_chain(factors, n_factors, batch, x_dtype, y_dtype);
+    if (rc != KSMM_OK) return rc;
+    const int64_t nb = chain_wants_transposed(factors, n_factors, batch, x_dtype, y_dtype, bs_last) ||
+                               chain_wants_padded(factors, n_factors, batch, x_dtype, y_dtype, bs_last)
+                           ? padded_batch(batch) : 0;
+    if (nb == 0) return ksmm_chain_workspace(factors, n_factors, batch, y_dtype);
+    int64_t widest = 0;
+    for (int i = 0; i < n_factors; ++i) {
+        int64_t o = (int64_t)factors[i].a * factors[i].b * factors[i].d;
+        if (o > widest) widest = o;
+    }
+    const int64_t in0 = (int64_t)factors[0].a * factors[0].c * factors[0].d;
+    return align256(in0 * nb * (int64_t)dtype_size(x_dtype)) +
+           2 * align256(widest * nb * (int64_t)dtype_size(y_dtype));
+}
+
+// Predicted time of a chain by the faster of its routes (< 0: no price); *copies: that is the one between copies
+float chain_best_us(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype, int bs_last, bool *copies)
+{
+    *copies = false;
+    const float direct = chain_us(f, n, nullptr, nullptr, batch, x_dtype, y_dtype, bs_last, false);
+    if (!(bs_last ? chain_wants_padded(f, n, batch, x_dtype, y_dtype, 1) : chain_wants_transposed(f, n, batch, x_dtype, y_dtype, 0))) return direct;
+    const float middle = chain_us(f, n, nullptr, nullptr, batch, x_dtype, y_dtype, bs_last, true);
+    if (middle < 0.f) return direct;
+    const int64_t bp = padded_batch(batch);
+    const ksmm_factor_desc &l = f[n - 1];
+    const float route = middle + copy_us((int64_t)f[0].a * f[0].c * f[0].d, batch, bp, (int)dtype_size(x_dtype), !bs_last) +
+                        copy_us((int64_t)l.a * l.b * l.d, batch, bp, (int)dtype_size(y_dtype), !bs_last);
+    *copies = direct < 0.f || route < direct;
+    return *copies ? route : direct;
+}
+
+// Factors of e4m3 weights on an fp16 input (all but the first of an e4m3 layer): the kernels that decode such weights
+// on the way to LDS take up to twice the time of the fp16 ones, of which there are more.  Decoded once a call, in one
+// launch for the chain and exactly, the weights run on those.  Whether that pays: `decoded` is the chain with such
+// weights (w is not set).  The decoding is priced at a launch (4 us with its host time) and 3 bytes a weight, and has to be
+// ahead by the error of the prices, unless it saves the copies of a route or a split-K kernel on thousands of rows, whose
+// price is too low by up to 3: measured on the projections of feed-forward
+// blocks of widths 192 .. 1024 at ten batches, what was predicted to take less than 0.855 of the time was 1.08 to 2.7 times
+// faster, from there to 1 it was 0.88 to 1.4 times.  us a call without and with: (6,64,64,1)+(1,768,192,2) on
+// 25088 columns 143 / 52, on rows 103 / 65, (3,64,256,1)+(1,64,64,3) on 4800 rows 36 / 15, (12,64,256,1)+(1,256,256,3) on
+// 10070 rows 79 / 44, on 25088 125 / 101.
+bool decode_pays(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype, int bs_last, ksmm_factor_desc *decoded)
+{
+    if (batch < 512 || y_dtype != KSMM_F16) return false;
+    int64_t weights = 0;
+    bool split = false;
+    for (int i = 0; i < n; ++i) {
+        decoded[i] = f[i];
+        if (f[i].w_dtype != KSMM_FP8_E4M3 || (i == 0 ? x_dtype : y_dtype) != KSMM_F16) continue;
+        decoded[i].w_dtype = KSMM_F16;
+        auto on_split = [&](int w_dtype) {
+            const Choice c = pick_of(Problem{nullptr, nullptr, nullptr, batch, f[i].a, f[i].b, f[i].c, f[i].d, KSMM_F16, w_dtype, y_dtype,
+                                             bs_last, 1.f, nullptr}, true).c;
+            return c.algo == KSMM_ALGO_TILE && (c.variant >> 24) == 5;
+        };
+        split |= batch >= 4096 && on_split(KSMM_FP8_E4M3) && !on_split(KSMM_F16);
+        weights += (int64_t)f[i].a * f[i].b * f[i].c * f[i].d;
+    }
+    if (weights == 0) return false;
+    // (chains of one kernel read their weights once a workgroup)
+    if (chain16r_run(f, n, nullptr, nullptr, batch, x_dtype, y_dtype, bs_last ? 1 : 0, false, nullptr, nullptr) == KSMM_OK) return false;
+    // (short chains cannot win a launch back: no more than their own prices is looked up)
+    const float direct = chain_us(f, n, nullptr, nullptr, batch, x_dtype, y_dtype, bs_last, false);
+    if (direct >= 0.f && direct < 12.f) return false;
+    bool copied, copied_then;
+    const float now = chain_best_us(f, n, batch, x_dtype, y_dtype, bs_last, &copied);
+    const float then = chain_best_us(decoded, n, batch, x_dtype, y_dtype, bs_last, &copied_then) + 4.f + (float)weights * 1.5e-6f;
+    return now > 0.f && then > 4.f && then < ((split || copied) && !copied_then ? 1.f : 0.855f) * now;
+}
+
+// Workspace of a chain with decoded weights: that of either chain, then (from *at) the fp16 weights
+int64_t decode_layout(const ksmm_factor_desc *f, const ksmm_factor_desc *decoded, int n, int64_t batch, int x_dtype, int y_dtype,
+                      int bs_last, int64_t *at)
+{
+    const int64_t one = chain_layout(f, n, batch, x_dtype, y_dtype, bs_last), two = chain_layout(decoded, n, batch, x_dtype, y_dtype, bs_last);
+    *at = align256(one > two ? one : two);
+    int64_t bytes = *at;
+    for (int i = 0; i < n; ++i)
+        if (decoded[i].w_dtype != f[i].w_dtype) bytes += align256((int64_t)f[i].a * f[i].b * f[i].c * f[i].d * 2);
+    return bytes;
+}
+
 // The chain launcher behind ksmm_chain_forward, ksmm_chain_forward_ep and
 // ksmm_chain_forward_static: `ep` (may be null) belongs to the last factor, `x_scale` (device
 // memory, may be null) multiplies the first one's scale.
@@ -621,10 +707,28 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
             return KSMM_ERR_ALIAS;
         if (((uintptr_t)workspace & 15) != 0) return KSMM_ERR_WORKSPACE;
     }
+    ksmm_factor_desc decoded[KSMM_MAX_FACTORS];
+    if (workspace && decode_pays(factors, n_factors, batch, x_dtype, y_dtype, bs_last, decoded)) {
+        int64_t at;
+        if (workspace_bytes >= decode_layout(factors, decoded, n_factors, batch, x_dtype, y_dtype, bs_last, &at)) {
+            DecodeJob jobs[KSMM_MAX_FACTORS];
+            int n_jobs = 0;
+            char *to = (char *)workspace + at;
+            for (int i = 0; i < n_factors; ++i) {
+                if (decoded[i].w_dtype == factors[i].w_dtype) continue;
+                const int64_t n = (int64_t)factors[i].a * factors[i].b * factors[i].c * factors[i].d;
+                jobs[n_jobs++] = DecodeJob{factors[i].w, to, n};
+                decoded[i].w = to;
+                to += align256(n * 2);
+            }
+            if ((rc = decode_run(jobs, n_jobs, (hipStream_t)stream)) != KSMM_OK) return rc;
+            return chain_forward_impl(decoded, n_factors, x, y, workspace, at, batch, x_dtype, y_dtype, bs_last, fuse, ep, stream, x_scale);
+        }
+    }
     auto ep_of = [&](int i) { return i == n_factors - 1 ? ep : nullptr; };
     // (with the workspace that the other routes ask for: a call that lacks it is refused whichever route is the faster)
     if (fuse && fused_rows_pay(factors, n_factors, x, y, batch, x_dtype, y_dtype, bs_last)) {
-        const int64_t asked = ksmm_chain_workspace_layout(factors, n_factors, batch, x_dtype, y_dtype, bs_last);
+        const int64_t asked = chain_layout(factors, n_factors, batch, x_dtype, y_dtype, bs_last);
         if (asked <= 0 || (workspace && workspace_bytes >= asked)) {
             rc = chain16r_run(factors, n_factors, x, y, batch, x_dtype, y_dtype, bs_last ? 1 : 0, true, (hipStream_t)stream, ep, x_scale);
             if (rc != KSMM_ERR_BAD_ALGO) return rc;
@@ -660,7 +764,7 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
         // (a workspace below what ksmm_chain_workspace_layout() asks for is an error, as it is for
         // ksmm_factor_forward_ws: the factor-by-factor route would land on the one-thread-per-output
         // kernel without a word)
-        const int64_t need_t = ksmm_chain_workspace_layout(factors, n_factors, batch, x_dtype, y_dtype, 0);
+        const int64_t need_t = chain_layout(factors, n_factors, batch, x_dtype, y_dtype, 0);
         if (!workspace || workspace_bytes < need_t) return KSMM_ERR_WORKSPACE;
         if (chain_route_pays(factors, n_factors, x, y, batch, x_dtype, y_dtype, 0, fuse != 0)) {
             const int64_t bp = padded_batch(batch);  // row length of the transposed copies
@@ -675,7 +779,7 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
         }
     } else if (chain_wants_padded(factors, n_factors, batch, x_dtype, y_dtype, bs_last)) {
         // pad the rows once, run the whole chain at the padded batch, cut the result rows back
-        const int64_t need_p = ksmm_chain_workspace_layout(factors, n_factors, batch, x_dtype, y_dtype, 1);
+        const int64_t need_p = chain_layout(factors, n_factors, batch, x_dtype, y_dtype, 1);
         if (!workspace || workspace_bytes < need_p) return KSMM_ERR_WORKSPACE;
         if (chain_route_pays(factors, n_factors, x, y, batch, x_dtype, y_dtype, 1, fuse != 0)) {
             const int64_t bp = padded_batch(batch);
@@ -943,20 +1047,12 @@ int64_t ksmm_chain_workspace(const ksmm_factor_desc *factors, int n_factors, int
 int64_t ksmm_chain_workspace_layout(const ksmm_factor_desc *factors, int n_factors, int64_t batch,
                                     int x_dtype, int y_dtype, int bs_last)
 {
-    int rc = check_chain(factors, n_factors, batch, x_dtype, y_dtype);
-    if (rc != KSMM_OK) return rc;
-    const int64_t nb = chain_wants_transposed(factors, n_factors, batch, x_dtype, y_dtype, bs_last) ||
-                               chain_wants_padded(factors, n_factors, batch, x_dtype, y_dtype, bs_last)
-                           ? padded_batch(batch) : 0;
-    if (nb == 0) return ksmm_chain_workspace(factors, n_factors, batch, y_dtype);
-    int64_t widest = 0;
-    for (int i = 0; i < n_factors; ++i) {
-        int64_t o = (int64_t)factors[i].a * factors[i].b * factors[i].d;
-        if (o > widest) widest = o;
-    }
-    const int64_t in0 = (int64_t)factors[0].a * factors[0].c * factors[0].d;
-    return align256(in0 * nb * (int64_t)dtype_size(x_dtype)) +
-           2 * align256(widest * nb * (int64_t)dtype_size(y_dtype));
+    const int64_t need = chain_layout(factors, n_factors, batch, x_dtype, y_dtype, bs_last);
+    if (need < 0) return need;
+    ksmm_factor_desc decoded[KSMM_MAX_FACTORS];
+    if (!decode_pays(factors, n_factors, batch, x_dtype, y_dtype, bs_last, decoded)) return need;
+    int64_t at;
+    return decode_layout(factors, decoded, n_factors, batch, x_dtype, y_dtype, bs_last, &at);
 }
 
 int ksmm_chain_forward(const ksmm_factor_desc *factors, int n_factors, const void *x, void *y,
@@ -1014,21 +1110,24 @@ int ksmm_chain_forward_quant(const ksmm_factor_desc *factors, int n_factors, con
                              int64_t workspace_bytes, int64_t batch, int x_dtype, int y_dtype, int bs_last, int fuse,
                              const ksmm_epilogue *epilogue, void *stream)
 {
-    const int64_t need = ksmm_chain_quant_workspace(factors, n_factors, batch, x_dtype, y_dtype, bs_last);
-    if (need < 0) return (int)need;
+    // (more is asked for than a chain without decoded weights needs: with less it runs without them)
+    const int64_t asked = ksmm_chain_quant_workspace(factors, n_factors, batch, x_dtype, y_dtype, bs_last);
+    if (asked < 0) return (int)asked;
+    int64_t maxima;
+    const int64_t own = quant_layout(factors, batch, &maxima);
+    int64_t need = own + chain_layout(factors, n_factors, batch, KSMM_FP8_E4M3, y_dtype, bs_last);
     int rc = check_epilogue(epilogue);
     if (rc != KSMM_OK) return rc;
     if (!x || !y) return KSMM_ERR_NULL_POINTER;
     for (int i = 0; i < n_factors; ++i)
         if (!factors[i].w) return KSMM_ERR_NULL_POINTER;
     if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15) != 0) return KSMM_ERR_WORKSPACE;
+    if (workspace_bytes >= asked) need = asked;
     const ksmm_factor_desc &last = factors[n_factors - 1];
     const int64_t n = (int64_t)factors[0].a * factors[0].c * factors[0].d * batch, xbytes = n * (int64_t)dtype_size(x_dtype);
     const int64_t ybytes = (int64_t)last.a * last.b * last.d * batch * (int64_t)dtype_size(y_dtype);
     if (overlaps(x, xbytes, y, ybytes) || overlaps(workspace, need, x, xbytes) || overlaps(workspace, need, y, ybytes))
         return KSMM_ERR_ALIAS;
-    int64_t maxima;
-    const int64_t own = quant_layout(factors, batch, &maxima);
     char *ws = (char *)workspace;
     float *scale = (float *)(ws + own - 256);
     rc = quantize_run(x, x_dtype, ws, scale, ws + maxima, n, (hipStream_t)stream);
@@ -1177,7 +1276,7 @@ int ksmm_chain_forward_static(const ksmm_factor_desc *factors, int n_factors, co
                               const ksmm_epilogue *epilogue, void *stream)
 {
     // what the chain would ask a caller to lend (0 when it needs no scratch at all)
-    const int64_t need = ksmm_chain_workspace_layout(factors, n_factors, batch, x_dtype, y_dtype, bs_last);
+    const int64_t need = chain_layout(factors, n_factors, batch, x_dtype, y_dtype, bs_last);
     if (need < 0) return (int)need;
     if (need > KSMM_STATIC_SCRATCH_BYTES) return KSMM_ERR_WORKSPACE;
     void *buf = nullptr;

@@ -242,6 +242,13 @@ int chain16_run(const ksmm_factor_desc *f, int n, const void *x, void *y, int64_
 // the same chains in either layout, fp32 and any batch (ksmm_chain16r.hip)
 int chain16r_run(const ksmm_factor_desc *f, int n, const void *x, void *y, int64_t batch, int x_dtype, int y_dtype, int bs_last,
                  bool launch, hipStream_t stream, const ksmm_epilogue *ep, const float *x_scale = nullptr);
+// fp16 values (16-byte aligned) of e4m3fn codes (ksmm_quant.hip)
+struct DecodeJob {
+    const void *codes;
+    void *to;
+    int64_t n;
+};
+int decode_run(const DecodeJob *jobs, int n, hipStream_t stream);
 // codes (e4m3fn) and scale of a tensor of n values (ksmm_quant.hip)
 int64_t quantize_scratch_bytes();
 int quantize_run(const void *x, int x_dtype, void *codes, float *scale, void *scratch, int64_t n, hipStream_t stream);

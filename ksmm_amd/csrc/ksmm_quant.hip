@@ -181,6 +181,41 @@ __global__ __launch_bounds__(1024) void ks_quant_small_kernel(const T *__restric
 // 512 KB 13.4 / 13.2 and 13.0 / 11.7, 768 KB 13.3 / 13.3 and 14.7 / 13.5; fp32 within 0.5 of these.
 constexpr int64_t SMALL_BYTES = 384 << 10;
 
+// e4m3fn codes as fp16 (exact), for the weights of a whole chain in one launch
+struct DecodeArgs {
+    struct {
+        const uint8_t *codes;
+        half_t *to;
+        int64_t n;
+        uint32_t first;  // the job's first workgroup
+    } job[KSMM_MAX_FACTORS];
+    int jobs;
+};
+
+__global__ __launch_bounds__(256) void ks_decode_kernel(DecodeArgs d)
+{
+    int k = 0;
+    while (k + 1 < d.jobs && blockIdx.x >= d.job[k + 1].first) ++k;
+    const uint8_t *codes = d.job[k].codes;
+    half_t *to = d.job[k].to;
+    const int64_t n = d.job[k].n, at = ((int64_t)(blockIdx.x - d.job[k].first) * 256 + threadIdx.x) * RUN;
+    if (at >= n) return;
+    if (at + RUN <= n) {
+        uint4_t v;
+        __builtin_memcpy(&v, codes + at, 16);  // (any alignment)
+        uint4_t o[2];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            o[w >> 1][2 * (w & 1)] = __builtin_bit_cast(uint32_t, fp8x2_to_half2(v[w]));
+            o[w >> 1][2 * (w & 1) + 1] = __builtin_bit_cast(uint32_t, fp8x2_hi_to_half2(v[w]));
+        }
+        ((uint4_t *)(to + at))[0] = o[0];
+        ((uint4_t *)(to + at))[1] = o[1];
+    } else {
+        for (int64_t i = at; i < n; ++i) to[i] = fp8_to_half(codes[i]);
+    }
+}
+
 template <typename T> int launch(const void *x, void *q, uint32_t *part, float *scale, int64_t n, hipStream_t s)
 {
     const bool aligned = ((uintptr_t)x & 15) == 0;
@@ -201,6 +236,24 @@ template <typename T> int launch(const void *x, void *q, uint32_t *part, float *
 }
 
 }  // namespace
+
+int decode_run(const DecodeJob *jobs, int n, hipStream_t stream)
+{
+    DecodeArgs d;
+    int64_t blocks = 0;
+    d.jobs = n;
+    for (int i = 0; i < n; ++i) {
+        d.job[i].codes = (const uint8_t *)jobs[i].codes;
+        d.job[i].to = (half_t *)jobs[i].to;
+        d.job[i].n = jobs[i].n;
+        d.job[i].first = (uint32_t)blocks;
+        blocks += (jobs[i].n + 256 * RUN - 1) / (256 * RUN);
+        if (blocks > 0x7fffffffLL) return KSMM_ERR_TOO_LARGE;
+    }
+    if (blocks < 1) return KSMM_OK;
+    hipLaunchKernelGGL(ks_decode_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, d);
+    return hipGetLastError() == hipSuccess ? KSMM_OK : KSMM_ERR_LAUNCH;
+}
 
 int64_t quantize_scratch_bytes() { return 4 * QUANT_BLOCKS; }
 

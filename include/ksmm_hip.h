@@ -166,7 +166,8 @@ int ksmm_factor_forward(const void *x, const void *w, void *y, int64_t batch, in
  * instance v (how the automatic choice reports an instance it takes for a problem that has no kernel
  * of its own at full batches: a ragged batch, strided batch-size-first blocks); KSMM_ALGO_WAVE
  * instance | tiles-per-wave << 8 | round-robin << 16, 1000 + i = batch-size-first row kernel i;
- * KSMM_ALGO_TILE sub-family << 24 | instance (0 k-loop, 1 weight-stationary, 2 stream,
+ * KSMM_ALGO_TILE sub-family << 24 | instance (0 k-loop, | 1 << 8 where batch-size-last rows that no
+ * 16-byte vector divides are to be taken; 1 weight-stationary, 2 stream,
  * 3 batch-size-first d > 1, 4 direct-to-LDS GEMM, 5 split-K: instance | waves << 8); KSMM_ALGO_AUTO -1 = measured table, then
  * heuristics, -3 = heuristics only.  An instance that cannot run the problem returns
  * KSMM_ERR_BAD_ALGO. */

@@ -133,11 +133,18 @@ float predicted_us(const Problem &p, const ksmm_tile &t)
     return r ? price(*r, p, t) : -1.f;
 }
 
+// The k-loop tiles on batch-size-last rows that no vector divides, against whole ones: 1.00 to 1.04 times the time in fp32
+// and e4m3, up to 1.2 in fp16 (seven patterns at 6500 and 6501 columns: vectors off their alignment).  Against the
+// split-K kernel, which alone took such rows before (us at 6501 / 25061 columns): (4,192,192,1) fp16 18 / 38 and 9 / 22,
+// (1,256,256,3) fp16 24 / 46 and 12 / 26, (1,1536,384,2) fp16 47 / 184 and 36 / 112, fp32 166 / 560 and 143 / 507.
+constexpr float RAGGED_H = 1.1f;
+
 Choice cheapest_instance(const Problem &p, bool split_only)
 {
     Choice best{KSMM_ALGO_AUTO, -1, -1.f};
     const int combo = combo_of(p.x_dtype, p.w_dtype, p.y_dtype);
     if (combo < 0) return best;
+    const bool ragged = p.bs_last && p.batch % (16 / (int64_t)dtype_size(p.x_dtype)) != 0;
     auto offer = [&](int algo, int variant) {
         ksmm_tile t;
         memset(&t, 0, sizeof(t));
@@ -145,7 +152,7 @@ Choice cheapest_instance(const Problem &p, bool split_only)
         if (rc != KSMM_OK) return;
         const CostRow *r = row_of(p, combo, t.algo, t.variant);
         if (!r || (t.threads & 63) || t.tile_d < 1) return;
-        const float us = price(*r, p, t);
+        const float us = price(*r, p, t) * (algo == KSMM_ALGO_TILE && (variant >> 24) == 0 && ragged && combo == 1 ? RAGGED_H : 1.f);
         if (best.us < 0.f || us < best.us) best = Choice{t.algo, t.variant, us};
     };
     const CostIndex &ix = cost_index();
@@ -153,7 +160,7 @@ Choice cheapest_instance(const Problem &p, bool split_only)
         offer(KSMM_ALGO_WAVE, -1);
         for (int sub = 0; sub < FAM_SPLIT; ++sub)
             for (int i = 0; i < ix.count[sub]; ++i)
-                if (ix.tile[sub][combo][p.bs_last][i]) offer(KSMM_ALGO_TILE, (sub << 24) | i);
+                if (ix.tile[sub][combo][p.bs_last][i]) offer(KSMM_ALGO_TILE, (sub << 24) | (sub == 0 && ragged ? 1 << 8 : 0) | i);
     }
     for (int i = 0; i < ix.count[FAM_SPLIT]; ++i) {
         if (!ix.tile[FAM_SPLIT][combo][p.bs_last][i]) continue;

@@ -129,12 +129,14 @@ __global__ __launch_bounds__(64 * WM * WN) void ks_tile_kernel(const TX *__restr
             if (C::X_VECS % C::THREADS == 0 || v < C::X_VECS) {
                 if (BS_LAST) {
                     const int kk = v / (TN / C::X_EPV), nn = (v % (TN / C::X_EPV)) * C::X_EPV;
-                    // columns past the end are clamped to the last valid vector (never stored)
+                    // vectors past the end of the row, or across it, are those that end with it (and are stored
+                    // there, see below); rows of any length: element alignment (global memory takes
+                    // unaligned vector accesses)
                     const int col = min(n0 + nn, batch - C::X_EPV);
                     if (k0 + kk >= c)
                         xreg[i].v = uint4_t{0u, 0u, 0u, 0u};
                     else
-                        xreg[i].load(xg + (size_t)(k0 + kk) * x_kstride + col);
+                        __builtin_memcpy(&xreg[i].v, xg + (size_t)(k0 + kk) * x_kstride + col, 16);
                 } else {
                     const int nn = v / (TK / C::X_EPV), kk = (v % (TK / C::X_EPV)) * C::X_EPV;
                     const int row = min(n0 + nn, batch - 1);
@@ -247,9 +249,13 @@ __global__ __launch_bounds__(64 * WM * WN) void ks_tile_kernel(const TX *__restr
                 const int r = q / CPR, cc = (q % CPR) * OEPC;
                 const int row = pass * RPP + r;
                 if (row >= TM) break;
-                const int m = m0 + row, n = n0 + cc;
-                if (n < batch && (!RB || m < b))
-                    *(uint4_t *)(y + ((size_t)(a_i * b + m) * d + d_i) * batch + n) = *(const uint4_t *)(out + r * RC + cc);
+                // (a vector of inputs that was moved back to end with the row has its results there: some of them
+                // are written twice, the same)
+                const int group = cc / C::X_EPV * C::X_EPV, m = m0 + row, n = min(n0 + group, batch - C::X_EPV) + (cc - group);
+                if (n0 + group < batch && (!RB || m < b)) {
+                    const uint4_t v = *(const uint4_t *)(out + r * RC + cc);
+                    __builtin_memcpy(y + ((size_t)(a_i * b + m) * d + d_i) * batch + n, &v, 16);
+                }
             }
         }
     } else {
@@ -611,7 +617,8 @@ const TileInst tile_insts[] = {
 };
 constexpr int N_TILE_INSTS = sizeof(tile_insts) / sizeof(TileInst);
 
-bool tile_fits(const TileInst &t, const Problem &p, int combo)
+// ragged: batch-size-last rows that no 16-byte vector divides are taken too
+bool tile_fits(const TileInst &t, const Problem &p, int combo, bool ragged = false)
 {
     if (t.combo != combo || t.bs_last != p.bs_last) return false;
     if (!p.bs_last && p.c % t.tk) return false;  // batch-size-last tiles zero-fill the K tail
@@ -626,7 +633,7 @@ bool tile_fits(const TileInst &t, const Problem &p, int combo)
         return false;
     }
     if (p.bs_last) {
-        if (p.batch % x_epv || p.batch < x_epv) return false;
+        if ((p.batch % x_epv && !ragged) || p.batch < x_epv) return false;
     } else {
         if (p.d != 1) return false;  // batch-size-first with d > 1 is not handled by this family
         if (((int64_t)p.a * p.c) % x_epv || p.c % x_epv) return false;
@@ -662,7 +669,8 @@ int tile_run(const Problem &p, int variant, bool launch, ksmm_tile *tile)
     if (combo < 0) return KSMM_ERR_BAD_DTYPE;
     // variant layout: bits 24-27 sub-family (0 k-loop tiles, 1 weight-stationary, 2 stream,
     // 3 batch-size-first with d > 1, 4 direct-to-LDS GEMM), bits 0-7 instance (0xff: first that fits), bits 8-23 a
-    // sub-family parameter (persistent workgroups per block); -1: everything automatic
+    // sub-family parameter (persistent workgroups per block; k-loop tiles: 1 takes ragged rows); -1: everything automatic
+    bool ragged = false;
     if (variant >= 0) {
         const int sub = (variant >> 24) & 15, inst = variant & 0xff, par = (variant >> 8) & 0xffff;
         if (sub == 5) return split_run(p, inst == 0xff ? -1 : inst | (par << 8), launch, tile);
@@ -671,6 +679,7 @@ int tile_run(const Problem &p, int variant, bool launch, ksmm_tile *tile)
         if (sub == 2) return stream_run(p, (inst == 0xff ? 0x7f : inst) | (par << 7), launch, tile);
         if (sub == 1) return ws_run(p, inst == 0xff ? -1 : inst, par, launch, tile);
         variant = inst == 0xff ? -2 : inst;  // -2: heuristic among the k-loop tiles only
+        ragged = par == 1;
     } else {
         int rc = gemm_run(p, -1, launch, tile);  // large blocks: matrix-core-bound
         if (rc != KSMM_ERR_BAD_ALGO) return rc;
@@ -690,7 +699,7 @@ int tile_run(const Problem &p, int variant, bool launch, ksmm_tile *tile)
     }
     int pick = -1;
     if (variant >= 0) {
-        if (variant < N_TILE_INSTS && tile_fits(tile_insts[variant], p, combo)) pick = variant;
+        if (variant < N_TILE_INSTS && tile_fits(tile_insts[variant], p, combo, ragged)) pick = variant;
     } else {  // -1 or -2
         // heuristic: the largest TM that divides b (fewest re-reads of the input), then a batch
         // tile that still leaves >= 2 workgroups per CU
@@ -720,7 +729,7 @@ int tile_run(const Problem &p, int variant, bool launch, ksmm_tile *tile)
     if (grid > 0x7fffffffLL) return KSMM_ERR_TOO_LARGE;
     if (tile) {
         tile->algo = KSMM_ALGO_TILE;
-        tile->variant = pick;
+        tile->variant = pick | (ragged ? 1 << 8 : 0);
         tile->tile_m = t.tm;
         tile->tile_n = t.tn;
         tile->tile_k = t.tk;

@@ -13,8 +13,8 @@
 // that share the loaded cache lines (all of them for d <= 8, eight otherwise), times the tiles of a
 // block or the neighbouring blocks, up to four waves (more only where d asks for them).
 //
-// What bounds it: at full batches the latency of a slab (load, transpose, two barriers), three or
-// four slabs of 16 KB in flight per CU; four waves a workgroup, three workgroups a CU.  Eight-wave
+// What bounds it: at full batches the latency of a slab (load, transpose, two barriers, or one: two_slabs()), three
+// or four slabs of 16 KB in flight per CU; four waves a workgroup, three workgroups a CU.  Eight-wave
 // workgroups read less through L2 but leave one workgroup a CU: 83 us instead of 52 on the second
 // shape below.  128 registers a wave (four waves a SIMD) spill: 74 us.
 // Against transposed copies of both operands in HBM and the batch-size-last kernel on them, fp16 at
@@ -82,7 +82,8 @@ template <int CH> __device__ __forceinline__ int lds_unit(int row, int ch)
 }
 
 // acc_out: one slice of partial sums per split; dw (used when there is one split): the result.
-template <typename T, int TT, int CH>
+// TWO: two slabs in LDS, see two_slabs()
+template <typename T, int TT, int CH, bool TWO>
 __global__ __launch_bounds__(512) void ks_wgrad_bf_kernel(const T *__restrict__ dy, const T *__restrict__ x,
                                                           float *__restrict__ acc_out, T *__restrict__ dw, WgradBf g)
 {
@@ -201,29 +202,55 @@ __global__ __launch_bounds__(512) void ks_wgrad_bf_kernel(const T *__restrict__ 
 #pragma unroll
         for (int j = 0; j < TT; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
 
-    load();
-    for (int64_t n = n_begin; n < n_end; n += SLAB) {
-        __syncthreads();  // the slab in LDS is consumed
+    auto store = [&](uint4_t *to) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
             for (int e = 0; e < N; ++e)
-                lds[e & 1 ? dst[u][e / 2] >> 16 : dst[u][e / 2] & 0xffffu] = V::column(v[u], e);
-        __syncthreads();
-        if (n + SLAB < n_end) load();
+                to[e & 1 ? dst[u][e / 2] >> 16 : dst[u][e / 2] & 0xffffu] = V::column(v[u], e);
+    };
+    auto multiply = [&](const uint4_t *from) {
 #pragma unroll
         for (int ks = 0; ks < CH / 4; ++ks) {
             int ua = ra, ub = rb;
             asm volatile("" : "+v"(ua), "+v"(ub));  // the positions are recomputed per slab: held, they would cost a wave per SIMD
             vec_t fa[TT];
 #pragma unroll
-            for (int i = 0; i < TT; ++i) fa[i] = __builtin_bit_cast(vec_t, lds[lds_unit<CH>(ua + 16 * i, 4 * ks + q)]);
+            for (int i = 0; i < TT; ++i) fa[i] = __builtin_bit_cast(vec_t, from[lds_unit<CH>(ua + 16 * i, 4 * ks + q)]);
 #pragma unroll
             for (int j = 0; j < TT; ++j) {
-                const vec_t fb = __builtin_bit_cast(vec_t, lds[lds_unit<CH>(ub + 16 * j, 4 * ks + q)]);
+                const vec_t fb = __builtin_bit_cast(vec_t, from[lds_unit<CH>(ub + 16 * j, 4 * ks + q)]);
 #pragma unroll
                 for (int i = 0; i < TT; ++i) acc[i][j] = V::mfma(fa[i], fb, acc[i][j]);
             }
+        }
+    };
+
+    load();
+    if constexpr (TWO) {
+        // one barrier a slab: the next one goes to the other buffer while other waves still multiply
+        uint4_t *now = lds, *next = lds + dump + 1;
+        store(now);
+        if (n_begin + SLAB < n_end) load();
+        __syncthreads();
+        for (int64_t n = n_begin; n < n_end; n += SLAB) {
+            multiply(now);
+            if (n + SLAB < n_end) {
+                store(next);
+                if (n + 2 * SLAB < n_end) load();
+            }
+            __syncthreads();
+            uint4_t *const was = now;
+            now = next;
+            next = was;
+        }
+    } else {
+        for (int64_t n = n_begin; n < n_end; n += SLAB) {
+            __syncthreads();  // the slab in LDS is consumed
+            store(lds);
+            __syncthreads();
+            if (n + SLAB < n_end) load();
+            multiply(lds);
         }
     }
 
@@ -318,16 +345,25 @@ WgradBf plan(int64_t batch, int a, int b, int c, int d, int dtype, float scale)
     return g;
 }
 
-template <typename T, int TT> int launch(const void *dy, const void *x, float *acc, void *dw, const WgradBf &g, hipStream_t s)
+// Tiles of 64 x 64 leave registers for twelve waves a CU: one workgroup of the five to eight that d asks for.  Nobody
+// multiplies while that one waits at the two barriers of a slab, and LDS has room for a second slab: one barrier.  us with one
+// and with two, 25088 rows: fp16 (2,96,384,8) 196 / 156, (1,192,192,32) 712 / 547, (2,64,64,6) 36.0 / 35.0, (1,100,70,5) 45.2 / 43.3;
+// fp32, 12544 rows: 393 / 372, 747 / 677, 49.2 / 49.0, 77.6 / 75.2.  Where several workgroups share a CU they fill each other's
+// waits and the second slab costs some of them their place: (1,512,512,2) 70.6 / 75, (16,64,64,1) 34.6 / 36.5, 48 x 48 tiles
+// (1,48,48,16) 27.2 / 29.2; from 0.9 to 1.1 elsewhere.
+constexpr bool two_slabs(int edge, int waves) { return edge == 4 && waves > 4; }
+
+template <typename T, int TT, bool TWO> int launch(const void *dy, const void *x, float *acc, void *dw, const WgradBf &g, hipStream_t s)
 {
     constexpr int CH = TT == 1 ? 16 : TT == 2 ? 8 : 4;
     const int64_t tiles = (int64_t)g.a_groups * g.d_groups * g.m_groups * g.n_groups;
     const int64_t blocks = g.splits >= 8 ? (int64_t)((g.splits + 7) / 8 * 8) * tiles : g.splits * tiles;
     if (blocks > 0x7fffffffLL) return KSMM_ERR_TOO_LARGE;
-    const int lds = (g.ta * g.td * (g.wm + g.wn) * 16 * TT * CH + 1) * 16;
-    const int rc = ensure_dynamic_lds((const void *)ks_wgrad_bf_kernel<T, TT, CH>, lds);
+    const int lds = (TWO ? 2 : 1) * (g.ta * g.td * (g.wm + g.wn) * 16 * TT * CH + 1) * 16;
+    constexpr int MOST = (TWO ? 2 : 1) * (8 * 2 * 16 * TT * CH + 1) * 16;  // eight waves (the limit is set once a kernel)
+    const int rc = ensure_dynamic_lds((const void *)ks_wgrad_bf_kernel<T, TT, CH, TWO>, MOST);
     if (rc != KSMM_OK) return rc;
-    hipLaunchKernelGGL((ks_wgrad_bf_kernel<T, TT, CH>), dim3((unsigned)blocks), dim3(64 * g.ta * g.td * g.wm * g.wn), lds, s,
+    hipLaunchKernelGGL((ks_wgrad_bf_kernel<T, TT, CH, TWO>), dim3((unsigned)blocks), dim3(64 * g.ta * g.td * g.wm * g.wn), lds, s,
                        (const T *)dy, (const T *)x, acc, (T *)dw, g);
     return hipGetLastError() == hipSuccess ? KSMM_OK : KSMM_ERR_LAUNCH;
 }
@@ -335,10 +371,11 @@ template <typename T, int TT> int launch(const void *dy, const void *x, float *a
 template <typename T> int launch_edge(int t, const void *dy, const void *x, float *acc, void *dw, const WgradBf &g, hipStream_t s)
 {
     switch (t) {
-    case 1: return launch<T, 1>(dy, x, acc, dw, g, s);
-    case 2: return launch<T, 2>(dy, x, acc, dw, g, s);
-    case 3: return launch<T, 3>(dy, x, acc, dw, g, s);
-    default: return launch<T, 4>(dy, x, acc, dw, g, s);
+    case 1: return launch<T, 1, false>(dy, x, acc, dw, g, s);
+    case 2: return launch<T, 2, false>(dy, x, acc, dw, g, s);
+    case 3: return launch<T, 3, false>(dy, x, acc, dw, g, s);
+    default:
+        return two_slabs(t, g.ta * g.td * g.wm * g.wn) ? launch<T, 4, true>(dy, x, acc, dw, g, s) : launch<T, 4, false>(dy, x, acc, dw, g, s);
     }
 }
 

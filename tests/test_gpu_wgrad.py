@@ -43,3 +43,23 @@ def test_weight_gradient_edges(dt, bs_last, offset):
         want = 0.5 * torch.bmm(xs, ys).reshape(a * d * c, b)
         err = ((got.double() - want).norm() / want.norm()).item()
         assert err <= TOL[dt], ((a, b, c, d), n, err)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16])
+@pytest.mark.parametrize("d", [5, 6, 8, 11])
+def test_weight_gradient_slab_counts(dt, d):
+    """Workgroups of five to eight waves on 64 x 64 tiles hold two slabs (32 rows in fp16, 16 in fp32): none, one, an odd
+    and an even number of whole ones, a remainder of one row."""
+    from ksmm_amd import Kernel
+
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    a, b, c = 2, 64, 80
+    for n in (1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 96, 97, 129, 160):
+        x, dy = (torch.randn(n, a * s * d, generator=gen, device="cuda").to(dt) for s in (c, b))
+        factor = torch.zeros(a * c * d, b, device="cuda", dtype=dt)
+        got = Kernel.backward(dy, x, factor, False, a, b, c, d, need_input=False)[1]
+        xs = x.t().double().reshape(a, c, d, n).permute(0, 2, 1, 3).reshape(a * d, c, n)
+        ys = dy.t().double().reshape(a, b, d, n).permute(0, 2, 3, 1).reshape(a * d, n, b).contiguous()
+        want = torch.bmm(xs, ys).reshape(a * d * c, b)
+        err = ((got.double() - want).norm() / want.norm()).item()
+        assert err <= TOL[dt], (n, err)

@@ -138,6 +138,10 @@ float predicted_us(const Problem &p, const ksmm_tile &t)
 // split-K kernel, which alone took such rows before (us at 6501 / 25061 columns): (4,192,192,1) fp16 18 / 38 and 9 / 22,
 // (1,256,256,3) fp16 24 / 46 and 12 / 26, (1,1536,384,2) fp16 47 / 184 and 36 / 112, fp32 166 / 560 and 143 / 507.
 constexpr float RAGGED_H = 1.1f;
+// and where they fill their last tile of outputs in part, whose prices are too low there: us on the kernel that took such rows
+// before / with the prices as they are / with the factor, (12,48,192,6) fp16 at 997 columns 10.6 / 15.6 / 11.1, (12,48,48,4) fp32 at
+// 4531 22.5 / 24.7 / 23.4; (6,96,384,2) fp16 at 9259, 42 before, keeps its tile at 26.
+constexpr float RAGGED_PART = 1.3f;
 
 Choice cheapest_instance(const Problem &p, bool split_only)
 {
@@ -152,7 +156,8 @@ Choice cheapest_instance(const Problem &p, bool split_only)
         if (rc != KSMM_OK) return;
         const CostRow *r = row_of(p, combo, t.algo, t.variant);
         if (!r || (t.threads & 63) || t.tile_d < 1) return;
-        const float us = price(*r, p, t) * (algo == KSMM_ALGO_TILE && (variant >> 24) == 0 && ragged && combo == 1 ? RAGGED_H : 1.f);
+        float us = price(*r, p, t);
+        if (algo == KSMM_ALGO_TILE && (variant >> 24) == 0 && ragged) us *= (combo == 1 ? RAGGED_H : 1.f) * (p.b % t.tile_m ? RAGGED_PART : 1.f);
         if (best.us < 0.f || us < best.us) best = Choice{t.algo, t.variant, us};
     };
     const CostIndex &ix = cost_index();

@@ -34,14 +34,16 @@ namespace ksmm {
 
 namespace {
 
-// GELU for tiles that wait for their epilogue's vector instructions (the other kernels, through epi_finish, wait for memory
-// or their launch, with gelu_erf): x * Phi(x) = max(x, 0) - |x| * tail, tail = erfc(|x| / sqrt 2) / 2 = 2^P(|x|).  log2 of the tail is
-// smooth, and a polynomial of degree 8, fitted to the smallest largest error of the GELU, gives that to 1e-8 before
-// rounding; its leading coefficient is negative, so the tail falls to 0 behind the fitted range (6.5) as well.  11 vector
+// GELU for tiles that write fp16 and wait for their epilogue's vector instructions (the other kernels, through epi_finish, wait
+// for memory or their launch, with gelu_erf): x * Phi(x) = max(x, 0) - |x| * tail, tail = erfc(|x| / sqrt 2) / 2 = 2^P(|x|).
+// log2 of the tail is smooth, and a polynomial of degree 8, fitted to the smallest largest error of the GELU, gives that to 1e-8
+// before rounding; its leading coefficient is negative, so the tail falls to 0 behind the fitted range (6.5) as well.  11 vector
 // instructions per value, one of them transcendental, which is what an epilogue with GELU costs next to the
 // multiplications.  Against Abramowitz & Stegun 7.1.26 for the tail (12 instructions, a reciprocal and an exponential):
-// largest error in fp32 2.5e-7 for 3.3e-7, root mean square over normal values 2.0e-8 for 5.4e-8, and
-// (1,1536,384,2) fp16 at 25088 rows 118.6 -> 109.5 us, (1,768,192,2) 51.4 -> 46.8.
+// largest error before rounding 2.5e-7 for 3.3e-7, root mean square over normal values 2.0e-8 for 5.4e-8, every fp16 input within
+// 0.66 units in the last place for 1.28, and (1,1536,384,2) fp16 at 25088 rows 118.6 -> 109.5 us, (1,768,192,2) 51.4 -> 46.8.
+// fp32 results keep gelu_erf: small differences from 0 count there, and below -4.7 its relative error is the smaller one
+// (-5: 1.6e-3 for 4.9e-3, -6: 3.6e-3 for 6.6e-2).
 __device__ __forceinline__ float gelu_pow2(float x)
 {
     const float ax = fabsf(x);
@@ -54,6 +56,12 @@ __device__ __forceinline__ float gelu_pow2(float x)
     p = fmaf(p, ax, -1.1511097f);
     p = fmaf(p, ax, -0.999999881f);
     return fmaf(-ax, __builtin_amdgcn_exp2f(p), fmaxf(x, 0.f));
+}
+
+template <typename TY> __device__ __forceinline__ float gelu_of(float x)
+{
+    if constexpr (sizeof(TY) == 4) return gelu_erf(x);
+    else return gelu_pow2(x);
 }
 
 constexpr int vmcnt_imm(int n) { return (n & 15) | (7 << 4) | (15 << 8) | (((n >> 4) & 3) << 14); }
@@ -520,7 +528,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void ks_gemm_kernel(const CT *__
 #pragma unroll
                         for (int dd = 0; dd < DD; ++dd) {
                             const float v = fmaf(acc[dd][i][j][e], scale, bias_at(e, dd));
-                            acc[dd][i][j][e] = decltype(gelu)::value ? gelu_pow2(v) : v;
+                            acc[dd][i][j][e] = decltype(gelu)::value ? gelu_of<TY>(v) : v;
                         }
             };
             auto finish_act = [&](int i, const auto &bias_at) {
@@ -962,7 +970,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void ks_gemm_pbf_kernel(const CT
 #pragma unroll
                                 for (int dd = 0; dd < DD; ++dd) {
                                     const float v = fmaf(acc[dd][i][j][4 * eg + u], scale, (float)bb[i][eg][DD * u + dd]);
-                                    acc[dd][i][j][4 * eg + u] = decltype(gelu)::value ? gelu_pow2(v) : v;
+                                    acc[dd][i][j][4 * eg + u] = decltype(gelu)::value ? gelu_of<TY>(v) : v;
                                 }
             };
             // one branch for the tile, as in ks_gemm_kernel.  (1,1536,384,2) at 25088 rows with bias / and GELU: 99.9 / 120.9 us
@@ -1281,7 +1289,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void ks_gemm_pbl_kernel(const CT
 #pragma unroll
                         for (int e = 0; e < 16; ++e) {
                             const float v = fmaf(acc[i][j][e], scale, bl[i]);
-                            acc[i][j][e] = decltype(gelu)::value ? gelu_pow2(v) : v;
+                            acc[i][j][e] = decltype(gelu)::value ? gelu_of<TY>(v) : v;
                         }
             };
             if (ep.act == KSMM_ACT_GELU) finish(std::true_type());

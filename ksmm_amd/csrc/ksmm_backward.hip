@@ -24,13 +24,15 @@ namespace {
 // out block g (b x c, c contiguous)  <-  in block g (c x b, b contiguous); both in "kernel format"
 // of their own pattern: in = (a*d*c, b) of (a,b,c,d), out = (a*d*b, c) of (a,c,b,d).  One launch takes
 // the weights of a whole layer.  A workgroup moves a 64 x 64 square through LDS, so that both sides are
-// whole lines; what bounds it is the launch.
+// whole lines; few elements, and blocks that leave most of their squares empty, are moved an element a thread (their
+// lines stay in the cache): a square each would be a workgroup per block, however small.  What bounds it is the launch.
 struct TransposeArgs {
     struct {
         const void *in;
         void *out;
-        int b, c, b_tiles, c_tiles;
-        uint32_t first;  // the job's first workgroup
+        int b, c, b_tiles, c_tiles;  // b_tiles 0: element by element
+        uint32_t total;              // elements
+        uint32_t first;              // the job's first workgroup
     } job[KSMM_MAX_FACTORS];
     int jobs;
 };
@@ -44,6 +46,13 @@ template <typename T> __global__ __launch_bounds__(256) void ks_block_transpose_
     const T *in = (const T *)t.job[k].in;
     T *out = (T *)t.job[k].out;
     uint32_t id = blockIdx.x - t.job[k].first;
+    if (bt == 0) {
+        const uint32_t total = t.job[k].total, size = (uint32_t)b * c;  // (at most 2^31)
+        const uint32_t at = id * 256 + threadIdx.x, g = at / size, rem = at - g * size;
+        const uint32_t bi = rem / c, ci = rem - bi * c;
+        if (at < total) out[at] = in[(size_t)g * size + ci * b + bi];
+        return;
+    }
     const int b0 = (int)(id % bt) * 64;
     id /= bt;
     const int c0 = (int)(id % ct) * 64;
@@ -57,8 +66,8 @@ template <typename T> __global__ __launch_bounds__(256) void ks_block_transpose_
     __syncthreads();
     if (c0 + x < c)
 #pragma unroll
-        for (int i = y; i < 64; i += 4)
-            if (b0 + i < b) out[block + (size_t)(b0 + i) * c + c0 + x] = square[x][i];
+        for (int i = 0; i < 16; ++i)
+            if (b0 + y + 4 * i < b) out[block + (size_t)(b0 + y + 4 * i) * c + c0 + x] = square[x][y + 4 * i];
 }
 
 // out[i] = scale * (sum of the slices); slices are n floats apart.  One launch takes all the sums of a
@@ -585,7 +594,14 @@ int block_transpose_run(const TransposeJob *jobs, int n, int dtype, hipStream_t 
         o.b_tiles = (j.b + 63) / 64;
         o.c_tiles = (j.c + 63) / 64;
         o.first = (uint32_t)blocks;
-        blocks += j.blocks * o.b_tiles * o.c_tiles;
+        const int64_t total = j.blocks * j.b * j.c, squares = j.blocks * o.b_tiles * o.c_tiles;
+        o.total = (uint32_t)total;
+        // Element by element: squares that are filled to an eighth or less, and few elements, whose time is the latency of
+        // one workgroup.  dX of 16 rows in fp16, us with squares / by elements: (1,2,2,131072) 166 / 19, (64,16,16,64)
+        // 14.7 / 10.6, (6,64,64,1) 6.5 / 5.6, (1,192,192,2) 9.5 / 8.4, (1,512,512,1) 8.5 / 8.3, but (1,512,512,2)
+        // 11.7 / 12.5, (16,64,64,16) 8.9 / 10.3, (6,192,192,16) 19 / 28.
+        if (total <= squares * 512 || total <= 1 << 18) o.b_tiles = 0;
+        blocks += o.b_tiles ? squares : (total + 255) / 256;
         if (blocks > 0x7fffffffLL) return KSMM_ERR_TOO_LARGE;
     }
     if (n < 1) return KSMM_OK;

@@ -59,3 +59,21 @@ def test_layer_backward_refuses_what_the_single_calls_refuse():
     assert lib.ksmm_layer_backward_workspace(d, 2, 0, _lib.KSMM_F32, 0, _lib.ACT_NONE) < 0
     d[1].c = 15
     assert lib.ksmm_layer_backward_workspace(d, 2, 8, _lib.KSMM_F32, 0, _lib.ACT_NONE) < 0  # sizes out of line
+
+
+@pytest.mark.parametrize("pattern", [(1, 1, 1, 1 << 24), (1 << 24, 1, 1, 1), (1 << 12, 3, 5, 17), (3, 16, 16, 64), (2, 33, 31, 5),
+                                     (1, 1, 700, 3), (2, 700, 1, 3), (1, 512, 512, 1), (1, 513, 512, 1), (260, 32, 32, 1),
+                                     (5000, 7, 65, 1), (3, 100, 70, 65)])
+def test_gradient_through_blocks_of_any_size(pattern):
+    """Transposes element by element (few elements, small and thin blocks) and in squares, at both sides of the rule's lines,
+    and more blocks than a launch may have workgroups of 256: against the products in float64, one row, whole numbers."""
+    from ksmm_amd import Kernel
+
+    a, b, c, d = pattern
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    w, g = (torch.randint(-1, 2, s, generator=gen, device="cuda").half() for s in ((a * d * c, b), (1, a * b * d)))
+    dx, _ = Kernel.backward(g, torch.empty(1, a * c * d, device="cuda").half(), w, False, a, b, c, d, need_weight=False)
+    gd = g.view(a, b, d).permute(0, 2, 1).double()
+    for k in range(0, c, 99):  # dx[a, c, d] = sum over b of w[a, d, c, b] g[a, b, d], at most 700
+        want = (w.view(a, d, c, b)[:, :, k].double() * gd).sum(-1)
+        assert torch.equal(dx.view(a, c, d)[:, k].double(), want), (pattern, k)

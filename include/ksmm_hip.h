@@ -292,7 +292,8 @@ int ksmm_epilogue_backward(const void *dy, const void *z, void *dz, void *dbias,
  * activation was applied to (KSMM_ACT_NONE: not read).  Writes dx, dw[i] (kernel format) and dbias, each
  * of which may be NULL where it is not wanted.  Against one call per factor and epilogue it transposes
  * all blocks in one launch and adds all partial sums in one.  Needs ksmm_layer_backward_workspace() bytes
- * of 16-byte aligned device memory. */
+ * of 16-byte aligned device memory, more than the largest of those calls does: the partial sums of all factors,
+ * their transposed blocks and the gradients between them (one for two factors) are held until the end. */
 int64_t ksmm_layer_backward_workspace(const ksmm_factor_desc *factors, int n_factors, int64_t batch, int dtype,
                                       int bs_last, int act);
 int ksmm_layer_backward(const ksmm_factor_desc *factors, int n_factors, const void *const *inputs, const void *z,

@@ -821,7 +821,7 @@ struct LayerBackward {
     int64_t dz, bias_sums;               // gradient of what the activation was applied to; partial sums of the bias's
     int64_t blocks[KSMM_MAX_FACTORS];    // transposed blocks of each factor
     int64_t sums[KSMM_MAX_FACTORS];      // partial sums of each weight gradient: all are added at the end
-    int64_t grads[2];                    // gradients between factors
+    int64_t grads[2];                    // gradient of factor i's input, 0 < i, at grads[i & 1]
     int64_t forward;                     // what the forward kernels of the transposed factors ask for
 };
 
@@ -832,7 +832,7 @@ int64_t layer_backward_layout(const ksmm_factor_desc *f, int n, int64_t batch, i
     int rc = check_chain(f, n, batch, dtype, dtype);
     if (rc != KSMM_OK) return rc;
     const int64_t es = (int64_t)dtype_size(dtype), out = (int64_t)f[n - 1].a * f[n - 1].b * f[n - 1].d;
-    int64_t at = 0, widest = 0, forward = 0;
+    int64_t at = 0, widest[2] = {0, 0}, forward = 0;
     auto take = [&](int64_t bytes) {
         const int64_t was = at;
         at += align256(bytes);
@@ -847,10 +847,10 @@ int64_t layer_backward_layout(const ksmm_factor_desc *f, int n, int64_t batch, i
         if (need < 0) return need;
         if (need > forward) forward = need;
         const int64_t in = (int64_t)f[i].a * f[i].c * f[i].d;
-        if (i > 0 && in > widest) widest = in;
+        if (i > 0 && in > widest[i & 1]) widest[i & 1] = in;
     }
-    l->grads[0] = take(widest * batch * es);
-    l->grads[1] = take(widest * batch * es);
+    l->grads[0] = take(widest[0] * batch * es);
+    l->grads[1] = take(widest[1] * batch * es);
     l->forward = take(forward);
     return at;
 }

@@ -245,6 +245,26 @@ def test_workspace_queries_need_no_gpu():
     assert lib.ksmm_chain_workspace_layout(descs, 2, 512, F16, F16, 0) == 3 * (3072 * 512 * 2)
 
 
+def test_layer_backward_asks_for_the_gradients_it_writes(lib):
+    """Gradients between factors: one buffer for two factors, for more two that are as wide as what lands in them."""
+    from ksmm_amd import _lib
+
+    def more(patterns, n):
+        d = (_lib.KsmmFactorDesc * len(patterns))()
+        for i, (a, b, c, e) in enumerate(patterns):
+            d[i].a, d[i].b, d[i].c, d[i].d, d[i].w_dtype, d[i].scale = a, b, c, e, _lib.KSMM_F16, 1.0
+        single = sum(lib.ksmm_factor_backward_workspace(n, *p, _lib.KSMM_F16, 1) for p in patterns)
+        a, b, _, e = patterns[-1]
+        single += lib.ksmm_epilogue_backward_workspace(n, a * b * e, _lib.KSMM_F16, 1)
+        return lib.ksmm_layer_backward_workspace(d, len(patterns), n, _lib.KSMM_F16, 1, _lib.ACT_NONE) - single
+
+    n, ends = 25088, 256 * 16  # every piece ends on 256 bytes
+    assert more([(1, 64, 64, 1)], n) <= ends
+    assert more([(6, 64, 64, 1), (1, 768, 192, 2)], n) <= 384 * n * 2 + ends
+    assert more([(2, 64, 64, 1), (1, 256, 128, 1), (1, 64, 256, 1)], n) <= (128 + 256) * n * 2 + ends
+    assert more([(2, 64, 64, 1), (1, 256, 128, 1), (1, 64, 256, 1), (1, 32, 64, 1)], n) <= (128 + 256) * n * 2 + ends
+
+
 def test_gelu_constants_of_the_kernel_epilogue():
     """The epilogue's GELU (gelu_erf in ksmm_common.h) is x * Phi(x) with erfc by Abramowitz &
     Stegun 7.1.26 and the formula's factors folded into its constants.  The constants are read

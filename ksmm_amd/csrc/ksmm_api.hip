@@ -258,7 +258,7 @@ bool find_transposed(const Problem &p)
 }
 
 // Batch-size-last rows are `batch` elements long: when that is not a multiple of the 16-byte
-// vector only the split-K and the one-thread-per-output kernels take the problem.  With a workspace it runs on a
+// vector only the k-loop tiles, the split-K and the one-thread-per-output kernels take the problem.  With a workspace it runs on a
 // copy whose rows are zero-filled to the next multiple of 16 columns (the vector of every type)
 // and the result rows are cut back: two copies more, but on the kernel of the padded batch, where that
 // is priced lower (route_pays).

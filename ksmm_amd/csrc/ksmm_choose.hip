@@ -77,6 +77,24 @@ const CostIndex &cost_index()
 
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// batch-size-last rows that no 16-byte vector divides
+bool ragged_rows(const Problem &p) { return p.bs_last && p.batch % (16 / (int64_t)dtype_size(p.x_dtype)) != 0; }
+
+// The k-loop tiles on batch-size-last rows that no vector divides, against whole ones: 1.00 to 1.04 times the time in fp32
+// and e4m3, up to 1.2 in fp16 (seven patterns at 6500 and 6501 columns: vectors off their alignment).  Against the
+// split-K kernel, which alone took such rows before (us at 6501 / 25061 columns): (4,192,192,1) fp16 18 / 38 and 9 / 22,
+// (1,256,256,3) fp16 24 / 46 and 12 / 26, (1,1536,384,2) fp16 47 / 184 and 36 / 112, fp32 166 / 560 and 143 / 507.
+constexpr float RAGGED_H = 1.1f;
+// and where they fill their last tile of outputs in part, by which they have to be ahead: the split-K kernel skips some of
+// what is not there, and its price is up to 1.4 times too high on such blocks.  us on that kernel / on the tile: (12,48,192,6)
+// fp16 at 997 columns 11.8 / 16.5 and (12,48,48,4) fp32 at 4531 23.0 / 25.3 stay where they are for it; (6,96,384,2) fp16 at
+// 9259, 41.0 / 24.5, has its tile.
+// What both factors give: on 8519 drawn ragged problems the choice takes 0.965 (fp32), 0.930 (fp16), 0.963 and 0.946 (e4m3, e4m3
+// weights) of the time without these tiles in the geometric mean; on 127 of them, 1.5 percent, it is more than 3 percent slower,
+// by 1.09 in their mean.  Prices of these tiles fitted to such rows instead gave 0.963, 0.923, 0.963 and 0.945 with 120 that are
+// slower: the tiles' own prices are within 3 percent there, the error is that of the split-K prices (a factor of 1.2 to 1.4).
+constexpr float RAGGED_PART = 1.3f;
+
 float price(const CostRow &r, const Problem &p, const ksmm_tile &t)
 {
     const double ex = (double)dtype_size(p.x_dtype), ew = (double)dtype_size(p.w_dtype), ey = (double)dtype_size(p.y_dtype);
@@ -107,6 +125,8 @@ float price(const CostRow &r, const Problem &p, const ksmm_tile &t)
     const double v[COST_TERMS] = {1., s, cu * s, s * w, cu * s * w, (double)cu, by, by * w, by > 25. ? by - 25. : 0.};
     double us = 0.;
     for (int i = 0; i < COST_TERMS; ++i) us += r.f[i] * v[i];
+    if (t.algo == KSMM_ALGO_TILE && t.variant >> 24 == 0 && ragged_rows(p))
+        us *= (p.x_dtype == KSMM_F16 && p.w_dtype == KSMM_F16 ? RAGGED_H : 1.f) * (p.b % t.tile_m ? RAGGED_PART : 1.f);
     return (float)us;
 }
 
@@ -133,22 +153,12 @@ float predicted_us(const Problem &p, const ksmm_tile &t)
     return r ? price(*r, p, t) : -1.f;
 }
 
-// The k-loop tiles on batch-size-last rows that no vector divides, against whole ones: 1.00 to 1.04 times the time in fp32
-// and e4m3, up to 1.2 in fp16 (seven patterns at 6500 and 6501 columns: vectors off their alignment).  Against the
-// split-K kernel, which alone took such rows before (us at 6501 / 25061 columns): (4,192,192,1) fp16 18 / 38 and 9 / 22,
-// (1,256,256,3) fp16 24 / 46 and 12 / 26, (1,1536,384,2) fp16 47 / 184 and 36 / 112, fp32 166 / 560 and 143 / 507.
-constexpr float RAGGED_H = 1.1f;
-// and where they fill their last tile of outputs in part, whose prices are too low there: us on the kernel that took such rows
-// before / with the prices as they are / with the factor, (12,48,192,6) fp16 at 997 columns 10.6 / 15.6 / 11.1, (12,48,48,4) fp32 at
-// 4531 22.5 / 24.7 / 23.4; (6,96,384,2) fp16 at 9259, 42 before, keeps its tile at 26.
-constexpr float RAGGED_PART = 1.3f;
-
 Choice cheapest_instance(const Problem &p, bool split_only)
 {
     Choice best{KSMM_ALGO_AUTO, -1, -1.f};
     const int combo = combo_of(p.x_dtype, p.w_dtype, p.y_dtype);
     if (combo < 0) return best;
-    const bool ragged = p.bs_last && p.batch % (16 / (int64_t)dtype_size(p.x_dtype)) != 0;
+    const bool ragged = ragged_rows(p);
     auto offer = [&](int algo, int variant) {
         ksmm_tile t;
         memset(&t, 0, sizeof(t));
@@ -156,8 +166,7 @@ Choice cheapest_instance(const Problem &p, bool split_only)
         if (rc != KSMM_OK) return;
         const CostRow *r = row_of(p, combo, t.algo, t.variant);
         if (!r || (t.threads & 63) || t.tile_d < 1) return;
-        float us = price(*r, p, t);
-        if (algo == KSMM_ALGO_TILE && (variant >> 24) == 0 && ragged) us *= (combo == 1 ? RAGGED_H : 1.f) * (p.b % t.tile_m ? RAGGED_PART : 1.f);
+        const float us = price(*r, p, t);
         if (best.us < 0.f || us < best.us) best = Choice{t.algo, t.variant, us};
     };
     const CostIndex &ix = cost_index();

@@ -720,3 +720,22 @@ def test_tile_instances_of_small_problems_are_priced_by_the_number_they_are_repo
     t = query_tile(33 * 197, (4, 192, 192, 1), torch.float16, None, True)  # ragged rows: a split-K tile, as generic 16 + v
     assert t["algo"] == 1 and t["variant"] >= 16
     assert lib.ksmm_price(33 * 197, 4, 192, 192, 1, 1, 1, 1, 1, 0, -1, us) == 0 and us.value > 0
+
+
+def test_choice_on_ragged_rows_is_the_cheapest_by_reported_prices(lib):
+    """What ksmm_price reports for the automatic choice is what it was made with: no k-loop or split-K tile that takes such
+    rows has a lower price (the tiles' factors for ragged rows are part of theirs)."""
+    us = ctypes.c_float()
+
+    def price(problem, combo, algo, variant):
+        a, b, c, d, n = problem
+        types = [(0, 0, 0), (1, 1, 1), (2, 2, 1), (1, 2, 1)][combo]
+        return us.value if lib.ksmm_price(n, a, b, c, d, *types, 1, algo, variant, us) == 0 else None
+
+    for combo, problem in [(0, (12, 48, 48, 4, 4531)), (1, (12, 48, 192, 6, 997)), (1, (4, 192, 192, 1, 6501)), (2, (2, 141, 256, 4, 3871)),
+                           (3, (6, 96, 384, 2, 9259)), (0, (16, 192, 48, 8, 1322))]:
+        chosen = price(problem, combo, 0, -1)
+        tiles = [price(problem, combo, 3, i | 1 << 8) for i in range(128)]
+        tiles += [price(problem, combo, 3, 5 << 24 | w << 8 | i) for i in range(128) for w in (1, 2, 4, 8, 16)]
+        tiles = [t for t in tiles if t is not None and t >= 0]
+        assert len(tiles) > 5 and chosen <= min(tiles) * (1 + 1e-6), (combo, problem, chosen, min(tiles))

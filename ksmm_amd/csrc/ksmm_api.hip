@@ -564,20 +564,20 @@ bool fused_pays(const ksmm_factor_desc *f, int n, const void *x, void *y, int64_
 }
 
 // Whether the fused chain of ksmm_chain16r.hip is the fastest way through a chain that it takes.  Measured on chains of
-// 256, 512 and 1024 features in three types, us a call of the routes below / this one at 197, 2050, 9408 and 25088 rows:
-// batch-size-first always (1024 features: fp32 14 / 11, 21 / 12, 51 / 32, 119 / 68; fp16 14 / 8, 16 / 9, 39 / 20, 81 / 35;
-// e4m3 21 / 9, 24 / 9, 29 / 20, 54 / 32).  Batch-size-last fp32 as well (13 / 12, 29 / 15, 49 / 31, 108 / 64), but where
-// a second round of chunks is nearly empty (1024 features at 4800 columns: 24.1 / 25.8, at 5300 equal).  The 16-bit
-// kernel for whole batch-size-last vectors (ksmm_chain16.hip) has longer chunks and is ahead once this one needs a second
-// round (fp16 4800 columns 17 / 11, 9408 19 / 23; e4m3 13 / 11.5, 14.5 / 23); on other row lengths it needs
-// padded copies (9409 columns: 38 / 28).  Narrower chains leave most of a workgroup idle: one round only.
+// 256, 512 and 1024 features, us of the routes below / this one: batch-size-first always (1024 features at 197, 2050, 9408 and
+// 25088 rows: fp32 14 / 11, 21 / 12, 51 / 31, 119 / 66; fp16 14 / 7, 16 / 8, 39 / 16, 81 / 28; e4m3 21 / 8, 24 / 9, 29 / 16,
+// 54 / 26).  Batch-size-last fp32 and fp16 as well (fp32 13 / 11.5, 29 / 15.5, 49 / 29, 107 / 58; at 4800 columns, where the second
+// round of chunks is nearly empty, 24 / 21; fp16, whose routes below are the kernel for whole vectors, ksmm_chain16.hip, 4800 columns
+// 16.4 / 11.3, 9408 18.7 / 16.9, 25088 33.2 / 29.7, with e4m3 weights 18.6 / 17.4 and 33.1 / 30.4).  On e4m3 inputs that kernel, with
+// its longer chunks, is ahead once this one needs a second round (4800 columns 12.9 / 11.7, 8192 13.3 / 12.3, 9408 14.5 / 17.0,
+// 25088 24.0 / 26.7); on other row lengths it needs padded copies.  Narrower chains leave most of a workgroup idle: one
+// round only.
 bool fused_rows_pay(const ksmm_factor_desc *f, int n, const void *x, void *y, int64_t batch, int x_dtype, int y_dtype, int bs_last)
 {
     if (chain16r_run(f, n, x, y, batch, x_dtype, y_dtype, bs_last ? 1 : 0, false, nullptr, nullptr) != KSMM_OK) return false;
     const int64_t features = (int64_t)f[0].a * f[0].c * f[0].d, round = 256 * 16;
     if (features < 256) return batch <= round;
-    if (!bs_last) return true;
-    if (x_dtype == KSMM_F32) return !(features > 512 && batch > round && batch <= round + round / 4);
+    if (!bs_last || x_dtype != KSMM_FP8_E4M3) return true;
     return batch <= 2 * round || chain16_run(f, n, x, y, batch, x_dtype, y_dtype, 1, false, nullptr, nullptr) != KSMM_OK;
 }
 

@@ -19,11 +19,11 @@
 //
 // What bounds it: a small batch is one launch instead of one per factor, and then the latency of a chunk
 // (weights, input, a barrier per factor, output), 6 us of it on the GPU; full batches the rounds of chunks, one
-// workgroup a CU with the next chunk's input in flight (1024 features, 25088 rows, fp16: 35 us, 3.1 rounds of 32 rows,
+// workgroup a CU with the next chunk's input in flight (1024 features, 25088 rows, fp16: 28 us, 3.1 rounds of 32 rows,
 // where the memory would take 18).  us a call before (a launch per factor, batch-size-first 16-bit chains between
-// two transposes) and now, three factors of 1024 features, 197 / 9408 / 25088 rows: fp32 14 / 51 / 119 -> 11 / 32 / 68,
-// fp16 14 / 39 / 81 -> 8 / 20 / 35, e4m3 21 / 29 / 54 -> 9 / 20 / 32.  64 registers a wave, for two workgroups a CU,
-// spill (fp16 80 us); fp32 with two planes does too.
+// two transposes) and of a replay now, three factors of 1024 features, 197 / 9408 / 25088 rows: fp32 14 / 51 / 119 and
+// 10.5 / 31 / 66, fp16 14 / 39 / 81 and 7.3 / 16 / 28, e4m3 21 / 29 / 54 and 8.2 / 16 / 26.  64 registers a wave, for two
+// workgroups a CU, spill (fp16 80 us); fp32 with two planes does too.
 //
 // Reference counterpart: the Python loop over factors of KSLinear.forward_bs_first / forward_bs_last
 // (src/ksmm_py/layer/kronecker_sparse/interface.py:193-211, 269-291).
@@ -388,9 +388,13 @@ int chain16r_run(const ksmm_factor_desc *f, int n, const void *x, void *y, int64
     const bool aligned = (((uintptr_t)x | (uintptr_t)y) & 15) == 0;
     if (!bs_last && !aligned) return KSMM_ERR_BAD_ALGO;
     if (!launch) return KSMM_OK;
-    // two planes a chunk once every CU has a chunk of two
+    // two planes a chunk where chunks of one would need a second round
     const int ns = combo != 0 && batch > 256 * 16 ? 2 : 1;
-    const int64_t chunks = (batch + 16 * ns - 1) / (16 * ns), most = 512;
+    // One workgroup a CU: with twice as many, the second half starts cold (weights, first input) behind the first.  us with
+    // 512 / 256, 1024 features at 9409 and 25087 rows: batch-size-last fp16 27.4 / 19.9 and 44.9 / 42.3, e4m3 26.6 / 19.4
+    // and 47.5 / 43.3, fp32 34.5 / 32.4 and 71.3 / 73.0, batch-size-first fp16 18.5 / 16.4 and 30.2 / 28.3; 256 features
+    // 1.1 to 1.3 times as fast; the one loss is fp32 beyond 40000 rows of 1024 features, 130 / 133 at 50000.
+    const int64_t chunks = (batch + 16 * ns - 1) / (16 * ns), most = 256;
     const void *fn = combo == 0   ? fn_of<float, float>(n, bs_last, ns)
                      : combo == 1 ? fn_of<half_t, half_t>(n, bs_last, ns)
                      : combo == 2 ? fn_of<fp8_t, fp8_t>(n, bs_last, ns)

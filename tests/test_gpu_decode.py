@@ -68,5 +68,30 @@ def test_room_for_decoded_weights_is_asked_for_where_it_pays():
     plain = lambda n: lib.ksmm_chain_workspace(d, 2, n, _lib.KSMM_F16)
     assert need(64) == plain(64)
     assert need(25088) == plain(25088) + 2 * 768 * 192 * 2
-    # the entry point with its own scratch refuses what it refused: 2 x 384 x 20000 x 2 bytes fit its 32 MiB
-    assert plain(20000) <= lib.ksmm_static_scratch_bytes() < need(21840)
+
+
+def test_the_entry_point_with_its_own_scratch_takes_what_it_took():
+    """Up to what the chain alone needs, with room for decoded weights or without; beyond that it is refused."""
+    from ksmm_amd import KSLinear, _lib
+    from ksmm_amd.kernel import dtype_code
+
+    lib = _lib.load()
+    patterns = [(6, 64, 64, 1), (1, 768, 192, 2)]
+    layer = KSLinear(patterns, algo="kernel", dtype=FP8, bs_last=True, device="cuda", bias=False)
+    d = (_lib.KsmmFactorDesc * 2)()
+    for i, (f, p) in enumerate(zip(layer.factors, patterns)):
+        d[i].w, d[i].w_dtype, d[i].scale = f.data_ptr(), dtype_code(f.dtype), layer.w_scales[i]
+        d[i].a, d[i].b, d[i].c, d[i].d = p
+    xd, yd, room = dtype_code(FP8), _lib.KSMM_F16, lib.ksmm_static_scratch_bytes()
+    most = max(n for n in range(16, 1 << 16, 16) if lib.ksmm_chain_workspace(d, 2, n, yd) <= room)
+    asked = lambda n: lib.ksmm_chain_workspace_layout(d, 2, n, xd, yd, 1)
+    assert asked(20000) <= room < asked(most)
+    stream = torch.cuda.current_stream().cuda_stream
+    for n, rc in ((20000, 0), (most, 0), (most + 16, -9)):
+        codes = torch.randn(layer.in_size, n, device="cuda").to(FP8)
+        y = torch.empty(layer.out_size, n, dtype=torch.float16, device="cuda")
+        assert lib.ksmm_chain_forward_static(d, 2, codes.data_ptr(), y.data_ptr(), n, xd, yd, 1, 1, None, stream) == rc
+        if rc == 0:
+            with torch.no_grad():
+                want = layer(codes, x_scale=1.0)
+            assert O.rel_fro_error(y.double().cpu().numpy(), want.double().cpu().numpy()) <= 1e-3

@@ -12,7 +12,9 @@
 // 256 bytes, all banks, hold 8 or 4 rows: the rows of such a line are permuted, and the pieces of a row, by
 // `key`, the XOR of the row number's 4-bit fields, which takes 16 values on the rows r0 + i*d of a block for
 // any power-of-two d.  So the 16 rows that a 16-lane group of accumulators writes lie in different banks, and so do
-// the 4 rows that such a group reads.  The map is linear over GF(2): the position of row0 ^ off is the XOR of both.
+// the 4 rows that such a group reads.  That is not the whole of it: the counters show conflicts in 0.12 of the LDS-active
+// cycles in fp32 and 0.43 in fp16, where staging and output (lanes 8 rows apart) hit a bank twice and the rest is not
+// accounted for.  The map is linear over GF(2): the position of row0 ^ off is the XOR of both.
 //
 // MFMA roles: A = X^T (rows = batch elements; fp16: transpose loads), B = W^T (lanes = outputs): a lane
 // holds 4 batch elements of one output, one piece.

@@ -239,7 +239,7 @@ int ksmm_chain_forward_ep(const ksmm_factor_desc *factors, int n_factors, const 
                           void *stream);
 
 /* The chain in one launch that needs no workspace, where that is the fastest way through it (radix-16 chains of at most
- * 1024 features); KSMM_ERR_BAD_ALGO, and nothing launched, otherwise.  ksmm_chain_forward_ep with `fuse` takes the same
+ * 1024 features, two factors on small batches); KSMM_ERR_BAD_ALGO, and nothing launched, otherwise.  ksmm_chain_forward_ep with `fuse` takes the same
  * launch. */
 int ksmm_chain_forward_fused(const ksmm_factor_desc *factors, int n_factors, const void *x, void *y, int64_t batch,
                              int x_dtype, int y_dtype, int bs_last, const ksmm_epilogue *epilogue, void *stream);

@@ -4,6 +4,7 @@
 #include <atomic>
 
 #include "ksmm_choose.h"
+#include "ksmm_pair.h"
 
 using namespace ksmm;
 
@@ -671,6 +672,19 @@ bool decode_pays(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, i
     return now > 0.f && then > 4.f && then < ((split || copied) && !copied_then ? 1.f : 0.855f) * now;
 }
 
+// Whether two factors run in one launch (ksmm_pair.hip): where that is priced below the other routes.
+bool pair_pays(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype, int bs_last, PairShape *shape)
+{
+    if (n != 2 || f[0].d != 1 || (f[0].b == 16 && f[0].c == 16)) return false;  // (radix-16 chains have kernels of their own)
+    const float us = pair_us(f, n, batch, x_dtype, y_dtype, bs_last, shape);
+    if (us < 0.f) return false;
+    bool copies;
+    ksmm_factor_desc decoded[2];
+    if (decode_pays(f, n, batch, x_dtype, y_dtype, bs_last, decoded) && us >= chain_best_us(decoded, n, batch, x_dtype, y_dtype, bs_last, &copies) + 4.f)
+        return false;
+    return us < chain_best_us(f, n, batch, x_dtype, y_dtype, bs_last, &copies);
+}
+
 // Workspace of a chain with decoded weights: that of either chain, then (from *at) the fp16 weights
 int64_t decode_layout(const ksmm_factor_desc *f, const ksmm_factor_desc *decoded, int n, int64_t batch, int x_dtype, int y_dtype,
                       int bs_last, int64_t *at)
@@ -707,6 +721,13 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
             return KSMM_ERR_ALIAS;
         if (((uintptr_t)workspace & 15) != 0) return KSMM_ERR_WORKSPACE;
     }
+    PairShape shape;
+    if (fuse && pair_pays(factors, n_factors, batch, x_dtype, y_dtype, bs_last, &shape)) {
+        // (with the workspace that the other routes ask for: a call that lacks it is refused whichever route is the faster)
+        const int64_t asked = chain_layout(factors, n_factors, batch, x_dtype, y_dtype, bs_last);
+        if (asked <= 0 || (workspace && workspace_bytes >= asked))
+            return pair_run(factors, n_factors, x, y, batch, x_dtype, y_dtype, bs_last, shape, (hipStream_t)stream, ep, x_scale);
+    }
     ksmm_factor_desc decoded[KSMM_MAX_FACTORS];
     if (workspace && decode_pays(factors, n_factors, batch, x_dtype, y_dtype, bs_last, decoded)) {
         int64_t at;
@@ -726,7 +747,6 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
         }
     }
     auto ep_of = [&](int i) { return i == n_factors - 1 ? ep : nullptr; };
-    // (with the workspace that the other routes ask for: a call that lacks it is refused whichever route is the faster)
     if (fuse && fused_rows_pay(factors, n_factors, x, y, batch, x_dtype, y_dtype, bs_last)) {
         const int64_t asked = chain_layout(factors, n_factors, batch, x_dtype, y_dtype, bs_last);
         if (asked <= 0 || (workspace && workspace_bytes >= asked)) {
@@ -1085,6 +1105,9 @@ int ksmm_chain_forward_fused(const ksmm_factor_desc *factors, int n_factors, con
     if (overlaps(x, (int64_t)factors[0].a * factors[0].c * factors[0].d * batch * (int64_t)dtype_size(x_dtype), y,
                  (int64_t)l.a * l.b * l.d * batch * (int64_t)dtype_size(y_dtype)))
         return KSMM_ERR_ALIAS;
+    PairShape shape;
+    if (pair_pays(factors, n_factors, batch, x_dtype, y_dtype, bs_last ? 1 : 0, &shape))
+        return pair_run(factors, n_factors, x, y, batch, x_dtype, y_dtype, bs_last ? 1 : 0, shape, (hipStream_t)stream, epilogue);
     if (!fused_rows_pay(factors, n_factors, x, y, batch, x_dtype, y_dtype, bs_last)) return KSMM_ERR_BAD_ALGO;
     return chain16r_run(factors, n_factors, x, y, batch, x_dtype, y_dtype, bs_last ? 1 : 0, true, (hipStream_t)stream, epilogue);
 }

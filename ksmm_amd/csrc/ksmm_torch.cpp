@@ -132,8 +132,9 @@ int forward(const at::Tensor &x, const Layer &l, int64_t batch, const c10::Small
     const int xd = code_of(x.scalar_type()), yd = code_of(out_type);
     void *const stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
     const ksmm_epilogue *const epilogue = ep.bias || ep.act ? &ep : nullptr;
-    // chains of one launch need no workspace (1.7 us); they are of 16 x 16 blocks (asking costs the others 0.4 us)
-    if (fuse && !quantise && l.n > 1 && l.f[0].b == 16 && l.f[0].c == 16) {
+    // chains of one launch need no workspace (1.7 us); they are of 16 x 16 blocks, or of two factors on small batches (asking
+    // costs the others 0.4 us)
+    if (fuse && !quantise && l.n > 1 && ((l.f[0].b == 16 && l.f[0].c == 16) || (l.n == 2 && l.f[0].d == 1 && batch <= 4096))) {
         at::Tensor out = at::empty(shape, x.options().dtype(out_type));
         const int rc = ksmm_chain_forward_fused(l.f, l.n, x.const_data_ptr(), out.mutable_data_ptr(), batch, xd, yd, bs_last, epilogue, stream);
         *y = std::move(out);

@@ -198,66 +198,46 @@ template <> struct wg_vec<half_t> {
     }
 };
 
-// Batch-size-last.  One wavefront owns a (16*MT) x (16*NT)
-// tile of one block's b x c gradient and a range of batch columns.  Lane (r = lane % 16,
-// q = lane / 16) loads N consecutive batch elements of operand row r at column n + N*q; MFMA e
+// Batch-size-last blocks of at most 16 x 16.  One wavefront owns one block's gradient and a range of batch columns.  Lane
+// (r = lane % 16, q = lane / 16) loads N consecutive batch elements of operand row r at column n + N*q; MFMA e
 // multiplies element group e of every lane, i.e. its k-set is {n + N*q + e ...}: the same set for
-// both operands, and the order of a sum's terms is free.
-// NTL: non-temporal loads, for blocks of a single tile (every operand row is read by one wave only;
-// with several tiles per block the rows are shared through the caches)
+// both operands, and the order of a sum's terms is free.  Loads are non-temporal: every operand row is read by one wave.
 // ANY: rows of any length and alignment (a batch that the vector does not divide): vectors at element
 // alignment, and the last one of a row pulled back to end with it, its first elements cleared where
 // the vector before has them.
-template <typename T, int MT, int NT, bool NTL, bool ANY>
+template <typename T, bool ANY>
 __global__ __launch_bounds__(256) void ks_wgrad_bl_kernel(const T *__restrict__ dy, const T *__restrict__ x,
                                                           float *__restrict__ acc_out, int batch, int a, int b,
-                                                          int c, int d, int m_tiles, int n_tiles, int splits,
-                                                          int cols_per_split, int64_t slice)
+                                                          int c, int d, int splits, int cols_per_split, int64_t slice)
 {
     typedef wg_vec<T> V;
     constexpr int STEP = 4 * V::N;  // batch columns per step (4 lane groups)
     const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
-    int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int split = (int)(wave % splits);
-    wave /= splits;
-    const int nt = (int)(wave % n_tiles);
-    wave /= n_tiles;
-    const int mt = (int)(wave % m_tiles);
-    const int64_t g = wave / m_tiles;
+    const int64_t g = wave / splits;
     if (g >= (int64_t)a * d) return;
     const int a_i = (int)(g / d), d_i = (int)(g - (int64_t)a_i * d);
-    const int m0 = mt * 16 * MT, c0 = nt * 16 * NT;
     const int n_begin = split * cols_per_split, n_end = min(batch, n_begin + cols_per_split);
     if (n_begin >= n_end) return;
     const size_t row_stride = (size_t)d * batch;
     // rows behind b (or c) are clamped to the last valid one and dropped at the end
-    const T *ap[MT], *bp[NT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-        ap[i] = dy + ((size_t)a_i * b * d + d_i) * batch + (size_t)min(m0 + 16 * i + r, b - 1) * row_stride;
-#pragma unroll
-    for (int j = 0; j < NT; ++j)
-        bp[j] = x + ((size_t)a_i * c * d + d_i) * batch + (size_t)min(c0 + 16 * j + r, c - 1) * row_stride;
-    float4_t acc[MT][NT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+    const T *const ap = dy + ((size_t)a_i * b * d + d_i) * batch + (size_t)min(r, b - 1) * row_stride;
+    const T *const bp = x + ((size_t)a_i * c * d + d_i) * batch + (size_t)min(r, c - 1) * row_stride;
+    float4_t acc = {0.f, 0.f, 0.f, 0.f};
     typedef typename V::type vec_t;
     // U sub-steps per iteration, all their loads issued before the first MFMA: a row is then read
     // in runs of U * 64 bytes, and the loads of the whole iteration are in flight together
-    constexpr int U = (MT + NT) * 4 <= 24 ? 4 : 2;
+    constexpr int U = 4;
     for (int n = n_begin; n < n_end; n += U * STEP) {
-        vec_t av[U][MT], bv[U][NT];
+        vec_t av[U], bv[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int col = n + u * STEP + V::N * q;
             const bool live = col < n_end;          // whole vectors: batch and the split are multiples of N
             const int lcol = ANY ? min(col, batch - V::N) : live ? col : n_begin;  // (a valid address; the value is zeroed)
-#pragma unroll
-            for (int i = 0; i < MT; ++i) av[u][i] = wg_load<NTL, ANY, vec_t>(ap[i] + lcol);
-#pragma unroll
-            for (int j = 0; j < NT; ++j) bv[u][j] = wg_load<NTL, ANY, vec_t>(bp[j] + lcol);
+            av[u] = wg_load<!ANY, ANY, vec_t>(ap + lcol);
+            bv[u] = wg_load<!ANY, ANY, vec_t>(bp + lcol);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -266,35 +246,20 @@ __global__ __launch_bounds__(256) void ks_wgrad_bl_kernel(const T *__restrict__ 
                 // elements in front of `drop` are not this vector's (n_end is the batch where ANY gets here with col < n_end)
                 const int drop = ANY && col < n_end ? col - min(col, batch - V::N) : V::N;
 #pragma unroll
-                for (int i = 0; i < MT; ++i)
-#pragma unroll
-                    for (int e = 0; e < V::N; ++e) av[u][i][e] = e < drop ? (T)0 : av[u][i][e];
-#pragma unroll
-                for (int j = 0; j < NT; ++j)
-#pragma unroll
-                    for (int e = 0; e < V::N; ++e) bv[u][j][e] = e < drop ? (T)0 : bv[u][j][e];
+                for (int e = 0; e < V::N; ++e) {
+                    av[u][e] = e < drop ? (T)0 : av[u][e];
+                    bv[u][e] = e < drop ? (T)0 : bv[u][e];
+                }
             }
 #pragma unroll
-            for (int e = 0; e < V::MFMAS; ++e)
-#pragma unroll
-                for (int i = 0; i < MT; ++i)
-#pragma unroll
-                    for (int j = 0; j < NT; ++j) acc[i][j] = V::mfma(e, av[u][i], bv[u][j], acc[i][j]);
+            for (int e = 0; e < V::MFMAS; ++e) acc = V::mfma(e, av[u], bv[u], acc);
         }
     }
-    // D: lane holds column (c index) r and rows (b index) 4*q .. 4*q + 3 of each 16 x 16 tile
+    // D: lane holds column (c index) r and rows (b index) 4*q .. 4*q + 3
+    if (r >= c) return;
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j) {
-            const int cc = c0 + 16 * j + r;
-            if (cc >= c) continue;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int m = m0 + 16 * i + 4 * q + e;
-                if (m < b) acc_out[(size_t)split * slice + ((size_t)g * c + cc) * b + m] = acc[i][j][e];
-            }
-        }
+    for (int e = 0; e < 4; ++e)
+        if (4 * q + e < b) acc_out[(size_t)split * slice + ((size_t)g * c + r) * b + 4 * q + e] = acc[e];
 }
 
 // Any layout, any batch: 16 x 16 threads compute a 16 x 16 tile of one block's gradient over a
@@ -342,151 +307,191 @@ __global__ __launch_bounds__(256) void ks_wgrad_tiled_kernel(const T *__restrict
     if (m < b && cc < c) acc_out[(size_t)split * slice + ((size_t)g * c + cc) * b + m] = acc;
 }
 
-// Batch splits of the two weight-gradient kernels (every split is non-empty and writes a slice of
-// a*b*c*d partial sums of its own): columns per split and their number.
-// Weight gradient of large fp16 blocks (b and c multiples of 128), batch-size-last operands: a
-// 128 x 128 tile of one block's gradient and a range of batch columns per workgroup (4 waves, 2 x 2,
-// 64 x 64 each on v_mfma_f32_32x32x16_f16).  Both operands have the batch axis contiguous, so a slab
-// of 64 columns is 128 rows x 128 bytes per operand: it goes through registers into LDS (16-byte
-// chunks, the chunk index XORed with row / 2 so that the operand reads of 16 consecutive rows hit
-// different banks), double-buffered, one barrier per slab.  Against the wave-per-tile kernel above,
-// which re-reads every operand row once per 64 x 64 tile through L2 (1.85 GB for (1,1536,384,2) at
-// batch 25088), the traffic drops to a quarter.  D = X-rows x dY-rows^T, so a lane holds one output
-// feature m (contiguous in kernel format) and 16 inputs k.
+// Weight gradient of blocks beyond 16 x 16 on batch-size-last operands: a TM x TN tile of one block's
+// gradient and a range of batch columns per workgroup (4 waves, 2 x 2, on 32x32 MFMA tiles).  Both operands have the batch
+// axis contiguous, so a slab is 128 bytes (64 columns in fp16, 32 in fp32) of TM + TN rows: it goes through registers into LDS
+// (16-byte chunks, the chunk index XORed with row / 2 so that the operand reads of 16 consecutive rows hit different
+// banks), double-buffered, one barrier per slab.  fp32: a lane's chunk is four of the sum's elements, one for each of
+// four MFMAs, the same four for both operands.  D = X-rows x dY-rows^T, so a lane holds one output feature m (contiguous in
+// kernel format) and 16 inputs k.  Rows behind b (or c) repeat the last valid one and are dropped at the end.
+// What bounds it: in fp32 the matrix cores (at half their rate); in fp16 the latency of a slab, two to five workgroups of 32
+// to 64 KB on a CU.  With the sums of the slices, us / us before, where a wave per 64 x 64 tile loaded its operands itself
+// (one batch of loads in flight, every row read once a tile; fp16 multiples of 128 had the 128 x 128 tile): 25088 columns
+// fp16 (1,768,192,2) 123 / 41, (6,64,256,1) 60 / 28, (1,1536,384,2) 133 / 101; fp32 237 / 146; 6272 columns fp32
+// (1,768,192,2) 83 / 49, (6,64,64,1) 33 / 16; 197 columns (6,64,256,1) 28 / 10; (3,200,768,3) fp16 at 9850 337 / 95.
 // ANY as in the kernel above.
-constexpr int WG_TM = 128, WG_TN = 128, WG_TK = 64;
-template <bool ANY>
-__global__ __launch_bounds__(256, 2) void ks_wgrad_gemm_h_kernel(const half_t *__restrict__ dy,
-                                                                 const half_t *__restrict__ x,
-                                                                 float *__restrict__ acc_out, int batch, int a, int b,
-                                                                 int c, int d, int m_tiles, int n_tiles, int splits,
-                                                                 int cols, int64_t slice)
+template <typename T, int TM, int TN, bool ANY>
+__global__ __launch_bounds__(256, 2) void ks_wgrad_gemm_kernel(const T *__restrict__ dy, const T *__restrict__ x,
+                                                               float *__restrict__ acc_out, int batch, int a, int b, int c,
+                                                               int d, int m_tiles, int n_tiles, int splits, int cols, int64_t slice)
 {
-    __shared__ __attribute__((aligned(16))) half_t sa[2][WG_TM * WG_TK], sb[2][WG_TN * WG_TK];
-    int id = blockIdx.x;
-    const int split = id % splits;
-    id /= splits;
+    constexpr int N = wg_vec<T>::N, TK = 8 * N, VA = TM / 32, VB = TN / 32, MT = TM / 64, NT = TN / 64;
+    extern __shared__ __attribute__((aligned(16))) uint4_t wg_lds[];  // [2][TM + TN rows][8 chunks]
+    // an XCD takes an eighth of the workgroups, the tiles of a split side by side: they share its rows in that L2
+    const int tiles = a * d * m_tiles * n_tiles, per_xcd = (tiles * splits + 7) / 8;
+    const int lid = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (lid >= tiles * splits) return;
+    const int split = lid / tiles;
+    int id = lid - split * tiles;
     const int mt = id % m_tiles;
     id /= m_tiles;
     const int nt = id % n_tiles, g = id / n_tiles;
     const int a_i = g / d, d_i = g - a_i * d;
-    const int m0 = mt * WG_TM, n0 = nt * WG_TN;
+    const int m0 = mt * TM, n0 = nt * TN;
     const int k_begin = split * cols, k_end = min(k_begin + cols, batch);
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, lq = lane >> 5;
     const int wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
-    // staging: 4 vectors per operand and thread; vector v = tid + 256 * i is row v / 8, physical
-    // chunk v % 8, which holds the logical chunk (v % 8) ^ ((row / 2) % 8)
-    const half_t *ga[4], *gb[4];
-    int lcol[4];
+    // staging: vector v = tid + 256 * i is row v / 8, physical chunk v % 8, which holds the logical
+    // chunk (v % 8) ^ ((row / 2) % 8): the same one for all vectors of a thread
+    const int row0 = tid >> 3, lc = ((tid & 7) ^ ((row0 >> 1) & 7)) * N;
+    const T *ga[VA], *gb[VB];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int v = tid + 256 * i, row = v >> 3, lc = (v & 7) ^ ((row >> 1) & 7);
-        lcol[i] = lc * 8;
-        ga[i] = dy + ((size_t)(a_i * b + m0 + row) * d + d_i) * batch + lc * 8;
-        gb[i] = x + ((size_t)(a_i * c + n0 + row) * d + d_i) * batch + lc * 8;
-    }
-    uint4_t ra[4], rb[4];
+    for (int i = 0; i < VA; ++i) ga[i] = dy + ((size_t)(a_i * b + min(m0 + row0 + 32 * i, b - 1)) * d + d_i) * batch;
+#pragma unroll
+    for (int i = 0; i < VB; ++i) gb[i] = x + ((size_t)(a_i * c + min(n0 + row0 + 32 * i, c - 1)) * d + d_i) * batch;
+    uint4_t ra[VA], rb[VB];
+    // (whole vectors of a row that the batch ends in, or the one that ends with it: a valid address, and no branch around
+    // the loads; what is not of this slab is cleared on the way to LDS)
     auto gload = [&](int k) {
+        const int col = min(k + lc, batch - N);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int col = k + lcol[i];
-            ra[i] = rb[i] = uint4_t{0u, 0u, 0u, 0u};
-            if (col >= k_end) continue;  // (without ANY, k_end is a multiple of 8)
-            const int back = ANY ? max(col + 8 - batch, 0) : 0;
-            ra[i] = wg_load<false, ANY, uint4_t>(ga[i] + k - back);
-            rb[i] = wg_load<false, ANY, uint4_t>(gb[i] + k - back);
-            if (ANY && back > 0) {
+        for (int i = 0; i < VA; ++i) ra[i] = wg_load<false, ANY, uint4_t>(ga[i] + col);
+#pragma unroll
+        for (int i = 0; i < VB; ++i) rb[i] = wg_load<false, ANY, uint4_t>(gb[i] + col);
+    };
+    auto lstore = [&](uint4_t *to, int k) {
+        if (k + TK > k_end) {
+            // elements before `from` are not of this vector, those from `until` on not of this split
+            const int col = k + lc, back = col - min(col, batch - N), from = min(back, N), until = min(max(k_end - col, 0) + from, N);
+            auto keep = [&](uint4_t &v) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const uint32_t keep = (2 * e >= back ? 0xffffu : 0u) | (2 * e + 1 >= back ? 0xffff0000u : 0u);
-                    ra[i][e] &= keep;
-                    rb[i][e] &= keep;
+                    uint32_t mask = 0u;
+                    if constexpr (N == 8) {
+                        if (2 * e >= from && 2 * e < until) mask |= 0xffffu;
+                        if (2 * e + 1 >= from && 2 * e + 1 < until) mask |= 0xffff0000u;
+                    } else if (e >= from && e < until) {
+                        mask = 0xffffffffu;
+                    }
+                    v[e] &= mask;
                 }
-            }
+            };
+#pragma unroll
+            for (int i = 0; i < VA; ++i) keep(ra[i]);
+#pragma unroll
+            for (int i = 0; i < VB; ++i) keep(rb[i]);
         }
+#pragma unroll
+        for (int i = 0; i < VA; ++i) to[tid + 256 * i] = ra[i];
+#pragma unroll
+        for (int i = 0; i < VB; ++i) to[TM * 8 + tid + 256 * i] = rb[i];
     };
-    auto lstore = [&](int buf) {
+    float16_t acc[NT][MT];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            *(uint4_t *)(sa[buf] + (tid + 256 * i) * 8) = ra[i];
-            *(uint4_t *)(sb[buf] + (tid + 256 * i) * 8) = rb[i];
-        }
-    };
-    float16_t acc[2][2];
+    for (int i = 0; i < NT; ++i)
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < MT; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-    if (k_begin < k_end) {
-        gload(k_begin);
-        lstore(0);
-    }
+    uint4_t *now = wg_lds, *next = wg_lds + (TM + TN) * 8;
+    gload(k_begin);
+    lstore(now, k_begin);
     __syncthreads();
-    int buf = 0;
-    for (int k = k_begin; k < k_end; k += WG_TK) {
-        const bool more = k + WG_TK < k_end;
-        if (more) gload(k + WG_TK);
+    for (int k = k_begin; k < k_end; k += TK) {
+        gload(k + TK);  // (behind the last slab: of the last columns, and not used)
 #pragma unroll
-        for (int ks = 0; ks < WG_TK / 16; ++ks) {
-            half8_t fx[2], fy[2];
+        for (int ks = 0; ks < 4; ++ks) {
+            uint4_t fx[NT], fy[MT];
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int rx = wn * 64 + i * 32 + l32, ry = wm * 64 + i * 32 + l32;
-                fx[i] = *(const half8_t *)(sb[buf] + (rx * 8 + ((2 * ks + lq) ^ ((rx >> 1) & 7))) * 8);
-                fy[i] = *(const half8_t *)(sa[buf] + (ry * 8 + ((2 * ks + lq) ^ ((ry >> 1) & 7))) * 8);
+            for (int i = 0; i < NT; ++i) {
+                const int r = wn * (TN / 2) + i * 32 + l32;
+                fx[i] = now[TM * 8 + r * 8 + ((2 * ks + lq) ^ ((r >> 1) & 7))];
             }
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int j = 0; j < MT; ++j) {
+                const int r = wm * (TM / 2) + j * 32 + l32;
+                fy[j] = now[r * 8 + ((2 * ks + lq) ^ ((r >> 1) & 7))];
+            }
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fx[i], fy[j], acc[i][j], 0, 0, 0);
+            for (int e = 0; e < (N == 4 ? 4 : 1); ++e)
+#pragma unroll
+                for (int i = 0; i < NT; ++i)
+#pragma unroll
+                    for (int j = 0; j < MT; ++j) {
+                        if constexpr (N == 4)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__builtin_bit_cast(float, (uint32_t)fx[i][e]),
+                                                                             __builtin_bit_cast(float, (uint32_t)fy[j][e]), acc[i][j], 0, 0, 0);
+                        else
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, fx[i]),
+                                                                               __builtin_bit_cast(half8_t, fy[j]), acc[i][j], 0, 0, 0);
+                    }
         }
-        if (more) lstore(buf ^ 1);
+        if (k + TK < k_end) lstore(next, k + TK);
         __syncthreads();
-        buf ^= 1;
+        uint4_t *const was = now;
+        now = next;
+        next = was;
     }
     // D[k'][m]: lane l32 = output feature m, rows k' = 8 * (e / 4) + 4 * lq + e % 4
     float *out = acc_out + (size_t)split * slice + (size_t)g * c * b;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < NT; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < MT; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
-                const int kk = n0 + wn * 64 + i * 32 + 8 * (e >> 2) + 4 * lq + (e & 3);
-                const int m = m0 + wm * 64 + j * 32 + l32;
-                out[(size_t)kk * b + m] = acc[i][j][e];
+                const int kk = n0 + wn * (TN / 2) + i * 32 + 8 * (e >> 2) + 4 * lq + (e & 3);
+                const int m = m0 + wm * (TM / 2) + j * 32 + l32;
+                if (kk < c && m < b) out[(size_t)kk * b + m] = acc[i][j][e];
             }
 }
 
-bool wgrad_gemm_ok(int b, int c, int dtype) { return dtype == KSMM_F16 && b % WG_TM == 0 && c % WG_TN == 0; }
-
-// batch ranges of the tiled kernel: two workgroups per CU, at least 8 slabs each
-void wgrad_gemm_splits(int64_t batch, int64_t tiles, int64_t *splits_out, int64_t *cols_out)
+// Batch ranges: every one is non-empty and writes a slice of a*b*c*d partial sums of its own.
+struct WgradSplit {
+    int64_t splits, cols;
+};
+// `want` of them, of whole `step`s and at least `least` columns, and beyond `fill` no more partial sums (written, then read)
+// than the operands have bytes or 24 MB
+WgradSplit wgrad_split(int64_t batch, int a, int b, int c, int d, int dtype, int64_t want, int64_t fill, int64_t least, int64_t step)
 {
-    int64_t splits = (512 + tiles - 1) / tiles;
-    const int64_t max_splits = (batch + 8 * WG_TK - 1) / (8 * WG_TK);
-    if (splits > max_splits) splits = max_splits;
-    if (splits < 1) splits = 1;
-    int64_t cols = (batch + splits - 1) / splits;
-    cols = (cols + WG_TK - 1) / WG_TK * WG_TK;
-    *splits_out = (batch + cols - 1) / cols;
-    *cols_out = cols;
-}
-
-void wgrad_bl_splits(int64_t batch, int64_t tiles, int step, int64_t *splits_out, int64_t *cols_out)
-{
-    // about 16 waves per CU; at least 4 loop iterations per wave
-    int64_t splits = (4096 + tiles - 1) / tiles;
-    const int64_t max_splits = (batch + 4 * step - 1) / (4 * step);
-    if (splits > max_splits) splits = max_splits;
+    const int64_t bytes = batch * a * (b + c) * d * (int64_t)dtype_size(dtype), slice = (int64_t)a * b * c * d;
+    const int64_t by_traffic = (bytes > (24ll << 20) ? bytes : 24ll << 20) / (8 * slice), by_cols = (batch + least - 1) / least;
+    int64_t splits = want < by_cols ? want : by_cols;
+    const int64_t most = by_traffic > fill ? by_traffic : fill;
+    if (splits > most) splits = most;
     if (splits < 1) splits = 1;
     int64_t cols = (batch + splits - 1) / splits;
     cols = (cols + step - 1) / step * step;
-    *splits_out = (batch + cols - 1) / cols;
-    *cols_out = cols;
+    return WgradSplit{(batch + cols - 1) / cols, cols};
+}
+
+// Blocks of 16 x 16 leave fifteen sixteenths of the GEMM tile empty.  Beyond that it is ahead of the wave-per-tile kernel with
+// tiles of 32, 48 and 64 as well (us with those / on it, 25088 columns: (1,32,32,32) fp32 75.4 / 74.6, fp16 37.4 / 26.3, (1,48,48,16)
+// 63.0 / 48.7 and 32.9 / 22.3; 9000 columns: (6,16,32,8) fp16 20.0 / 17.3).
+bool wgrad_gemm_ok(int b, int c) { return b > 16 || c > 16; }
+
+// An edge of 128 where that pads the block by no more than a tenth beyond what 64 does
+int wgrad_gemm_edge(int n)
+{
+    const int wide = (n + 127) / 128 * 128, narrow = (n + 63) / 64 * 64;
+    return 10 * wide <= 11 * narrow ? 128 : 64;
+}
+// as many workgroups as the CUs' LDS has room for at once, of at least two slabs each; one a CU whatever the partial sums cost
+WgradSplit wgrad_gemm_split(int64_t batch, int a, int b, int c, int d, int dtype)
+{
+    const int tm = wgrad_gemm_edge(b), tn = wgrad_gemm_edge(c), slab = 128 / (int)dtype_size(dtype);
+    const int64_t tiles = (int64_t)a * d * ((b + tm - 1) / tm) * ((c + tn - 1) / tn), room = 256 * (tm + tn == 256 ? 2 : tm + tn == 192 ? 3 : 4);
+    return wgrad_split(batch, a, b, c, d, dtype, room / tiles, (256 + tiles - 1) / tiles, 2 * slab, slab);
+}
+
+// about 16 waves per CU; at least 4 loop iterations per wave, or one where that leaves SIMDs without a wave
+WgradSplit wgrad_bl_split(int64_t batch, int a, int b, int c, int d, int dtype)
+{
+    const int step = 16 * (16 / (int)dtype_size(dtype));  // columns per loop iteration (four sub-steps)
+    const int64_t tiles = (int64_t)a * d;
+    const int64_t long_ones = (batch + 4 * step - 1) / (4 * step);
+    if (long_ones * tiles >= 1024) return wgrad_split(batch, a, b, c, d, dtype, (4096 + tiles - 1) / tiles, (1024 + tiles - 1) / tiles, 4 * step, step);
+    return wgrad_split(batch, a, b, c, d, dtype, (1024 + tiles - 1) / tiles, 1, step, step);
 }
 
 void wgrad_tiled_splits(int64_t batch, int64_t tiles, int64_t *splits_out, int64_t *cols_out)
@@ -501,12 +506,6 @@ void wgrad_tiled_splits(int64_t batch, int64_t tiles, int64_t *splits_out, int64
     *cols_out = cols;
 }
 
-// tile of the MFMA kernel for a block shape: 16 * t rows and columns
-int wgrad_bl_tile(int b, int c)
-{
-    return (b <= 16 && c <= 16) ? 1 : (b <= 32 && c <= 32) ? 2 : (b % 64 && c % 64 && b % 48 == 0 && c % 48 == 0) ? 3 : 4;
-}
-
 // Batch-size-last with at least one vector per row.  Against the tiled kernel at 6501 columns, which
 // the vector does not divide: (1,768,192,2) fp16 310 -> 58 us, fp32 310 -> 82.
 bool wgrad_mfma_ok(int64_t batch, int dtype, int bs_last) { return bs_last && batch >= 16 / (int)dtype_size(dtype); }
@@ -517,24 +516,17 @@ bool wgrad_aligned(const void *dy, const void *x, int64_t batch, int dtype)
     return batch % (16 / (int)dtype_size(dtype)) == 0 && ((((uintptr_t)dy | (uintptr_t)x) & 15) == 0);
 }
 
-template <typename T, int MT, int NT>
+template <typename T>
 int launch_wgrad_bl(const void *dy, const void *x, float *acc, int64_t batch, int a, int b, int c, int d,
                     hipStream_t s, int *splits_used)
 {
-    const int m_tiles = (b + 16 * MT - 1) / (16 * MT), n_tiles = (c + 16 * NT - 1) / (16 * NT);
-    const int64_t tiles = (int64_t)a * d * m_tiles * n_tiles;
-    constexpr int STEP = 16 * wg_vec<T>::N;  // columns per loop iteration of the kernel (four sub-steps)
-    int64_t splits, cols;
-    wgrad_bl_splits(batch, tiles, STEP, &splits, &cols);
-    const int64_t waves = tiles * splits, blocks = (waves + 3) / 4;
+    const auto [splits, cols] = wgrad_bl_split(batch, a, b, c, d, elem<T>::dtype);
+    const int64_t waves = (int64_t)a * d * splits, blocks = (waves + 3) / 4;
     if (blocks > 0x7fffffffLL) return KSMM_ERR_TOO_LARGE;
     *splits_used = (int)splits;
-    const bool one = m_tiles == 1 && n_tiles == 1, any = !wgrad_aligned(dy, x, batch, elem<T>::dtype);
-    const auto fn = any   ? &ks_wgrad_bl_kernel<T, MT, NT, false, true>
-                    : one ? &ks_wgrad_bl_kernel<T, MT, NT, true, false>
-                          : &ks_wgrad_bl_kernel<T, MT, NT, false, false>;
+    const auto fn = wgrad_aligned(dy, x, batch, elem<T>::dtype) ? &ks_wgrad_bl_kernel<T, false> : &ks_wgrad_bl_kernel<T, true>;
     hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(256), 0, s, (const T *)dy, (const T *)x, acc, (int)batch, a, b, c, d,
-                       m_tiles, n_tiles, (int)splits, (int)cols, (int64_t)a * b * c * d);
+                       (int)splits, (int)cols, (int64_t)a * b * c * d);
     return hipGetLastError() == hipSuccess ? KSMM_OK : KSMM_ERR_LAUNCH;
 }
 
@@ -559,21 +551,39 @@ int launch_wgrad_tiled(const void *dy, const void *x, float *acc, int64_t batch,
     return hipGetLastError() == hipSuccess ? KSMM_OK : KSMM_ERR_LAUNCH;
 }
 
+template <typename T, int TM, int TN>
+int launch_wgrad_gemm_tile(const void *dy, const void *x, float *acc, int64_t batch, int a, int b, int c, int d,
+                           hipStream_t s, int *splits_used)
+{
+    const int m_tiles = (b + TM - 1) / TM, n_tiles = (c + TN - 1) / TN;
+    const int64_t tiles = (int64_t)a * d * m_tiles * n_tiles;
+    const auto [splits, cols] = wgrad_gemm_split(batch, a, b, c, d, elem<T>::dtype);
+    const int64_t blocks = (splits * tiles + 7) / 8 * 8;
+    if (blocks > 0x7fffffffLL) return KSMM_ERR_TOO_LARGE;
+    *splits_used = (int)splits;
+    const auto fn = wgrad_aligned(dy, x, batch, elem<T>::dtype) ? &ks_wgrad_gemm_kernel<T, TM, TN, false> : &ks_wgrad_gemm_kernel<T, TM, TN, true>;
+    const int lds = 2 * (TM + TN) * 128;
+    hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(256), lds, s, (const T *)dy, (const T *)x, acc, (int)batch, a, b, c, d,
+                       m_tiles, n_tiles, (int)splits, (int)cols, (int64_t)a * b * c * d);
+    return hipGetLastError() == hipSuccess ? KSMM_OK : KSMM_ERR_LAUNCH;
+}
+template <typename T>
 int launch_wgrad_gemm(const void *dy, const void *x, float *acc, int64_t batch, int a, int b, int c, int d,
                       hipStream_t s, int *splits_used)
 {
-    const int m_tiles = b / WG_TM, n_tiles = c / WG_TN;
-    const int64_t tiles = (int64_t)a * d * m_tiles * n_tiles;
-    int64_t splits, cols;
-    wgrad_gemm_splits(batch, tiles, &splits, &cols);
-    const int64_t blocks = tiles * splits;
-    if (blocks > 0x7fffffffLL) return KSMM_ERR_TOO_LARGE;
-    *splits_used = (int)splits;
-    const auto fn = wgrad_aligned(dy, x, batch, KSMM_F16) ? &ks_wgrad_gemm_h_kernel<false> : &ks_wgrad_gemm_h_kernel<true>;
-    hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(256), 0, s, (const half_t *)dy,
-                       (const half_t *)x, acc, (int)batch, a, b, c, d, m_tiles, n_tiles, (int)splits, (int)cols,
-                       (int64_t)a * b * c * d);
-    return hipGetLastError() == hipSuccess ? KSMM_OK : KSMM_ERR_LAUNCH;
+    const int tm = wgrad_gemm_edge(b), tn = wgrad_gemm_edge(c);
+    const auto fn = tm == 128 ? (tn == 128 ? launch_wgrad_gemm_tile<T, 128, 128> : launch_wgrad_gemm_tile<T, 128, 64>)
+                              : (tn == 128 ? launch_wgrad_gemm_tile<T, 64, 128> : launch_wgrad_gemm_tile<T, 64, 64>);
+    return fn(dy, x, acc, batch, a, b, c, d, s, splits_used);
+}
+
+// the batch-size-last kernels, and the one for rows shorter than a vector in either layout
+template <typename T>
+int wgrad_last(const void *dy, const void *x, float *acc, int64_t batch, int a, int b, int c, int d, int bs_last, hipStream_t s, int *splits)
+{
+    if (!wgrad_mfma_ok(batch, elem<T>::dtype, bs_last)) return launch_wgrad_tiled<T>(dy, x, acc, batch, a, b, c, d, bs_last, s, splits);
+    return wgrad_gemm_ok(b, c) ? launch_wgrad_gemm<T>(dy, x, acc, batch, a, b, c, d, s, splits)
+                               : launch_wgrad_bl<T>(dy, x, acc, batch, a, b, c, d, s, splits);
 }
 
 }  // namespace
@@ -618,17 +628,11 @@ int64_t wgrad_partial_floats(int64_t batch, int a, int b, int c, int d, int dtyp
 {
     if (!bs_last && wgrad_bf_ok(a, b, c, d, dtype)) return wgrad_bf_partial_floats(batch, a, b, c, d, dtype);
     const int64_t n = (int64_t)a * b * c * d;
-    int64_t splits, cols, most = 1;
-    const int t = wgrad_bl_tile(b, c);
-    const int64_t tiles_bl = (int64_t)a * d * ((b + 16 * t - 1) / (16 * t)) * ((c + 16 * t - 1) / (16 * t));
-    wgrad_bl_splits(batch, tiles_bl, 16 * (16 / (int)dtype_size(dtype)), &splits, &cols);
-    if (splits > most) most = splits;
-    wgrad_tiled_splits(batch, (int64_t)a * d * ((b + 15) / 16) * ((c + 15) / 16), &splits, &cols);
-    if (splits > most) most = splits;
-    if (wgrad_gemm_ok(b, c, dtype)) {
-        wgrad_gemm_splits(batch, (int64_t)a * d * (b / WG_TM) * (c / WG_TN), &splits, &cols);
-        if (splits > most) most = splits;
-    }
+    int64_t cols, most = 1;
+    if (wgrad_mfma_ok(batch, dtype, bs_last))
+        most = (wgrad_gemm_ok(b, c) ? wgrad_gemm_split : wgrad_bl_split)(batch, a, b, c, d, dtype).splits;
+    else
+        wgrad_tiled_splits(batch, (int64_t)a * d * ((b + 15) / 16) * ((c + 15) / 16), &most, &cols);
     return most * n;
 }
 
@@ -666,31 +670,15 @@ int wgrad_run(const void *dy, const void *x, void *dw, float *acc, int64_t batch
               int dtype, int bs_last, float scale, hipStream_t stream, FinishJob *rest)
 {
     const int64_t n = (int64_t)a * b * c * d;
-    const bool mfma_ok = wgrad_mfma_ok(batch, dtype, bs_last);
-    const int t = wgrad_bl_tile(b, c);
     int rc, splits = 1;
     *rest = FinishJob{acc, dw, n, 0, scale};
     if (!bs_last && wgrad_bf_ok(a, b, c, d, dtype)) {
         rc = wgrad_bf_run(dy, x, dw, acc, batch, a, b, c, d, dtype, scale, stream, &splits);
         if (rc != KSMM_OK || splits == 1) return rc;
     } else if (dtype == KSMM_F32) {
-        if (mfma_ok)
-            rc = t == 1   ? launch_wgrad_bl<float, 1, 1>(dy, x, acc, batch, a, b, c, d, stream, &splits)
-                 : t == 2 ? launch_wgrad_bl<float, 2, 2>(dy, x, acc, batch, a, b, c, d, stream, &splits)
-                 : t == 3 ? launch_wgrad_bl<float, 3, 3>(dy, x, acc, batch, a, b, c, d, stream, &splits)
-                          : launch_wgrad_bl<float, 4, 4>(dy, x, acc, batch, a, b, c, d, stream, &splits);
-        else
-            rc = launch_wgrad_tiled<float>(dy, x, acc, batch, a, b, c, d, bs_last, stream, &splits);
+        rc = wgrad_last<float>(dy, x, acc, batch, a, b, c, d, bs_last, stream, &splits);
     } else if (dtype == KSMM_F16) {
-        if (mfma_ok && wgrad_gemm_ok(b, c, dtype))
-            rc = launch_wgrad_gemm(dy, x, acc, batch, a, b, c, d, stream, &splits);
-        else if (mfma_ok)
-            rc = t == 1   ? launch_wgrad_bl<half_t, 1, 1>(dy, x, acc, batch, a, b, c, d, stream, &splits)
-                 : t == 2 ? launch_wgrad_bl<half_t, 2, 2>(dy, x, acc, batch, a, b, c, d, stream, &splits)
-                 : t == 3 ? launch_wgrad_bl<half_t, 3, 3>(dy, x, acc, batch, a, b, c, d, stream, &splits)
-                          : launch_wgrad_bl<half_t, 4, 4>(dy, x, acc, batch, a, b, c, d, stream, &splits);
-        else
-            rc = launch_wgrad_tiled<half_t>(dy, x, acc, batch, a, b, c, d, bs_last, stream, &splits);
+        rc = wgrad_last<half_t>(dy, x, acc, batch, a, b, c, d, bs_last, stream, &splits);
     } else {
         return KSMM_ERR_BAD_DTYPE;
     }

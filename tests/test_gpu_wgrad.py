@@ -63,3 +63,23 @@ def test_weight_gradient_slab_counts(dt, d):
         want = torch.bmm(xs, ys).reshape(a * d * c, b)
         err = ((got.double() - want).norm() / want.norm()).item()
         assert err <= TOL[dt], (n, err)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16])
+@pytest.mark.parametrize("shape", [(1, 128, 64, 2), (2, 64, 128, 1), (1, 120, 250, 1), (3, 17, 40, 3)])
+def test_weight_gradient_slabs_batch_last(dt, shape):
+    """Each tile of the batch-size-last GEMM kernel on no more than its first slab (64 columns in fp16, 32 in fp32), whole and
+    ragged ones behind it, and several splits whose last one is short; rows that hold one vector only."""
+    from ksmm_amd import Kernel
+
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    a, b, c, d = shape
+    for n in (4, 8, 9, 31, 32, 33, 63, 64, 65, 127, 128, 129, 130, 192, 200, 1025, 3001):
+        x, dy = (torch.randn(a * s * d, n, generator=gen, device="cuda").to(dt) for s in (c, b))
+        factor = torch.zeros(a * c * d, b, device="cuda", dtype=dt)
+        got = Kernel.backward(dy, x, factor, True, a, b, c, d, need_input=False)[1]
+        xs = x.double().reshape(a, c, d, n).permute(0, 2, 1, 3).reshape(a * d, c, n)
+        ys = dy.double().reshape(a, b, d, n).permute(0, 2, 3, 1).reshape(a * d, n, b).contiguous()
+        want = torch.bmm(xs, ys).reshape(a * d * c, b)
+        err = ((got.double() - want).norm() / want.norm()).item()
+        assert err <= TOL[dt], (n, err)

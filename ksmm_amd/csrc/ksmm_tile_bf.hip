@@ -316,24 +316,20 @@ __global__ __launch_bounds__(64 * WM * WN * NG, (WM * WN * NG >= 8 ? 1 : 2)) voi
         asm volatile("" : "+v"(lv));  // opaque: stays a mask
         return 0u - (uint32_t)lv;
     };
-    auto gload_w = [&](int slot, int k0, bool live) {
-        const uint32_t mk = live_mask(live);
-#pragma unroll
-        for (int i = 0; i < W_PER_T; ++i) wreg[slot][i].load(wt + ((woff[i] + (uint32_t)(k0 * b)) & mk));
-    };
-    auto gload_x = [&](int slot, int k0, bool live) {
-        const uint32_t mk = live_mask(live);
-#pragma unroll
-        for (int i = 0; i < XQ_PER_T; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-                // (32 fp16 blocks per workgroup: few workgroups share a line of x, and read without the
-                // temporal hint it leaves more of L2 to the weights: (8,128,128,64) 2546 -> 2396 us,
-                // (1,192,192,128) 1394 -> 1273; 1-6 % slower with 16 blocks, e4m3 input and in fp32)
-                if constexpr (NG == 4 && sizeof(TX) == 2)
-                    xreg[slot][i][j] = __builtin_nontemporal_load((const xvec_t *)(xt + ((xoff[i] + (uint32_t)((k0 + KH * j) * d)) & mk)));
-                else
-                    xreg[slot][i][j] = *(const xvec_t *)(xt + ((xoff[i] + (uint32_t)((k0 + KH * j) * d)) & mk));
+    // load i of a slab: the weights', then the input's
+    constexpr int LOADS = W_PER_T + 2 * XQ_PER_T;
+    auto gload = [&](int i, int wslot, int wk0, uint32_t wmk, int xslot, int xk0, uint32_t xmk) {
+        if (i < W_PER_T) {
+            wreg[wslot][i < W_PER_T ? i : 0].load(wt + ((woff[i < W_PER_T ? i : 0] + (uint32_t)(wk0 * b)) & wmk));
+        } else {
+            const int q = i >= W_PER_T ? (i - W_PER_T) / 2 : 0, j = (i - W_PER_T) & 1;
+            const xvec_t *const at = (const xvec_t *)(xt + ((xoff[q] + (uint32_t)((xk0 + KH * j) * d)) & xmk));
+            // (32 fp16 blocks per workgroup: few workgroups share a line of x, and read without the
+            // temporal hint it leaves more of L2 to the weights: (8,128,128,64) 2546 -> 2396 us,
+            // (1,192,192,128) 1394 -> 1273; 1-6 % slower with 16 blocks, e4m3 input and in fp32)
+            if constexpr (NG == 4 && sizeof(TX) == 2) xreg[xslot][q][j] = __builtin_nontemporal_load(at);
+            else xreg[xslot][q][j] = *at;
+        }
     };
     auto lstore = [&](int wslot, int slot, int buf) {
 #pragma unroll
@@ -395,58 +391,80 @@ __global__ __launch_bounds__(64 * WM * WN * NG, (WM * WN * NG >= 8 ? 1 : 2)) voi
         const int n = (wn * NT + j) * 32 + l32;
         xrow[j] = TK == 16 ? n * TK + ((lq ^ ((n >> 3) & 1)) << 3) : n * TK + 4 * (lq ^ ((n >> 4) & 1));
     }
-    auto multiply = [&](int buf) {
+    // operands of block dd: TK = 8 has 4 k a lane (one transpose load, one 8-byte read)
+    typedef typename std::conditional<TK == 16, half8_t, half4_t>::type op_t;
+    op_t fw[DD][MT], fx[DD][NT];
+    auto operands = [&](int dd, int buf) {
+        const half_t *wb = ws(buf, wg * DD + dd), *xb = xs(buf, wg * DD + dd);
 #pragma unroll
-        for (int dd = 0; dd < DD; ++dd) {
-            const half_t *wb = ws(buf, wg * DD + dd), *xb = xs(buf, wg * DD + dd);
-            if constexpr (TK == 16) {
-                half8_t fw[MT], fx[NT];
-#pragma unroll
-                for (int i = 0; i < MT; ++i) fw[i] = frag<half_t>::k_outer(wb, LDW, (wm * MT + i) * 32, 0, lane);
-#pragma unroll
-                for (int j = 0; j < NT; ++j) fx[j] = *(const half8_t *)(xb + xrow[j]);
-#pragma unroll
-                for (int i = 0; i < MT; ++i)
-#pragma unroll
-                    for (int j = 0; j < NT; ++j) acc[dd][i][j] = frag<half_t>::mfma(fx[j], fw[i], acc[dd][i][j]);
-            } else {
-                // 8 k per slab: the lane's operand is 4 k (one transpose load, one 8-byte read)
-                half4_t fw[MT], fx[NT];
-#pragma unroll
-                for (int i = 0; i < MT; ++i) fw[i] = frag<half_t>::k_outer4(wb, LDW, (wm * MT + i) * 32, 0, lane);
-#pragma unroll
-                for (int j = 0; j < NT; ++j) fx[j] = *(const half4_t *)(xb + xrow[j]);
-#pragma unroll
-                for (int i = 0; i < MT; ++i)
-#pragma unroll
-                    for (int j = 0; j < NT; ++j)
-                        acc[dd][i][j] = __builtin_amdgcn_mfma_f32_32x32x8f16(fx[j], fw[i], acc[dd][i][j], 0, 0, 0);
-            }
+        for (int i = 0; i < MT; ++i) {
+            if constexpr (TK == 16) fw[dd][i] = frag<half_t>::k_outer(wb, LDW, (wm * MT + i) * 32, 0, lane);
+            else fw[dd][i] = frag<half_t>::k_outer4(wb, LDW, (wm * MT + i) * 32, 0, lane);
         }
+#pragma unroll
+        for (int j = 0; j < NT; ++j) fx[dd][j] = *(const op_t *)(xb + xrow[j]);
+    };
+    auto products = [&](int dd) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                if constexpr (TK == 16) acc[dd][i][j] = frag<half_t>::mfma(fx[dd][j], fw[dd][i], acc[dd][i][j]);
+                else acc[dd][i][j] = __builtin_amdgcn_mfma_f32_32x32x8f16(fx[dd][j], fw[dd][i], acc[dd][i][j], 0, 0, 0);
+            }
     };
 
     const int steps = c / TK;
+    // (wide groups: neighbouring batch tiles begin a slab apart: rows of x that are a multiple of 4 KB long put the same slab
+    // of all of them in the same channels of the L2)
+    const int rot = FL ? nt_id % steps : 0;
+    auto k_of = [&](int s) {
+        s += rot;
+        return (s >= steps ? s - steps : s) * TK;
+    };
     // slab s: request weights PDW and input PDX slabs ahead into the slots slab s came from (it
     // went to LDS an iteration ago), multiply slab s, move slab s + 1 from its registers to
     // the other LDS buffer.  The weights come from L2 and get the shorter lead; they are
     // requested first, so that waiting for them leaves the younger input loads in flight.
+    // Wide groups have one workgroup on a CU, and nobody multiplies while its waves issue their loads: these are spread over
+    // the products, whose operands are read two blocks ahead.  us before / so, and with the batch tiles in step: (6,192,192,64)
+    // on 25088 rows 3841 / 3717, (8,128,128,64) on 12544 rows 1210 / 1151, (1,256,64,64) on 25088 457 / 418, (1,192,192,128) on
+    // 12544 653 / 644, (1,512,128,16) on 25088 257 / 247; with the LDS stores among the products as well 3686 / 1130 / 410, but
+    // 683 and 263.  Groups of 8, two workgroups a CU: registers that spill.
     constexpr int PERIOD = PDX * PDW / (PDX % PDW == 0 ? PDW : PDW % PDX == 0 ? PDX : 1);
     static_assert(PERIOD % PDX == 0 && PERIOD % PDW == 0, "slots repeat after PERIOD slabs");
     auto slab = [&](int u, int s) {
-        gload_w(u % PDW, (s + PDW) * TK, s + PDW < steps);
-        gload_x(u % PDX, (s + PDX) * TK, s + PDX < steps);
-        // (the permutes of the next slab's vectors must not move up here: they would wait for
-        // that slab before this one is multiplied)
+        const uint32_t wmk = live_mask(s + PDW < steps), xmk = live_mask(s + PDX < steps);
+        const int buf = s & 1, wk = k_of(min(s + PDW, steps - 1)), xk = k_of(min(s + PDX, steps - 1));
+        auto request = [&](int i) { gload(i, u % PDW, wk, wmk, u % PDX, xk, xmk); };
+        constexpr int AHEAD = FL ? 2 : 0;
+#pragma unroll
+        for (int i = 0; i < LOADS && !FL; ++i) request(i);
+#pragma unroll
+        for (int dd = 0; dd < AHEAD; ++dd) operands(dd, buf);
         __builtin_amdgcn_sched_barrier(0);
-        multiply(s & 1);
+#pragma unroll
+        for (int dd = 0; dd < DD; ++dd) {
+            if (!FL) operands(dd, buf);
+            products(dd);
+            if (FL) {
+                if (dd + AHEAD < DD) operands(dd + AHEAD, buf);
+#pragma unroll
+                for (int i = dd * LOADS / DD; i < (dd + 1) * LOADS / DD; ++i) request(i);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        // (the permutes of the next slab's vectors must not move up beyond this: they would wait for that slab)
         __builtin_amdgcn_sched_barrier(0);
-        lstore((u + 1) % PDW, (u + 1) % PDX, (s & 1) ^ 1);  // behind the last slab: whatever the idle loads brought
+        lstore((u + 1) % PDW, (u + 1) % PDX, buf ^ 1);  // behind the last slab: whatever the idle loads brought
         __syncthreads();
     };
 #pragma unroll
     for (int u = 0; u < (PDX > PDW ? PDX : PDW); ++u) {
-        if (u < PDW) gload_w(u, u * TK, u < steps);
-        if (u < PDX) gload_x(u, u * TK, u < steps);
+        const uint32_t mk = live_mask(u < steps);
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i)
+            if (i < W_PER_T ? u < PDW : u < PDX) gload(i, u % PDW, k_of(min(u, steps - 1)), mk, u % PDX, k_of(min(u, steps - 1)), mk);
     }
     lstore(0, 0, 0);
     __syncthreads();

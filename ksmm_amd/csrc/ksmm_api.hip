@@ -682,7 +682,9 @@ bool pair_pays(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int
     ksmm_factor_desc decoded[2];
     if (decode_pays(f, n, batch, x_dtype, y_dtype, bs_last, decoded) && us >= chain_best_us(decoded, n, batch, x_dtype, y_dtype, bs_last, &copies) + 4.f)
         return false;
-    return us < chain_best_us(f, n, batch, x_dtype, y_dtype, bs_last, &copies);
+    // (ahead by a part of the prices' error, except where the launch that the host saves is worth more)
+    const float best = chain_best_us(f, n, batch, x_dtype, y_dtype, bs_last, &copies);
+    return (us < 12.f ? 1.f : 1.05f) * us < best;
 }
 
 // Workspace of a chain with decoded weights: that of either chain, then (from *at) the fp16 weights

@@ -16,7 +16,7 @@
 //   far those beyond 125 MB, which the last-level cache does not keep for the next kernel
 // with non-negative coefficients fitted per instance to its measured times, and the cheapest one is
 // taken.  The table comes from `python -m ksmm_amd.prices`, which also says how good the choice is on
-// problems that were held back from the fit (1.05 to 1.07 times the fastest instance in the geometric
+// problems that were held back from the fit (1.04 to 1.08 times the fastest instance in the geometric
 // mean by type and layout); instances that it lists as having no price are not offered.  The generic kernels are priced for the comparison only: they are the choice at full batches
 // of what has no other kernel, or of blocks of a few elements.
 #include <math.h>

@@ -1471,6 +1471,19 @@ const GemmInst gemm_insts[] = {
     GEMM_INST_PL(2, fp8_t, half_t, 64, 128, 64, 2, 2, 5, 2),
     GEMM_INST_PLM(2, fp8_t, half_t, 64, 256, 64, 1, 4, 3, 2, true),
     GEMM_INST_PLM(2, fp8_t, half_t, 64, 128, 64, 2, 2, 5, 2, true),
+    // 64 x 64, two to four workgroups a CU, for what is not a full batch: the tiles above give it a workgroup a CU or less there.
+    // Chosen by price (below 8192 columns), which is 1.08 of the fitted one: the measured choice with them is then 0.89 to 0.998 of
+    // the time without in the geometric mean by type, layout and d = 2 or not, and 7 of 1520 problems are more than 3 percent
+    // slower.  us before / on them: fp32 (1,192,768,2) feature-major at 6272 columns 65 / 37.6, (6,64,256,1) 20.5 / 16.8; fp16
+    // (1,768,768,1) on 1024 rows 9.0 / 5.7, (12,64,256,1) 6.9 / 4.6, (1,768,192,2) 6.0 / 4.8
+    GEMM_INST_O(0, float, true, 1, 64, 64, 16, 2, 2, 4, 4),
+    GEMM_INST_O(0, float, true, 1, 64, 64, 32, 2, 2, 3, 3),
+    GEMM_INST_O(1, half_t, true, 1, 64, 64, 32, 2, 2, 4, 4),
+    GEMM_INST_O(1, half_t, true, 1, 64, 64, 64, 2, 2, 3, 3),
+    GEMM_INST_O(1, half_t, false, 1, 64, 64, 32, 2, 2, 4, 4),
+    GEMM_INST_O(1, half_t, false, 1, 64, 64, 64, 2, 2, 3, 3),
+    GEMM_INST_O(1, half_t, false, 2, 64, 64, 32, 2, 2, 3, 3),
+    GEMM_INST_T(2, fp8_t, half_t, true, 1, 64, 128, 64, 2, 2, 4, 3),
 };
 constexpr int GEMM_PF = 4;             // GemmCfg::PF
 constexpr int N_GEMM_INSTS = sizeof(gemm_insts) / sizeof(GemmInst);

@@ -195,6 +195,14 @@ const TunedRow *tuned_lookup(const Problem &p)
     return nullptr;
 }
 
+// Whether a measured row names an instance of the library for the problem
+bool tuned_for(const Problem &p)
+{
+    const TunedRow *row = p.batch >= TUNED_MIN_BATCH ? tuned_lookup(p) : nullptr;
+    int variant;
+    return row && row->algo != KSMM_ALGO_AUTO && resolve_variant(row->algo, row->id, row->param, row->combo, row->bs_last, &variant);
+}
+
 // A family's kernel, or its own choice (variant < 0).
 int family_run(const Problem &p, int algo, int variant, bool launch, ksmm_tile *tile)
 {
@@ -286,11 +294,23 @@ struct Pick {
     float us;     // predicted time, < 0: no model of it
 };
 
+// Full batches that no row of the table names.  The heuristics were made on the patterns of the table; the prices, fitted on
+// batches up to 16384, find instances that they pass by: (12,64,256,1) fp32 at 25088 rows 221 us / 111, (12,256,64,1) feature-major
+// 131 / 55, (3,128,128,2) fp16 at 17040 rows 27.7 / 11.2, (6,256,64,1) e4m3 at 19440 41.8 / 21.2.  How far below the
+// heuristics' price an instance has to be priced is from 2400 drawn problems of 8192 .. 25088 columns, us of the priced one / of
+// the heuristics' in the geometric mean over those that change: fp32 at 0.9 0.77 feature-major and 0.67 rows (117 problems, 2 of them
+// more than 3 percent slower, by 1.06), the others at 0.85 0.57 .. 0.84 (195 problems, 11 slower, by 1.15 at most); at 0.9
+// 23 of 267 are slower, at 0.97 56 of 469.  (e4m3 weights on fp16 inputs keep the heuristics' choice: what they lose to fp16 weights
+// is what decode_pays goes by.)
+constexpr float HEURISTIC_MARGIN_F = 0.9f, HEURISTIC_MARGIN_H = 0.85f;
+constexpr int64_t HEURISTIC_LAST = 25088;  // the largest batch that this was measured at
+
 // Whether the kernels that move aligned 16-byte vectors take a problem's tensors (null: they will be).
 bool on_vectors(const Problem &p) { return (((uintptr_t)p.x | (uintptr_t)p.w | (uintptr_t)p.y) & 15) == 0; }
 
 // Below TUNED_MIN_BATCH, and where the full-batch choice is the one-thread-per-output kernel, the
-// cheapest instance by the model of ksmm_choose.hip; else the full-batch choice.  Tensors off the
+// cheapest instance by the model of ksmm_choose.hip; else the full-batch choice, a row of the table, or the heuristics' one
+// unless an instance is priced well below it (HEURISTIC_MARGIN).  Tensors off the
 // vector take the cheapest of the kernels that do not need it.  A function of the sizes, types and that
 // alignment alone: each thread remembers its last answers (pricing every instance takes tens
 // of microseconds, a launch five).
@@ -322,8 +342,8 @@ Pick pick_of(const Problem &given, bool table)
     // be slower: it stays.  The one-thread-per-output kernel has to be ahead by the error of its fit (0.3):
     // on 14900 measured problems that it takes, chosen / fastest is 1.059 in the geometric mean so, 1.062 without
     // the margin and 1.081 (up to 13.5) if it is never taken.
-    auto replace = [&](const Choice &c) {
-        if (c.algo == KSMM_ALGO_AUTO || (k.us < 0.f ? k.direct : c.us >= (k.direct ? 1.f : 1.3f) * k.us)) return;
+    auto replace = [&](const Choice &c, float margin) {
+        if (c.algo == KSMM_ALGO_AUTO || (k.us < 0.f ? k.direct : c.us >= (k.direct ? margin : 1.3f) * k.us)) return;
         k.c = c;
         k.us = c.us;
     };
@@ -331,11 +351,12 @@ Pick pick_of(const Problem &given, bool table)
         k.direct = false;
         generic_run(p, 0, false, &t);
         k.us = predicted_us(p, t);
-        replace(cheapest_instance(p, true));
+        replace(cheapest_instance(p, true), 1.f);
     } else if (table_run(p, table, false, &t) == KSMM_OK) {
         k.direct = t.algo != KSMM_ALGO_GENERIC || t.variant == 1;
         k.us = predicted_us(p, t);
-        if (p.batch < TUNED_MIN_BATCH || !k.direct) replace(cheapest_instance(p, false));
+        if (p.batch < TUNED_MIN_BATCH || !k.direct) replace(cheapest_instance(p, false), 1.f);
+        else if (!(table && tuned_for(p)) && p.batch <= HEURISTIC_LAST && p.w_dtype == p.x_dtype) replace(cheapest_instance(p, false), p.x_dtype == KSMM_F32 ? HEURISTIC_MARGIN_F : HEURISTIC_MARGIN_H);
     }
     Entry &e = memo[set][oldest[set]++ % WAYS];
     e.batch = p.batch;

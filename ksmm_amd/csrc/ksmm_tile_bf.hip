@@ -17,7 +17,7 @@
 // Reference counterpart: kernel_bs_first_float / kernel_bs_first_half2
 // (src/ksmm_py/layer/kronecker_sparse/template_kernels_float.cuh:85-286,
 //  template_kernels_half.cuh:103-299), which gather the strided inputs with scalar loads.
-#include "ksmm_mfma.h"
+#include "ksmm_swizzle.h"
 #include <type_traits>
 
 namespace ksmm {
@@ -804,6 +804,235 @@ __global__ __launch_bounds__(64 * WM * WN * NG, (WM * WN * NG >= 8 ? 1 : 2)) voi
 }
 
 // LDS of the whole-d form: one buffer of planes, or the staged result tile if that is larger
+// Whole d of any small number, 3 and 6 among them, where no 16-byte vector is a run of all d_i: a thread loads 8 k (fp32: 4)
+// of all DD blocks of a row, DD vectors in a row, and sorts them by d_i on the way to LDS (16-bit types: one v_perm per word;
+// fp32: a renaming).  A vector of a plane is one chunk of a row, so LDS has no padding and its chunks are swizzled as in the GEMM
+// tiles; the weights are k-outer rows as there.  Both operands go through registers a slab ahead of the products,
+// double-buffered, one barrier a slab; two to three workgroups of four waves on a CU fill each other's waits.  Roles as in
+// the batch-size-first GEMM tiles (A = W, lanes = batch rows): a lane holds 4 outputs x DD blocks of a row, one run of y, and the
+// waves turn their 32 x 32 blocks around in LDS to store whole lines.  Outputs behind b are dropped.
+//
+// What bounds it: LDS reads (24 to 32 bytes a lane and product) on blocks of 192 and more, before that the latency of a slab.
+// Such d ran between two transposes, on the split-K or on the row kernel; us of those / of this one: fp16 (1,256,256,3) at 25088
+// rows 49 / 32 (10 would take the bytes), at 6304 22.5 / 12.6, at 1000 18 / 7.7; (4,96,384,3) 185 / 96, (1,128,128,3) 15.3 / 12.2;
+// e4m3 (1,192,192,3) 33 / 20.5; fp32 (1,256,256,3) 142 / 109; fp16 (12,128,128,6) at
+// 12131 rows 307 / 169.  In the geometric mean over 150 drawn problems of 32 .. 25088 rows it takes 0.7 (fp32), 0.60 (fp16) and 0.70
+// (e4m3) of the time.
+template <typename TX> struct whole_op {
+    typedef half_t type;
+};
+template <> struct whole_op<float> {
+    typedef float type;
+};
+template <typename TX, typename TW, int DD, int TM, int TN, int TK, int WM, int WN> struct WholeCfg {
+    typedef typename whole_op<TX>::type CT;
+    static constexpr int ES = (int)sizeof(CT), EPC = 16 / ES, THREADS = 64 * WM * WN;
+    static constexpr int MT = TM / WM / 32, NT = TN / WN / 32;
+    static constexpr int XC = TK / EPC, WC = TM / EPC;           // chunks of a plane's row, of a weight row
+    static constexpr int X_BYTES = DD * TN * TK * ES, W_BYTES = DD * TK * TM * ES, STAGE = X_BYTES + W_BYTES;
+    // per thread (where they do not come out even some are loaded and written twice): units of DD vectors of x, vectors of w
+    static constexpr int X_UNITS = TN * XC, UNITS = (X_UNITS + THREADS - 1) / THREADS;
+    static constexpr int W_EPV = stage<TW, CT>::EPV, W_VECS = DD * TK * TM / W_EPV, W_PER_T = (W_VECS + THREADS - 1) / THREADS;
+    static constexpr int OP = 32 * DD * ES + 16;                 // bytes per row of a wave's output piece
+    static constexpr int OUT_BYTES = WM * WN * 32 * OP;
+    static constexpr int LDS_BYTES = 2 * STAGE > OUT_BYTES ? 2 * STAGE : OUT_BYTES;
+    // (the swizzle of the weight rows moves chunks over 64 outputs)
+    static_assert(TM % (32 * WM) == 0 && TM >= 64 && TN % (32 * WN) == 0 && (XC == 2 || XC == 4) && LDS_BYTES <= 160 * 1024, "tiling");
+};
+template <int XC> __device__ __forceinline__ int whole_swz(int row) { return XC == 4 ? (row >> 2) & 3 : (row >> 3) & 1; }
+
+template <typename TX, typename TW, typename TY, int DD, int TM, int TN, int TK, int WM, int WN, int OCC>
+__global__ __launch_bounds__(64 * WM * WN, OCC) void ks_whole_bf_kernel(const TX *__restrict__ x, const TW *__restrict__ w,
+                                                                       TY *__restrict__ y, int batch, int a, int b, int c, int d,
+                                                                       Epi ep, int m_tiles, int n_tiles, int blocks)
+{
+    epi_load<TX>(ep);
+    typedef WholeCfg<TX, TW, DD, TM, TN, TK, WM, WN> C;
+    typedef typename C::CT CT;
+    constexpr bool F32 = sizeof(CT) == 4;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    // the TM-tiles of one batch tile run side by side on one XCD
+    const int per_xcd = (blocks + 7) / 8;
+    const int lid = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if (lid >= blocks) return;
+    const int mt_id = lid % m_tiles, rest = lid / m_tiles, nt_id = rest % n_tiles, a_i = rest / n_tiles;
+    const int m0 = mt_id * TM, n0 = nt_id * TN;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave / WN, wn = wave % WN;
+    const int l32 = lane & 31, lq = lane >> 5;
+    const size_t in_size = (size_t)a * c * DD, out_size = (size_t)a * b * DD;
+
+    // ---- staging ----
+    typedef typename std::conditional<sizeof(TX) == 1, uint2_t, uint4_t>::type xvec_t;  // e4m3: 8 codes
+    const TX *xp[C::UNITS];
+    int xdst[C::UNITS];
+#pragma unroll
+    for (int i = 0; i < C::UNITS; ++i) {
+        const int u = (tid + i * C::THREADS) % C::X_UNITS, row = u / C::XC, kc = u % C::XC;
+        xp[i] = x + (size_t)min(n0 + row, batch - 1) * in_size + ((size_t)a_i * c + kc * C::EPC) * DD;
+        xdst[i] = row * (TK * C::ES) + ((kc ^ whole_swz<C::XC>(row)) << 4);
+    }
+    const TW *wp[C::W_PER_T];
+    int wdst[C::W_PER_T];
+#pragma unroll
+    for (int i = 0; i < C::W_PER_T; ++i) {
+        constexpr int WV = TM / C::W_EPV;
+        const int v = (tid + i * C::THREADS) % C::W_VECS, mv = v % WV, k = v / WV % TK, dd = v / (WV * TK);
+        wp[i] = w + ((size_t)(a_i * DD + dd) * c + k) * b + min(m0 + mv * C::W_EPV, b - C::W_EPV);
+        const int chunk = mv * C::W_EPV / C::EPC;
+        wdst[i] = C::X_BYTES + (dd * TK + k) * (TM * C::ES) + ((chunk ^ (F32 ? 8 * ((k >> 2) & 1) : swz_outer<half_t, C::WC>(k))) << 4);
+    }
+    xvec_t xreg[C::UNITS][DD];
+    stage<TW, CT> wreg[C::W_PER_T];
+    auto gload = [&](int s) {
+#pragma unroll
+        for (int i = 0; i < C::UNITS; ++i)
+#pragma unroll
+            for (int j = 0; j < DD; ++j) xreg[i][j] = ((const xvec_t *)(xp[i] + (size_t)s * (TK * DD)))[j];
+#pragma unroll
+        for (int i = 0; i < C::W_PER_T; ++i) wreg[i].load(wp[i] + (size_t)s * TK * b);
+    };
+    auto lstore = [&](unsigned char *to) {
+#pragma unroll
+        for (int i = 0; i < C::UNITS; ++i) {
+            // word q of the unit: 16-bit elements 2 q and 2 q + 1 (element k * DD + dd), or fp32 element q
+            uint32_t word[4 * DD];
+#pragma unroll
+            for (int j = 0; j < DD; ++j) {
+                if constexpr (sizeof(TX) == 1) {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        word[4 * j + 2 * h] = __builtin_bit_cast(uint32_t, fp8x2_to_half2(xreg[i][j][h]));
+                        word[4 * j + 2 * h + 1] = __builtin_bit_cast(uint32_t, fp8x2_hi_to_half2(xreg[i][j][h]));
+                    }
+                } else {
+#pragma unroll
+                    for (int h = 0; h < 4; ++h) word[4 * j + h] = xreg[i][j][h];
+                }
+            }
+#pragma unroll
+            for (int dd = 0; dd < DD; ++dd) {
+                uint4_t v;
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    if constexpr (F32) {
+                        v[p] = word[p * DD + dd];
+                    } else {
+                        const int e0 = 2 * p * DD + dd, e1 = (2 * p + 1) * DD + dd;
+                        v[p] = __builtin_amdgcn_perm(word[e1 >> 1], word[e0 >> 1], ((e0 & 1) ? 0x0302u : 0x0100u) | ((e1 & 1) ? 0x07060000u : 0x05040000u));
+                    }
+                }
+                *(uint4_t *)(to + xdst[i] + dd * (TN * TK * C::ES)) = v;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < C::W_PER_T; ++i) wreg[i].store((CT *)(to + wdst[i]));
+    };
+
+    float16_t acc[DD][C::MT][C::NT];
+#pragma unroll
+    for (int dd = 0; dd < DD; ++dd)
+#pragma unroll
+        for (int i = 0; i < C::MT; ++i)
+#pragma unroll
+            for (int j = 0; j < C::NT; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[dd][i][j][e] = 0.f;
+    const uint32_t base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
+    auto multiply = [&](int buf) {
+        const unsigned char *const xs = smem + buf * C::STAGE;
+#pragma unroll
+        for (int dd = 0; dd < DD; ++dd) {
+#pragma unroll
+            for (int ks = 0; ks < C::XC / 2; ++ks) {
+                uint4_t fx[C::NT];  // chunk 2 ks + lq of the lane's row
+#pragma unroll
+                for (int j = 0; j < C::NT; ++j) {
+                    const int row = (wn * C::NT + j) * 32 + l32;
+                    fx[j] = *(const uint4_t *)(xs + dd * (TN * TK * C::ES) + row * (TK * C::ES) + (((2 * ks + lq) ^ whole_swz<C::XC>(row)) << 4));
+                }
+#pragma unroll
+                for (int i = 0; i < C::MT; ++i) {
+                    const int col = (wm * C::MT + i) * 32;
+                    if constexpr (F32) {
+                        const float *const wr = (const float *)(xs + C::X_BYTES) + (dd * TK + 8 * ks + 4 * lq) * TM;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const int m = col + l32;
+                            const float fw = wr[e * TM + ((((m >> 2) ^ (8 * lq)) << 2) | (m & 3))];
+#pragma unroll
+                            for (int j = 0; j < C::NT; ++j)
+                                acc[dd][i][j] = frag<float>::mfma(fw, __builtin_bit_cast(float, (uint32_t)fx[j][e]), acc[dd][i][j]);
+                        }
+                    } else {
+                        const half8_t fw = outer_frag<half_t, TM>::read(base + buf * C::STAGE + C::X_BYTES + dd * (TK * TM * 2) + outer_frag<half_t, TM>::off(col, lane), 16 * ks);
+#pragma unroll
+                        for (int j = 0; j < C::NT; ++j) acc[dd][i][j] = frag<half_t>::mfma(fw, __builtin_bit_cast(half8_t, fx[j]), acc[dd][i][j]);
+                    }
+                }
+            }
+        }
+    };
+
+    const int steps = c / TK;
+    gload(0);
+    lstore(smem);
+    __syncthreads();
+    for (int s = 0; s < steps; ++s) {
+        gload(min(s + 1, steps - 1));  // (behind the last slab: repeats of it, not used)
+        multiply(s & 1);
+        if (s + 1 < steps) lstore(smem + ((s + 1) & 1) * C::STAGE);
+        __syncthreads();
+    }
+
+    // lane: row n = l32 of the block, outputs 8 eg + 4 lq .. + 3 of every d_i: 4 DD consecutive elements
+    unsigned char *const piece = smem + wave * (32 * C::OP);
+    struct alignas(4 * sizeof(TY)) Run {
+        TY v[4 * DD];
+    };
+#pragma unroll
+    for (int i = 0; i < C::MT; ++i) {
+        const int mb = m0 + (wm * C::MT + i) * 32;
+        float bv[4][4 * DD];
+#pragma unroll
+        for (int eg = 0; eg < 4; ++eg) {
+            const int m = min(mb + 8 * eg + 4 * lq, b - 4);
+            Run r = {};
+            if (ep.bias) __builtin_memcpy(&r, (const TY *)ep.bias + ((size_t)a_i * b + m) * DD, sizeof(r));
+#pragma unroll
+            for (int q = 0; q < 4 * DD; ++q) bv[eg][q] = (float)r.v[q];
+        }
+#pragma unroll
+        for (int j = 0; j < C::NT; ++j) {
+            const int nb = n0 + (wn * C::NT + j) * 32;
+            auto turn = [&](auto gelu) {
+#pragma unroll
+                for (int eg = 0; eg < 4; ++eg) {
+                    Run o;
+#pragma unroll
+                    for (int q = 0; q < 4 * DD; ++q) {
+                        const float v = fmaf(acc[q % DD][i][j][4 * eg + q / DD], ep.scale, bv[eg][q]);
+                        o.v[q] = (TY)(decltype(gelu)::value ? gelu_erf(v) : v);
+                    }
+                    *(Run *)(piece + l32 * C::OP + (8 * eg + 4 * lq) * (DD * C::ES)) = o;
+                }
+            };
+            // (one branch for the block)
+            if (ep.act == KSMM_ACT_GELU) turn(std::true_type());
+            else turn(std::false_type());
+            __builtin_amdgcn_wave_barrier();
+            constexpr int RV = 32 * DD * C::ES / 16;  // vectors of a row
+#pragma unroll
+            for (int q = 0; q < 32 * RV / 64; ++q) {
+                const int v = lane + 64 * q, row = v / RV, at = v % RV;
+                if (nb + row < batch && at * 16 < (b - mb) * (DD * C::ES))
+                    *(uint4_t *)((unsigned char *)(y + (size_t)(nb + row) * out_size + ((size_t)a_i * b + mb) * DD) + at * 16) =
+                        *(const uint4_t *)(piece + row * C::OP + at * 16);
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+}
+
 constexpr int bf8l_lds(int ng, int tk, int tm, int tn)
 {
     const int ldw = tm == 32 ? 32 : pads<half_t>::outer(tm);
@@ -818,8 +1047,12 @@ constexpr int bf4l_lds(int ng, int tk, int tm, int tn)
 struct BfInst {
     int combo, dd, tm, tn, tk, threads, lds, wm;
     const void *fn;
-    int pd;  // slabs in flight in registers, input * 16 + weights (ks_tile_bf8_kernel); 0: the plain kernel
+    int pd;  // slabs in flight in registers, input * 16 + weights (ks_tile_bf8_kernel); 0: the plain kernel; WHOLE: ks_whole_bf_kernel
 };
+constexpr int WHOLE = 1024;
+#define WHOLE_INST(COMBO_, TX_, TW_, TY_, DD_, TM_, TN_, TK_, WM_, WN_, OCC_)                      \
+    {COMBO_, DD_, TM_, TN_, TK_, 64 * WM_ * WN_, WholeCfg<TX_, TW_, DD_, TM_, TN_, TK_, WM_, WN_>::LDS_BYTES, WM_, \
+     (const void *)ks_whole_bf_kernel<TX_, TW_, TY_, DD_, TM_, TN_, TK_, WM_, WN_, OCC_>, WHOLE}
 #define BF_INST(COMBO_, CT_, TW_, DD_, TM_, TN_, TK_, WM_, WN_)                                  \
     {COMBO_, DD_, TM_, TN_, TK_, 64 * WM_ * WN_, BfCfg<CT_, TW_, DD_, TM_, TN_, TK_, WM_, WN_>::LDS_BYTES, WM_, \
      (const void *)ks_tile_bf_kernel<CT_, TW_, CT_, DD_, TM_, TN_, TK_, WM_, WN_>}
@@ -852,6 +1085,9 @@ struct BfInst {
      (const void *)ks_tile_bf4_kernel<TM_, TN_, WM_, WN_, PDX_, PDW_, NG_, TK_>, 256 + PDX_ * 16 + PDW_}
 #define BF8_SET(COMBO_, TX_, TW_)                                                                \
     BF8_INST(COMBO_, TX_, TW_, 64, 64, 2, 2, 2, 2), BF8_INST(COMBO_, TX_, TW_, 64, 128, 2, 4, 2, 2)
+#define WHOLE_SET(COMBO_, TX_, TW_, TK_)                                                             \
+    WHOLE_INST(COMBO_, TX_, TW_, half_t, 3, 64, 64, TK_, 2, 2, 3), WHOLE_INST(COMBO_, TX_, TW_, half_t, 3, 64, 128, TK_, 2, 4, 4), \
+        WHOLE_INST(COMBO_, TX_, TW_, half_t, 3, 128, 128, TK_, 4, 2, 2), WHOLE_INST(COMBO_, TX_, TW_, half_t, 6, 64, 64, TK_ / 2, 2, 2, 2)
 const BfInst bf_insts[] = {
     BF_SET_H(1, half_t),
     BF_SET_H(3, fp8_t),
@@ -902,12 +1138,28 @@ const BfInst bf_insts[] = {
     // 16-bit groups of 8 on a 128 x 64 tile, 8 waves
     BF8_INST(1, half_t, half_t, 128, 64, 4, 2, 2, 2), BF8_INST(3, half_t, fp8_t, 128, 64, 4, 2, 2, 2),
     BF8_INST(2, fp8_t, fp8_t, 128, 64, 4, 2, 2, 2),
+    // whole d = 3 and 6 (fp32: 64 x 128 never won; fp16 (1,64,64,3) and (1,128,128,3) at 25088 rows have no row in the measured table:
+    // the row kernels are ahead on inputs out of memory, 8.2 us / 8.7 and 14.8 / 15.5, and behind on just written ones, 8.1 / 7.2
+    // and 15.0 / 12.3; e4m3 weights on fp16 inputs, which come behind a chain's first factor, are decoded for the fp16 form)
+    WHOLE_SET(1, half_t, half_t, 32),
+    WHOLE_SET(2, fp8_t, fp8_t, 32),
+    WHOLE_INST(0, float, float, float, 3, 64, 64, 16, 2, 2, 3), WHOLE_INST(0, float, float, float, 3, 128, 128, 16, 4, 2, 2),
+    WHOLE_INST(0, float, float, float, 6, 64, 64, 8, 2, 2, 2),
 };
 constexpr int N_BF_INSTS = sizeof(bf_insts) / sizeof(BfInst);
 
 bool bf_fits(const BfInst &t, const Problem &p, int combo)
 {
     if (t.combo != combo || p.bs_last || p.d % t.dd) return false;
+    if (t.pd == WHOLE) {
+        // vectors of weights, of a unit of x (8 k in 16-bit types, 4 in fp32) and of y's rows; a short last TM-tile
+        const int ws = (int)dtype_size(p.w_dtype), xs = (int)dtype_size(p.x_dtype), ys = (int)dtype_size(p.y_dtype), xv = xs == 1 ? 8 : 16;
+        // (fp32 d = 6, whose planes leave one workgroup a CU: a tile filled in part was up to 1.17 times the time of the
+        // transposed route, full ones 0.59 to 1.00)
+        if (combo == 0 && t.dd == 6 && p.b % t.tm) return false;
+        return p.d == t.dd && p.b >= 32 && p.b % (16 / ws) == 0 && p.c % t.tk == 0 && (int64_t)p.a * p.c * p.d * xs % xv == 0 &&
+               (int64_t)p.c * p.d * xs % xv == 0 && (int64_t)p.b * p.d * ys % 16 == 0;
+    }
     if (p.b % t.tm || p.c % t.tk) return false;
     const int x_epv = 16 / (int)dtype_size(p.x_dtype), w_epv = 16 / (int)dtype_size(p.w_dtype);
     // d > DD: the DD elements of one (row, k) must fill the 16-byte vector
@@ -949,7 +1201,7 @@ int tile_bf_run(const Problem &p, int variant, bool launch, ksmm_tile *tile)
         int64_t best = -1;
         for (int i = 0; i < N_BF_INSTS; ++i) {
             const BfInst &t = bf_insts[i];
-            if (!bf_fits(t, p, combo)) continue;
+            if (t.pd == WHOLE || !bf_fits(t, p, combo)) continue;  // (those are chosen by price)
             // Groups out of a larger d: every line of x is shared by d/DD groups x b/TM tiles, and
             // the loads are 16-byte pieces d elements apart.  Against the transposed route (two
             // extra passes, but the fastest kernels in between) this wins while b x d stays
@@ -1027,7 +1279,7 @@ int tile_bf_run(const Problem &p, int variant, bool launch, ksmm_tile *tile)
     }
     if (pick < 0) return KSMM_ERR_BAD_ALGO;
     const BfInst &t = bf_insts[pick];
-    const int m_tiles = p.b / t.tm;
+    const int m_tiles = (p.b + t.tm - 1) / t.tm;
     const int64_t n_tiles = (p.batch + t.tn - 1) / t.tn;
     const int64_t blocks = (int64_t)p.a * (p.d / t.dd) * m_tiles * n_tiles;
     const int64_t grid = (blocks + 7) / 8 * 8;

@@ -1,0 +1,68 @@
+"""Batch-size-first tiles that take all of d = 3 or 6 at once: every instance, at batches around its tiles, with blocks that
+fill its tiles of outputs and blocks that do not, against float64.
+
+Tolerances: fp32 1e-5, fp16 and e4m3 operands 2e-3 (one rounding of the result to 2^-11; the operands are exact and the sums
+fp32)."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+FP8 = torch.float8_e4m3fn
+
+
+@pytest.mark.parametrize("dts", [(torch.float32, torch.float32), (torch.float16, torch.float16), (FP8, FP8)])
+@pytest.mark.parametrize("pattern", [(2, 192, 64, 3), (1, 32, 32, 3), (3, 80, 96, 3), (1, 144, 128, 3), (2, 64, 48, 6), (3, 128, 32, 6), (1, 208, 16, 6)])
+def test_whole_d(dts, pattern):
+    from ksmm_amd import Kernel, _lib
+    from ksmm_amd._lib import KsmmError
+    from ksmm_amd.kernel import query_tile
+
+    (a, b, c, d), (xt, wt) = pattern, dts
+    w = (torch.rand(a * d * c, b, device="cuda") * 2 - 1).div(math.sqrt(c)).to(wt)
+    wk = w.float().double().view(a, d, c, b)
+    seen = set()
+    for n in (1, 33, 63, 64, 65, 127, 129, 515):
+        x = torch.randn(n, a * c * d, device="cuda").to(xt)
+        flat = torch.full((a * b * d * n + 64,), 7.0, device="cuda", dtype=torch.float32 if xt == torch.float32 else torch.float16)
+        y = flat[:a * b * d * n].view(n, a * b * d)
+        xk = x.float().double().view(n, a, c, d)
+        want = torch.stack([torch.stack([xk[:, i, :, j].contiguous() @ wk[i, j] for j in range(d)], -1) for i in range(a)], 1)
+        want = want.reshape(n, -1)
+        for i in range(128):
+            variant = 3 << 24 | i
+            try:
+                tile = query_tile(n, pattern, xt, wt, False, _lib.ALGO_TILE, variant)
+            except KsmmError:
+                continue
+            if tile["tile_d"] != d:
+                continue
+            seen.add(i)
+            flat.fill_(7.0)
+            Kernel.forward(x, w, False, a, b, c, d, out=y, algo=_lib.ALGO_TILE, variant=variant)
+            err = ((y.double() - want).norm() / want.norm()).item()
+            assert err <= (1e-5 if xt == torch.float32 else 2e-3), (n, i, err)
+            assert bool((flat[a * b * d * n:] == 7.0).all())
+    least = (1 if b % 64 == 0 else 0) if xt == torch.float32 and d == 6 else 2 if xt == torch.float32 else 1 if d == 6 else 3
+    assert len(seen) >= (least if c % (32 if d == 3 else 16) == 0 else 0), seen
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16, FP8])
+def test_whole_d_epilogue(dt):
+    """Bias and GELU of a layer whose factor the tiles take, and what they refuse: a stride or block off the vector."""
+    from ksmm_amd import KSLinear, quantize_fp8
+
+    for pattern in ((1, 192, 192, 3), (2, 80, 192, 3), (1, 72, 96, 3), (1, 100, 96, 3)):
+        w4 = (torch.rand(pattern) * 2 - 1) / math.sqrt(pattern[2])
+        layer = KSLinear([pattern], weights=[w4], algo="kernel", dtype=dt, device="cuda", act="gelu")
+        dense = layer.get_dense_product(torch.float64)
+        for n in (197, 1001):
+            x = torch.randn(n, layer.in_size, device="cuda")
+            x, scale = quantize_fp8(x) if dt == FP8 else (x.to(dt), None)
+            with torch.no_grad():
+                y = layer(x, x_scale=scale)
+                z = x.double() * (float(scale) if scale is not None else 1.0) @ dense.T + layer.bias.double()
+            want = z * 0.5 * (1 + torch.erf(z / math.sqrt(2)))
+            assert ((y.double() - want).norm() / want.norm()).item() <= {torch.float32: 1e-5, torch.float16: 2e-3, FP8: 5e-3}[dt]

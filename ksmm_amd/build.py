@@ -14,7 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "build")
 LIB = os.path.join(HERE, "libksmm_hip.so")
-SOURCES = ["ksmm_api.hip", "ksmm_generic.hip", "ksmm_wave.hip", "ksmm_tile.hip", "ksmm_stream.hip", "ksmm_tile_bf.hip", "ksmm_rows_bf.hip", "ksmm_gemm.hip", "ksmm_split.hip", "ksmm_pair.hip", "ksmm_choose.hip", "ksmm_chain16.hip", "ksmm_chain16r.hip", "ksmm_transpose.hip", "ksmm_backward.hip", "ksmm_wgrad_bf.hip", "ksmm_act_bwd.hip", "ksmm_quant.hip"]
+SOURCES = ["ksmm_api.hip", "ksmm_generic.hip", "ksmm_wave.hip", "ksmm_tile.hip", "ksmm_stream.hip", "ksmm_tile_bf.hip", "ksmm_rows_bf.hip", "ksmm_gemm.hip", "ksmm_split.hip", "ksmm_pair.hip", "ksmm_choose.hip", "ksmm_chain16.hip", "ksmm_chain16r.hip", "ksmm_transpose.hip", "ksmm_backward.hip", "ksmm_wgrad_bf.hip", "ksmm_wgrad_wide.hip", "ksmm_act_bwd.hip", "ksmm_quant.hip"]
 # measurement aids of bench.py: a library of their own, outside the drop-in ABI
 BENCH_LIB = os.path.join(HERE, "libksmm_bench.so")
 BENCH_SOURCES = ["ksmm_probe.hip"]

@@ -17,10 +17,14 @@
 // or four slabs of 16 KB in flight per CU; four waves a workgroup, three workgroups a CU.  Eight-wave
 // workgroups read less through L2 but leave one workgroup a CU: 83 us instead of 52 on the second
 // shape below.  128 registers a wave (four waves a SIMD) spill: 74 us.
+// (fp16 blocks of 48 and more with d up to 4 have ksmm_wgrad_wide.hip.)
 // Against transposed copies of both operands in HBM and the batch-size-last kernel on them, fp16 at
 // 25088 rows: (1,768,192,2) 156 -> 52 us, (6,64,256,1) 90 -> 35, (1,128,128,3) 38 -> 23,
 // (1,1536,384,2) 213 -> 157 (180 on another box), (1,16,16,64) 70 -> 46; fp32: 323 -> 200, 193 -> 72, 108 -> 52, 1083 -> 680, 148 -> 52.
+#include <algorithm>
+
 #include "ksmm_common.h"
+#include "ksmm_wgrad_wide.h"
 
 namespace ksmm {
 
@@ -389,14 +393,17 @@ bool wgrad_bf_ok(int a, int b, int c, int d, int dtype)
 
 int64_t wgrad_bf_partial_floats(int64_t batch, int a, int b, int c, int d, int dtype)
 {
+    // (which of the two kernels runs depends on the tensors' alignment)
     const WgradBf g = plan(batch, a, b, c, d, dtype, 1.f);
-    return g.splits > 1 ? g.splits * g.slice : 0;
+    return std::max(g.splits > 1 ? g.splits * g.slice : 0, wgrad_wide_partial_floats(batch, a, b, c, d, dtype));
 }
 
 // dw is complete when *splits is 1; otherwise acc holds *splits slices of partial sums.
 int wgrad_bf_run(const void *dy, const void *x, void *dw, float *acc, int64_t batch, int a, int b, int c, int d, int dtype,
                  float scale, hipStream_t stream, int *splits)
 {
+    const int rc = wgrad_wide_run(dy, x, dw, acc, batch, a, b, c, d, dtype, scale, stream, splits);
+    if (rc != KSMM_ERR_BAD_ALGO) return rc;
     const WgradBf g = plan(batch, a, b, c, d, dtype, scale);
     *splits = g.splits;
     const int t = edge_of(b, c);

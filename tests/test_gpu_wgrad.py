@@ -83,3 +83,37 @@ def test_weight_gradient_slabs_batch_last(dt, shape):
         want = torch.bmm(xs, ys).reshape(a * d * c, b)
         err = ((got.double() - want).norm() / want.norm()).item()
         assert err <= TOL[dt], (n, err)
+
+
+@pytest.mark.parametrize("d", [1, 2, 3, 4])
+def test_weight_gradient_wide(d):
+    """Batch-size-first fp16 blocks of 48 and more (ksmm_wgrad_wide.hip): tiles of 64 and 128 filled and in part, no whole slab, whole
+    ones and a remainder of one row, one split and several."""
+    from ksmm_amd import Kernel
+
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    for a, b, c in ((1, 64, 64), (3, 48, 56), (2, 128, 72), (1, 72, 128), (1, 200, 136), (5, 64, 192), (1, 520, 264)):
+        for n in (1, 32, 63, 64, 65, 97, 129, 1025, 1100, 2304) if b * c < 20000 else (64, 1031, 4000):
+            x, dy = (torch.randn(n, a * s * d, generator=gen, device="cuda").half() for s in (c, b))
+            factor = torch.zeros(a * c * d, b, device="cuda", dtype=torch.float16)
+            got = Kernel.backward(dy, x, factor, False, a, b, c, d, scale=0.5, need_input=False)[1]
+            xs = x.t().double().reshape(a, c, d, n).permute(0, 2, 1, 3).reshape(a * d, c, n)
+            ys = dy.t().double().reshape(a, b, d, n).permute(0, 2, 3, 1).reshape(a * d, n, b).contiguous()
+            want = 0.5 * torch.bmm(xs, ys).reshape(a * d * c, b)
+            err = ((got.double() - want).norm() / want.norm()).item()
+            assert err <= TOL[torch.float16], ((a, b, c, d), n, err)
+
+
+def test_weight_gradient_wide_bytes():
+    """Rows behind a split's end and features behind a block's do not reach the sums: infinities there would."""
+    from ksmm_amd import Kernel
+
+    a, b, c, d, n = 2, 72, 56, 2, 1100
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    rows = [torch.full((n + 200, a * s * d), float("inf"), device="cuda", dtype=torch.float16) for s in (c, b)]
+    for r in rows:
+        r[:n] = torch.randn(n, r.shape[1], generator=gen, device="cuda").half()
+        r[:n].view(n, a, -1)[:, 1] = float("inf")  # the second block: its own gradient only
+    factor = torch.zeros(a * c * d, b, device="cuda", dtype=torch.float16)
+    got = Kernel.backward(rows[1][:n], rows[0][:n], factor, False, a, b, c, d, need_input=False)[1].view(a, -1)
+    assert bool(got[0].isfinite().all()) and not bool(got[1].isfinite().any())

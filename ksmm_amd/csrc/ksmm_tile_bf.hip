@@ -804,7 +804,7 @@ __global__ __launch_bounds__(64 * WM * WN * NG, (WM * WN * NG >= 8 ? 1 : 2)) voi
 }
 
 // LDS of the whole-d form: one buffer of planes, or the staged result tile if that is larger
-// Whole d of any small number, 3 and 6 among them, where no 16-byte vector is a run of all d_i: a thread loads 8 k (fp32: 4)
+// Whole d of a small number, 3 and 6 among them, where no 16-byte vector is a run of all d_i: a thread loads 8 k (fp32: 4)
 // of all DD blocks of a row, DD vectors in a row, and sorts them by d_i on the way to LDS (16-bit types: one v_perm per word;
 // fp32: a renaming).  A vector of a plane is one chunk of a row, so LDS has no padding and its chunks are swizzled as in the GEMM
 // tiles; the weights are k-outer rows as there.  Both operands go through registers a slab ahead of the products,
@@ -817,7 +817,10 @@ __global__ __launch_bounds__(64 * WM * WN * NG, (WM * WN * NG >= 8 ? 1 : 2)) voi
 // rows 49 / 32 (10 would take the bytes), at 6304 22.5 / 12.6, at 1000 18 / 7.7; (4,96,384,3) 185 / 96, (1,128,128,3) 15.3 / 12.2;
 // e4m3 (1,192,192,3) 33 / 20.5; fp32 (1,256,256,3) 142 / 109; fp16 (12,128,128,6) at
 // 12131 rows 307 / 169.  In the geometric mean over 150 drawn problems of 32 .. 25088 rows it takes 0.7 (fp32), 0.60 (fp16) and 0.70
-// (e4m3) of the time.
+// (e4m3) of the time.  With d = 2 and 4 a vector is such a run, and the plain kernel above, whose planes are padded and whose slabs
+// are one in flight between two barriers, takes them too: e4m3 (3,512,128,2) at 25088 rows 87 / 42, (6,128,128,2) 52 / 26,
+// (1,256,256,4) 43.6 / 33.4, 0.755 of the time over 67 drawn problems; fp32 (1,768,192,2) 167 / 141, 0.93 over 20.  fp16 has the GEMM
+// tiles for d = 2, and d = 4 was behind on this kernel (1.11 over 37).
 template <typename TX> struct whole_op {
     typedef half_t type;
 };
@@ -1145,6 +1148,10 @@ const BfInst bf_insts[] = {
     WHOLE_SET(2, fp8_t, fp8_t, 32),
     WHOLE_INST(0, float, float, float, 3, 64, 64, 16, 2, 2, 3), WHOLE_INST(0, float, float, float, 3, 128, 128, 16, 4, 2, 2),
     WHOLE_INST(0, float, float, float, 6, 64, 64, 8, 2, 2, 2),
+    // and of d = 2 and 4
+    WHOLE_INST(0, float, float, float, 2, 64, 64, 16, 2, 2, 4), WHOLE_INST(0, float, float, float, 2, 128, 128, 16, 4, 2, 2),
+    WHOLE_INST(2, fp8_t, fp8_t, half_t, 4, 64, 64, 32, 2, 2, 2),
+    WHOLE_INST(2, fp8_t, fp8_t, half_t, 2, 64, 64, 32, 2, 2, 4), WHOLE_INST(2, fp8_t, fp8_t, half_t, 2, 128, 128, 32, 4, 2, 4),
 };
 constexpr int N_BF_INSTS = sizeof(bf_insts) / sizeof(BfInst);
 
@@ -1155,8 +1162,11 @@ bool bf_fits(const BfInst &t, const Problem &p, int combo)
         // vectors of weights, of a unit of x (8 k in 16-bit types, 4 in fp32) and of y's rows; a short last TM-tile
         const int ws = (int)dtype_size(p.w_dtype), xs = (int)dtype_size(p.x_dtype), ys = (int)dtype_size(p.y_dtype), xv = xs == 1 ? 8 : 16;
         // (fp32 d = 6, whose planes leave one workgroup a CU: a tile filled in part was up to 1.17 times the time of the
-        // transposed route, full ones 0.59 to 1.00)
-        if (combo == 0 && t.dd == 6 && p.b % t.tm) return false;
+        // transposed route, full ones 0.59 to 1.00; d = 2, whose other kernel is 1.06 times slower on full tiles, likewise, 24.0 us / 27.0
+        // on (6,96,96,2) at 5950 rows, and on fewer rows than a tile or long c, (12,768,192,2) at 37 10.2 / 12.9, (1,192,768,2) at
+        // 5051 44 / 51)
+        if (combo == 0 && (t.dd == 2 || t.dd == 6) && p.b % 64) return false;
+        if (combo == 0 && t.dd == 2 && (p.batch < 64 || p.c > 512)) return false;
         return p.d == t.dd && p.b >= 32 && p.b % (16 / ws) == 0 && p.c % t.tk == 0 && (int64_t)p.a * p.c * p.d * xs % xv == 0 &&
                (int64_t)p.c * p.d * xs % xv == 0 && (int64_t)p.b * p.d * ys % 16 == 0;
     }

@@ -694,18 +694,44 @@ bool decode_pays(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, i
 }
 
 // Whether two factors run in one launch (ksmm_pair.hip): where that is priced below the other routes.
-bool pair_pays(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype, int bs_last, PairShape *shape)
+bool pair_priced_lower(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype, int bs_last, PairShape *shape)
 {
-    if (n != 2 || f[0].d != 1 || (f[0].b == 16 && f[0].c == 16)) return false;  // (radix-16 chains have kernels of their own)
     const float us = pair_us(f, n, batch, x_dtype, y_dtype, bs_last, shape);
     if (us < 0.f) return false;
     bool copies;
     ksmm_factor_desc decoded[2];
     if (decode_pays(f, n, batch, x_dtype, y_dtype, bs_last, decoded) && us >= chain_best_us(decoded, n, batch, x_dtype, y_dtype, bs_last, &copies) + 4.f)
         return false;
-    // (ahead by a part of the prices' error, except where the launch that the host saves is worth more)
+    // (ahead by a part of the prices' error; short ones, which wait for the host's launches, may be behind by a part of the launch
+    // that they save: (6,64,64,1)+(1,768,192,2) fp32 on 32 columns 9.6 us on the GPU for 8.6, 8.9 a call for 10.5)
     const float best = chain_best_us(f, n, batch, x_dtype, y_dtype, bs_last, &copies);
-    return (us < 12.f ? 1.f : 1.05f) * us < best;
+    return us < 12.f ? us < best + 1.f : 1.05f * us < best;
+}
+
+// A function of the sizes and types alone, asked up to three times a call: each thread remembers its last answers (2 us
+// otherwise, of a call of 10).
+bool pair_pays(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype, int bs_last, PairShape *shape)
+{
+    if (n != 2 || f[0].d != 1 || (f[0].b == 16 && f[0].c == 16)) return false;  // (radix-16 chains have kernels of their own)
+    struct Entry {
+        int64_t batch;  // 0: empty
+        int key[13];
+        PairShape shape;
+        bool pays;
+    };
+    constexpr unsigned ENTRIES = 128;
+    static thread_local Entry memo[ENTRIES];
+    const int key[13] = {f[0].a, f[0].b, f[0].c, f[0].d, f[0].w_dtype, f[1].a, f[1].b, f[1].c, f[1].d, f[1].w_dtype, x_dtype, y_dtype, bs_last != 0};
+    uint64_t h = (uint64_t)batch;
+    for (int v : key) h = (h ^ (uint64_t)v) * 0x9E3779B97F4A7C15ull;
+    Entry &e = memo[(h >> 40) % ENTRIES];
+    if (e.batch != batch || memcmp(e.key, key, sizeof(key)) != 0) {
+        e.batch = batch;
+        memcpy(e.key, key, sizeof(key));
+        e.pays = pair_priced_lower(f, n, batch, x_dtype, y_dtype, bs_last, &e.shape);
+    }
+    *shape = e.shape;
+    return e.pays;
 }
 
 // Workspace of a chain with decoded weights: that of either chain, then (from *at) the fp16 weights

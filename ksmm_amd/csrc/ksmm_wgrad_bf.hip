@@ -17,7 +17,7 @@
 // or four slabs of 16 KB in flight per CU; four waves a workgroup, three workgroups a CU.  Eight-wave
 // workgroups read less through L2 but leave one workgroup a CU: 83 us instead of 52 on the second
 // shape below.  128 registers a wave (four waves a SIMD) spill: 74 us.
-// (fp16 blocks of 48 and more with d up to 4 have ksmm_wgrad_wide.hip.)
+// (fp16 blocks of 48 and more with d up to 4 or 6 have ksmm_wgrad_wide.hip.)
 // Against transposed copies of both operands in HBM and the batch-size-last kernel on them, fp16 at
 // 25088 rows: (1,768,192,2) 156 -> 52 us, (6,64,256,1) 90 -> 35, (1,128,128,3) 38 -> 23,
 // (1,1536,384,2) 213 -> 157 (180 on another box), (1,16,16,64) 70 -> 46; fp32: 323 -> 200, 193 -> 72, 108 -> 52, 1083 -> 680, 148 -> 52.

@@ -1,4 +1,4 @@
-// Weight gradients of batch-size-first fp16 blocks of 64 and more (ksmm_wgrad_wide.hip)
+// Weight gradients of batch-size-first fp16 blocks of 48 and more (ksmm_wgrad_wide.hip)
 #pragma once
 #include "ksmm_common.h"
 

@@ -1,4 +1,4 @@
-// Weight gradient of a Kronecker-sparse factor on batch-size-first fp16 tensors, blocks of 64 and more with d up to 4:
+// Weight gradient of a Kronecker-sparse factor on batch-size-first fp16 tensors, blocks of 48 and more with d up to 4 or 6:
 //   dW[a_i, m, k, d_i] = sum_n dY[n, (a_i b + m) d + d_i] * X[n, (a_i c + k) d + d_i]
 // A slab of rows n is staged as it lies, one plane of [n][features] per d_i and operand: a thread loads 8 features of all d_i of a
 // row, d vectors in a row, sorts them by d_i (one v_perm per word, nothing at d = 1) and writes a vector into each plane.  The
@@ -11,8 +11,8 @@
 // blocks the launch of the sum over the splits.  One workgroup a CU reaches it, so there are few splits, and big tiles read less.
 // fp16, us with the sum, the kernel of ksmm_wgrad_bf.hip / this one at 25088 rows: (1,1536,384,2) 168 / 100 (35 would take the
 // bytes), (1,768,192,2) 61 / 46, (6,64,256,1) 40 / 26.5, (6,64,64,1) 23 / 15.7, (1,128,128,3) 23.4 / 22.1, (1,96,96,4) 25.0 / 21.5;
-// (1,768,192,2) at 3000 rows 25.5 / 17.0, (6,64,64,1) at 1000 11.2 / 8.3.  Over 28 shapes 1.31 times as fast in the geometric mean.
-// That kernel keeps fp32, which waits for its matrix cores, d beyond 4, blocks below 48 and what no 16-byte vector divides.
+// (1,768,192,2) at 3000 rows 25.5 / 17.0, (6,64,64,1) at 1000 11.2 / 8.3; (12,64,64,6) at 9000 64.5 / 46.3.  Over 28 shapes 1.31 times as fast in the geometric mean.
+// That kernel keeps fp32, which waits for its matrix cores, other d, blocks below 48 and what no 16-byte vector divides.
 #include <algorithm>
 #include <type_traits>
 
@@ -237,6 +237,8 @@ const WideInst wide_insts[] = {
     WIDE_INST(2, 64, 64, 4, 64, 2), WIDE_INST(2, 128, 64, 2, 64, 2), WIDE_INST(2, 64, 128, 2, 64, 2), WIDE_INST(2, 128, 128, 1, 32, 2),
     WIDE_INST(3, 64, 64, 2, 96, 2), WIDE_INST(3, 128, 64, 1, 48, 2), WIDE_INST(3, 64, 128, 1, 48, 2),
     WIDE_INST(4, 64, 64, 2, 64, 2),
+    // (d = 8: 0.56 to 0.77 of the other kernel's speed, its rows fill half of a load)
+    WIDE_INST(6, 64, 64, 1, 32, 2),
 };
 
 struct WidePlan {
@@ -247,10 +249,10 @@ struct WidePlan {
 WidePlan wide_plan(int64_t batch, int a, int b, int c, int d, int dtype, float scale)
 {
     WidePlan p{};
-    // (32-bit offsets inside a slab; slabs of three and four d_i take longer to fill than few rows take on the other kernel:
-    // (1,128,128,3) on 196 rows 9.7 us there and 10.5 here, (1,64,256,4) on 777 12.1 and 12.4)
-    if (d > 2 && batch < 1024) return p;
-    if (dtype != KSMM_F16 || d > 4 || b % 8 || c % 8 || b < 48 || c < 48 || (int64_t)a * (b > c ? b : c) * d > 1 << 24) return p;
+    // (32-bit offsets inside a slab; slabs of three and more d_i take longer to fill than few rows take on the other kernel:
+    // (1,128,128,3) on 196 rows 9.7 us there and 10.5 here, (1,64,256,4) on 777 12.1 and 12.4, (1,96,96,6) on 1100 13.8 and 14.1)
+    if (batch < (d > 4 ? 2048 : d > 2 ? 1024 : 0)) return p;
+    if (dtype != KSMM_F16 || d > 6 || b % 8 || c % 8 || b < 48 || c < 48 || (int64_t)a * (b > c ? b : c) * d > 1 << 24) return p;
     const int64_t slice = (int64_t)a * b * c * d, by_rows = batch <= 1024 ? (batch + 63) / 64 : (batch + 127) / 128;
     // The tile and the splits: 1 .. 4 rounds of a workgroup a CU, whose rows arrive at 42 bytes a ns, and partial sums written and
     // read at 5 TB/s

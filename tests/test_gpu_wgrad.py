@@ -85,7 +85,7 @@ def test_weight_gradient_slabs_batch_last(dt, shape):
         assert err <= TOL[dt], (n, err)
 
 
-@pytest.mark.parametrize("d", [1, 2, 3, 4])
+@pytest.mark.parametrize("d", [1, 2, 3, 4, 6])
 def test_weight_gradient_wide(d):
     """Batch-size-first fp16 blocks of 48 and more (ksmm_wgrad_wide.hip): tiles of 64 and 128 filled and in part, no whole slab, whole
     ones and a remainder of one row, one split and several."""

@@ -415,28 +415,21 @@ __global__ __launch_bounds__(64 * WM * WN * NG, (WM * WN * NG >= 8 ? 1 : 2)) voi
     };
 
     const int steps = c / TK;
-    // (wide groups: neighbouring batch tiles begin a slab apart: rows of x that are a multiple of 4 KB long put the same slab
-    // of all of them in the same channels of the L2)
-    const int rot = FL ? nt_id % steps : 0;
-    auto k_of = [&](int s) {
-        s += rot;
-        return (s >= steps ? s - steps : s) * TK;
-    };
     // slab s: request weights PDW and input PDX slabs ahead into the slots slab s came from (it
     // went to LDS an iteration ago), multiply slab s, move slab s + 1 from its registers to
     // the other LDS buffer.  The weights come from L2 and get the shorter lead; they are
     // requested first, so that waiting for them leaves the younger input loads in flight.
     // Wide groups have one workgroup on a CU, and nobody multiplies while its waves issue their loads: these are spread over
-    // the products, whose operands are read two blocks ahead.  us before / so, and with the batch tiles in step: (6,192,192,64)
-    // on 25088 rows 3841 / 3717, (8,128,128,64) on 12544 rows 1210 / 1151, (1,256,64,64) on 25088 457 / 418, (1,192,192,128) on
-    // 12544 653 / 644, (1,512,128,16) on 25088 257 / 247; with the LDS stores among the products as well 3686 / 1130 / 410, but
-    // 683 and 263.  Groups of 8, two workgroups a CU: registers that spill.
+    // the products, whose operands are read two blocks ahead.  us before / so: (6,192,192,64) on 25088 rows 3845 / 3738,
+    // (8,128,128,64) on 12544 rows 1196 / 1168, (1,256,64,64) on 25088 457 / 448, (1,192,192,128) on 12544 652 / 642, (1,512,128,16)
+    // on 25088 256 / 251.  Groups of 8, two workgroups a CU: registers that spill.  Batch tiles that begin a slab apart take another
+    // 0 to 6 percent off (3715, 1143, 419), but a row's sum would then have the order of its tile: equal rows keep equal bits.
     constexpr int PERIOD = PDX * PDW / (PDX % PDW == 0 ? PDW : PDW % PDX == 0 ? PDX : 1);
     static_assert(PERIOD % PDX == 0 && PERIOD % PDW == 0, "slots repeat after PERIOD slabs");
     auto slab = [&](int u, int s) {
         const uint32_t wmk = live_mask(s + PDW < steps), xmk = live_mask(s + PDX < steps);
-        const int buf = s & 1, wk = k_of(min(s + PDW, steps - 1)), xk = k_of(min(s + PDX, steps - 1));
-        auto request = [&](int i) { gload(i, u % PDW, wk, wmk, u % PDX, xk, xmk); };
+        const int buf = s & 1;
+        auto request = [&](int i) { gload(i, u % PDW, (s + PDW) * TK, wmk, u % PDX, (s + PDX) * TK, xmk); };
         constexpr int AHEAD = FL ? 2 : 0;
 #pragma unroll
         for (int i = 0; i < LOADS && !FL; ++i) request(i);
@@ -464,7 +457,7 @@ __global__ __launch_bounds__(64 * WM * WN * NG, (WM * WN * NG >= 8 ? 1 : 2)) voi
         const uint32_t mk = live_mask(u < steps);
 #pragma unroll
         for (int i = 0; i < LOADS; ++i)
-            if (i < W_PER_T ? u < PDW : u < PDX) gload(i, u % PDW, k_of(min(u, steps - 1)), mk, u % PDX, k_of(min(u, steps - 1)), mk);
+            if (i < W_PER_T ? u < PDW : u < PDX) gload(i, u % PDW, u * TK, mk, u % PDX, u * TK, mk);
     }
     lstore(0, 0, 0);
     __syncthreads();

@@ -51,3 +51,23 @@ def test_unaligned_tensors_between_aligned_ones(dt, bs_last):
                 # sums of c products of type dt in fp32, one rounding: 2e-7 sqrt(c) in fp32, 2.9e-4 in fp16
                 assert ((y.double() - want).norm() / want.norm()).item() <= (5e-6 if dt == torch.float32 else 4e-4)
                 assert torch.equal(y, bits.setdefault((i, j), y)), (i, j)
+
+
+@pytest.mark.parametrize("dts", [(torch.float32, torch.float32), (torch.float16, torch.float16), (torch.float8_e4m3fn, torch.float8_e4m3fn),
+                                 (torch.float16, torch.float8_e4m3fn)])
+@pytest.mark.parametrize("bs_last", [False, True])
+def test_equal_rows_have_equal_bits(dts, bs_last):
+    """A row's result does not depend on where in the batch it lies: every tile sums in the same order."""
+    from ksmm_amd import Kernel
+
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    # wide groups of blocks first, then a shape per family
+    for a, b, c, d in [(1, 192, 192, 64), (2, 128, 128, 32), (1, 256, 64, 16), (1, 48, 48, 16), (3, 64, 64, 1), (1, 768, 192, 2), (1, 128, 128, 3),
+                       (2, 96, 96, 4), (1, 64, 256, 6), (4, 192, 192, 1), (1, 100, 36, 1), (3, 4, 4, 16), (16, 16, 16, 4), (1, 451, 64, 1)]:
+        w = (torch.randn(a * d * c, b, generator=gen, device="cuda") / c ** 0.5).to(dts[1])
+        row = torch.randn(a * c * d, generator=gen, device="cuda").to(dts[0])
+        for n in (33, 197, 1000, 2050, 8192):
+            x = torch.empty((a * c * d, n) if bs_last else (n, a * c * d), device="cuda", dtype=dts[0])
+            x.copy_(row[:, None] if bs_last else row)
+            y = Kernel.forward(x, w, bs_last, a, b, c, d)
+            assert bool((y == (y[:, :1] if bs_last else y[:1])).all()), (a, b, c, d, n)

@@ -292,6 +292,7 @@ struct Pick {
     bool direct;
     bool transposed, padded;  // the problem has that route
     float us;     // predicted time, < 0: no model of it
+    bool own;     // it has the transposed route, and a whole-d tile that is priced below it: no copies, no workspace
 };
 
 // Full batches that no row of the table names.  The heuristics were made on the patterns of the table; the prices, fitted on
@@ -314,6 +315,7 @@ bool on_vectors(const Problem &p) { return (((uintptr_t)p.x | (uintptr_t)p.w | (
 // vector take the cheapest of the kernels that do not need it.  A function of the sizes, types and that
 // alignment alone: each thread remembers its last answers (pricing every instance takes tens
 // of microseconds, a launch five).
+float route_us(const Problem &p);
 Pick pick_of(const Problem &given, bool table)
 {
     const bool aligned = on_vectors(given);
@@ -337,7 +339,7 @@ Pick pick_of(const Problem &given, bool table)
         if (e.batch == p.batch && memcmp(e.key, key, sizeof(key)) == 0) return e.pick;
     ksmm_tile t;
     memset(&t, 0, sizeof(t));
-    Pick k{{KSMM_ALGO_AUTO, -1, -1.f}, true, find_transposed(p), find_padded(p), -1.f};
+    Pick k{{KSMM_ALGO_AUTO, -1, -1.f}, true, find_transposed(p), find_padded(p), -1.f, false};
     // in place of the full-batch choice, priced at k.us.  A kernel of its own that has no price is not known to
     // be slower: it stays.  The one-thread-per-output kernel has to be ahead by the error of its fit (0.3):
     // on 14900 measured problems that it takes, chosen / fastest is 1.059 in the geometric mean so, 1.062 without
@@ -358,6 +360,13 @@ Pick pick_of(const Problem &given, bool table)
         if (p.batch < TUNED_MIN_BATCH || !k.direct) replace(cheapest_instance(p, false), 1.f);
         else if (!(table && tuned_for(p)) && p.batch <= HEURISTIC_LAST && p.w_dtype == p.x_dtype) replace(cheapest_instance(p, false), p.x_dtype == KSMM_F32 ? HEURISTIC_MARGIN_F : HEURISTIC_MARGIN_H);
     }
+    if (k.transposed && !aligned) {
+        k.own = pick_of(p, table).own;
+    } else if (k.transposed && k.c.algo == KSMM_ALGO_TILE && (k.c.variant >> 24) == 3 && bf_inst_whole(k.c.variant & 0xff)) {
+        const float route = route_us(p);
+        k.own = route >= 0.f && k.us <= route;
+        k.direct |= k.own;
+    }
     Entry &e = memo[set][oldest[set]++ % WAYS];
     e.batch = p.batch;
     memcpy(e.key, key, sizeof(key));
@@ -365,7 +374,11 @@ Pick pick_of(const Problem &given, bool table)
     return k;
 }
 
-bool wants_transposed(const Problem &p) { return pick_of(p, true).transposed; }
+bool wants_transposed(const Problem &p)
+{
+    const Pick k = pick_of(p, true);
+    return k.transposed && !k.own;
+}
 bool wants_padded(const Problem &p) { return pick_of(p, true).padded; }
 
 int dispatch(const Problem &p, int algo, int variant, bool launch, ksmm_tile *tile)
@@ -399,16 +412,22 @@ Problem twin_of(const Problem &p)
     return q;
 }
 
-// Whether the transposed or padded-rows route of a problem that has one beats the kernel that takes
-// it as it is: small problems are done before the first copy would be.
-bool route_pays(const Problem &p)
+// Predicted time of the transposed or padded-rows route of a problem that has one (< 0: no model of it)
+float route_us(const Problem &p)
 {
-    const Pick k = pick_of(p, true), q = pick_of(twin_of(p), true);
-    if (k.us < 0.f || q.us < 0.f) return true;
+    const Pick q = pick_of(twin_of(p), true);
+    if (q.us < 0.f) return -1.f;
     const int64_t bp = padded_batch(p.batch);
     const float copies = copy_us((int64_t)p.a * p.c * p.d, p.batch, bp, (int)dtype_size(p.x_dtype), !p.bs_last) +
                          copy_us((int64_t)p.a * p.b * p.d, p.batch, bp, (int)dtype_size(p.y_dtype), !p.bs_last);
-    return copies + q.us < k.us;
+    return copies + q.us;
+}
+
+// Whether it beats the kernel that takes the problem as it is: small problems are done before the first copy would be.
+bool route_pays(const Problem &p)
+{
+    const float now = pick_of(p, true).us, route = route_us(p);
+    return now < 0.f || route < 0.f || route < now;
 }
 
 int64_t align256(int64_t v) { return (v + 255) / 256 * 256; }
@@ -519,7 +538,11 @@ int check_chain(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, in
     return KSMM_OK;
 }
 
-// batch-size-first chain with at least one factor that needs the transposed route
+bool chain_route_pays(const ksmm_factor_desc *f, int n, const void *x, void *y, int64_t batch, int x_dtype, int y_dtype, int bs_last,
+                      bool fuse);
+
+// batch-size-first chain with at least one factor that needs the transposed route, or where one pair of copies for all of its
+// factors is priced below their own tiles
 bool chain_wants_transposed(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype,
                             int bs_last)
 {
@@ -528,12 +551,18 @@ bool chain_wants_transposed(const ksmm_factor_desc *f, int n, int64_t batch, int
     // transposes instead of one pass per factor
     if (chain16_run(f, n, nullptr, nullptr, padded_batch(batch), x_dtype, y_dtype, 1, false, nullptr, nullptr) == KSMM_OK)
         return true;
+    // (a function of the sizes and types: what is asked for is what a call needs, wherever its tensors lie)
+    ksmm_factor_desc sizes[KSMM_MAX_FACTORS];
+    bool own = false;
     for (int i = 0; i < n; ++i) {
-        Problem p{nullptr, nullptr, nullptr, batch, f[i].a, f[i].b, f[i].c, f[i].d, i == 0 ? x_dtype : y_dtype,
-                  f[i].w_dtype, y_dtype, 0, 1.f, nullptr};
-        if (wants_transposed(p)) return true;
+        sizes[i] = f[i];
+        sizes[i].w = nullptr;
+        const Pick k = pick_of(Problem{nullptr, nullptr, nullptr, batch, f[i].a, f[i].b, f[i].c, f[i].d, i == 0 ? x_dtype : y_dtype,
+                                       f[i].w_dtype, y_dtype, 0, 1.f, nullptr}, true);
+        if (k.transposed && !k.own) return true;
+        own |= k.own;
     }
-    return false;
+    return own && n > 1 && chain_route_pays(sizes, n, nullptr, nullptr, batch, x_dtype, y_dtype, 0, false);
 }
 
 // batch-size-last chain whose batch is not a multiple of the vector, with at least one factor

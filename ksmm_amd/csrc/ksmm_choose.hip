@@ -153,7 +153,7 @@ float predicted_us(const Problem &p, const ksmm_tile &t)
     return r ? price(*r, p, t) : -1.f;
 }
 
-Choice cheapest_instance(const Problem &p, bool split_only)
+Choice cheapest_instance(const Problem &p, bool any_alignment)
 {
     Choice best{KSMM_ALGO_AUTO, -1, -1.f};
     const int combo = combo_of(p.x_dtype, p.w_dtype, p.y_dtype);
@@ -170,12 +170,14 @@ Choice cheapest_instance(const Problem &p, bool split_only)
         if (best.us < 0.f || us < best.us) best = Choice{t.algo, t.variant, us};
     };
     const CostIndex &ix = cost_index();
-    if (!split_only) {
+    if (!any_alignment) {
         offer(KSMM_ALGO_WAVE, -1);
         for (int sub = 0; sub < FAM_SPLIT; ++sub)
             for (int i = 0; i < ix.count[sub]; ++i)
                 if (ix.tile[sub][combo][p.bs_last][i]) offer(KSMM_ALGO_TILE, (sub << 24) | (sub == 0 && ragged ? 1 << 8 : 0) | i);
     }
+    for (int i = 0; any_alignment && i < ix.count[3]; ++i)
+        if (bf_inst_whole(i) && ix.tile[3][combo][p.bs_last][i]) offer(KSMM_ALGO_TILE, (3 << 24) | i);
     for (int i = 0; i < ix.count[FAM_SPLIT]; ++i) {
         if (!ix.tile[FAM_SPLIT][combo][p.bs_last][i]) continue;
         for (int waves = 1; waves <= 16; waves *= 2) offer(KSMM_ALGO_TILE, (FAM_SPLIT << 24) | (waves << 8) | i);

@@ -178,6 +178,7 @@ int ws_inst_count();
 uint32_t ws_inst_id(int i);
 int bf_inst_count();
 uint32_t bf_inst_id(int i);
+bool bf_inst_whole(int i);  // all of d at once, at any alignment
 int gemm_inst_count();
 uint32_t gemm_inst_id(int i);
 int split_inst_count();

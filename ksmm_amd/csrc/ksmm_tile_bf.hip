@@ -803,7 +803,8 @@ __global__ __launch_bounds__(64 * WM * WN * NG, (WM * WN * NG >= 8 ? 1 : 2)) voi
 // tiles; the weights are k-outer rows as there.  Both operands go through registers a slab ahead of the products,
 // double-buffered, one barrier a slab; two to three workgroups of four waves on a CU fill each other's waits.  Roles as in
 // the batch-size-first GEMM tiles (A = W, lanes = batch rows): a lane holds 4 outputs x DD blocks of a row, one run of y, and the
-// waves turn their 32 x 32 blocks around in LDS to store whole lines.  Outputs behind b are dropped.
+// waves turn their 32 x 32 blocks around in LDS to store whole lines.  Outputs behind b are dropped.  Vectors of all three tensors are
+// taken at the alignment of their elements: such problems ask for no workspace, which tensors off 16 bytes would need elsewhere.
 //
 // What bounds it: LDS reads (24 to 32 bytes a lane and product) on blocks of 192 and more, before that the latency of a slab.
 // Such d ran between two transposes, on the split-K or on the row kernel; us of those / of this one: fp16 (1,256,256,3) at 25088
@@ -883,9 +884,9 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void ks_whole_bf_kernel(const TX
 #pragma unroll
         for (int i = 0; i < C::UNITS; ++i)
 #pragma unroll
-            for (int j = 0; j < DD; ++j) xreg[i][j] = ((const xvec_t *)(xp[i] + (size_t)s * (TK * DD)))[j];
+            for (int j = 0; j < DD; ++j) __builtin_memcpy(&xreg[i][j], (const char *)(xp[i] + (size_t)s * (TK * DD)) + j * sizeof(xvec_t), sizeof(xvec_t));
 #pragma unroll
-        for (int i = 0; i < C::W_PER_T; ++i) wreg[i].load(wp[i] + (size_t)s * TK * b);
+        for (int i = 0; i < C::W_PER_T; ++i) __builtin_memcpy(&wreg[i].v, wp[i] + (size_t)s * TK * b, 16);
     };
     auto lstore = [&](unsigned char *to) {
 #pragma unroll
@@ -1020,9 +1021,9 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void ks_whole_bf_kernel(const TX
 #pragma unroll
             for (int q = 0; q < 32 * RV / 64; ++q) {
                 const int v = lane + 64 * q, row = v / RV, at = v % RV;
+                const uint4_t o = *(const uint4_t *)(piece + row * C::OP + at * 16);
                 if (nb + row < batch && at * 16 < (b - mb) * (DD * C::ES))
-                    *(uint4_t *)((unsigned char *)(y + (size_t)(nb + row) * out_size + ((size_t)a_i * b + mb) * DD) + at * 16) =
-                        *(const uint4_t *)(piece + row * C::OP + at * 16);
+                    __builtin_memcpy((unsigned char *)(y + (size_t)(nb + row) * out_size + ((size_t)a_i * b + mb) * DD) + at * 16, &o, 16);
             }
             __builtin_amdgcn_wave_barrier();
         }
@@ -1183,6 +1184,7 @@ bool bf_fits(const BfInst &t, const Problem &p, int combo)
 }  // namespace
 
 int bf_inst_count() { return N_BF_INSTS; }
+bool bf_inst_whole(int i) { return i >= 0 && i < N_BF_INSTS && bf_insts[i].pd == WHOLE; }
 
 uint32_t bf_inst_id(int i)
 {

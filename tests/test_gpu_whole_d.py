@@ -68,3 +68,47 @@ def test_whole_d_epilogue(dt):
                 z = x.double() * (float(scale) if scale is not None else 1.0) @ dense.T + layer.bias.double()
             want = z * 0.5 * (1 + torch.erf(z / math.sqrt(2)))
             assert ((y.double() - want).norm() / want.norm()).item() <= {torch.float32: 1e-5, torch.float16: 2e-3, FP8: 5e-3}[dt]
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16, FP8])
+def test_whole_d_without_workspace_at_any_alignment(dt):
+    """What asks for no workspace runs without one, on tensors that start an element behind 16 bytes as well, and writes nothing
+    but its result; a chain on its intermediates alone."""
+    from ksmm_amd import Kernel, KSLinear, _lib
+    from ksmm_amd.kernel import dtype_code
+
+    lib = _lib.load()
+    yt = torch.float32 if dt == torch.float32 else torch.float16
+    xd, yd, tol = dtype_code(dt), dtype_code(yt), 1e-5 if dt == torch.float32 else 2e-3
+    for (a, b, c, d), n in [((1, 256, 256, 3), 2050), ((3, 80, 96, 3), 2051), ((2, 128, 32, 6), 2111), ((1, 192, 48, 2), 6304), ((2, 64, 256, 4), 4099)]:
+        def tensor(size, off, dtype):
+            return torch.empty(size + 64, device="cuda", dtype=dtype)[off:off + size]
+
+        full_x = torch.randn(n * a * c * d, device="cuda").to(dt)
+        full_w = ((torch.rand(a * d * c * b, device="cuda") * 2 - 1) / math.sqrt(c)).to(dt)
+        xk, wk = full_x.float().double().view(n, a, c, d), full_w.float().double().view(a, d, c, b)
+        want = torch.stack([torch.stack([xk[:, i, :, j].contiguous() @ wk[i, j] for j in range(d)], -1) for i in range(a)], 1).reshape(n, -1)
+        need = lib.ksmm_factor_workspace(n, a, b, c, d, xd, xd, yd, 0)
+        for offs in ((0, 0, 0), (1, 0, 0), (0, 1, 0), (0, 0, 1), (1, 3, 1)):
+            x, w = tensor(full_x.numel(), offs[0], dt).copy_(full_x), tensor(full_w.numel(), offs[1], dt).copy_(full_w)
+            flat = torch.full((want.numel() + 64,), 7.0, device="cuda", dtype=yt)
+            y = flat[offs[2]:offs[2] + want.numel()]
+            stream = torch.cuda.current_stream().cuda_stream
+            rc = lib.ksmm_factor_forward_ws(x.data_ptr(), w.data_ptr(), y.data_ptr(), n, a, b, c, d, xd, xd, yd, 0, 1.0, None, 0, stream)
+            assert rc == (0 if need == 0 else -9), (a, b, c, d, rc)
+            if rc:
+                continue
+            err = ((y.view(n, -1).double() - want).norm() / want.norm()).item()
+            assert err <= tol, ((a, b, c, d), offs, err)
+            assert bool((flat[:offs[2]] == 7.0).all()) and bool((flat[offs[2] + want.numel():] == 7.0).all())
+    if dt == FP8:
+        return
+    patterns, n = [(12, 64, 256, 1), (1, 256, 256, 3)], 2050
+    layer = KSLinear(patterns, bias=False, algo="kernel", dtype=dt, device="cuda")
+    flat = torch.randn(n * layer.in_size + 1, device="cuda").to(dt)
+    for off in (0, 1):
+        x = flat[off:off + n * layer.in_size].view(n, layer.in_size)
+        with torch.no_grad():
+            y = layer(x)
+            want = x.double() @ layer.get_dense_product(torch.float64).t()
+        assert ((y.double() - want).norm() / want.norm()).item() <= tol

@@ -245,6 +245,35 @@ def test_workspace_queries_need_no_gpu():
     assert lib.ksmm_chain_workspace_layout(descs, 2, 512, F16, F16, 0) == 3 * (3072 * 512 * 2)
 
 
+def test_tiles_of_a_whole_stride_ask_for_no_workspace(lib):
+    """Batch-size-first blocks of d = 3 and 6 (fp32 and e4m3: 2, e4m3: 4 as well) that run on a tile of their own ask for nothing,
+    chains of them for their intermediates only; what takes the transposed route asks for its copies."""
+    from ksmm_amd import _lib
+    from ksmm_amd.kernel import query_tile
+
+    f32, f16, f8 = torch.float32, torch.float16, torch.float8_e4m3fn
+    code = {f32: _lib.KSMM_F32, f16: _lib.KSMM_F16, f8: _lib.KSMM_FP8_E4M3}
+    for dt, pattern in [(f32, (1, 256, 256, 3)), (f16, (1, 256, 256, 3)), (f8, (1, 192, 192, 3)), (f32, (2, 128, 32, 6)), (f16, (4, 96, 384, 3)),
+                        (f32, (1, 192, 48, 2)), (f8, (2, 64, 256, 4))]:
+        x, y = code[dt], code[f32 if dt == f32 else f16]
+        for n in (2050, 6304, 8191, 8192, 25088, 25090):
+            t = query_tile(n, pattern, dt, None, False)
+            whole = t["algo"] == _lib.ALGO_TILE and t["variant"] >> 24 == 3 and t["tile_d"] == pattern[3]
+            assert whole, (dt, pattern, n, t)
+            assert lib.ksmm_factor_workspace(n, *pattern, x, x, y, 0) == 0, (dt, pattern, n)
+    descs = (_lib.KsmmFactorDesc * 2)()
+    for n in (6304, 25088):
+        for w in (0, 4096, 4098):  # (the weights' place does not matter)
+            for i, p in enumerate([(12, 64, 256, 1), (1, 256, 256, 3)]):
+                descs[i].w, descs[i].w_dtype, descs[i].scale = w, _lib.KSMM_F16, 1.0
+                descs[i].a, descs[i].b, descs[i].c, descs[i].d = p
+            plain = lib.ksmm_chain_workspace(descs, 2, n, _lib.KSMM_F16)
+            assert lib.ksmm_chain_workspace_layout(descs, 2, n, _lib.KSMM_F16, _lib.KSMM_F16, 0) == plain
+    assert lib.ksmm_factor_workspace(25088, 1, 192, 192, 12, _lib.KSMM_F16, _lib.KSMM_F16, _lib.KSMM_F16, 0) > 0
+    # (a tile takes this one too, but the copies and the kernel between them are priced below it)
+    assert lib.ksmm_factor_workspace(25088, 12, 128, 128, 6, _lib.KSMM_F32, _lib.KSMM_F32, _lib.KSMM_F32, 0) > 0
+
+
 def test_layer_backward_asks_for_the_gradients_it_writes(lib):
     """Gradients between factors: one buffer for two factors, for more two that are as wide as what lands in them."""
     from ksmm_amd import _lib

@@ -301,17 +301,24 @@ struct Pick {
 // heuristics' price an instance has to be priced is from 2400 drawn problems of 8192 .. 25088 columns, us of the priced one / of
 // the heuristics' in the geometric mean over those that change: fp32 at 0.9 0.77 feature-major and 0.67 rows (117 problems, 2 of them
 // more than 3 percent slower, by 1.06), the others at 0.85 0.57 .. 0.84 (195 problems, 11 slower, by 1.15 at most); at 0.9
-// 23 of 267 are slower, at 0.97 56 of 469.  (e4m3 weights on fp16 inputs keep the heuristics' choice: what they lose to fp16 weights
-// is what decode_pays goes by.)
-constexpr float HEURISTIC_MARGIN_F = 0.9f, HEURISTIC_MARGIN_H = 0.85f;
-constexpr int64_t HEURISTIC_LAST = 25088;  // the largest batch that this was measured at
+// 23 of 267 are slower, at 0.97 56 of 469.  Beyond, the error of the prices that are extrapolated furthest grows; from 900 problems
+// of 25089 .. 110000 columns whose choice would change: fp32 at 0.9 0.69 rows and 0.77 feature-major (285 problems, 5 slower), e4m3
+// rows at 0.85 0.64 (209, 3 slower); fp16 rows at 0.85 0.95 (84, 23 slower, up to 1.54) and at 0.75 0.90 (24, 1 slower by 1.07);
+// fp16 and e4m3 feature-major at 0.85 0.85 and 0.75 (321, 115 slower, up to 1.33), at 0.7 0.64 and 0.50 (135, 8 slower, up to 1.13).
+// (e4m3 weights on fp16 inputs keep the heuristics' choice: what they lose to fp16 weights is what decode_pays goes by.)
+float heuristic_margin(const Problem &p)
+{
+    if (p.x_dtype == KSMM_F32) return 0.9f;
+    if (p.batch <= 25088 || (p.x_dtype == KSMM_FP8_E4M3 && !p.bs_last)) return 0.85f;
+    return p.bs_last ? 0.7f : 0.75f;
+}
 
 // Whether the kernels that move aligned 16-byte vectors take a problem's tensors (null: they will be).
 bool on_vectors(const Problem &p) { return (((uintptr_t)p.x | (uintptr_t)p.w | (uintptr_t)p.y) & 15) == 0; }
 
 // Below TUNED_MIN_BATCH, and where the full-batch choice is the one-thread-per-output kernel, the
 // cheapest instance by the model of ksmm_choose.hip; else the full-batch choice, a row of the table, or the heuristics' one
-// unless an instance is priced well below it (HEURISTIC_MARGIN).  Tensors off the
+// unless an instance is priced well below it (heuristic_margin).  Tensors off the
 // vector take the cheapest of the kernels that do not need it.  A function of the sizes, types and that
 // alignment alone: each thread remembers its last answers (pricing every instance takes tens
 // of microseconds, a launch five).
@@ -358,7 +365,7 @@ Pick pick_of(const Problem &given, bool table)
         k.direct = t.algo != KSMM_ALGO_GENERIC || t.variant == 1;
         k.us = predicted_us(p, t);
         if (p.batch < TUNED_MIN_BATCH || !k.direct) replace(cheapest_instance(p, false), 1.f);
-        else if (!(table && tuned_for(p)) && p.batch <= HEURISTIC_LAST && p.w_dtype == p.x_dtype) replace(cheapest_instance(p, false), p.x_dtype == KSMM_F32 ? HEURISTIC_MARGIN_F : HEURISTIC_MARGIN_H);
+        else if (!(table && tuned_for(p)) && p.w_dtype == p.x_dtype) replace(cheapest_instance(p, false), heuristic_margin(p));
     }
     if (k.transposed && !aligned) {
         k.own = pick_of(p, table).own;

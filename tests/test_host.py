@@ -274,6 +274,17 @@ def test_tiles_of_a_whole_stride_ask_for_no_workspace(lib):
     assert lib.ksmm_factor_workspace(25088, 12, 128, 128, 6, _lib.KSMM_F32, _lib.KSMM_F32, _lib.KSMM_F32, 0) > 0
 
 
+def test_choice_does_not_end_with_the_measured_batches():
+    """One row more than the largest batch that the choice was first measured at takes the same kernel."""
+    from ksmm_amd.kernel import query_tile
+
+    f32, f16, f8 = torch.float32, torch.float16, torch.float8_e4m3fn
+    for dt, pattern, last in [(f32, (12, 64, 256, 1), False), (f32, (12, 256, 64, 1), True), (f32, (1, 256, 256, 3), False), (f16, (1, 256, 256, 3), False),
+                              (f8, (6, 256, 64, 1), False), (f8, (2, 64, 256, 2), False), (f8, (1, 16, 64, 16), True), (f32, (1, 768, 192, 2), False)]:
+        at, behind = (query_tile(n, pattern, dt, None, last) for n in (25088, 25088 + 16))
+        assert (behind["algo"], behind["variant"]) == (at["algo"], at["variant"]), (dt, pattern, last, at, behind)
+
+
 def test_layer_backward_asks_for_the_gradients_it_writes(lib):
     """Gradients between factors: one buffer for two factors, for more two that are as wide as what lands in them."""
     from ksmm_amd import _lib

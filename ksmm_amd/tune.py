@@ -34,6 +34,7 @@ import torch
 
 DT = {"fp32": torch.float32, "fp16": torch.float16, "fp8": torch.float8_e4m3fn}
 COMBO = {"fp32": 0, "fp16": 1, "fp8": 2}
+TABLE_FROM = 8192  # the smallest batch that the library looks the table up for
 
 
 def _time_graph(fn, n_sets, steps):
@@ -246,13 +247,23 @@ def _entry_id(e):
     return None
 
 
+def _spares_copies(e, batch):
+    """Whether an entry's kernel is one of its own (not the generic family's, family 1) where the heuristics have none: such
+    problems ask for the copies of the transposed route."""
+    from .kernel import query_tile
+
+    return e["algo"] != 1 and any(query_tile(n, tuple(e["pattern"]), DT[e["prec"]], None, e["bs_last"], variant=-3)["algo"] == 1
+                                  for n in (TABLE_FROM, batch))
+
+
 def emit(entries, path, batch):
-    """Write the C table: one row per entry where the tuned choice beats the heuristic by > 3 %."""
+    """Write the C table: one row per entry where the tuned choice beats the heuristic by > 3 %, or is as fast and spares the
+    workspace that the heuristic's choice asks for on the smallest batch of the table's range or at ``batch``."""
     rows = []
     for e in entries:
         if e.get("best_us") is None or e.get("auto_us") is None or e["algo"] == 0:
             continue
-        if not e["best_us"] < 0.97 * e["auto_us"]:
+        if not e["best_us"] < 0.97 * e["auto_us"] and not (e["best_us"] <= e["auto_us"] and _spares_copies(e, batch)):
             continue
         a, b, c, d = e["pattern"]
         named = _entry_id(e)
@@ -268,7 +279,8 @@ def emit(entries, path, batch):
     with open(path, "w") as f:
         f.write("// Generated by `python -m ksmm_amd.tune` on MI355X (gfx950) at batch %d: fastest measured\n" % batch)
         f.write("// (family, instance id, parameter) per (a, b, c, d, element-type combination, layout), kept only\n")
-        f.write("// where it beats the heuristic choice by more than 3 %.  Sorted by key for binary search.\n")
+        f.write("// where it beats the heuristic choice by more than 3 %, or spares a workspace that this one asks for.  Sorted by key\n")
+        f.write("// for binary search.\n")
         f.write("// {a, b, c, d, combo, bs_last, algo, instance id, parameter},  // tuned us (heuristic us)\n")
         for r in rows:
             f.write("{%d, %d, %d, %d, %d, %d, %d, %du, %d},  // %.1f (%.1f)\n" % r)

@@ -515,6 +515,31 @@ def test_tuner_emit_keeps_one_sorted_row_per_key_above_the_threshold(tmp_path):
     assert variant_from_id(2, iid, par, 1, True) == 1
 
 
+def test_tuner_emit_keeps_rows_that_spare_a_workspace(tmp_path):
+    """Within 3 % a row stays where the heuristics have no kernel of the problem's own, which then asks for the copies of the
+    transposed route; every row of the table within 3 % is of that kind."""
+    from ksmm_amd import _lib
+    from ksmm_amd.kernel import query_tile
+    from ksmm_amd.tune import TABLE_FROM, emit
+
+    f32 = torch.float32
+    e = {"pattern": [1, 192, 768, 2], "prec": "fp32", "bs_last": False, "auto_us": 173.0, "best_us": 170.0, "algo": 3, "variant": (3 << 24) | 16}
+    path = tmp_path / "t.inc"
+    assert emit([e], str(path), 25088) == 1
+    assert emit([dict(e, best_us=173.1)], str(path), 25088) == 0                                                     # slower
+    assert emit([dict(e, pattern=[1, 48, 48, 16], bs_last=True, algo=2, variant=0x700)], str(path), 25088) == 0       # nothing to spare
+    table = open(os.path.join(_lib.HERE, "csrc", "ksmm_tuned.inc")).read()
+    types = {0: (f32, f32), 1: (torch.float16,) * 2, 2: (torch.float8_e4m3fn,) * 2, 3: (torch.float16, torch.float8_e4m3fn)}
+    close = 0
+    for a, b, c, d, combo, last, best, was in re.findall(r"^\{(\d+), (\d+), (\d+), (\d+), (\d), (\d), \d+, \d+u, -?\d+\},\s*// ([\d.]+) \(([\d.]+)\)", table, re.M):
+        if float(best) - 0.05 < 0.97 * (float(was) + 0.05):  # (printed to a tenth)
+            continue
+        algos = [query_tile(n, (int(a), int(b), int(c), int(d)), *types[int(combo)], last == "1", variant=-3)["algo"] for n in (TABLE_FROM, 25088)]
+        assert _lib.ALGO_GENERIC in algos, (a, b, c, d, combo, last, best, was)
+        close += 1
+    assert close
+
+
 def test_tuner_best_files_have_the_reference_columns(tmp_path):
     """ksmm_amd.tune.emit_best: `batch a b c d <kernel> ms std mse` per pattern, one file per
     element type and layout, named like the reference's *.best files."""

@@ -745,7 +745,7 @@ bool pair_priced_lower(const ksmm_factor_desc *f, int n, int64_t batch, int x_dt
 }
 
 // A function of the sizes and types alone, asked up to three times a call: each thread remembers its last answers (2 us
-// otherwise, of a call of 10).
+// otherwise, of a call of 10), in sets of four as pick_of does: two layers of a network that share an entry would ask anew each call.
 bool pair_pays(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype, int bs_last, PairShape *shape)
 {
     if (n != 2 || f[0].d != 1 || (f[0].b == 16 && f[0].c == 16)) return false;  // (radix-16 chains have kernels of their own)
@@ -755,19 +755,25 @@ bool pair_pays(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int
         PairShape shape;
         bool pays;
     };
-    constexpr unsigned ENTRIES = 128;
-    static thread_local Entry memo[ENTRIES];
+    constexpr unsigned SETS = 64, WAYS = 4;
+    static thread_local Entry memo[SETS][WAYS];
+    static thread_local uint8_t oldest[SETS];
     const int key[13] = {f[0].a, f[0].b, f[0].c, f[0].d, f[0].w_dtype, f[1].a, f[1].b, f[1].c, f[1].d, f[1].w_dtype, x_dtype, y_dtype, bs_last != 0};
     uint64_t h = (uint64_t)batch;
     for (int v : key) h = (h ^ (uint64_t)v) * 0x9E3779B97F4A7C15ull;
-    Entry &e = memo[(h >> 40) % ENTRIES];
-    if (e.batch != batch || memcmp(e.key, key, sizeof(key)) != 0) {
+    const unsigned set = (h >> 40) % SETS;
+    const Entry *hit = nullptr;
+    for (const Entry &e : memo[set])
+        if (e.batch == batch && memcmp(e.key, key, sizeof(key)) == 0) hit = &e;
+    if (!hit) {
+        Entry &e = memo[set][oldest[set]++ % WAYS];
         e.batch = batch;
         memcpy(e.key, key, sizeof(key));
         e.pays = pair_priced_lower(f, n, batch, x_dtype, y_dtype, bs_last, &e.shape);
+        hit = &e;
     }
-    *shape = e.shape;
-    return e.pays;
+    *shape = hit->shape;
+    return hit->pays;
 }
 
 // Workspace of a chain with decoded weights: that of either chain, then (from *at) the fp16 weights

@@ -274,6 +274,43 @@ def test_tiles_of_a_whole_stride_ask_for_no_workspace(lib):
     assert lib.ksmm_factor_workspace(25088, 12, 128, 128, 6, _lib.KSMM_F32, _lib.KSMM_F32, _lib.KSMM_F32, 0) > 0
 
 
+def test_chains_asked_in_turn_are_remembered(lib):
+    """Whether two factors run in one launch is asked for on every call, and finding out takes microseconds: two chains asked in
+    turn are both remembered, whichever they are."""
+    import time
+
+    from ksmm_amd import _lib
+
+    def question(n):
+        d = (_lib.KsmmFactorDesc * 2)()
+        for i, p in enumerate([(16, 64, 256, 1), (1, 256, 256, 4)]):
+            d[i].w, d[i].w_dtype, d[i].scale = 1 << 16, _lib.KSMM_FP8_E4M3, 1.0
+            d[i].a, d[i].b, d[i].c, d[i].d = p
+        return d, 2, 1 << 36, 2 << 36, n, _lib.KSMM_FP8_E4M3, _lib.KSMM_F16, 0, None, None
+
+    asked = [question(n) for n in range(512, 1024)]  # (two launches take this chain: nothing is launched)
+    assert all(lib.ksmm_chain_forward_fused(*q) == -6 for q in asked)
+
+    def turns(a, b, tries):
+        best = 1.0
+        for _ in range(tries):
+            t = time.perf_counter()
+            for _ in range(8):
+                lib.ksmm_chain_forward_fused(*a)
+                lib.ksmm_chain_forward_fused(*b)
+            best = min(best, time.perf_counter() - t)
+        return best
+
+    # the slowest partners of the first chain, again and more often, next to ones from the middle: what is asked anew takes 1.4 times as long
+    order = sorted(asked[1:], key=lambda q: turns(asked[0], q, 10))
+    for slow, usual in zip(order[-8:], order[250:258]):
+        for _ in range(5):
+            a, b = turns(asked[0], slow, 50), turns(asked[0], usual, 50)
+            if a <= 1.2 * b:
+                break
+        assert a <= 1.2 * b, (a, b)
+
+
 def test_choice_does_not_end_with_the_measured_batches():
     """One row more than the largest batch that the choice was first measured at takes the same kernel."""
     from ksmm_amd.kernel import query_tile

@@ -240,7 +240,8 @@ int ksmm_chain_forward_ep(const ksmm_factor_desc *factors, int n_factors, const 
 
 /* The chain in one launch that needs no workspace, where that is the fastest way through it (radix-16 chains of at most
  * 1024 features, two factors on small batches); KSMM_ERR_BAD_ALGO, and nothing launched, otherwise.  ksmm_chain_forward_ep with `fuse` takes the same
- * launch. */
+ * launch.  Two factors may take it up to a microsecond of GPU time behind two launches, of which it spares the host one, but not on a stream that
+ * is being captured: there the last bits of a result can differ from those of a call of its own. */
 int ksmm_chain_forward_fused(const ksmm_factor_desc *factors, int n_factors, const void *x, void *y, int64_t batch,
                              int x_dtype, int y_dtype, int bs_last, const ksmm_epilogue *epilogue, void *stream);
 

@@ -729,31 +729,49 @@ bool decode_pays(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, i
     return now > 0.f && then > 4.f && then < ((split || copied) && !copied_then ? 1.f : 0.855f) * now;
 }
 
-// Whether two factors run in one launch (ksmm_pair.hip): where that is priced below the other routes.
-bool pair_priced_lower(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype, int bs_last, PairShape *shape)
+// Whether two factors run in one launch (ksmm_pair.hip): where that is priced below the other routes by PAIR_AHEAD.  Of 16270 measured
+// chains (see pair_us) it is so in 5590, which take 0.73 to 0.84 of the time of two launches by type and layout; 2.1 percent
+// of them are more than 3 percent slower.
+// A call that goes to the GPU as it is made costs the host 6.1 us with one launch and 9.7 with two, for which the GPU waits: there, up
+// to a time of HOST_US it may be priced up to a microsecond later.  (6,64,64,1)+(1,768,192,2) fp32 on 32 columns 8.9 us on the GPU
+// for 8.0, but 8.8 a call for 9.6.  In a graph that waits for nobody, the GPU's time alone decides.
+constexpr float PAIR_AHEAD = 0.5f, PAIR_AHEAD_LAST = 1.f, HOST_US = 9.5f;
+struct PairChoice {
+    PairShape shape;
+    bool on_gpu, on_call;  // in a graph, and as a call of its own
+};
+PairChoice pair_choice(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype, int bs_last)
 {
-    const float us = pair_us(f, n, batch, x_dtype, y_dtype, bs_last, shape);
-    if (us < 0.f) return false;
+    PairChoice c{{1, 1}, false, false};
+    float us = pair_us(f, n, batch, x_dtype, y_dtype, bs_last, &c.shape);
+    if (us < 0.f) return c;
     bool copies;
+    float best = chain_best_us(f, n, batch, x_dtype, y_dtype, bs_last, &copies);
     ksmm_factor_desc decoded[2];
-    if (decode_pays(f, n, batch, x_dtype, y_dtype, bs_last, decoded) && us >= chain_best_us(decoded, n, batch, x_dtype, y_dtype, bs_last, &copies) + 4.f)
-        return false;
-    // (ahead by a part of the prices' error; short ones, which wait for the host's launches, may be behind by a part of the launch
-    // that they save: (6,64,64,1)+(1,768,192,2) fp32 on 32 columns 9.6 us on the GPU for 8.6, 8.9 a call for 10.5)
-    const float best = chain_best_us(f, n, batch, x_dtype, y_dtype, bs_last, &copies);
-    return us < 12.f ? us < best + 1.f : 1.05f * us < best;
+    if (decode_pays(f, n, batch, x_dtype, y_dtype, bs_last, decoded)) best = fminf(best, chain_best_us(decoded, n, batch, x_dtype, y_dtype, bs_last, &copies) + 4.f);
+    us += bs_last ? PAIR_AHEAD_LAST : PAIR_AHEAD;
+    c.on_gpu = us < best;
+    c.on_call = us < best + fminf(fmaxf(HOST_US - best, 0.f), 1.f);
+    return c;
 }
 
-// A function of the sizes and types alone, asked up to three times a call: each thread remembers its last answers (2 us
-// otherwise, of a call of 10), in sets of four as pick_of does: two layers of a network that share an entry would ask anew each call.
-bool pair_pays(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype, int bs_last, PairShape *shape)
+// Whether a stream's launches go into a graph.  (The default stream's cannot, and asking about it fails while another one is captured.)
+bool captured(hipStream_t stream)
+{
+    hipStreamCaptureStatus status;
+    return stream && hipStreamIsCapturing(stream, &status) == hipSuccess && status == hipStreamCaptureStatusActive;
+}
+
+// A function of the sizes and types, and where these leave it open of whether the stream is captured; asked up to three times
+// a call: each thread remembers its last answers (2 us otherwise, of a call of 10), in sets of four as pick_of does: two layers of
+// a network that share an entry would ask anew each call.
+bool pair_pays(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype, int bs_last, hipStream_t stream, PairShape *shape)
 {
     if (n != 2 || f[0].d != 1 || (f[0].b == 16 && f[0].c == 16)) return false;  // (radix-16 chains have kernels of their own)
     struct Entry {
         int64_t batch;  // 0: empty
         int key[13];
-        PairShape shape;
-        bool pays;
+        PairChoice choice;
     };
     constexpr unsigned SETS = 64, WAYS = 4;
     static thread_local Entry memo[SETS][WAYS];
@@ -769,11 +787,11 @@ bool pair_pays(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int
         Entry &e = memo[set][oldest[set]++ % WAYS];
         e.batch = batch;
         memcpy(e.key, key, sizeof(key));
-        e.pays = pair_priced_lower(f, n, batch, x_dtype, y_dtype, bs_last, &e.shape);
+        e.choice = pair_choice(f, n, batch, x_dtype, y_dtype, bs_last);
         hit = &e;
     }
-    *shape = hit->shape;
-    return hit->pays;
+    *shape = hit->choice.shape;
+    return hit->choice.on_gpu || (hit->choice.on_call && !captured(stream));
 }
 
 // Workspace of a chain with decoded weights: that of either chain, then (from *at) the fp16 weights
@@ -813,7 +831,7 @@ int chain_forward_impl(const ksmm_factor_desc *factors, int n_factors, const voi
         if (((uintptr_t)workspace & 15) != 0) return KSMM_ERR_WORKSPACE;
     }
     PairShape shape;
-    if (fuse && pair_pays(factors, n_factors, batch, x_dtype, y_dtype, bs_last, &shape)) {
+    if (fuse && pair_pays(factors, n_factors, batch, x_dtype, y_dtype, bs_last, (hipStream_t)stream, &shape)) {
         // (with the workspace that the other routes ask for: a call that lacks it is refused whichever route is the faster)
         const int64_t asked = chain_layout(factors, n_factors, batch, x_dtype, y_dtype, bs_last);
         if (asked <= 0 || (workspace && workspace_bytes >= asked))
@@ -1197,7 +1215,7 @@ int ksmm_chain_forward_fused(const ksmm_factor_desc *factors, int n_factors, con
                  (int64_t)l.a * l.b * l.d * batch * (int64_t)dtype_size(y_dtype)))
         return KSMM_ERR_ALIAS;
     PairShape shape;
-    if (pair_pays(factors, n_factors, batch, x_dtype, y_dtype, bs_last ? 1 : 0, &shape))
+    if (pair_pays(factors, n_factors, batch, x_dtype, y_dtype, bs_last ? 1 : 0, (hipStream_t)stream, &shape))
         return pair_run(factors, n_factors, x, y, batch, x_dtype, y_dtype, bs_last ? 1 : 0, shape, (hipStream_t)stream, epilogue);
     if (!fused_rows_pay(factors, n_factors, x, y, batch, x_dtype, y_dtype, bs_last)) return KSMM_ERR_BAD_ALGO;
     return chain16r_run(factors, n_factors, x, y, batch, x_dtype, y_dtype, bs_last ? 1 : 0, true, (hipStream_t)stream, epilogue);

@@ -16,7 +16,7 @@
 // load instruction, whatever its width: hence four outputs a lane and not two (those: 10.3 for 9.4 us where c0 is 256).
 // Eight waves of up to 256 registers: sixteen of 128 spill, 7.9 against 6.4 us.  us of a replay, two launches / this one:
 // (6,64,64,1)+(1,768,192,2) + GELU, 196 rows: fp16 9.8 / 7.1, fp32 13.5 / 9.4, e4m3 10.1 / 6.5, feature-major 9.0 / 6.8,
-// 10.1 / 9.6, 8.6 / 6.0; (12,64,64,1)+(1,1536,384,2) 14.3 / 11.4, 18.9 / 17.5, 13.8 / 9.5.  A call costs the host 2 us less as well.
+// 10.1 / 9.6, 8.6 / 6.0; on weights and inputs that no cache holds fp16 9.9 / 7.7, fp32 15.6 / 10.8; (12,64,64,1)+(1,1536,384,2) 14.3 / 11.4, 18.9 / 17.5, 13.8 / 9.5.  A call costs the host 2 us less as well.
 #include "ksmm_direct.h"
 #include "ksmm_pair.h"
 
@@ -355,23 +355,24 @@ bool pair_plan(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int
 
 // Predicted time in microseconds (< 0: the kernel does not take the chain, or no shape of it gives a single round of
 // workgroups: with more of them the first factor is repeated too often) and the shape that takes it.
-//     t = f . (1, p, q, l, l g, p nt, g, q nt, nt mg dg)
+//     t = f . (1, p, q, l, l g, p nt, g, q nt, nt mg dg, r nt, z r nt, p g, q g)
 //   p, q  steps that a wave does one after the other in the first and the second factor
 //   l     load instructions of a workgroup / 100: sixteen cycles each, whatever their width
 //   g     workgroups / 256
-// with non-negative coefficients fitted to 445 and 421 measured times a type and layout (feed-forward projections of widths
-// 192 .. 1024 at batches 1 .. 2048): within 0.86 .. 1.14 for nine in ten.  Taken where it is below the price of the two
-// launches, these batches take 0.89 and 0.97 (fp32, batch-size-first and -last), 0.92 and 0.93 (fp16), 0.80 and 0.88
-// (e4m3) of their time, the fastest of both each time 0.88 and 0.96, 0.89 and 0.91, 0.78 and 0.86.
+//   r     tasks that a wave does one after the other in the first factor: each writes its outputs to the planes,
+//   z     element by element (1) unless the planes hold all d_i and these are not three (0)
+// with non-negative coefficients fitted to 49600 replays below 25 us (16280 chains of feed-forward projections of widths 192 .. 1024
+// and of drawn pairs of factors, 1 .. 3000 rows or columns): within 0.87 .. 1.11 for nine in ten.
 float pair_us(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int y_dtype, int bs_last, PairShape *best)
 {
-    static const float coef[3][2][9] = {
-        {{3.211f, 0.000f, 0.000f, 0.354f, 0.189f, 0.313f, 2.013f, 0.798f, 0.000f},
-         {2.939f, 0.000f, 0.000f, 0.268f, 0.149f, 0.381f, 1.625f, 0.803f, 0.063f}},  // fp32
-        {{4.390f, 0.000f, 0.000f, 0.650f, 0.301f, 0.161f, 1.232f, 0.294f, 0.079f},
-         {4.111f, 0.149f, 0.000f, 0.484f, 0.349f, 0.000f, 0.000f, 0.154f, 0.257f}},  // fp16
-        {{4.485f, 0.000f, 0.000f, 0.186f, 0.210f, 0.198f, 1.219f, 0.361f, 0.039f},
-         {4.008f, 0.201f, 0.000f, 0.190f, 0.267f, 0.029f, 0.011f, 0.208f, 0.264f}},  // e4m3
+    constexpr int TERMS = 13;
+    static const float coef[3][2][TERMS] = {
+        {{2.452f, 0.f, 0.f, 0.812f, 0.018f, 0.211f, 2.739f, 0.548f, 0.161f, 0.716f, 0.333f, 0.f, 0.f},
+         {2.309f, 0.f, 0.f, 0.625f, 0.107f, 0.214f, 1.721f, 0.612f, 0.267f, 0.571f, 0.425f, 0.f, 0.f}},  // fp32
+        {{3.461f, 0.f, 0.f, 0.880f, 0.161f, 0.034f, 1.415f, 0.071f, 0.175f, 0.133f, 0.493f, 0.125f, 0.f},
+         {3.592f, 0.012f, 0.063f, 0.583f, 0.112f, 0.f, 0.661f, 0.064f, 0.274f, 0.064f, 0.426f, 0.151f, 0.f}},  // fp16
+        {{3.410f, 0.f, 0.f, 0.376f, 0.235f, 0.071f, 1.250f, 0.142f, 0.143f, 0.198f, 0.579f, 0.021f, 0.f},
+         {3.412f, 0.053f, 0.f, 0.314f, 0.f, 0.011f, 0.404f, 0.102f, 0.277f, 0.196f, 0.500f, 0.213f, 0.101f}},  // e4m3
     };
     float us = -1.f;
     for (int nt = 1; nt <= 2; ++nt)
@@ -380,14 +381,15 @@ float pair_us(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, int 
             PairPlan p;
             if (!pair_plan(f, n, batch, x_dtype, y_dtype, bs_last, s, &p) || p.grid > 256) continue;
             const int kv = p.combo == 0 ? 4 : 8, steps0 = f[0].c / (4 * kv), steps1 = f[1].c / (4 * kv);
-            const int tasks = f[1].c * f[1].d / f[0].b * ((f[0].b + 63) / 64);
-            const float first = (float)((tasks + PAIR_WAVES - 1) / PAIR_WAVES * steps0), second = (float)((steps1 + p.ks - 1) / p.ks);
+            const int tasks = f[1].c * f[1].d / f[0].b * ((f[0].b + 63) / 64), rounds = (tasks + PAIR_WAVES - 1) / PAIR_WAVES;
+            const float first = (float)(rounds * steps0), second = (float)((steps1 + p.ks - 1) / p.ks);
             const float loads = (float)(tasks * steps0 * (kv + (bs_last ? kv : nt)) + mg * p.dg * steps1 * kv) / 100.f;
-            const float g = (float)p.grid / 256.f;
-            const float v[9] = {1.f, first, second, loads, loads * g, first * nt, g, second * nt, (float)(nt * mg * p.dg)};
+            const float g = (float)p.grid / 256.f, put = (float)(rounds * nt);
+            const float v[TERMS] = {1.f, first, second, loads, loads * g, first * nt, g, second * nt, (float)(nt * mg * p.dg),
+                                    put, p.dg != 3 && f[1].d == p.dg ? 0.f : put, first * g, second * g};
             const float *c = coef[p.combo < 2 ? p.combo : 2][bs_last ? 1 : 0];
             float t = 0.f;
-            for (int i = 0; i < 9; ++i) t += c[i] * v[i];
+            for (int i = 0; i < TERMS; ++i) t += c[i] * v[i];
             if (us < 0.f || t < us) us = t, *best = s;
         }
     return us;

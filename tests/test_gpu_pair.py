@@ -67,3 +67,34 @@ def test_pair_takes_any_alignment_and_leaves_the_rest():
         x = torch.randn(33, layer.in_size, device="cuda").half()
         with torch.no_grad():
             assert not taken(layer, x, layer(x))
+
+
+def test_pair_in_a_graph_goes_by_the_gpus_time():
+    """A call of its own may take the one launch to spare the host the other; a graph takes it only where it is priced below two, and
+    its replays give what float64 gives, whichever it is."""
+    from ksmm_amd import KSLinear
+
+    up = [(6, 64, 64, 1), (1, 768, 192, 2)]
+    for dt, bs_last, n, in_graph in ((torch.float32, True, 32, False), (torch.float16, False, 196, True), (torch.float16, False, 33, True)):
+        layer = KSLinear(up, algo="kernel", dtype=dt, bs_last=bs_last, device="cuda")
+        dense = layer.get_dense_product(torch.float64)
+        x = torch.randn((layer.in_size, n) if bs_last else (n, layer.in_size), device="cuda").to(dt)
+        side = torch.cuda.Stream()
+        with torch.no_grad(), torch.cuda.stream(side):
+            spare = torch.empty_like(layer(x))
+            assert taken(layer, x, spare)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.no_grad(), torch.cuda.graph(graph):
+            assert taken(layer, x, spare) == in_graph, (dt, bs_last, n)
+            y = layer(x)
+        for k in range(3):
+            x.copy_(torch.randn(x.shape, device="cuda") * (k + 1))
+            graph.replay()
+            torch.cuda.synchronize()
+            with torch.no_grad():
+                eager = layer(x)
+                bias = layer.bias.double()
+                want = dense @ x.double() + bias if bs_last else x.double() @ dense.t() + bias
+            for got in (y, eager):
+                assert ((got.double() - want).norm() / want.norm()).item() <= TOL[dt], (dt, bs_last, n, k)

@@ -1,9 +1,10 @@
-"""Two factors in one launch (ksmm_pair.hip) against the layer's dense product in float64: edges of the batch tiles of 16 and
-32, output tiles filled in part, strides of one to four and of several groups, several blocks of the second factor, and
-whole and ragged rows in either layout.
+"""Two factors in one launch (ksmm_pair.hip) against the layer's dense product in float64: the shapes that layers choose by price, and
+every shape by itself (batch tiles of 16 and 32, output tiles of 64 and 128 filled in part), strides of one to four and of several
+groups, several blocks of the second factor, and whole and ragged rows in either layout.
 
 Tolerances are those of the other chain tests: fp32 1e-5; fp16 2e-3 (each factor rounds to 2^-11); e4m3 5e-3 against the
 oracle on the dequantised operands."""
+import ctypes
 import math
 
 import pytest
@@ -43,6 +44,63 @@ def test_pair_edges(dt, bs_last):
             err = O.rel_fro_error(y.double().cpu().numpy(), z.detach().numpy())
             assert err <= TOL[dt], (patterns, n, err)
     assert ran >= 24, ran  # (half of the calls: the others are priced lower on two launches)
+
+
+# (beside those: planes and partial sums that do not fit the LDS together, which share it)
+SHARED = [(32, 64, 32, 1), (1, 64, 512, 4)]
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16, FP8])
+@pytest.mark.parametrize("bs_last", [False, True])
+def test_pair_every_shape(dt, bs_last):
+    """Each workgroup shape that the kernel takes a chain with, whatever it is priced at, through the library's own launcher: full and
+    ragged batch tiles, odd feature-major rows of which two columns are written twice, bias and GELU, nothing written behind the end."""
+    from ksmm_amd import KSLinear, _lib, quantize_fp8
+    from ksmm_amd.kernel import dtype_code
+
+    launch = _lib.load()["_ZN4ksmm8pair_runEPK16ksmm_factor_desciPKvPvliiiRKNS_9PairShapeEP12ihipStream_tPK13ksmm_epiloguePKf"]
+    vp, i64, i32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int
+    launch.restype, launch.argtypes = i32, [vp, i32, vp, vp, i64, i32, i32, i32, vp, vp, vp, vp]
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    seen, shared = set(), 0
+    for k, patterns in enumerate(CHAINS + [SHARED]):
+        ws = [(torch.rand(p, generator=torch.Generator().manual_seed(k)) * 2 - 1) / math.sqrt(p[2]) for p in patterns]
+        layer = KSLinear(patterns, weights=ws, algo="kernel", dtype=dt, bs_last=bs_last, device="cuda", act="gelu" if k % 2 else None)
+        dense, bias = layer.get_dense_product(torch.float64), layer.bias.double()
+        d = (_lib.KsmmFactorDesc * 2)()
+        for i, (f, p) in enumerate(zip(layer.factors, patterns)):
+            d[i].w, d[i].w_dtype, d[i].scale = f.data_ptr(), dtype_code(f.dtype), layer.w_scales[i]
+            d[i].a, d[i].b, d[i].c, d[i].d = p
+        ep = _lib.KsmmEpilogue(layer.bias.data_ptr(), _lib.ACT_GELU if layer.act else _lib.ACT_NONE)
+        d1, c1 = patterns[1][3], patterns[1][2]
+        dg = d1 if d1 <= 4 else 4 if d1 % 4 == 0 else 3 if d1 % 3 == 0 else 2 if d1 % 2 == 0 else 1
+        for n in (1, 2, 15, 31, 32, 33, 65):
+            x = torch.randn((layer.in_size, n) if bs_last else (n, layer.in_size), generator=gen, device="cuda")
+            x, scale = quantize_fp8(x) if dt == FP8 else (x.to(dt), None)
+            xs = scale.float().cuda().reshape(1) if dt == FP8 else None
+            x64 = x.float().double() * (float(scale) if dt == FP8 else 1.0)
+            want = dense @ x64 + bias if bs_last else x64 @ dense.t() + bias
+            if layer.act:
+                want = want * 0.5 * (1 + torch.erf(want / math.sqrt(2)))
+            for nt in (1, 2):
+                for mg in (1, 2):
+                    flat = torch.full((want.numel() + 64,), 7.0, device="cuda", dtype=layer.out_dtype)
+                    rc = launch(d, 2, x.data_ptr(), flat.data_ptr(), n, dtype_code(x.dtype), dtype_code(flat.dtype), int(bs_last),
+                                ctypes.byref((i32 * 2)(nt, mg)), torch.cuda.current_stream().cuda_stream, ctypes.byref(ep),
+                                xs.data_ptr() if dt == FP8 else None)
+                    if rc == -6:
+                        assert (bs_last and n < nt) or patterns is SHARED, (patterns, n, nt, mg)
+                        continue
+                    assert rc == 0, rc
+                    err = ((flat[:want.numel()].view(want.shape).double() - want).norm() / want.norm()).item()
+                    assert err <= TOL[dt], (patterns, n, nt, mg, err)
+                    assert bool((flat[want.numel():] == 7.0).all()), (patterns, n, nt, mg)
+                    if patterns is SHARED:
+                        shared += 1
+                    else:
+                        seen.add((nt, mg, dg))
+    assert seen == {(nt, mg, dg) for nt in (1, 2) for mg in (1, 2) for dg in (1, 2, 3, 4)}, seen
+    assert shared
 
 
 def test_pair_takes_any_alignment_and_leaves_the_rest():

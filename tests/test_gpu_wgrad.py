@@ -117,3 +117,26 @@ def test_weight_gradient_wide_bytes():
     factor = torch.zeros(a * c * d, b, device="cuda", dtype=torch.float16)
     got = Kernel.backward(rows[1][:n], rows[0][:n], factor, False, a, b, c, d, need_input=False)[1].view(a, -1)
     assert bool(got[0].isfinite().all()) and not bool(got[1].isfinite().any())
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16])
+@pytest.mark.parametrize("shape", [(2, 128, 64, 1), (2, 72, 130, 1), (1, 64, 192, 2), (2, 16, 16, 1), (1, 12, 9, 2)])
+def test_weight_gradient_rows_end_where_the_batch_does(dt, shape):
+    """Batch-size-last rows that no vector divides: what a vector reaches of the next row, and what a slab reaches of the next split, does
+    not get into the sums: infinities there would."""
+    from ksmm_amd import Kernel
+
+    a, b, c, d = shape
+    gen = torch.Generator(device="cuda").manual_seed(10)
+    for n in (9, 33, 65, 130, 1025, 3001):
+        pair = []
+        for s in (c, b):
+            t = torch.randn(a, s, d, n, generator=gen, device="cuda").to(dt)
+            (t[1] if a == 2 else t[:, :, 1]).fill_(float("inf"))  # the other block: its rows lie behind (d = 2: between) the finite ones
+            pair.append(t.view(a * s * d, n))
+        factor = torch.zeros(a * c * d, b, device="cuda", dtype=dt)
+        got = Kernel.backward(pair[1], pair[0], factor, True, a, b, c, d, need_input=False)[1].view(2, c, b)
+        xs, ys = (t.view(a, s, d, n)[0, :, 0].double() for t, s in zip(pair, (c, b)))
+        want = xs @ ys.t()
+        assert ((got[0].double() - want).norm() / want.norm()).item() <= TOL[dt], n
+        assert not bool(got[1].isfinite().any())

@@ -1,8 +1,9 @@
-"""Batch-size-first tiles that take all of d = 2, 3, 4 or 6 at once: every instance, at batches around its tiles, with blocks that
-fill its tiles of outputs and blocks that do not, against float64.
+"""Batch-size-first tiles that take all of d = 2, 3, 4 or 6 at once, at batches around their tiles, with blocks that fill their tiles of
+outputs and blocks that do not, and with bias and GELU, against float64; every instance of the library is one of those run.
 
 Tolerances: fp32 1e-5, fp16 and e4m3 operands 2e-3 (one rounding of the result to 2^-11; the operands are exact and the sums
 fp32)."""
+import ctypes
 import math
 
 import pytest
@@ -13,9 +14,12 @@ pytestmark = pytest.mark.gpu
 FP8 = torch.float8_e4m3fn
 
 
+PATTERNS = [(2, 192, 64, 3), (1, 32, 32, 3), (3, 80, 96, 3), (1, 144, 128, 3), (2, 64, 48, 6), (3, 128, 32, 6), (1, 208, 16, 6),
+            (2, 128, 64, 2), (1, 208, 96, 2), (2, 64, 64, 4), (1, 144, 32, 4), (1, 256, 32, 3), (1, 192, 32, 2)]
+
+
 @pytest.mark.parametrize("dts", [(torch.float32, torch.float32), (torch.float16, torch.float16), (FP8, FP8)])
-@pytest.mark.parametrize("pattern", [(2, 192, 64, 3), (1, 32, 32, 3), (3, 80, 96, 3), (1, 144, 128, 3), (2, 64, 48, 6), (3, 128, 32, 6), (1, 208, 16, 6),
-                                     (2, 128, 64, 2), (1, 208, 96, 2), (2, 64, 64, 4), (1, 144, 32, 4)])
+@pytest.mark.parametrize("pattern", PATTERNS)
 def test_whole_d(dts, pattern):
     from ksmm_amd import Kernel, _lib
     from ksmm_amd._lib import KsmmError
@@ -49,6 +53,29 @@ def test_whole_d(dts, pattern):
     # (fp16 has other tiles for d = 2 and 4; fp32 with d = 2 and 6 takes full tiles only)
     takes = {torch.float16: d in (3, 6), torch.float32: d == 3 or b % 64 == 0, FP8: True}[xt]
     assert seen or not takes or c % (16 if d == 6 else 32)
+
+
+def test_every_whole_d_instance_takes_one_of_the_patterns():
+    """The patterns above reach all of these tiles, each with outputs that fill its last tile and outputs that do not where it takes both."""
+    from ksmm_amd import _lib
+    from ksmm_amd._lib import KsmmError
+    from ksmm_amd.kernel import query_tile
+
+    whole = _lib.load()["_ZN4ksmm13bf_inst_wholeEi"]
+    whole.restype = ctypes.c_bool
+    every, full, part = {i for i in range(128) if whole(i)}, set(), set()
+    for dt in (torch.float32, torch.float16, FP8):
+        for pattern in PATTERNS:
+            for i in every:
+                try:
+                    t = query_tile(129, pattern, dt, dt, False, _lib.ALGO_TILE, 3 << 24 | i)
+                except KsmmError:
+                    continue
+                assert t["tile_d"] == pattern[3]
+                (part if pattern[1] % t["tile_m"] else full).add(i)
+    assert len(every) >= 16 and full | part == every, every - full - part
+    # (fp32 with d = 2 and 6 takes whole blocks of 64: their two tiles of 64 are never filled in part)
+    assert full == every and len(every - part) == 2, (every - full, every - part)
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.float16, FP8])

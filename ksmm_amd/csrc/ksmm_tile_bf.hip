@@ -427,12 +427,17 @@ __global__ __launch_bounds__(64 * WM * WN * NG, (WM * WN * NG >= 8 ? 1 : 2)) voi
     constexpr int PERIOD = PDX * PDW / (PDX % PDW == 0 ? PDW : PDW % PDX == 0 ? PDX : 1);
     static_assert(PERIOD % PDX == 0 && PERIOD % PDW == 0, "slots repeat after PERIOD slabs");
     auto slab = [&](int u, int s) {
-        const uint32_t wmk = live_mask(s + PDW < steps), xmk = live_mask(s + PDX < steps);
         const int buf = s & 1;
+        uint32_t wmk = live_mask(s + PDW < steps), xmk = 0u;
         auto request = [&](int i) { gload(i, u % PDW, (s + PDW) * TK, wmk, u % PDX, (s + PDX) * TK, xmk); };
         constexpr int AHEAD = FL ? 2 : 0;
+        // (the weights' loads leave before the input's mask and addresses are made: with both first, groups of 8 take 1 to 9
+        // percent longer, e4m3 (3,64,384,16) on 713 rows 21.6 us / 23.6)
 #pragma unroll
-        for (int i = 0; i < LOADS && !FL; ++i) request(i);
+        for (int i = 0; i < W_PER_T && !FL; ++i) request(i);
+        xmk = live_mask(s + PDX < steps);
+#pragma unroll
+        for (int i = W_PER_T; i < LOADS && !FL; ++i) request(i);
 #pragma unroll
         for (int dd = 0; dd < AHEAD; ++dd) operands(dd, buf);
         __builtin_amdgcn_sched_barrier(0);
@@ -454,10 +459,12 @@ __global__ __launch_bounds__(64 * WM * WN * NG, (WM * WN * NG >= 8 ? 1 : 2)) voi
     };
 #pragma unroll
     for (int u = 0; u < (PDX > PDW ? PDX : PDW); ++u) {
-        const uint32_t mk = live_mask(u < steps);
+        const uint32_t wmk = live_mask(u < steps);
 #pragma unroll
-        for (int i = 0; i < LOADS; ++i)
-            if (i < W_PER_T ? u < PDW : u < PDX) gload(i, u % PDW, u * TK, mk, u % PDX, u * TK, mk);
+        for (int i = 0; i < W_PER_T && u < PDW; ++i) gload(i, u % PDW, u * TK, wmk, 0, 0, 0u);
+        const uint32_t xmk = live_mask(u < steps);
+#pragma unroll
+        for (int i = W_PER_T; i < LOADS && u < PDX; ++i) gload(i, 0, 0, 0u, u % PDX, u * TK, xmk);
     }
     lstore(0, 0, 0);
     __syncthreads();

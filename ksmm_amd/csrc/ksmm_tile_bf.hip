@@ -422,30 +422,33 @@ __global__ __launch_bounds__(64 * WM * WN * NG, (WM * WN * NG >= 8 ? 1 : 2)) voi
     // Wide groups have one workgroup on a CU, and nobody multiplies while its waves issue their loads: these are spread over
     // the products, whose operands are read two blocks ahead.  us before / so: (6,192,192,64) on 25088 rows 3845 / 3738,
     // (8,128,128,64) on 12544 rows 1196 / 1168, (1,256,64,64) on 25088 457 / 448, (1,192,192,128) on 12544 652 / 642, (1,512,128,16)
-    // on 25088 256 / 251.  Groups of 8, two workgroups a CU: registers that spill.  Batch tiles that begin a slab apart take another
-    // 0 to 6 percent off (3715, 1143, 419), but a row's sum would then have the order of its tile: equal rows keep equal bits.
+    // on 25088 256 / 251.  Groups of 8, two workgroups a CU: registers that spill.  Groups of 16 with e4m3 weights, which are decoded on
+    // the way to LDS: 1.00 to 1.05 of the time over 180 problems (0.97 over 12 with d = 16), up to 1.10: not there.
+    // Batch tiles that begin a slab apart take another 0 to 6 percent off (3715, 1143, 419), but a row's sum would then have the
+    // order of its tile: equal rows keep equal bits.
+    constexpr bool SPREAD = FL && (NG == 4 || sizeof(TW) == 2);
     constexpr int PERIOD = PDX * PDW / (PDX % PDW == 0 ? PDW : PDW % PDX == 0 ? PDX : 1);
     static_assert(PERIOD % PDX == 0 && PERIOD % PDW == 0, "slots repeat after PERIOD slabs");
     auto slab = [&](int u, int s) {
         const int buf = s & 1;
         uint32_t wmk = live_mask(s + PDW < steps), xmk = 0u;
         auto request = [&](int i) { gload(i, u % PDW, (s + PDW) * TK, wmk, u % PDX, (s + PDX) * TK, xmk); };
-        constexpr int AHEAD = FL ? 2 : 0;
+        constexpr int AHEAD = SPREAD ? 2 : 0;
         // (the weights' loads leave before the input's mask and addresses are made: with both first, groups of 8 take 1 to 9
         // percent longer, e4m3 (3,64,384,16) on 713 rows 21.6 us / 23.6)
 #pragma unroll
-        for (int i = 0; i < W_PER_T && !FL; ++i) request(i);
+        for (int i = 0; i < W_PER_T && !SPREAD; ++i) request(i);
         xmk = live_mask(s + PDX < steps);
 #pragma unroll
-        for (int i = W_PER_T; i < LOADS && !FL; ++i) request(i);
+        for (int i = W_PER_T; i < LOADS && !SPREAD; ++i) request(i);
 #pragma unroll
         for (int dd = 0; dd < AHEAD; ++dd) operands(dd, buf);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int dd = 0; dd < DD; ++dd) {
-            if (!FL) operands(dd, buf);
+            if (!SPREAD) operands(dd, buf);
             products(dd);
-            if (FL) {
+            if (SPREAD) {
                 if (dd + AHEAD < DD) operands(dd + AHEAD, buf);
 #pragma unroll
                 for (int i = dd * LOADS / DD; i < (dd + 1) * LOADS / DD; ++i) request(i);

@@ -730,12 +730,13 @@ bool decode_pays(const ksmm_factor_desc *f, int n, int64_t batch, int x_dtype, i
 }
 
 // Whether two factors run in one launch (ksmm_pair.hip): where that is priced below the other routes by PAIR_AHEAD.  Of 16270 measured
-// chains (see pair_us) it is so in 5590, which take 0.73 to 0.84 of the time of two launches by type and layout; 2.1 percent
-// of them are more than 3 percent slower.
+// chains (see pair_us) it is so in 5790, which take 0.73 to 0.84 of the time of two launches by type and layout; 2.2 percent
+// of them are more than 3 percent slower (9 percent of feature-major fp32 and e4m3 chains, whose two launches are priced too high by most,
+// if those need to be ahead by 0.7 only).
 // A call that goes to the GPU as it is made costs the host 6.1 us with one launch and 9.7 with two, for which the GPU waits: there, up
 // to a time of HOST_US it may be priced up to a microsecond later.  (6,64,64,1)+(1,768,192,2) fp32 on 32 columns 8.9 us on the GPU
 // for 8.0, but 8.8 a call for 9.6.  In a graph that waits for nobody, the GPU's time alone decides.
-constexpr float PAIR_AHEAD = 0.5f, PAIR_AHEAD_LAST = 1.f, HOST_US = 9.5f;
+constexpr float PAIR_AHEAD = 0.5f, PAIR_AHEAD_LAST = 1.f /* fp32 and e4m3 */, HOST_US = 9.5f;
 struct PairChoice {
     PairShape shape;
     bool on_gpu, on_call;  // in a graph, and as a call of its own
@@ -749,7 +750,7 @@ PairChoice pair_choice(const ksmm_factor_desc *f, int n, int64_t batch, int x_dt
     float best = chain_best_us(f, n, batch, x_dtype, y_dtype, bs_last, &copies);
     ksmm_factor_desc decoded[2];
     if (decode_pays(f, n, batch, x_dtype, y_dtype, bs_last, decoded)) best = fminf(best, chain_best_us(decoded, n, batch, x_dtype, y_dtype, bs_last, &copies) + 4.f);
-    us += bs_last ? PAIR_AHEAD_LAST : PAIR_AHEAD;
+    us += bs_last && f[0].w_dtype != KSMM_F16 ? PAIR_AHEAD_LAST : PAIR_AHEAD;
     c.on_gpu = us < best;
     c.on_call = us < best + fminf(fmaxf(HOST_US - best, 0.f), 1.f);
     return c;

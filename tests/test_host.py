@@ -286,18 +286,18 @@ def test_chains_asked_in_turn_are_remembered(lib):
         for i, p in enumerate([(16, 64, 256, 1), (1, 256, 256, 4)]):
             d[i].w, d[i].w_dtype, d[i].scale = 1 << 16, _lib.KSMM_FP8_E4M3, 1.0
             d[i].a, d[i].b, d[i].c, d[i].d = p
-        return d, 2, 1 << 36, 2 << 36, n, _lib.KSMM_FP8_E4M3, _lib.KSMM_F16, 0, None, None
+        return d, 2, 1 << 36, 2 << 36, None, 0, n, _lib.KSMM_FP8_E4M3, _lib.KSMM_F16, 0, 1, None, None
 
-    asked = [question(n) for n in range(512, 1024)]  # (two launches take this chain: nothing is launched)
-    assert all(lib.ksmm_chain_forward_fused(*q) == -6 for q in asked)
+    asked = [question(n) for n in range(512, 1024)]  # (without a workspace they are refused: nothing is launched)
+    assert all(lib.ksmm_chain_forward_ep(*q) == -9 for q in asked)
 
     def turns(a, b, tries):
         best = 1.0
         for _ in range(tries):
             t = time.perf_counter()
             for _ in range(8):
-                lib.ksmm_chain_forward_fused(*a)
-                lib.ksmm_chain_forward_fused(*b)
+                lib.ksmm_chain_forward_ep(*a)
+                lib.ksmm_chain_forward_ep(*b)
             best = min(best, time.perf_counter() - t)
         return best
 

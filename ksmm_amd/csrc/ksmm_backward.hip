@@ -198,14 +198,14 @@ template <> struct wg_vec<half_t> {
     }
 };
 
-// Batch-size-last blocks of at most 16 x 16.  One wavefront owns one block's gradient and a range of batch columns.  Lane
-// (r = lane % 16, q = lane / 16) loads N consecutive batch elements of operand row r at column n + N*q; MFMA e
+// Batch-size-last blocks of at most 16 MT x 16 MT.  One wavefront owns one block's gradient and a range of batch columns.  Lane
+// (r = lane % 16, q = lane / 16) loads N consecutive batch elements of operand rows r + 16 i at column n + N*q; MFMA e
 // multiplies element group e of every lane, i.e. its k-set is {n + N*q + e ...}: the same set for
-// both operands, and the order of a sum's terms is free.  Loads are non-temporal: every operand row is read by one wave.
+// both operands, and the order of a sum's terms is free.  NTL: non-temporal loads, every operand row is read by one wave.
 // ANY: rows of any length and alignment (a batch that the vector does not divide): vectors at element
 // alignment, and the last one of a row pulled back to end with it, its first elements cleared where
 // the vector before has them.
-template <typename T, bool ANY>
+template <typename T, int MT, bool NTL, bool ANY>
 __global__ __launch_bounds__(256) void ks_wgrad_bl_kernel(const T *__restrict__ dy, const T *__restrict__ x,
                                                           float *__restrict__ acc_out, int batch, int a, int b,
                                                           int c, int d, int splits, int cols_per_split, int64_t slice)
@@ -222,22 +222,33 @@ __global__ __launch_bounds__(256) void ks_wgrad_bl_kernel(const T *__restrict__ 
     if (n_begin >= n_end) return;
     const size_t row_stride = (size_t)d * batch;
     // rows behind b (or c) are clamped to the last valid one and dropped at the end
-    const T *const ap = dy + ((size_t)a_i * b * d + d_i) * batch + (size_t)min(r, b - 1) * row_stride;
-    const T *const bp = x + ((size_t)a_i * c * d + d_i) * batch + (size_t)min(r, c - 1) * row_stride;
-    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+    const T *ap[MT], *bp[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        ap[i] = dy + ((size_t)a_i * b * d + d_i) * batch + (size_t)min(16 * i + r, b - 1) * row_stride;
+        bp[i] = x + ((size_t)a_i * c * d + d_i) * batch + (size_t)min(16 * i + r, c - 1) * row_stride;
+    }
+    float4_t acc[MT][MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < MT; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
     typedef typename V::type vec_t;
     // U sub-steps per iteration, all their loads issued before the first MFMA: a row is then read
     // in runs of U * 64 bytes, and the loads of the whole iteration are in flight together
     constexpr int U = 4;
     for (int n = n_begin; n < n_end; n += U * STEP) {
-        vec_t av[U], bv[U];
+        vec_t av[U][MT], bv[U][MT];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int col = n + u * STEP + V::N * q;
             const bool live = col < n_end;          // whole vectors: batch and the split are multiples of N
             const int lcol = ANY ? min(col, batch - V::N) : live ? col : n_begin;  // (a valid address; the value is zeroed)
-            av[u] = wg_load<!ANY, ANY, vec_t>(ap + lcol);
-            bv[u] = wg_load<!ANY, ANY, vec_t>(bp + lcol);
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                av[u][i] = wg_load<NTL, ANY, vec_t>(ap[i] + lcol);
+                bv[u][i] = wg_load<NTL, ANY, vec_t>(bp[i] + lcol);
+            }
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -246,20 +257,34 @@ __global__ __launch_bounds__(256) void ks_wgrad_bl_kernel(const T *__restrict__ 
                 // elements in front of `drop` are not this vector's (n_end is the batch where ANY gets here with col < n_end)
                 const int drop = ANY && col < n_end ? col - min(col, batch - V::N) : V::N;
 #pragma unroll
-                for (int e = 0; e < V::N; ++e) {
-                    av[u][e] = e < drop ? (T)0 : av[u][e];
-                    bv[u][e] = e < drop ? (T)0 : bv[u][e];
-                }
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int e = 0; e < V::N; ++e) {
+                        av[u][i][e] = e < drop ? (T)0 : av[u][i][e];
+                        bv[u][i][e] = e < drop ? (T)0 : bv[u][i][e];
+                    }
             }
 #pragma unroll
-            for (int e = 0; e < V::MFMAS; ++e) acc = V::mfma(e, av[u], bv[u], acc);
+            for (int e = 0; e < V::MFMAS; ++e)
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < MT; ++j) acc[i][j] = V::mfma(e, av[u][i], bv[u][j], acc[i][j]);
         }
     }
-    // D: lane holds column (c index) r and rows (b index) 4*q .. 4*q + 3
-    if (r >= c) return;
+    // D: lane holds column (c index) r and rows (b index) 4*q .. 4*q + 3 of each 16 x 16 tile
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-        if (4 * q + e < b) acc_out[(size_t)split * slice + ((size_t)g * c + r) * b + 4 * q + e] = acc[e];
+    for (int j = 0; j < MT; ++j) {
+        const int k = 16 * j + r;
+        if (k >= c) continue;
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int m = 16 * i + 4 * q + e;
+                if (m < b) acc_out[(size_t)split * slice + ((size_t)g * c + k) * b + m] = acc[i][j][e];
+            }
+    }
 }
 
 // Any layout, any batch: 16 x 16 threads compute a 16 x 16 tile of one block's gradient over a
@@ -465,10 +490,16 @@ WgradSplit wgrad_split(int64_t batch, int a, int b, int c, int d, int dtype, int
     return WgradSplit{(batch + cols - 1) / cols, cols};
 }
 
-// Blocks of 16 x 16 leave fifteen sixteenths of the GEMM tile empty.  Beyond that it is ahead of the wave-per-tile kernel with
-// tiles of 32, 48 and 64 as well (us with those / on it, 25088 columns: (1,32,32,32) fp32 75.4 / 74.6, fp16 37.4 / 26.3, (1,48,48,16)
-// 63.0 / 48.7 and 32.9 / 22.3; 9000 columns: (6,16,32,8) fp16 20.0 / 17.3).
-bool wgrad_gemm_ok(int b, int c) { return b > 16 || c > 16; }
+// Blocks of 16 x 16 leave fifteen sixteenths of the GEMM tile empty, and in fp32, which waits for its matrix cores, those of 32 x 32 cost
+// three quarters of it: on 8670 drawn problems of 17 .. 32 rows the wave's kernel takes 0.85 of the tile's time, from 16 MB of
+// operands on 0.6 to 0.7 (1.00 below 4 MB): (16,32,32,4) on 10538 columns 61 us / 44, (6,20,16,32) on 12579 202 / 93.  In fp16 it takes
+// 1.01.  Beyond, the tile is ahead of waves with tiles of 32, 48 and 64 (us with those / on it): fp16 (1,32,32,32) at 25088 columns
+// 37.4 / 26.3, (1,48,48,16) fp32 63.0 / 48.7 and fp16 32.9 / 22.3.
+bool wgrad_gemm_ok(int b, int c, int dtype)
+{
+    const int edge = dtype == KSMM_F32 ? 32 : 16;
+    return b > edge || c > edge;
+}
 
 // An edge of 128 where that pads the block by no more than a tenth beyond what 64 does
 int wgrad_gemm_edge(int n)
@@ -524,7 +555,11 @@ int launch_wgrad_bl(const void *dy, const void *x, float *acc, int64_t batch, in
     const int64_t waves = (int64_t)a * d * splits, blocks = (waves + 3) / 4;
     if (blocks > 0x7fffffffLL) return KSMM_ERR_TOO_LARGE;
     *splits_used = (int)splits;
-    const auto fn = wgrad_aligned(dy, x, batch, elem<T>::dtype) ? &ks_wgrad_bl_kernel<T, false> : &ks_wgrad_bl_kernel<T, true>;
+    const bool whole = wgrad_aligned(dy, x, batch, elem<T>::dtype);
+    auto fn = whole ? &ks_wgrad_bl_kernel<T, 1, true, false> : &ks_wgrad_bl_kernel<T, 1, false, true>;
+    if constexpr (sizeof(T) == 4)
+        // (plain loads: 0.93 of the time of non-temporal ones)
+        if (b > 16 || c > 16) fn = whole ? &ks_wgrad_bl_kernel<T, 2, false, false> : &ks_wgrad_bl_kernel<T, 2, false, true>;
     hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(256), 0, s, (const T *)dy, (const T *)x, acc, (int)batch, a, b, c, d,
                        (int)splits, (int)cols, (int64_t)a * b * c * d);
     return hipGetLastError() == hipSuccess ? KSMM_OK : KSMM_ERR_LAUNCH;
@@ -582,7 +617,7 @@ template <typename T>
 int wgrad_last(const void *dy, const void *x, float *acc, int64_t batch, int a, int b, int c, int d, int bs_last, hipStream_t s, int *splits)
 {
     if (!wgrad_mfma_ok(batch, elem<T>::dtype, bs_last)) return launch_wgrad_tiled<T>(dy, x, acc, batch, a, b, c, d, bs_last, s, splits);
-    return wgrad_gemm_ok(b, c) ? launch_wgrad_gemm<T>(dy, x, acc, batch, a, b, c, d, s, splits)
+    return wgrad_gemm_ok(b, c, elem<T>::dtype) ? launch_wgrad_gemm<T>(dy, x, acc, batch, a, b, c, d, s, splits)
                                : launch_wgrad_bl<T>(dy, x, acc, batch, a, b, c, d, s, splits);
 }
 
@@ -630,7 +665,7 @@ int64_t wgrad_partial_floats(int64_t batch, int a, int b, int c, int d, int dtyp
     const int64_t n = (int64_t)a * b * c * d;
     int64_t cols, most = 1;
     if (wgrad_mfma_ok(batch, dtype, bs_last))
-        most = (wgrad_gemm_ok(b, c) ? wgrad_gemm_split : wgrad_bl_split)(batch, a, b, c, d, dtype).splits;
+        most = (wgrad_gemm_ok(b, c, dtype) ? wgrad_gemm_split : wgrad_bl_split)(batch, a, b, c, d, dtype).splits;
     else
         wgrad_tiled_splits(batch, (int64_t)a * d * ((b + 15) / 16) * ((c + 15) / 16), &most, &cols);
     return most * n;

@@ -120,7 +120,8 @@ def test_weight_gradient_wide_bytes():
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.float16])
-@pytest.mark.parametrize("shape", [(2, 128, 64, 1), (2, 72, 130, 1), (1, 64, 192, 2), (2, 16, 16, 1), (1, 12, 9, 2)])
+@pytest.mark.parametrize("shape", [(2, 128, 64, 1), (2, 72, 130, 1), (1, 64, 192, 2), (2, 16, 16, 1), (1, 12, 9, 2), (2, 32, 32, 1), (1, 17, 30, 2),
+                                   (2, 33, 32, 1)])
 def test_weight_gradient_rows_end_where_the_batch_does(dt, shape):
     """Batch-size-last rows that no vector divides: what a vector reaches of the next row, and what a slab reaches of the next split, does
     not get into the sums: infinities there would."""

@@ -155,7 +155,7 @@ float predicted_us(const Problem &p, const ksmm_tile &t)
 
 Choice cheapest_instance(const Problem &p, bool any_alignment)
 {
-    Choice best{KSMM_ALGO_AUTO, -1, -1.f};
+    Choice best{KSMM_ALGO_AUTO, -1, -1.f}, split = best;
     const int combo = combo_of(p.x_dtype, p.w_dtype, p.y_dtype);
     if (combo < 0) return best;
     const bool ragged = ragged_rows(p);
@@ -168,6 +168,7 @@ Choice cheapest_instance(const Problem &p, bool any_alignment)
         if (!r || (t.threads & 63) || t.tile_d < 1) return;
         const float us = price(*r, p, t);
         if (best.us < 0.f || us < best.us) best = Choice{t.algo, t.variant, us};
+        if (r->family == FAM_SPLIT && (split.us < 0.f || us < split.us)) split = Choice{t.algo, t.variant, us};
     };
     const CostIndex &ix = cost_index();
     if (!any_alignment) {
@@ -182,6 +183,12 @@ Choice cheapest_instance(const Problem &p, bool any_alignment)
         if (!ix.tile[FAM_SPLIT][combo][p.bs_last][i]) continue;
         for (int waves = 1; waves <= 16; waves *= 2) offer(KSMM_ALGO_TILE, (FAM_SPLIT << 24) | (waves << 8) | i);
     }
+    // 16-bit and e4m3 rows that fill the split-K kernel's 16 in part are priced too high there: what is beyond 5 us shrinks with
+    // them, to a quarter and less.  A whole-d tile has to be ahead of that: (16,256,256,3) e4m3 on one row, priced 9.0 and 8.0, takes
+    // 5.0 on split-K and 8.5 on the tile.
+    if (!p.bs_last && p.x_dtype != KSMM_F32 && p.batch < 16 && split.us > 5.f && best.algo == KSMM_ALGO_TILE && best.variant >> 24 == 3 &&
+        bf_inst_whole(best.variant & 0xff) && 5.f + (split.us - 5.f) * (0.25f + 0.75f / 16.f * p.batch) < best.us)
+        best = split;
     return best;
 }
 

@@ -311,6 +311,22 @@ def test_chains_asked_in_turn_are_remembered(lib):
         assert a <= 1.2 * b, (a, b)
 
 
+def test_few_rows_on_heavy_blocks_stay_on_split_k():
+    """One to eight rows of large 16-bit and e4m3 blocks with d = 3, where a whole-d tile multiplies mostly nothing; from a batch tile on
+    it takes them."""
+    from ksmm_amd import _lib
+    from ksmm_amd.kernel import query_tile
+
+    for dt in (torch.float16, torch.float8_e4m3fn):
+        for pattern in ((16, 256, 256, 3), (12, 384, 384, 3)):
+            for n in (1, 4, 8):
+                t = query_tile(n, pattern, dt, None, False)
+                split = (t["variant"] - 16 if t["algo"] == _lib.ALGO_GENERIC else t["variant"]) >> 24 == 5
+                assert split, (dt, pattern, n, t)
+            t = query_tile(64, pattern, dt, None, False)
+            assert t["algo"] == _lib.ALGO_TILE and t["variant"] >> 24 == 3 and t["tile_d"] == 3, (dt, pattern, t)
+
+
 def test_choice_does_not_end_with_the_measured_batches():
     """One row more than the largest batch that the choice was first measured at takes the same kernel."""
     from ksmm_amd.kernel import query_tile

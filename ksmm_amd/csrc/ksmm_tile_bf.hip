@@ -806,7 +806,6 @@ __global__ __launch_bounds__(64 * WM * WN * NG, (WM * WN * NG >= 8 ? 1 : 2)) voi
         }
 }
 
-// LDS of the whole-d form: one buffer of planes, or the staged result tile if that is larger
 // Whole d of a small number, 3 and 6 among them, where no 16-byte vector is a run of all d_i: a thread loads 8 k (fp32: 4)
 // of all DD blocks of a row, DD vectors in a row, and sorts them by d_i on the way to LDS (16-bit types: one v_perm per word;
 // fp32: a renaming).  A vector of a plane is one chunk of a row, so LDS has no padding and its chunks are swizzled as in the GEMM
@@ -1040,6 +1039,7 @@ __global__ __launch_bounds__(64 * WM * WN, OCC) void ks_whole_bf_kernel(const TX
     }
 }
 
+// LDS of the pipelined forms: two buffers of planes, or the staged result tile if that is larger
 constexpr int bf8l_lds(int ng, int tk, int tm, int tn)
 {
     const int ldw = tm == 32 ? 32 : pads<half_t>::outer(tm);
